@@ -95,6 +95,15 @@ hipError_t workspace(hipStream_t s, size_t need, void** out) {
     return hipSuccess;
 }
 
+// The stream's workspace for a faster route that the call can do without: null where it cannot grow now (the
+// stream is capturing, or the allocation failed), and the call then takes the route that needs less.
+void* workspace_or_null(hipStream_t s, size_t need) {
+    void* p = nullptr;
+    if (workspace(s, need, &p) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 int workspace_fail(const char* what, hipError_t e, size_t need) {
     if (e == hipErrorStreamCaptureUnsupported)
         return fail(MTH_EUNSUPPORTED,
@@ -329,6 +338,12 @@ int mth_i2s_gemv(const uint8_t* packed, float w_scale, const int8_t* act, const 
     REQUIRE(M > 0 && K > 0 && batch > 0 && M < kMaxDim && K < (1ll << 24) && batch <= 65536,
             "mth_i2s_gemv: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
     REQUIRE(K % 4 == 0, "mth_i2s_gemv: K=%lld must be a multiple of 4", (long long)K);
+    if (mth::i2s_rows_supported(packed, act, false, M, K, batch)) {
+        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch)))
+            return check_launch(mth::launch_i2s_rows(packed, w_scale, nullptr, act, act_scale, y, M, K, batch, ws,
+                                                     S(stream)),
+                                "mth_i2s_gemv");
+    }
     const bool aligned = (((uintptr_t)packed | (uintptr_t)act) & 15u) == 0;
     if (aligned && mth::i2s_bt_supported(M, K, batch)) {
         void* partial = nullptr;
@@ -349,6 +364,12 @@ int mth_i2s_gemv_f32(const uint8_t* packed, float w_scale, const float* x, float
     REQUIRE(M > 0 && K > 0 && batch > 0 && M < kMaxDim && K < (1ll << 24) && batch <= 65536,
             "mth_i2s_gemv_f32: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
     REQUIRE(K % 4 == 0, "mth_i2s_gemv_f32: K=%lld must be a multiple of 4", (long long)K);
+    if (mth::i2s_rows_supported(packed, x, true, M, K, batch)) {
+        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch)))
+            return check_launch(mth::launch_i2s_rows(packed, w_scale, x, nullptr, nullptr, y, M, K, batch, ws,
+                                                     S(stream)),
+                                "mth_i2s_gemv_f32");
+    }
     return check_launch(mth::launch_i2s_gemv(packed, w_scale, x, nullptr, nullptr, y, M, K, batch, S(stream)),
                         "mth_i2s_gemv_f32");
 }

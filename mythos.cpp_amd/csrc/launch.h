@@ -123,6 +123,14 @@ hipError_t launch_i2s_gemv_bt_f32act_y(const uint8_t* packed, float w_scale, con
 hipError_t launch_i2s_gemv_bt_slices(const uint8_t* packed, float w_scale, const int8_t* act, const float* act_scale,
                                     float* y, int64_t M, int64_t K, int64_t batch, float* partial, Slices* out,
                                     hipStream_t s);
+// Token rows of any K % 4 == 0, FP32 rows (x: quantised per token) or int8 rows (act, act_scale): the
+// rows as padded int8 in ws (i2s_rows_workspace_bytes), then the batched kernel (up to 16 tokens) or the int8
+// MFMA GEMM; the same bits as launch_i2s_gemv.
+bool i2s_rows_supported(const uint8_t* packed, const void* x, bool f32, int64_t M, int64_t K, int64_t batch);
+size_t i2s_rows_workspace_bytes(int64_t M, int64_t K, int64_t batch);
+hipError_t launch_i2s_rows(const uint8_t* packed, float w_scale, const float* x, const int8_t* act,
+                           const float* act_scale, float* y, int64_t M, int64_t K, int64_t batch, void* ws,
+                           hipStream_t s);
 // Batch 1, int8 activations, with the residual epilogue (ResidOut,
 // common.h) in place of y; *nparts: partials per token.
 bool i2s_resid_supported(const uint8_t* packed, const int8_t* act, int64_t M, int64_t K);

@@ -950,6 +950,74 @@ __device__ __forceinline__ uint32_t byte_t4x4(uint32_t a, uint32_t b, uint32_t c
            (((d >> (8 * s)) & 0xffu) << 24);
 }
 
+// Codes of rows that are not whole aligned 16-byte pieces (K % 64 != 0, or K % 256 != 0 where a step of 256
+// columns runs past the row): 8 bytes at byte pos of a matrix of `end` >= 8 bytes.  Bytes past the row are the
+// next row's (or, past the matrix, zeros): the activations there are zeros (the padded rows of
+// i2s_quant_rows_k / i2s_pad_rows_k), so their codes add nothing.
+__device__ __forceinline__ uint2 ld_codes8(const uint8_t* w, int64_t pos, int64_t end) {
+    const int64_t p = min(pos, end - 8);
+    uint64_t v;
+    __builtin_memcpy(&v, w + p, 8);
+    const int64_t past = pos - p;  // bytes of the piece that lie before pos
+    v = past >= 8 ? 0ull : v >> (8 * past);
+    return make_uint2((uint32_t)v, (uint32_t)(v >> 32));
+}
+
+// quantize_per_token of FP32 rows (src/int8_quant.cpp:8-31) into rows of Kp >= K bytes, zeros past K: the
+// operand of the batched kernels and the GEMM, which then need no bounds of their own.  One workgroup of 16
+// waves per row, the row read once (16384 columns in registers; longer rows read the rest twice).  VEC: 16-byte
+// aligned rows (x aligned, K % 4 == 0).  Latency-bound (one round trip, two barriers): 16 x 11008 takes 4.0 us
+// where quantising inside the GEMV, token after token in every workgroup, took 8 us per token (4096 x 11008).
+constexpr int kQrT = 1024, kQrN = 4;
+template <bool VEC>
+__global__ __launch_bounds__(kQrT) void i2s_quant_rows_k(const float* __restrict__ x, int K, int Kp,
+                                                         int8_t* __restrict__ q, float* __restrict__ inv) {
+    __shared__ float red[kQrT / 64];
+    const int tid = threadIdx.x;
+    const float* xr = x + (int64_t)blockIdx.x * K;
+    auto load = [&](int i) {  // columns 4i .. 4i + 3 (K % 4 == 0)
+        if (4 * i >= K) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if constexpr (VEC) return ldf4(xr + 4 * i);
+        else return make_float4(xr[4 * i], xr[4 * i + 1], xr[4 * i + 2], xr[4 * i + 3]);
+    };
+    auto amax4 = [](const float4& v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); };
+    float4 v[kQrN];
+#pragma unroll
+    for (int j = 0; j < kQrN; ++j) v[j] = load(tid + j * kQrT);
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kQrN; ++j) m = fmaxf(m, amax4(v[j]));
+    for (int i = tid + kQrN * kQrT; 4 * i < K; i += kQrT) m = fmaxf(m, amax4(load(i)));
+    m = wave_max(m);
+    if ((tid & 63) == 0) red[tid >> 6] = m;
+    __syncthreads();
+    m = red[0];
+#pragma unroll
+    for (int w = 1; w < kQrT / 64; ++w) m = fmaxf(m, red[w]);
+    if (m < 1e-10f) m = 1e-10f;
+    const float sc = __fdiv_rn(127.0f, m);
+    uint32_t* dst = (uint32_t*)(q + (int64_t)blockIdx.x * Kp);
+    auto store = [&](int i, const float4& f) {
+        const uint32_t b0 = (uint32_t)quant_i8(f.x, sc) & 0xffu, b1 = (uint32_t)quant_i8(f.y, sc) & 0xffu;
+        const uint32_t b2 = (uint32_t)quant_i8(f.z, sc) & 0xffu, b3 = (uint32_t)quant_i8(f.w, sc) & 0xffu;
+        if (4 * i < Kp) dst[i] = 4 * i < K ? b0 | (b1 << 8) | (b2 << 16) | (b3 << 24) : 0u;
+    };
+#pragma unroll
+    for (int j = 0; j < kQrN; ++j) store(tid + j * kQrT, v[j]);
+    for (int i = tid + kQrN * kQrT; 4 * i < Kp; i += kQrT) store(i, load(i));
+    if (tid == 0) inv[blockIdx.x] = __fdiv_rn(m, 127.0f);
+}
+
+// int8 rows of K bytes (K % 4 == 0, any alignment) into rows of Kp bytes, zeros past K.
+__global__ __launch_bounds__(kWG) void i2s_pad_rows_k(const int8_t* __restrict__ a, int K, int Kp,
+                                                      int8_t* __restrict__ q) {
+    const int i = blockIdx.x * kWG + threadIdx.x;
+    if (4 * i >= Kp) return;
+    uint32_t v = 0;
+    if (4 * i < K) __builtin_memcpy(&v, a + (int64_t)blockIdx.y * K + 4 * i, 4);
+    *(uint32_t*)(q + (int64_t)blockIdx.y * Kp + 4 * i) = v;
+}
+
 // FP32 activations (the decode step of a batch, FA): act[t * lda + k] =
 // silu(g * ni) * (u * ni) with amax[t][nmx] the maxima of |act| over blocks
 // of it (oil4_gemv_bt_swiglu); the kernel quantises per token as
@@ -972,8 +1040,8 @@ constexpr int kIbFaMx = 4, kIbFaChunks = 4;  // FA: block maxima per thread, chu
 // and quantised with the token's scale sc while staging; in the first round
 // sc is derived from the block maxima mxv (loaded at the kernel's start)
 // after the weights are issued.
-template <int NC, bool FA = false>
-__device__ __forceinline__ void ib_round(const uint8_t* wrow, const int8_t* arow, bool sv, bool stager, int c0,
+template <int NC, bool FA = false, bool TAIL = false>
+__device__ __forceinline__ void ib_round(const uint8_t* wrow, int64_t wend, const int8_t* arow, bool sv, bool stager, int c0,
                                          bool first, uint32_t (*qs)[kIbTok * kIbTokStride], int st, int sg, int r,
                                          int g, int& asum, i32x4& acc, const float* arowf = nullptr,
                                          float* sc = nullptr, const float* mxv = nullptr,
@@ -995,7 +1063,15 @@ __device__ __forceinline__ void ib_round(const uint8_t* wrow, const int8_t* arow
     __builtin_amdgcn_s_barrier();  // every wave's activations are issued before any weights
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) wv[c] = ld_stream(wrow + (int64_t)(c0 + c) * 64);
+    for (int c = 0; c < NC; ++c) {
+        const int64_t o = (int64_t)(c0 + c) * 64;
+        if constexpr (TAIL) {
+            const uint2 lo = ld_codes8(wrow, o, wend), hi = ld_codes8(wrow, o + 8, wend);
+            wv[c] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        } else {
+            wv[c] = ld_stream(wrow + o);
+        }
+    }
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (FA) {
         if (first && stager) {  // the token's scale: 16 threads (sg) per token
@@ -1057,11 +1133,13 @@ __device__ __forceinline__ void ib_round(const uint8_t* wrow, const int8_t* arow
     }
 }
 
-template <int MAXC, int WV, bool FA = false>
+// lda: bytes per activation row (K, or the padded row's).  TAIL: K % 256 != 0 (K % 4 == 0, any alignment of the
+// codes): activation rows padded with zeros to whole chunks, codes loaded by ld_codes8.
+template <int MAXC, int WV, bool FA = false, bool TAIL = false>
 __global__ __launch_bounds__(WV * 64) void i2s_gemv_bt(const uint8_t* packed, float w_scale, const int8_t* act,
-                                                       const float* __restrict__ act_scale, float* __restrict__ y,
-                                                       float* __restrict__ partial, int M, int K, int batch,
-                                                       I2sF32Act fa = I2sF32Act{}) {
+                                                       int64_t lda, const float* __restrict__ act_scale,
+                                                       float* __restrict__ y, float* __restrict__ partial, int M, int K,
+                                                       int batch, I2sF32Act fa = I2sF32Act{}) {
     static_assert(MAXC >= 1 && MAXC <= 8, "ib_round is dispatched for 1..8 chunks");
     // [chunk][token][16-col group][4 dwords], token stride kIbTokStride (64 + 4 dwords: the 16 tokens of an
     // MFMA operand read land on distinct banks)
@@ -1071,15 +1149,16 @@ __global__ __launch_bounds__(WV * 64) void i2s_gemv_bt(const uint8_t* packed, fl
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, g = lane >> 4;
     const int m0 = blockIdx.x * (WV * 16) + wave * 16;
-    const int nsc = K / 256, S = gridDim.y;
+    const int nsc = TAIL ? (K + 255) / 256 : K / 256, S = gridDim.y;
     const int sc0 = (int)((int64_t)blockIdx.y * nsc / S), sc1 = (int)((int64_t)(blockIdx.y + 1) * nsc / S);
     const int bpr = K / 4;
     const uint8_t* wrow = packed + (int64_t)min(m0 + r, M - 1) * bpr + 16 * g;  // clamped rows
+    const int64_t wend = (int64_t)M * bpr - (wrow - packed);                    // bytes from wrow to the end
     // staging by the first 4 waves: thread = token st, 16-column group sg
     const int st = (tid >> 4) & 15, sg = tid & 15;
     const bool stager = __builtin_amdgcn_readfirstlane(wave) < 4;
     const bool sv = st < batch;
-    const int8_t* arow = act + (int64_t)(sv ? st : 0) * K + 16 * sg;
+    const int8_t* arow = act + (int64_t)(sv ? st : 0) * lda + 16 * sg;
     // FA: the token's block maxima first (16 threads per token, clamped)
     const float* arowf = FA ? fa.act + (int64_t)(sv ? st : 0) * fa.lda + 16 * sg : nullptr;
     float mxv[kIbFaMx], sc = 0.0f;
@@ -1094,14 +1173,14 @@ __global__ __launch_bounds__(WV * 64) void i2s_gemv_bt(const uint8_t* packed, fl
         const int nc = min(MAXC, sc1 - c0);
         const bool first = c0 == sc0;
         switch (nc) {
-            case 1: ib_round<1, FA>(wrow, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 2: ib_round<2, FA>(wrow, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 3: ib_round<3, FA>(wrow, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 4: ib_round<4, FA>(wrow, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 5: ib_round<5 <= MAXC ? 5 : 1, FA>(wrow, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 6: ib_round<6 <= MAXC ? 6 : 1, FA>(wrow, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 7: ib_round<7 <= MAXC ? 7 : 1, FA>(wrow, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            default: ib_round<MAXC, FA>(wrow, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 1: ib_round<1, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 2: ib_round<2, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 3: ib_round<3, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 4: ib_round<4, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 5: ib_round<5 <= MAXC ? 5 : 1, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 6: ib_round<6 <= MAXC ? 6 : 1, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 7: ib_round<7 <= MAXC ? 7 : 1, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            default: ib_round<MAXC, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
         }
     }
     if (stager) asum_p[st][sg] = asum;
@@ -1126,12 +1205,11 @@ __global__ __launch_bounds__(WV * 64) void i2s_gemv_bt(const uint8_t* packed, fl
 
 __global__ __launch_bounds__(kWG) void i2s_bt_reduce(const float* __restrict__ partial, float w_scale,
                                                      const float* __restrict__ act_scale, float* __restrict__ y, int M,
-                                                     int batch, int nslice) {
+                                                     int batch, int nslice, int64_t zs) {
     const int64_t i = (int64_t)blockIdx.x * kWG + threadIdx.x;
     if (i >= (int64_t)batch * M) return;
-    const int64_t t = i / M, m = i - t * M;
-    const float* p = partial + t * M + m;
-    const int64_t zs = (int64_t)kIbTok * M;
+    const int64_t t = i / M;
+    const float* p = partial + i;
     float v[kMaxSlices];  // every load before the first add (at most kMaxSlices slices)
 #pragma unroll
     for (int z = 0; z < kMaxSlices; ++z) v[z] = z < nslice ? p[z * zs] : 0.0f;
@@ -1146,7 +1224,7 @@ __global__ __launch_bounds__(kWG) void i2s_bt_reduce(const float* __restrict__ p
 // least 4 chunks of 256 columns per slice, at most kIbChunks where 16 slices
 // allow.
 inline int ib_slices(int64_t M, int64_t K) {
-    const int64_t groups = (M + kIbRows - 1) / kIbRows, nsc = K / 256;
+    const int64_t groups = (M + kIbRows - 1) / kIbRows, nsc = (K + 255) / 256;
     int64_t S = std::min<int64_t>((256 + groups - 1) / groups, std::max<int64_t>(1, nsc / 4));
     S = std::max<int64_t>(S, (nsc + kIbChunks - 1) / kIbChunks);
     return (int)std::max<int64_t>(1, std::min<int64_t>({S, 16, nsc}));
@@ -1202,11 +1280,15 @@ __device__ __forceinline__ uint4 group_t4x4(const uint4& v) {
 // 8 waves, two per SIMD (one SIMD's pair interleaves its decode, LDS reads and MFMAs: 41.2 -> 39.7 us against
 // 4 waves of all four chunks at 4096 x 512 x 11008): wave (wr, wk) holds rows 32 wr .. 32 wr + 31 x all 64
 // tokens for chunks 2 wk, 2 wk + 1 of every step; the two K halves' sums meet through LDS at the end.
+// lda: bytes per activation row.  TAIL: K % 256 != 0 (K % 4 == 0, codes of any alignment): activation rows padded
+// with zeros to whole steps, codes loaded by ld_codes8.  gridDim.y > 1 (ROWS): K slices of whole steps; slice z
+// leaves its exact integer sums in partial[z][N][M] for i2s_bt_reduce.
 constexpr int TGT = 512;
-template <bool ROWS = false>
+template <bool ROWS = false, bool TAIL = false>
 __global__ __launch_bounds__(TGT) void i2s_gemm_mfma(const uint8_t* w, const int8_t* a, float* __restrict__ out, int M,
-                                                     int N, int K, float w_scale = 0.0f,
-                                                     const float* __restrict__ inv = nullptr) {
+                                                     int N, int K, int lda, float w_scale = 0.0f,
+                                                     const float* __restrict__ inv = nullptr,
+                                                     float* __restrict__ partial = nullptr) {
     __shared__ __align__(16) uint8_t bt[2][TGN * TGK];
     __shared__ int asum[2][TGN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1214,7 +1296,10 @@ __global__ __launch_bounds__(TGT) void i2s_gemm_mfma(const uint8_t* w, const int
     const int r16 = lane & 15, g = lane >> 4;
     const int tn = (N + TGN - 1) / TGN;
     const int m0 = (blockIdx.x / tn) * TGM, n0 = (blockIdx.x % tn) * TGN;
-    const int bpr = K / 4, steps = K / TGK;
+    const int bpr = K / 4, all = TAIL ? (K + TGK - 1) / TGK : K / TGK;
+    const int st0 = ROWS ? (int)((int64_t)blockIdx.y * all / gridDim.y) : 0;
+    const int steps = (ROWS ? (int)((int64_t)(blockIdx.y + 1) * all / gridDim.y) : all) - st0;
+    const uint32_t wtotal = (uint32_t)M * (uint32_t)bpr;
 
     // ---- codes: lane (r16, g), row tile i: row m0 + 32 wr + 16 i + r16, code dwords 4g + 2wk and 4g + 2wk + 1
     // of the step (16 columns each): the planes of dword 4g + c are the lane's A fragment of chunk c, so chunk
@@ -1228,16 +1313,20 @@ __global__ __launch_bounds__(TGT) void i2s_gemm_mfma(const uint8_t* w, const int
     uint2 cw[LEAD + 1][2];
     // ---- activations: wave (wr, wk) loads token n0 + 16 wr + r16, bytes 64 c + 16 g (group 4c + g) of the
     // step for c = 2 wk, 2 wk + 1
-    const uint32_t boff = (uint32_t)min(n0 + 16 * wr + r16, N - 1) * (uint32_t)K + 16 * g + 128 * wk;
+    const uint32_t boff = (uint32_t)min(n0 + 16 * wr + r16, N - 1) * (uint32_t)lda + 16 * g + 128 * wk;
     uint4 bw[LEAD + 1][2];
     int tsum = 0;  // sum of the bytes this lane loads of its token
     auto load_codes = [&](int step, uint2 (&dst)[2]) {
-        const uint8_t* base = w + (int64_t)min(step, steps - 1) * (TGK / 4);
+        const int64_t o = (int64_t)(st0 + min(step, steps - 1)) * (TGK / 4);
+        const uint8_t* base = w + o;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) dst[i] = *(const uint2*)(base + woff[i]);
+        for (int i = 0; i < 2; ++i) {
+            if constexpr (TAIL) dst[i] = ld_codes8(w, o + woff[i], wtotal);
+            else dst[i] = *(const uint2*)(base + woff[i]);
+        }
     };
     auto load_acts = [&](int step, uint4 (&dst)[2]) {
-        const int8_t* base = a + (int64_t)min(step, steps - 1) * TGK;
+        const int8_t* base = a + (int64_t)(st0 + min(step, steps - 1)) * TGK;
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc) dst[cc] = ld16(base + boff + 64 * cc);
     };
@@ -1348,14 +1437,15 @@ __global__ __launch_bounds__(TGT) void i2s_gemm_mfma(const uint8_t* w, const int
         if (n >= N) continue;
         const int as = asum[0][16 * j + r16] + asum[1][16 * j + r16];
         if constexpr (ROWS) {
-            const float ts = inv[n];
+            const bool split = gridDim.y > 1;
+            const float ts = split ? 1.0f : inv[n], ws = split ? 1.0f : w_scale;
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int m = m0 + 32 * wr + 16 * i + 4 * g;
                 float v[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = fmul_rn(fmul_rn((float)(acc[i][j][r] - as), w_scale), ts);
-                float* dst = out + (int64_t)n * M + m;
+                for (int r = 0; r < 4; ++r) v[r] = fmul_rn(fmul_rn((float)(acc[i][j][r] - as), ws), ts);
+                float* dst = split ? partial + ((int64_t)blockIdx.y * N + n) * M + m : out + (int64_t)n * M + m;
                 if (m + 3 < M && ((uintptr_t)dst & 15u) == 0) {
                     *(float4*)dst = make_float4(v[0], v[1], v[2], v[3]);
                 } else {
@@ -1520,22 +1610,115 @@ hipError_t launch_i2s_gemv_bt(const uint8_t* packed, float w_scale, const int8_t
     const dim3 grid(ceil_div(M, kIbRows), (unsigned)S);
     for (int64_t t0 = 0; t0 < batch; t0 += kIbTok) {
         const int b = (int)(batch - t0 < kIbTok ? batch - t0 : kIbTok);
-        i2s_gemv_bt<kIbChunks, kIbWaves><<<grid, kIbWaves * 64, 0, s>>>(packed, w_scale, act + t0 * K, act_scale + t0, y + t0 * M, partial, (int)M,
-                                         (int)K, b);
+        i2s_gemv_bt<kIbChunks, kIbWaves><<<grid, kIbWaves * 64, 0, s>>>(packed, w_scale, act + t0 * K, K,
+                                                                        act_scale + t0, y + t0 * M, partial, (int)M,
+                                                                        (int)K, b);
         if (S > 1)
             i2s_bt_reduce<<<ceil_div((int64_t)b * M, kWG), kWG, 0, s>>>(partial, w_scale, act_scale + t0, y + t0 * M,
-                                                                        (int)M, b, S);
+                                                                        (int)M, b, S, kIbTok * M);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
+// ---- token rows of any K % 4 == 0 ---------------------------------------------
+// workspace: the activation rows as int8 padded to whole 256-column chunks, their inverse scales (FP32 rows), the
+// K slices' sums
+namespace {
+inline int64_t rows_kp(int64_t K) { return (K + 255) / 256 * 256; }
+inline size_t al256(size_t n) { return (n + 255) & ~(size_t)255; }
+// the GEMM's K slices: about one workgroup per CU, at least 4 steps each, at most 16 (i2s_bt_reduce)
+inline int rows_slices(int64_t M, int64_t K, int64_t batch) {
+    const int64_t tiles = ((M + TGM - 1) / TGM) * ((batch + TGN - 1) / TGN), steps = (K + TGK - 1) / TGK;
+    return (int)std::max<int64_t>(1, std::min<int64_t>({(256 + tiles - 1) / tiles, steps / 4, 16}));
+}
+inline size_t rows_partial(int64_t M, int64_t K, int64_t batch) {
+    if (batch <= kIbTok) return i2s_bt_partial_bytes(M, K);
+    const int S = rows_slices(M, K, batch);
+    return S > 1 ? (size_t)(S * batch * M * 4) : 0;
+}
+// Whether the two or three launches of launch_i2s_rows (12 us eagerly without a K split, 15 us with one) beat the
+// one launch of the kernels that walk the tokens one after another (8 us eagerly for any little work).  Those take
+// per token (measured at M = 512 .. 8192, K = 512 .. 8256, 1 .. 16 tokens): the codes of any alignment about
+// K (3300 + M) / 2e6 us; whole 64-column pieces of int8 tokens (K + 1500)(1800 + M) / 1.2e7 us; quantising FP32
+// tokens 0.25 us + K / 3000 us and M K / 1e7 us.  At 12 tokens and more the walk was never faster.
+inline bool rows_pay(bool f32, bool whole, int64_t M, int64_t K, int64_t batch) {
+    if (batch >= 12) return true;
+    if (!whole) return batch * K * (3300 + M) >= 30000000;
+    if (f32) return batch * (K + 3000) >= 44000 || batch * M * K >= 120000000;
+    return batch * (K + 1500) * (1800 + M) >= 175000000;
+}
+}  // namespace
+
+bool i2s_rows_supported(const uint8_t* packed, const void* x, bool f32, int64_t M, int64_t K, int64_t batch) {
+    // int8 rows the batched kernel takes as they are (a decode group of whole aligned chunks) stay on it; exact
+    // integer sums in FP32 (K < 2^17) and 32-bit lane offsets as i2s_gemm_mfma_ok
+    if (!f32 && batch <= kIbTok && i2s_bt_supported(M, K, batch) && aligned16(packed) && aligned16(x)) return false;
+    const bool whole = K % 64 == 0 && K <= 64 * 256 && aligned16(packed) && aligned16(x);
+    if (batch == 1 && whole) return false;
+    return batch >= 1 && rows_pay(f32, whole, M, K, batch) && K % 4 == 0 && K >= 64 && K < (1 << 24) / 128 && M < (1ll << 31) &&
+           M * (K / 4) >= 16 && M * (K / 4) < (1ll << 32) - 256 && batch * rows_kp(K) < (1ll << 32) &&
+           ((M + TGM - 1) / TGM) * ((batch + TGN - 1) / TGN) < (1ll << 31) && batch <= 65535;
+}
+
+size_t i2s_rows_workspace_bytes(int64_t M, int64_t K, int64_t batch) {
+    return al256((size_t)(batch * rows_kp(K))) + al256((size_t)batch * 4) + rows_partial(M, K, batch);
+}
+
+hipError_t launch_i2s_rows(const uint8_t* packed, float w_scale, const float* x, const int8_t* act,
+                           const float* act_scale, float* y, int64_t M, int64_t K, int64_t batch, void* ws,
+                           hipStream_t s) {
+    const int64_t Kp = rows_kp(K);
+    int8_t* q = (int8_t*)ws;
+    float* inv = (float*)((char*)ws + al256((size_t)(batch * Kp)));
+    float* partial = (float*)((char*)inv + al256((size_t)batch * 4));
+    const int8_t* a = q;
+    int64_t lda = Kp;
+    if (x) {
+        if (aligned16(x))
+            i2s_quant_rows_k<true><<<(unsigned)batch, kQrT, 0, s>>>(x, (int)K, (int)Kp, q, inv);
+        else
+            i2s_quant_rows_k<false><<<(unsigned)batch, kQrT, 0, s>>>(x, (int)K, (int)Kp, q, inv);
+        act_scale = inv;
+    } else if (Kp != K || !aligned16(act)) {
+        i2s_pad_rows_k<<<dim3((unsigned)ceil_div(Kp, 4 * kWG), (unsigned)batch), kWG, 0, s>>>(act, (int)K, (int)Kp, q);
+    } else {
+        a = act;
+        lda = K;
+    }
+    const bool tail = K % 256 != 0 || !aligned16(packed);
+    const int m = (int)M, k = (int)K, n = (int)batch;
+    if (batch <= kIbTok) {
+        const int S = ib_slices(M, K);
+        const dim3 grid(ceil_div(M, kIbRows), (unsigned)S);
+        if (tail)
+            i2s_gemv_bt<kIbChunks, kIbWaves, false, true><<<grid, kIbWaves * 64, 0, s>>>(packed, w_scale, a, lda,
+                                                                                       act_scale, y, partial, m, k, n);
+        else
+            i2s_gemv_bt<kIbChunks, kIbWaves><<<grid, kIbWaves * 64, 0, s>>>(packed, w_scale, a, lda, act_scale, y,
+                                                                            partial, m, k, n);
+        if (S > 1)
+            i2s_bt_reduce<<<ceil_div(batch * M, kWG), kWG, 0, s>>>(partial, w_scale, act_scale, y, m, n, S,
+                                                                   kIbTok * M);
+        return hipGetLastError();
+    }
+    const int S = rows_slices(M, K, batch);
+    const dim3 grid((unsigned)(((M + TGM - 1) / TGM) * ((batch + TGN - 1) / TGN)), (unsigned)S);
+    if (tail)
+        i2s_gemm_mfma<true, true><<<grid, TGT, 0, s>>>(packed, a, y, m, n, k, (int)lda, w_scale, act_scale, partial);
+    else
+        i2s_gemm_mfma<true><<<grid, TGT, 0, s>>>(packed, a, y, m, n, k, (int)lda, w_scale, act_scale, partial);
+    if (S > 1)
+        i2s_bt_reduce<<<ceil_div(batch * M, kWG), kWG, 0, s>>>(partial, w_scale, act_scale, y, m, n, S, batch * M);
+    return hipGetLastError();
+}
+
 hipError_t launch_i2s_gemv_bt_slices(const uint8_t* packed, float w_scale, const int8_t* act, const float* act_scale,
                                     float* y, int64_t M, int64_t K, int64_t batch, float* partial, Slices* out,
                                     hipStream_t s) {
     const int S = ib_slices(M, K);
-    i2s_gemv_bt<kIbChunks, kIbWaves><<<dim3(ceil_div(M, kIbRows), (unsigned)S), kIbWaves * 64, 0, s>>>(packed, w_scale, act, act_scale, y, partial,
+    i2s_gemv_bt<kIbChunks, kIbWaves><<<dim3(ceil_div(M, kIbRows), (unsigned)S), kIbWaves * 64, 0, s>>>(packed, w_scale, act, K, act_scale, y, partial,
                                                                         (int)M, (int)K, (int)batch);
     *out = S == 1 ? plain_slices(y, M) : Slices{partial, M, kIbTok * M, S, w_scale, act_scale};
     return hipGetLastError();
@@ -1549,7 +1732,7 @@ hipError_t launch_i2s_gemv_bt_f32act(const uint8_t* packed, float w_scale, const
     const int S = ib_slices(M, K);
     const I2sF32Act fa{act, lda, amax, nmx, inv};
     i2s_gemv_bt<kIbFaChunks, kIbWaves, true><<<dim3(ceil_div(M, kIbRows), (unsigned)S), kIbWaves * 64, 0, s>>>(
-        packed, w_scale, nullptr, nullptr, y, partial, (int)M, (int)K, (int)batch, fa);
+        packed, w_scale, nullptr, 0, nullptr, y, partial, (int)M, (int)K, (int)batch, fa);
     *out = S == 1 ? plain_slices(y, M) : Slices{partial, M, kIbTok * M, S, w_scale, inv};
     return hipGetLastError();
 }
@@ -1561,7 +1744,8 @@ hipError_t launch_i2s_gemv_bt_f32act_y(const uint8_t* packed, float w_scale, con
     const hipError_t e = launch_i2s_gemv_bt_f32act(packed, w_scale, act, lda, amax, nmx, inv, y, M, K, batch, partial,
                                                    &out, s);
     if (e != hipSuccess || out.n == 1) return e;
-    i2s_bt_reduce<<<ceil_div(batch * M, kWG), kWG, 0, s>>>(partial, w_scale, inv, y, (int)M, (int)batch, out.n);
+    i2s_bt_reduce<<<ceil_div(batch * M, kWG), kWG, 0, s>>>(partial, w_scale, inv, y, (int)M, (int)batch, out.n,
+                                                           kIbTok * M);
     return hipGetLastError();
 }
 
@@ -1581,7 +1765,7 @@ hipError_t launch_i2s_gemm_vnni(const uint8_t* w, const int8_t* a, float* o, int
                                 hipStream_t s) {
     if (i2s_gemm_mfma_ok(M, N, K) && (((uintptr_t)w | (uintptr_t)a) & 15u) == 0) {
         const unsigned grid = (unsigned)(((M + TGM - 1) / TGM) * ((N + TGN - 1) / TGN));
-        i2s_gemm_mfma<<<grid, TGT, 0, s>>>(w, a, o, (int)M, (int)N, (int)K);
+        i2s_gemm_mfma<<<grid, TGT, 0, s>>>(w, a, o, (int)M, (int)N, (int)K, (int)K);
         return hipGetLastError();
     }
     i2s_gemm_vnni_k<<<ceil_div(M * N, kWaves), kWG, 0, s>>>(w, a, o, M, N, K);
@@ -1592,7 +1776,7 @@ hipError_t launch_i2s_gemm_rows(const uint8_t* w, float w_scale, const int8_t* a
                                 int64_t N, int64_t K, hipStream_t s) {
     if (!i2s_gemm_mfma_ok(M, N, K) || (((uintptr_t)w | (uintptr_t)a) & 15u) != 0) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)(((M + TGM - 1) / TGM) * ((N + TGN - 1) / TGN));
-    i2s_gemm_mfma<true><<<grid, TGT, 0, s>>>(w, a, y, (int)M, (int)N, (int)K, w_scale, inv);
+    i2s_gemm_mfma<true><<<grid, TGT, 0, s>>>(w, a, y, (int)M, (int)N, (int)K, (int)K, w_scale, inv);
     return hipGetLastError();
 }
 
