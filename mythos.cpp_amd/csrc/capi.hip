@@ -628,6 +628,14 @@ int mth_attention_decode(const float* q, const float* kcache, const float* vcach
             (long long)head_dim, (long long)max_seq);
     REQUIRE(ctx >= 1 && ctx <= max_seq, "mth_attention_decode: ctx=%lld outside 1..%lld", (long long)ctx,
             (long long)max_seq);
+    if (mth::attention_split_supported(q, kcache, vcache, batch, (int)heads, (int)kv_heads, (int)head_dim, (int)ctx,
+                                       (int)max_seq)) {
+        if (void* ws = workspace_or_null(S(stream), mth::attention_split_workspace_bytes(batch, (int)heads, (int)kv_heads,
+                                                                                         (int)head_dim, (int)ctx)))
+            return check_launch(mth::launch_attention_split(q, kcache, vcache, out, (int)ctx, batch, (int)heads,
+                                                            (int)kv_heads, (int)head_dim, (int)max_seq, ws, S(stream)),
+                                "mth_attention_decode");
+    }
     return check_launch(mth::launch_attention(q, kcache, vcache, out, nullptr, (int)ctx - 1, batch, (int)heads,
                                               (int)kv_heads, (int)head_dim, (int)max_seq, S(stream)),
                         "mth_attention_decode");

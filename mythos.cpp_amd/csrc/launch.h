@@ -256,6 +256,13 @@ hipError_t launch_rope_kv(float* q, const float* k, const float* v, const float*
 bool attention_supported(int head_dim, int max_seq);
 hipError_t launch_attention(const float* q, const float* kc, const float* vc, float* out, const int* step, int ctx0,
                             int64_t batch, int heads, int kv_heads, int head_dim, int max_seq, hipStream_t s);
+// Long contexts: the context split over workgroups (attn_split.hip), FP32 caches, partial results in ws
+// (attention_split_workspace_bytes); launch_attention's semantics for ctx positions.
+bool attention_split_supported(const float* q, const float* kc, const float* vc, int64_t batch, int heads,
+                               int kv_heads, int head_dim, int ctx, int max_seq);
+size_t attention_split_workspace_bytes(int64_t batch, int heads, int kv_heads, int head_dim, int ctx);
+hipError_t launch_attention_split(const float* q, const float* kc, const float* vc, float* out, int ctx, int64_t batch,
+                                  int heads, int kv_heads, int head_dim, int max_seq, void* ws, hipStream_t s);
 // RoPE of the current token's q/k at pos = *step, KV append, then attention
 // over pos + 1 positions (one launch).  Caches FP32, or bf16 bits (kv_bf16).
 hipError_t launch_rope_attention(const float* q, const float* k, const float* v, const float* cos_t,

@@ -81,3 +81,60 @@ def test_ternary_rows_under_capture(oracle, mth, dev):
             gr.replay()
         torch.cuda.synchronize()
         assert np.array_equal(y.cpu().numpy().reshape(batch, M), want), rep
+
+
+# -------------------------------------------------------------- attention --
+@pytest.mark.parametrize("B,H,KVH,D,ctx,S", [
+    (1, 8, 8, 128, 329, 400),        # shortest split context of 128, one head per workgroup, a slice of 9 rows
+    (2, 32, 8, 128, 1025, 1500),     # 4 heads per workgroup, a slice of one row
+    (1, 40, 5, 64, 2000, 2000),      # 8 heads per workgroup
+    (3, 12, 4, 64, 777, 1024),       # a group of 3: one head per workgroup
+    (2, 16, 1, 256, 400, 512),       # 16 heads of one kv head, two workgroup rows; D = 256
+    (1, 4, 2, 64, 16384, 16384),     # the longest context: slices at their limit
+    (16, 32, 2, 64, 1300, 1300),     # many workgroups, 16 rows per lane
+])
+def test_attention_split(B, H, KVH, D, ctx, S, mth, dev):
+    """The context split over workgroups against float64: scores of a spread
+    that leaves whole slices without weight, one row whose maximum sits in the
+    last slice.  FP32 sums of ctx products: a few 1e-7 of the output's norm."""
+    import torch
+    print(f"attention split B={B} H={H} KVH={KVH} D={D} ctx={ctx}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(ctx + D)
+    q = torch.randn(B, H, D, generator=g, device=dev) * 2
+    kc, vc = (torch.randn(B, KVH, S, D, generator=g, device=dev) for _ in range(2))
+    kc[0, 0, ctx - 1] = q[0, 0] * 0.5
+    kc[:, :, ctx:], vc[:, :, ctx:] = float("nan"), float("nan")      # rows past the context are never used
+    out = torch.full((B, H, D), float("nan"), device=dev)
+    mth.attention_decode(q, kc, vc, out, B, H, KVH, D, ctx, S)
+    torch.cuda.synchronize()
+    want = torch.empty(B, H, D, dtype=torch.float64, device=dev)
+    for b in range(B):
+        for h in range(H):
+            k, v = kc[b, h % KVH, :ctx].double(), vc[b, h % KVH, :ctx].double()
+            p = torch.softmax((k @ q[b, h].double()) / D ** 0.5, 0)
+            want[b, h] = p @ v
+    rel = ((out.double() - want).norm(dim=-1) / want.norm(dim=-1)).max().item()
+    assert rel <= 4e-6, rel
+
+
+def test_attention_split_specials(mth, dev):
+    """A slice whose scores are all -inf has no weight; a NaN in V reaches the
+    output (0 * NaN), as in the undivided sum."""
+    import torch
+    B, H, D, ctx = 1, 8, 128, 2000
+    g = torch.Generator(device=dev).manual_seed(5)
+    q = torch.rand(B, H, D, generator=g, device=dev) + 0.1
+    kc, vc = (torch.randn(B, H, ctx, D, generator=g, device=dev) for _ in range(2))
+    kc[:, :, 256:1400] = float("-inf")
+    vc[0, 3, 700, 5] = float("nan")
+    out = torch.empty(B, H, D, device=dev)
+    mth.attention_decode(q, kc, vc, out, B, H, H, D, ctx, ctx)
+    keep = [i for i in range(ctx) if not 256 <= i < 1400]
+    for h in range(H):
+        p = torch.softmax((kc[0, h, keep].double() @ q[0, h].double()) / D ** 0.5, 0)
+        want = p @ vc[0, h, keep].double()
+        got = out[0, h].double()
+        if h == 3:
+            assert torch.isnan(got[5]) and torch.isnan(got).sum() == 1
+            got[5] = want[5]
+        assert ((got - want).norm() / want.norm()).item() <= 4e-6
