@@ -190,7 +190,15 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
             "mth_oil8_gemv: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
     const bool aligned = (((uintptr_t)indices | (uintptr_t)x) & 15u) == 0;
     const mth::Oil8Seg seg{indices, codebook, y, M};
-    if (aligned && batch >= kGemmRows && mth::oil8_gemm_x32_supported(&seg, 1, batch, K)) {
+    const bool gemm = aligned && batch >= kGemmRows && mth::oil8_gemm_x32_supported(&seg, 1, batch, K);
+    const bool bt = aligned && mth::oil8_bt_supported(M, K, batch);
+    const bool walk = batch == 1 && aligned && K % 16 == 0 && K <= 4096 && M * K < (1ll << 32);
+    if (!walk && mth::oil8_rows_better(indices, M, K, batch, aligned, gemm, bt)) {
+        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch)))
+            return check_launch(mth::launch_oil8_rows(indices, codebook, x, y, M, K, batch, ws, S(stream)),
+                                "mth_oil8_gemv");
+    }
+    if (gemm) {
         // >= 128 tokens: the MFMA GEMM (each weight read once per 128 tokens)
         void* ws = nullptr;
         const size_t need = mth::oil8_gemm_x32_workspace_bytes(batch, K);
@@ -198,7 +206,7 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
         if (e != hipSuccess) return workspace_fail("mth_oil8_gemv", e, need);
         return check_launch(mth::launch_oil8_gemm_x32(x, &seg, 1, batch, K, ws, S(stream)), "mth_oil8_gemv");
     }
-    if (aligned && mth::oil8_bt_supported(M, K, batch)) {
+    if (bt) {
         void* partial = nullptr;
         const size_t need = mth::oil8_bt_partial_bytes(M, K);
         const hipError_t e = workspace(S(stream), need, &partial);
@@ -227,8 +235,16 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
     REQUIRE(cb_block == 0 || K % cb_block == 0, "mth_oil4_gemv: K=%lld not a multiple of cb_block=%lld",
             (long long)K, (long long)cb_block);
     const bool aligned = (((uintptr_t)packed | (uintptr_t)codebooks | (uintptr_t)x) & 15u) == 0;
-    if (aligned && ((uintptr_t)y & 15u) == 0 && batch >= kGemmRows &&
-        mth::oil4_gemm_x32_supported(batch, M, K, cb_block)) {
+    const bool gemm = aligned && ((uintptr_t)y & 15u) == 0 && batch >= kGemmRows &&
+                      mth::oil4_gemm_x32_supported(batch, M, K, cb_block);
+    const bool bt = aligned && mth::oil4_bt_supported(M, K, cb_block, batch);
+    const bool one = batch == 1 && aligned && K <= 4096;  // one token: its own kernels up to 4096 columns
+    if (!one && mth::oil4_rows_better(packed, codebooks, cb_block, M, K, batch, aligned, gemm, bt)) {
+        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch)))
+            return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, ws, S(stream)),
+                                "mth_oil4_gemv");
+    }
+    if (gemm) {
         // >= 128 tokens: the MFMA GEMM (each weight read once per 128 tokens)
         void* ws = nullptr;
         const size_t need = mth::oil4_gemm_x32_workspace_bytes(batch, K);
@@ -237,7 +253,7 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
         return check_launch(mth::launch_oil4_gemm_x32(x, packed, codebooks, cb_block, y, batch, M, K, ws, S(stream)),
                             "mth_oil4_gemv");
     }
-    if (aligned && mth::oil4_bt_supported(M, K, cb_block, batch)) {
+    if (bt) {
         void* partial = nullptr;
         const size_t need = mth::oil4_bt_partial_bytes(M, K);
         const hipError_t e = workspace(S(stream), need, &partial);
@@ -378,6 +394,10 @@ int mth_i2s_gemm(const uint8_t* w, const float* act, float* out, int64_t M, int6
                  mth_stream_t stream) {
     REQUIRE(w && act && out, "mth_i2s_gemm: null pointer");
     REQUIRE(M > 0 && N > 0 && K > 0 && M * N < kMaxDim && K < kMaxDim, "mth_i2s_gemm: bad sizes");
+    if (mth::tern_rows_better(M, K, N)) {
+        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, N)))
+            return check_launch(mth::launch_tern_rows(w, act, out, M, K, N, ws, S(stream)), "mth_i2s_gemm");
+    }
     return check_launch(mth::launch_i2s_gemm(w, act, out, M, N, K, S(stream)), "mth_i2s_gemm");
 }
 

@@ -369,6 +369,22 @@ __device__ __forceinline__ float norm_scale(const NormScale& ns, int t, double* 
 // SwiGLU of every decoder path uses this one definition).
 __device__ __forceinline__ float silu1(float g) { return (g / (1.0f + expf(-g))); }
 
+// ---- ternary codes at any alignment --------------------------------------------
+// 8 code bytes at byte pos of a matrix of `end` >= 8 bytes, for rows that are not whole aligned pieces (K / 4 bytes,
+// any K / 4).  Bytes past the row are the next row's: the activations there are zeros, so their codes add nothing.
+// Near the matrix's end the load is moved back into it, and codes8_at, at the use (a shift beside the load would
+// wait for it), puts the bytes in place again: needed only in tiles that hold the last row.
+__device__ __forceinline__ uint2 ld_codes8(const uint8_t* w, int64_t pos, int64_t end) {
+    uint2 v;
+    __builtin_memcpy(&v, w + min(pos, end - 8), 8);
+    return v;
+}
+__device__ __forceinline__ uint2 codes8_at(uint2 v, int64_t pos, int64_t end) {
+    const int past = (int)min(max(pos - (end - 8), (int64_t)0), (int64_t)7);  // (a piece past the end: any codes)
+    const uint64_t u = (v.x | ((uint64_t)v.y << 32)) >> (8 * past);
+    return make_uint2((uint32_t)u, (uint32_t)(u >> 32));
+}
+
 // ---- int8 helpers ---------------------------------------------------------
 // sum_{i<4} (int8)a.byte[i] * (int8)b.byte[i] + c   (v_dot4_i32_i8)
 __device__ __forceinline__ int dot4(uint32_t a, uint32_t b, int c) {

@@ -1,0 +1,562 @@
+// gemm_rows.hip — quantized weights times a batch of FP32 token rows on
+// gfx950 MFMA, for any row count, any token count and row lengths the tiled
+// prompt GEMMs do not take.
+//
+//   y[t][m] = sum_k W[m][k] x[t][k]       W: OIL8 (src/kernel_oil8.cpp:14-27), OIL4 with codebooks per cb_block
+//   columns or one per tensor (src/kernel_oil4.cpp:31-54), or ternary (src/kernel_i2s.cpp:42-65, o[m][t])
+//
+// Arithmetic (as the batched GEMVs and the prompt GEMMs): each token row is
+// scaled by a power of two and split into FP16 hi + lo (rows_split_k, once per
+// call); OIL4 and ternary weights are exact in FP16 (two products per weight
+// and token), OIL8 codebook entries are split the same way (three products;
+// lo x lo lies below FP32's rounding).  Products are exact in FP32, sums FP32
+// on v_mfma_f32_16x16x32_f16, the hi x hi products and the rest in accumulators
+// of their own.  A token tile that holds Inf or NaN, or a non-finite OIL8
+// codebook, takes FP32 FMAs over the reference's products instead.
+//
+// Tiling.  A workgroup of 4 waves takes 128 weight rows (32 per wave: two A
+// tiles share every B read, which otherwise bounds the kernel: a tile-step
+// reads 32 KB of B per wave from LDS) x 16 G tokens (G <= 4) over a K slice in
+// steps of 128 columns.  Weights go from memory straight into A registers (two
+// steps ahead), B fragments of a step through LDS (one step ahead in
+// registers); two workgroups per CU cover each other's barriers.  gridDim.z > 1:
+// K slices, whose sums rows_reduce_k adds in order.
+//
+// Bound: per workgroup ~5 us before the first step and after the last (load latency, table, output) and then, on a
+// full chip, LDS for OIL8 (a step's 256 gathers of ~6 cycles and its B reads, 1.35 us per step for two workgroups a
+// CU at 48 tokens) and half of the MFMA rate for the others (0.83 us).  Measured against the routes before it (one
+// call, eager): OIL8 4000 x 4096, 40 tokens 32.9 -> 19.3 us; 2000 x 8976, 256 tokens 9.9 ms -> 52 us; OIL4 5000 x
+// 9088 (codebooks per 64), 64 tokens 5.4 ms -> 36 us; ternary 4096 x 4096, 300 tokens 5.8 ms -> 36 us.
+#include <algorithm>
+
+#include "common.h"
+#include "launch.h"
+#include "oil4_common.h"
+
+namespace mth {
+namespace {
+
+constexpr int kRmStep = 128;              // columns per step
+constexpr int kRmRows = 128, kRmT = 256;  // weight rows and threads per workgroup
+constexpr int kRmSlices = 16;             // most K slices (rows_reduce_k)
+
+enum RowsFmt { kOil8, kOil4, kTern };
+
+// ---- token rows -> FP16 hi / lo B fragments ------------------------------------
+// Row t: shift s with max|x| 2^s in [2^14, 2^15) into rsh[t] (kRowNonFinite for a row holding Inf / NaN), then
+// 2^s x = hi + lo, group t / 16, part (hi, lo), 32-column chunk c: 1 KB of [8-column piece m][token t % 16][8].
+// TERN: the pieces hold the columns in the order of the ternary codes' planes (element e of piece m: column
+// 16 (m / 2) + 2 (m % 2) + e / 4 + 4 (e % 4) of the chunk).  Columns past K are zeros; rows past the batch are not
+// written (their products only reach their own, discarded, outputs).  One workgroup per row, the row read once
+// (16384 columns in registers; the rest of a longer row twice).
+constexpr int kRsN = 4;
+template <bool TERN, bool VEC>
+__global__ __launch_bounds__(kRmT) void rows_split_k(const float* __restrict__ x, uint16_t* __restrict__ a16,
+                                                     int* __restrict__ rsh, int K, int chunks) {
+    __shared__ uint32_t red[kRmT / 64];
+    const int tid = threadIdx.x, row = blockIdx.x;
+    const float* xr = x + (int64_t)row * K;
+    const int n16 = 2 * chunks;  // 16-column groups
+    auto load = [&](int g, float (&v)[16]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = 16 * g + 4 * i;
+            if constexpr (VEC) {
+                const float4 f = g < n16 && k < K ? ldf4(xr + k) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                v[4 * i] = f.x, v[4 * i + 1] = f.y, v[4 * i + 2] = f.z, v[4 * i + 3] = f.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[4 * i + e] = g < n16 && k + e < K ? xr[k + e] : 0.0f;
+            }
+        }
+    };
+    float v[kRsN][16], u[16];
+#pragma unroll
+    for (int j = 0; j < kRsN; ++j) load(tid + j * kRmT, v[j]);
+    uint32_t mb = 0;
+#pragma unroll
+    for (int j = 0; j < kRsN; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mb = max(mb, __float_as_uint(v[j][i]) & 0x7fffffffu);
+    for (int g = tid + kRsN * kRmT; g < n16; g += kRmT) {
+        load(g, u);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mb = max(mb, __float_as_uint(u[i]) & 0x7fffffffu);
+    }
+    mb = group_reduce<64>(mb, UMaxOp{});
+    if ((tid & 63) == 0) red[tid >> 6] = mb;
+    __syncthreads();
+    mb = max(max(red[0], red[1]), max(red[2], red[3]));
+    const int sh = fp16_scale_shift(__uint_as_float(mb));
+    if (tid == 0) rsh[row] = mb >= 0x7f800000u ? kRowNonFinite : sh;
+    uint16_t* hi = a16 + (int64_t)(row >> 4) * 2 * chunks * 512 + 8 * (row & 15);
+    uint16_t* lo = hi + (int64_t)chunks * 512;
+    auto store = [&](int g, const float (&f)[16]) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            half8 h, l;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float xs = ldexpf(f[TERN ? 2 * p + (e >> 2) + 4 * (e & 3) : 8 * p + e], sh);
+                h[e] = (_Float16)xs;
+                l[e] = (_Float16)(xs - (float)h[e]);
+            }
+            const int64_t off = (int64_t)(g >> 1) * 512 + 128 * (2 * (g & 1) + p);
+            *(half8*)(hi + off) = h;
+            *(half8*)(lo + off) = l;
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < kRsN; ++j)
+        if (tid + j * kRmT < n16) store(tid + j * kRmT, v[j]);
+    for (int g = tid + kRsN * kRmT; g < n16; g += kRmT) {
+        load(g, u);
+        store(g, u);
+    }
+}
+
+// ---- the product ----------------------------------------------------------------
+struct RowsArgs {
+    const uint8_t* w;      // OIL8 indices [M][K], OIL4 nibbles [M][K / 2], ternary codes [M][K / 4]
+    const void* cb;        // OIL8: 256 floats; OIL4: FP16 codebooks
+    const uint16_t* a16;   // rows_split_k's fragments
+    const int* rsh;
+    const float* x;        // [batch][K]
+    float* out;            // [batch][M] (ternary: [M][batch])
+    float* partial;        // [slice] of the same
+    int M, K, batch, steps, cb_block;
+};
+
+// a weight tile's registers of one step: 16 rows x 128 columns
+template <int FMT>
+struct RowsTile;
+template <>
+struct RowsTile<kOil8> {
+    uint4 x, y;  // rows 0-7 / 8-15, 8 lanes of 16 bytes per row (128-byte runs); h3_pieces hands them out
+};
+template <>
+struct RowsTile<kOil4> {
+    uint4 n, c0, c1;  // the lane's row: nibbles of columns 32 q .., its block's 16 entries
+};
+template <>
+struct RowsTile<kTern> {
+    uint2 c;  // the lane's row: codes of columns 32 q ..
+};
+
+__device__ __forceinline__ uint32_t rows_hl(float c) {
+    const _Float16 h = (_Float16)c;
+    const _Float16 l = (_Float16)(c - (float)h);
+    return (uint32_t)__builtin_bit_cast(uint16_t, h) | ((uint32_t)__builtin_bit_cast(uint16_t, l) << 16);
+}
+
+// 8 ternary weights (planes f, f + 1 of a code dword) as FP16: code 0 -> -1, 1 -> 0, 2 and 3 -> 1.  A byte lookup
+// gives the high bytes 0xBC, 0, 0x3C, 0x3C; the low bytes are 0.
+__device__ __forceinline__ half8 rows_tern8(uint32_t d, int f) {
+    typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+    const uint32_t h0 = __builtin_amdgcn_perm(0u, 0x3c3c00bcu, (d >> (2 * f)) & 0x03030303u);
+    const uint32_t h1 = __builtin_amdgcn_perm(0u, 0x3c3c00bcu, (d >> (2 * f + 2)) & 0x03030303u);
+    const u32x4v r = {__builtin_amdgcn_perm(0u, h0, 0x010c000cu), __builtin_amdgcn_perm(0u, h0, 0x030c020cu),
+                      __builtin_amdgcn_perm(0u, h1, 0x010c000cu), __builtin_amdgcn_perm(0u, h1, 0x030c020cu)};
+    return __builtin_bit_cast(half8, r);
+}
+
+// FP32 products over columns [k0, k1) of one output, the reference's arithmetic in column order.
+template <int FMT>
+__device__ float rows_fma(const RowsArgs& p, int row, int tok, int k0, int k1) {
+    const float* x = p.x + (int64_t)tok * p.K;
+    float s = 0.0f;
+    if constexpr (FMT == kOil8) {
+        const uint8_t* w = p.w + (int64_t)row * p.K;
+        const float* cb = (const float*)p.cb;
+        for (int k = k0; k < k1; ++k) s = fmaf(cb[w[k]], x[k], s);
+    } else if constexpr (FMT == kOil4) {
+        const uint8_t* w = p.w + (int64_t)row * (p.K >> 1);
+        const uint16_t* cb = (const uint16_t*)p.cb;
+        for (int k = k0; k < k1; ++k) {
+            const int e = (w[k >> 1] >> (4 * (k & 1))) & 15;
+            const int64_t b = p.cb_block ? (int64_t)row * (p.K / p.cb_block) + k / p.cb_block : 0;
+            s = fmaf(h2f(cb[b * 16 + e]), x[k], s);
+        }
+    } else {
+        const uint8_t* w = p.w + (int64_t)row * (p.K >> 2);
+        for (int k = k0; k < k1; ++k) {
+            const int c = (w[k >> 2] >> (2 * (k & 3))) & 3;
+            s += c == 1 ? 0.0f : (c == 0 ? -x[k] : x[k]);
+        }
+    }
+    return s;
+}
+
+template <int FMT, int G>
+__global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p) {
+    constexpr int NB = 2 * G;  // 16-byte pieces of a step's B per thread (8 KB per token group)
+    __shared__ __align__(16) uint8_t bs[G * 8192];
+    __shared__ uint32_t tab[FMT == kOil8 ? 256 : 1];
+    __shared__ float wred[kRmT / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int j = lane & 15, q = lane >> 4;
+    const int row0 = blockIdx.x * kRmRows + wave * 32, tok0 = blockIdx.y * 16 * G;
+    const int S = gridDim.z;
+    const int s0 = (int)((int64_t)blockIdx.z * p.steps / S), s1 = (int)((int64_t)(blockIdx.z + 1) * p.steps / S);
+    const int M = p.M, K = p.K;
+
+    // ---- loads of a step: every address in bounds (rows past M - 1: row M - 1; columns past the row: its last
+    // 16 bytes, whose products meet zeros; steps past the slice: its last)
+    RowsTile<FMT> wt[2][2];  // [step parity][tile]
+    const int64_t tend = FMT == kTern ? (int64_t)M * (K >> 2) : 0;
+    auto load_w = [&](int step, RowsTile<FMT> (&dst)[2]) {
+        const int st = min(step, s1 - 1);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if constexpr (FMT == kOil8) {
+                const int col = min(kRmStep * st + 16 * (2 * q + (j >> 3)), K - 16);
+                dst[t].x = ld_stream(p.w + (int64_t)min(row0 + 16 * t + (j & 7), M - 1) * K + col);
+                dst[t].y = ld_stream(p.w + (int64_t)min(row0 + 16 * t + 8 + (j & 7), M - 1) * K + col);
+            } else if constexpr (FMT == kOil4) {
+                const int64_t row = min(row0 + 16 * t + j, M - 1);
+                const int col = min(kRmStep * st + 32 * q, K - 32);
+                dst[t].n = ld_stream(p.w + row * (K >> 1) + (col >> 1));
+                const uint16_t* cb = (const uint16_t*)p.cb;
+                if (p.cb_block) cb += (row * (K / p.cb_block) + col / p.cb_block) * 16;
+                dst[t].c0 = ld16(cb);
+                dst[t].c1 = ld16(cb + 8);
+            } else {
+                const int64_t pos = (int64_t)min(row0 + 16 * t + j, M - 1) * (K >> 2) + (kRmStep / 4) * st + 8 * q;
+                dst[t].c = ld_codes8(p.w, pos, tend);
+            }
+        }
+    };
+    uint4 bv[NB];
+    // B: thread's pieces tid + 256 i of [group][part][4 KB of the step's 4 chunks]
+    const int64_t part_bytes = (int64_t)p.steps * 4096;
+    const uint8_t* a16 = (const uint8_t*)p.a16 + (int64_t)(tok0 >> 4) * 2 * part_bytes + 16 * tid;
+    auto load_b = [&](int step) {
+        const uint8_t* base = a16 + (int64_t)min(step, s1 - 1) * 4096;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) bv[i] = ld16(base + i * part_bytes);
+    };
+    // the small operands first (the CU returns loads in issue order), then B and the weights
+    int rs[G];  // this lane's tokens' shifts (rows past the batch: the last row's)
+#pragma unroll
+    for (int g = 0; g < G; ++g) rs[g] = p.rsh[min(tok0 + 16 * g + j, p.batch - 1)];
+    float cbv = 0.0f;
+    if constexpr (FMT == kOil8) cbv = ((const float*)p.cb)[tid];
+    __builtin_amdgcn_sched_barrier(0);
+    load_b(s0);
+    load_w(s0, wt[0]);
+    load_w(s0 + 1, wt[1]);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the codebook's table, the scales, the non-finite check
+    bool fin = true;
+    if constexpr (FMT == kOil8) {
+        fin = __builtin_isfinite(cbv);
+        const float m = wave_max(fabsf(cbv));
+        if (lane == 0) wred[wave] = m;
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) fin = fin && rs[g] != kRowNonFinite;
+    const bool special = __syncthreads_or(!fin) != 0;
+    const int64_t zs = (int64_t)p.batch * M;
+    float* out = S == 1 ? p.out : p.partial + blockIdx.z * zs;
+    auto at = [&](int row, int tok) { return FMT == kTern ? (int64_t)row * p.batch + tok : (int64_t)tok * M + row; };
+    if (special) {
+        const int k0 = kRmStep * s0, k1 = min(K, kRmStep * s1), r0 = blockIdx.x * kRmRows;
+        for (int o = tid; o < kRmRows * 16 * G; o += kRmT) {
+            const int row = r0 + o % kRmRows, tok = tok0 + o / kRmRows;
+            if (row < M && tok < p.batch) out[at(row, tok)] = rows_fma<FMT>(p, row, tok, k0, k1);
+        }
+        return;
+    }
+    int sw = 0;
+    if constexpr (FMT == kOil8) {
+        sw = fp16_scale_shift(fmaxf(fmaxf(wred[0], wred[1]), fmaxf(wred[2], wred[3])));
+        tab[tid] = rows_hl(ldexpf(cbv, sw));
+    }
+    CbPlanes shared_planes;
+    if constexpr (FMT == kOil4)
+        if (!p.cb_block) shared_planes = cb_planes(wt[0][0].c0, wt[0][0].c1);
+
+    floatx4 ah[2][G], ax[2][G];  // hi x hi; the other products
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < G; ++g) ah[t][g] = ax[t][g] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    const bool edge = FMT == kTern && blockIdx.x == gridDim.x - 1;  // a tile with the matrix's last row
+    const uint8_t* brow = bs + q * 1024 + j * 16;  // lane (token j, chunk q) of piece m: + 256 m
+    auto step_body = [&](int step, RowsTile<FMT> (&w)[2]) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) *(uint4*)(bs + i * 4096 + 16 * tid) = bv[i];
+        __syncthreads();
+        load_b(step + 1);
+        RowsTile<FMT> cur[2] = {w[0], w[1]};
+        load_w(step + 2, w);
+        __builtin_amdgcn_sched_barrier(0);
+        uint4 wa[2], wb[2];  // OIL8: the lane's 32 index bytes
+        CbPlanes pl[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if constexpr (FMT == kOil8) {
+                wa[t] = make_uint4(dpp_mix<0xc>(cur[t].x.x, cur[t].y.x), dpp_mix<0xc>(cur[t].x.y, cur[t].y.y),
+                                   dpp_mix<0xc>(cur[t].x.z, cur[t].y.z), dpp_mix<0xc>(cur[t].x.w, cur[t].y.w));
+                wb[t] = make_uint4(dpp_mix<0x3>(cur[t].y.x, cur[t].x.x), dpp_mix<0x3>(cur[t].y.y, cur[t].x.y),
+                                   dpp_mix<0x3>(cur[t].y.z, cur[t].x.z), dpp_mix<0x3>(cur[t].y.w, cur[t].x.w));
+            } else if constexpr (FMT == kOil4) {
+                pl[t] = p.cb_block ? cb_planes(cur[t].c0, cur[t].c1) : shared_planes;
+                if (kRmStep * step + 32 * q >= K) {  // columns past the row: weight 0 (an Inf entry would meet 0)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) pl[t].l[e] = pl[t].h[e] = 0;
+                }
+            } else if (edge) {
+                const int64_t pos = (int64_t)min(row0 + 16 * t + j, M - 1) * (K >> 2) + (kRmStep / 4) * step + 8 * q;
+                cur[t].c = codes8_at(cur[t].c, pos, tend);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            half8 bh[G], bl[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                bh[g] = *(const half8*)(brow + g * 8192 + 256 * m);
+                bl[g] = *(const half8*)(brow + g * 8192 + 4096 + 256 * m);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                half8 Ah, Al;
+                if constexpr (FMT == kOil8) {
+                    const uint32_t w0 = m == 0 ? wa[t].x : m == 1 ? wa[t].z : m == 2 ? wb[t].x : wb[t].z;
+                    const uint32_t w1 = m == 0 ? wa[t].y : m == 1 ? wa[t].w : m == 2 ? wb[t].y : wb[t].w;
+                    uint32_t gv[8];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        gv[e] = tab[(w0 >> (8 * e)) & 0xffu];
+                        gv[4 + e] = tab[(w1 >> (8 * e)) & 0xffu];
+                    }
+                    u32x4 hv, lv;
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        hv[d] = __builtin_amdgcn_perm(gv[2 * d + 1], gv[2 * d], 0x05040100u);
+                        lv[d] = __builtin_amdgcn_perm(gv[2 * d + 1], gv[2 * d], 0x07060302u);
+                    }
+                    Ah = __builtin_bit_cast(half8, hv);
+                    Al = __builtin_bit_cast(half8, lv);
+                } else if constexpr (FMT == kOil4) {
+                    Ah = lookup8_natural(u4get(cur[t].n, m), pl[t]);
+                } else {
+                    Ah = rows_tern8(m < 2 ? cur[t].c.x : cur[t].c.y, 2 * (m & 1));
+                }
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    ah[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh[g], ah[t][g], 0, 0, 0);
+                    ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bl[g], ax[t][g], 0, 0, 0);
+                    if constexpr (FMT == kOil8)
+                        ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, bh[g], ax[t][g], 0, 0, 0);
+                }
+            }
+        }
+        __syncthreads();
+    };
+    for (int step = s0; step < s1; step += 2) {
+        step_body(step, wt[0]);
+        if (step + 1 < s1) step_body(step + 1, wt[1]);
+    }
+
+    // ---- D: lane (j, q) holds rows 4q + i of token j
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const int tok = tok0 + 16 * g + j;
+        if (tok >= p.batch) continue;
+        const int sh = rs[g] + sw;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int row = row0 + 16 * t + 4 * q;
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                v[i] = ldexpf(FMT == kOil8 ? ah[t][g][i] + ax[t][g][i] : oil4_hi_lo(ah[t][g][i], ax[t][g][i]), -sh);
+            float* dst = out + at(row, tok);
+            if (FMT != kTern && row + 3 < M && ((uintptr_t)dst & 15u) == 0) {
+                *(float4*)dst = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (row + i < M) out[at(row + i, tok)] = v[i];
+            }
+        }
+    }
+}
+
+// out[i] = sum over slices z = 0, 1, ... of partial[z][i] (a fixed order); all loads before the first add.  Four
+// values per thread where both arrays are 16-byte aligned (n % 4 == 0).
+template <bool VEC>
+__global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ partial, float* __restrict__ out,
+                                                      int64_t n, int S) {
+    const int64_t i = ((int64_t)blockIdx.x * kRmT + threadIdx.x) * (VEC ? 4 : 1);
+    if (i >= n) return;
+    if constexpr (VEC) {
+        float4 v[kRmSlices];
+#pragma unroll
+        for (int z = 0; z < kRmSlices; ++z) v[z] = z < S ? ldf4(partial + z * n + i) : make_float4(0, 0, 0, 0);
+        float4 s = v[0];
+#pragma unroll
+        for (int z = 1; z < kRmSlices; ++z)
+            if (z < S) s = make_float4(s.x + v[z].x, s.y + v[z].y, s.z + v[z].z, s.w + v[z].w);
+        *(float4*)(out + i) = s;
+    } else {
+        float v[kRmSlices];
+#pragma unroll
+        for (int z = 0; z < kRmSlices; ++z) v[z] = z < S ? partial[z * n + i] : 0.0f;
+        float s = v[0];
+#pragma unroll
+        for (int z = 1; z < kRmSlices; ++z)
+            if (z < S) s += v[z];
+        out[i] = s;
+    }
+}
+
+struct RowsPlan {
+    int G, tiles, S, steps;
+    int64_t rtiles;
+};
+inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch) {
+    RowsPlan p{};
+    p.steps = (int)((K + kRmStep - 1) / kRmStep);
+    const int64_t nt = (batch + 63) / 64;
+    p.G = (int)((batch + 16 * nt - 1) / (16 * nt));  // token tiles of 16, 32, 48 or 64, as even as they go
+    p.tiles = (int)((batch + 16 * p.G - 1) / (16 * p.G));
+    p.rtiles = (M + kRmRows - 1) / kRmRows;
+    const int64_t wgs = p.rtiles * p.tiles;
+    // K slices: about one workgroup per CU (a workgroup's fixed cost, ~5 us of load latency, table and output, is then
+    // paid once per CU: 4096 x 4096 at 40 tokens 24.2 / 19.5 / 23.0 us for 4 / 8 / 16 slices); two per CU for long
+    // slices (16384 x 11008: 87 -> 80 us) or where one leaves a CU in three idle (4096 x 4096 at 300 tokens, 160
+    // workgroups: 51 / 43 / 37 us for 1 / 2 / 3 slices); one slice for more workgroups than CUs.
+    const int64_t per = wgs > 256 ? 1 : wgs > 128 ? (p.steps >= 16 ? 512 / wgs : 1)
+                      : wgs >= 64 && p.steps >= 48 ? 512 / wgs : 256 / wgs;
+    p.S = (int)std::max<int64_t>(1, std::min<int64_t>({per, p.steps / 2, kRmSlices}));
+    return p;
+}
+inline size_t al256r(size_t n) { return (n + 255) & ~(size_t)255; }
+inline size_t rows_a16_bytes(const RowsPlan& p) { return (size_t)p.tiles * p.G * 2 * p.steps * 4096; }
+
+template <int FMT>
+hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s) {
+    const int64_t n = (int64_t)a.M * a.batch;
+    uint16_t* a16 = (uint16_t*)ws;
+    int* rsh = (int*)((char*)ws + rows_a16_bytes(p));
+    float* partial = (float*)((char*)rsh + al256r((size_t)a.batch * 4));
+    a.a16 = a16;
+    a.rsh = rsh;
+    a.partial = partial;
+    a.steps = p.steps;
+    const bool vec = ((uintptr_t)a.x & 15u) == 0 && a.K % 4 == 0;
+    if (vec)
+        rows_split_k<FMT == kTern, true><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps);
+    else
+        rows_split_k<FMT == kTern, false><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps);
+    const dim3 grid((unsigned)p.rtiles, (unsigned)p.tiles, (unsigned)p.S);
+    switch (p.G) {
+        case 1: rows_mfma_k<FMT, 1><<<grid, kRmT, 0, s>>>(a); break;
+        case 2: rows_mfma_k<FMT, 2><<<grid, kRmT, 0, s>>>(a); break;
+        case 3: rows_mfma_k<FMT, 3><<<grid, kRmT, 0, s>>>(a); break;
+        default: rows_mfma_k<FMT, 4><<<grid, kRmT, 0, s>>>(a); break;
+    }
+    if (p.S > 1) {
+        if (n % 4 == 0 && ((uintptr_t)a.out & 15u) == 0)
+            rows_reduce_k<true><<<(unsigned)((n / 4 + kRmT - 1) / kRmT), kRmT, 0, s>>>(partial, a.out, n, p.S);
+        else
+            rows_reduce_k<false><<<(unsigned)((n + kRmT - 1) / kRmT), kRmT, 0, s>>>(partial, a.out, n, p.S);
+    }
+    return hipGetLastError();
+}
+
+inline bool rows_sizes(int64_t M, int64_t K, int64_t batch) {
+    return M >= 1 && M < (1ll << 31) - kRmRows && K >= 32 && K <= (1 << 20) && batch >= 1 && batch <= 65536 &&
+           M * batch < (1ll << 37);
+}
+
+}  // namespace
+
+size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch) {
+    const RowsPlan p = rows_plan(M, K, batch);
+    return rows_a16_bytes(p) + al256r((size_t)batch * 4) + (p.S > 1 ? (size_t)(p.S * M * batch * 4) : 0);
+}
+
+// ---- which route: estimated microseconds (eager calls, MI355X) ------------------
+namespace {
+// this file's three launches: 14.8 us for any little work (each launch costs the host ~3 us), 1.7 us (OIL8) or
+// 1.85 us (OIL4) per step of 128 columns of a full 128 x 64 tile on a CU, and for few tokens the weight stream
+double rows_us(int64_t M, int64_t K, int64_t batch, double step_us) {
+    const RowsPlan p = rows_plan(M, K, batch);
+    const double steps = (double)p.rtiles * p.tiles * p.steps / 256.0;
+    return 14.8 + std::max(steps * step_us * (p.G + 1) / 5.0 - 4.0, 0.0);
+}
+// the kernels that walk tokens one after another (a launch of their own: 8.7 us eagerly).  Measured at M = 512 ..
+// 16384, 1 .. 16 tokens: OIL8 rows of up to 4096 0.98 .. 11.9 us per token, OIL4 rows of up to 2048 / 4096 1.85 / 3.9
+// us per token up to 4400 rows, longer rows (one wave per output) 2.8 / 3.2 us per 1024 columns up to 1600 / 2900 rows
+double walk_us(int64_t M, int64_t K, int64_t batch, bool oil8, bool fast) {
+    if (!fast) return batch * (K / 1024.0) * (oil8 ? 2.8 * std::max(1.0, M / 1600.0) : 3.2 * std::max(1.0, M / 2900.0));
+    if (oil8) return batch * (0.7 + M / 4096.0 * (0.8 + K / 1860.0));
+    return batch * (K <= 2048 ? 1.85 : 3.9) * std::max(1.0, M / 4400.0);
+}
+}  // namespace
+
+// OIL8: K % 16 == 0, 16-byte aligned indices.  gemm: the prompt GEMM takes the call (128 tokens and more); bt: the
+// batched GEMV does (16 tokens per launch pair).
+bool oil8_rows_better(const uint8_t* idx, int64_t M, int64_t K, int64_t batch, bool aligned, bool gemm, bool bt) {
+    if (!rows_sizes(M, K, batch) || K % 16 != 0 || ((uintptr_t)idx & 15u) != 0) return false;
+    const double us = rows_us(M, K, batch, 1.7);
+    if (gemm) {
+        // a round of 256 tiles of 128 x 64 (54 us at K = 4096), or of 256 x 64 where those fill the chip (98 us)
+        const int64_t t = M / 64, wide = (batch + 255) / 256 * t, narrow = (batch + 127) / 128 * t;
+        const double g = wide >= 256 ? 5.0 + 23.3 * (K / 1024.0) * ((wide + 255) / 256)
+                                     : 5.0 + (12.2 + narrow / 110.0) * (K / 1024.0);
+        return us < g;
+    }
+    if (bt) return batch > 16;  // 17 tokens: 19 .. 49 us against 15 .. 31 us
+    return us < walk_us(M, K, batch, true, aligned && K <= 4096);
+}
+
+// OIL4: K % 32 == 0, codebook blocks of a multiple of 32 columns, 16-byte aligned weights.  Wider GEMM tiles (128
+// columns, 15.5 us per 1024 columns and round) as launch_oil4_gemm_x32 picks them.
+bool oil4_rows_better(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, int64_t M, int64_t K, int64_t batch,
+                      bool aligned, bool gemm, bool bt) {
+    if (!rows_sizes(M, K, batch) || K % 32 != 0 || cb_block % 32 != 0 || cb_block >= (1 << 30) ||
+        (((uintptr_t)nib | (uintptr_t)cbs) & 15u) != 0)
+        return false;
+    const double us = rows_us(M, K, batch, 1.85);
+    if (gemm) {
+        const int64_t tiles = (batch + 127) / 128;
+        const bool w128 = M % 128 == 0;
+        const int64_t t = tiles * (M / (w128 ? 128 : 64));
+        const double g = 5.0 + (w128 && t >= 128 ? 15.5 : 11.7) * (K / 1024.0) * ((t + 255) / 256);
+        return us < g;
+    }
+    if (bt) return batch > 16;  // 17 tokens: 18 .. 49 us against 15 .. 48 us
+    return us < walk_us(M, K, batch, false, aligned && K <= 4096);
+}
+
+// Ternary weights, FP32 tokens: against one wave per output (8 us for little work, 3.5 us per 1024 columns for up to
+// 8000 outputs).
+bool tern_rows_better(int64_t M, int64_t K, int64_t batch) {
+    return rows_sizes(M, K, batch) && K % 4 == 0 && M * (K / 4) >= 8 &&
+           K * std::max(1.0, (double)M * batch / 8000.0) > 4000.0;
+}
+
+hipError_t launch_oil8_rows(const uint8_t* idx, const float* cb, const float* x, float* y, int64_t M, int64_t K,
+                            int64_t batch, void* ws, hipStream_t s) {
+    RowsArgs a{idx, cb, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, 0};
+    return rows_run<kOil8>(a, rows_plan(M, K, batch), ws, s);
+}
+hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
+                            int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s) {
+    RowsArgs a{nib, cbs, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, (int)cb_block};
+    return rows_run<kOil4>(a, rows_plan(M, K, batch), ws, s);
+}
+hipError_t launch_tern_rows(const uint8_t* w, const float* x, float* out, int64_t M, int64_t K, int64_t batch,
+                            void* ws, hipStream_t s) {
+    RowsArgs a{w, nullptr, nullptr, nullptr, x, out, nullptr, (int)M, (int)K, (int)batch, 0, 0};
+    return rows_run<kTern>(a, rows_plan(M, K, batch), ws, s);
+}
+
+}  // namespace mth

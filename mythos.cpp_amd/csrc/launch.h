@@ -216,6 +216,24 @@ size_t oil8_gemm_x32_workspace_bytes(int64_t Mr, int64_t K);
 hipError_t launch_oil8_gemm_x32(const float* a, const Oil8Seg* seg, int nseg, int64_t Mr, int64_t K, void* ws,
                                 hipStream_t s);
 
+// ---- token rows of any count on MFMA (gemm_rows.hip) -----------------------------
+// y [batch][M] (ternary: out [M][batch]) for any M and batch; OIL8 rows of a multiple of 16, OIL4 rows and codebook
+// blocks of a multiple of 32 (16-byte aligned weights), ternary rows of a multiple of 4 (any alignment).
+// ws: rows_mfma_workspace_bytes.
+size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch);
+// Whether this route is the faster one (and takes the call): against the prompt GEMM (gemm), the batched GEMV (bt) or
+// the kernels that walk the tokens (x aligned to 16 bytes: aligned).
+bool oil8_rows_better(const uint8_t* idx, int64_t M, int64_t K, int64_t batch, bool aligned, bool gemm, bool bt);
+bool oil4_rows_better(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, int64_t M, int64_t K, int64_t batch,
+                      bool aligned, bool gemm, bool bt);
+bool tern_rows_better(int64_t M, int64_t K, int64_t batch);
+hipError_t launch_oil8_rows(const uint8_t* idx, const float* cb, const float* x, float* y, int64_t M, int64_t K,
+                            int64_t batch, void* ws, hipStream_t s);
+hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
+                            int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s);
+hipError_t launch_tern_rows(const uint8_t* w, const float* x, float* out, int64_t M, int64_t K, int64_t batch,
+                            void* ws, hipStream_t s);
+
 // ---- FP32 decode-step operators (dense.hip) ---------------------------------
 // x <- t + x (when t), then y = rms_norm(x) * gamma per row of dim.
 hipError_t launch_rms_norm(float* x, const float* t, const float* gamma, float* y, int64_t rows, int64_t dim,

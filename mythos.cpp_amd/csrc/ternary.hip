@@ -950,19 +950,6 @@ __device__ __forceinline__ uint32_t byte_t4x4(uint32_t a, uint32_t b, uint32_t c
            (((d >> (8 * s)) & 0xffu) << 24);
 }
 
-// Codes of rows that are not whole aligned 16-byte pieces (K % 64 != 0, or K % 256 != 0 where a step of 256
-// columns runs past the row): 8 bytes at byte pos of a matrix of `end` >= 8 bytes.  Bytes past the row are the
-// next row's (or, past the matrix, zeros): the activations there are zeros (the padded rows of
-// i2s_quant_rows_k / i2s_pad_rows_k), so their codes add nothing.
-__device__ __forceinline__ uint2 ld_codes8(const uint8_t* w, int64_t pos, int64_t end) {
-    const int64_t p = min(pos, end - 8);
-    uint64_t v;
-    __builtin_memcpy(&v, w + p, 8);
-    const int64_t past = pos - p;  // bytes of the piece that lie before pos
-    v = past >= 8 ? 0ull : v >> (8 * past);
-    return make_uint2((uint32_t)v, (uint32_t)(v >> 32));
-}
-
 // quantize_per_token of FP32 rows (src/int8_quant.cpp:8-31) into rows of Kp >= K bytes, zeros past K: the
 // operand of the batched kernels and the GEMM, which then need no bounds of their own.  One workgroup of 16
 // waves per row, the row read once (16384 columns in registers; longer rows read the rest twice).  VEC: 16-byte
@@ -1041,7 +1028,7 @@ constexpr int kIbFaMx = 4, kIbFaChunks = 4;  // FA: block maxima per thread, chu
 // sc is derived from the block maxima mxv (loaded at the kernel's start)
 // after the weights are issued.
 template <int NC, bool FA = false, bool TAIL = false>
-__device__ __forceinline__ void ib_round(const uint8_t* wrow, int64_t wend, const int8_t* arow, bool sv, bool stager, int c0,
+__device__ __forceinline__ void ib_round(const uint8_t* wrow, int64_t wend, bool edge, const int8_t* arow, bool sv, bool stager, int c0,
                                          bool first, uint32_t (*qs)[kIbTok * kIbTokStride], int st, int sg, int r,
                                          int g, int& asum, i32x4& acc, const float* arowf = nullptr,
                                          float* sc = nullptr, const float* mxv = nullptr,
@@ -1067,7 +1054,7 @@ __device__ __forceinline__ void ib_round(const uint8_t* wrow, int64_t wend, cons
         const int64_t o = (int64_t)(c0 + c) * 64;
         if constexpr (TAIL) {
             const uint2 lo = ld_codes8(wrow, o, wend), hi = ld_codes8(wrow, o + 8, wend);
-            wv[c] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            wv[c] = make_uint4(lo.x, lo.y, hi.x, hi.y);  // (codes8_at below)
         } else {
             wv[c] = ld_stream(wrow + o);
         }
@@ -1121,6 +1108,14 @@ __device__ __forceinline__ void ib_round(const uint8_t* wrow, int64_t wend, cons
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
+        if constexpr (TAIL) {
+            if (edge) {
+                const int64_t o = (int64_t)(c0 + c) * 64;
+                const uint2 lo = codes8_at(make_uint2(wv[c].x, wv[c].y), o, wend);
+                const uint2 hi = codes8_at(make_uint2(wv[c].z, wv[c].w), o + 8, wend);
+                wv[c] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            }
+        }
         const uint32_t wd[4] = {wv[c].x, wv[c].y, wv[c].z, wv[c].w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1154,6 +1149,7 @@ __global__ __launch_bounds__(WV * 64) void i2s_gemv_bt(const uint8_t* packed, fl
     const int bpr = K / 4;
     const uint8_t* wrow = packed + (int64_t)min(m0 + r, M - 1) * bpr + 16 * g;  // clamped rows
     const int64_t wend = (int64_t)M * bpr - (wrow - packed);                    // bytes from wrow to the end
+    const bool edge = blockIdx.x == gridDim.x - 1;  // a tile with the matrix's last row
     // staging by the first 4 waves: thread = token st, 16-column group sg
     const int st = (tid >> 4) & 15, sg = tid & 15;
     const bool stager = __builtin_amdgcn_readfirstlane(wave) < 4;
@@ -1173,14 +1169,14 @@ __global__ __launch_bounds__(WV * 64) void i2s_gemv_bt(const uint8_t* packed, fl
         const int nc = min(MAXC, sc1 - c0);
         const bool first = c0 == sc0;
         switch (nc) {
-            case 1: ib_round<1, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 2: ib_round<2, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 3: ib_round<3, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 4: ib_round<4, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 5: ib_round<5 <= MAXC ? 5 : 1, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 6: ib_round<6 <= MAXC ? 6 : 1, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            case 7: ib_round<7 <= MAXC ? 7 : 1, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
-            default: ib_round<MAXC, FA, TAIL>(wrow, wend, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 1: ib_round<1, FA, TAIL>(wrow, wend, edge, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 2: ib_round<2, FA, TAIL>(wrow, wend, edge, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 3: ib_round<3, FA, TAIL>(wrow, wend, edge, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 4: ib_round<4, FA, TAIL>(wrow, wend, edge, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 5: ib_round<5 <= MAXC ? 5 : 1, FA, TAIL>(wrow, wend, edge, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 6: ib_round<6 <= MAXC ? 6 : 1, FA, TAIL>(wrow, wend, edge, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            case 7: ib_round<7 <= MAXC ? 7 : 1, FA, TAIL>(wrow, wend, edge, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
+            default: ib_round<MAXC, FA, TAIL>(wrow, wend, edge, arow, sv, stager, c0, first, qs, st, sg, r, g, asum, acc, arowf, &sc, mxv, &fa, tinv); break;
         }
     }
     if (stager) asum_p[st][sg] = asum;
@@ -1300,6 +1296,7 @@ __global__ __launch_bounds__(TGT) void i2s_gemm_mfma(const uint8_t* w, const int
     const int st0 = ROWS ? (int)((int64_t)blockIdx.y * all / gridDim.y) : 0;
     const int steps = (ROWS ? (int)((int64_t)(blockIdx.y + 1) * all / gridDim.y) : all) - st0;
     const uint32_t wtotal = (uint32_t)M * (uint32_t)bpr;
+    const bool edge = TAIL && m0 + TGM >= M;  // a tile with the matrix's last row
 
     // ---- codes: lane (r16, g), row tile i: row m0 + 32 wr + 16 i + r16, code dwords 4g + 2wk and 4g + 2wk + 1
     // of the step (16 columns each): the planes of dword 4g + c are the lane's A fragment of chunk c, so chunk
@@ -1376,7 +1373,9 @@ __global__ __launch_bounds__(TGT) void i2s_gemm_mfma(const uint8_t* w, const int
             i32x4 af[2][2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const uint2 q = cw[u][i];
+                const uint2 q = TAIL && edge ? codes8_at(cw[u][i], (int64_t)(st0 + min(step, steps - 1)) * (TGK / 4) + woff[i],
+                                                         wtotal)
+                                             : cw[u][i];
                 const uint32_t d[2] = {q.x, q.y};
 #pragma unroll
                 for (int cc = 0; cc < 2; ++cc) {

@@ -138,3 +138,110 @@ def test_attention_split_specials(mth, dev):
             assert torch.isnan(got[5]) and torch.isnan(got).sum() == 1
             got[5] = want[5]
         assert ((got - want).norm() / want.norm()).item() <= 4e-6
+
+
+# ----------------------------------------------------- token rows on MFMA --
+def w64(kind, w, cb, M, K, blk, dev):
+    """[M][K] float64 weights."""
+    import torch
+    w = torch.from_numpy(w).to(dev)
+    if kind == "oil8":
+        return torch.from_numpy(cb).to(dev).double()[w.long()]
+    if kind == "oil4":
+        t = torch.from_numpy(synth.dequant_oil4(w.cpu().numpy(), cb, M, K, blk)).to(dev)
+        return t.double()
+    return torch.from_numpy(synth.dequant_ternary(w.cpu().numpy(), M, K, 1.0)).to(dev).double()
+
+
+def rows_inputs(kind, M, K, blk, g):
+    if kind == "oil8":
+        return g.integers(0, 256, (M, K), dtype=np.uint8), np.sort(g.normal(0, 0.02, 256)).astype(np.float32)
+    if kind == "oil4":
+        n = M * (K // blk) if blk else 1
+        return g.integers(0, 256, (M, K // 2), dtype=np.uint8), g.normal(0, 0.02, n * 16).astype(np.float16).view(np.uint16)
+    return g.integers(0, 256, (M, K // 4), dtype=np.uint8), None
+
+
+def rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev, shift=0):
+    import torch
+    y = empty(batch * M, torch.float32, dev)
+    xd = offset(to_dev(x, dev), shift)
+    if kind == "oil8":
+        mth.oil8_gemv(to_dev(w, dev), to_dev(cb, dev), xd, y, M, K, batch)
+    elif kind == "oil4":
+        mth.oil4_gemv(to_dev(w, dev), to_dev(cb, dev), blk, xd, y, M, K, batch)
+    else:
+        mth.i2s_gemm(offset(to_dev(w, dev), shift), xd, y, M, batch, K)
+    torch.cuda.synchronize()
+    return y.reshape(batch, M) if kind != "tern" else y.reshape(M, batch).T.contiguous()
+
+
+@pytest.mark.parametrize("kind,M,K,batch,blk,shift", [
+    ("oil8", 1, 4112, 1, 0, 0),          # one token, a row longer than the one-token kernel takes; 1 row
+    ("oil8", 129, 2064, 17, 0, 0),       # 2 row tiles, 16.1 steps: a last step of one 16-byte piece
+    ("oil8", 4000, 4096, 48, 0, 0),      # 3 token groups, K split 8 ways
+    ("oil8", 127, 1280, 65, 0, 0),       # 2 token tiles of 48
+    ("oil8", 300, 528, 40, 0, 4),        # x not 16-byte aligned
+    ("oil8", 640, 17024, 20, 0, 0),      # rows longer than the conversion keeps in registers
+    ("oil4", 100, 5120, 1, 64, 0),       # one token, codebooks per 64
+    ("oil4", 130, 1120, 33, 32, 0),      # codebooks per 32, a last step of 96 columns
+    ("oil4", 257, 3968, 64, 128, 0),
+    ("oil4", 255, 9088, 18, 0, 0),       # one codebook per tensor, two steps past 8192
+    ("oil4", 64, 640, 200, 64, 8),
+    ("tern", 33, 4100, 1, 0, 0),         # rows of 1025 code bytes
+    ("tern", 129, 1028, 40, 0, 0),
+    ("tern", 4096, 512, 300, 0, 0),
+    ("tern", 200, 2052, 64, 0, 4),
+])
+def test_token_rows(kind, M, K, batch, blk, shift, mth, dev):
+    """Token rows of magnitudes 2^-40 .. 2^40 and an all-zero row against
+    float64.  Bound: FP32 sums of K products in chunks of 32, so 1e-5 of
+    sum |w x| per element and 1e-6 of the row's norm."""
+    import torch
+    print(f"token rows {kind} M={M} K={K} batch={batch} blk={blk} shift={shift}", flush=True)
+    g = np.random.default_rng(M + K + batch)
+    w, cb = rows_inputs(kind, M, K, blk, g)
+    x = (g.normal(0, 1, (batch, K)) * np.exp2(g.integers(-40, 40, batch))[:, None]).astype(np.float32)
+    if batch > 2:
+        x[batch // 2] = 0.0
+    got = rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev, shift).double()
+    W, X = w64(kind, w, cb, M, K, blk, dev), torch.from_numpy(x).to(dev).double()
+    want, absw = X @ W.T.contiguous(), X.abs() @ W.abs().T.contiguous()
+    assert bool(((got - want).abs() <= 1e-5 * absw + 1e-30).all())
+    nrm = want.norm(dim=1)
+    assert bool(((got - want).norm(dim=1) <= 1e-6 * nrm + 1e-30).all())
+
+
+@pytest.mark.parametrize("kind", ["oil8", "oil4", "tern"])
+@pytest.mark.parametrize("what", ["x_inf", "x_nan", "codebook_inf"])
+def test_token_rows_non_finite(kind, what, mth, dev):
+    """Inf and NaN reach the outputs the reference's products give them: a
+    token's non-finite value its own outputs only, an infinite codebook entry
+    the rows that use it; a ternary weight of 0 skips its activation."""
+    import torch
+    if kind == "tern" and what == "codebook_inf":
+        pytest.skip("ternary weights have no codebook")
+    M, K, batch, blk = 300, 4096, 40, 128
+    g = np.random.default_rng(11)
+    w, cb = rows_inputs(kind, M, K, blk, g)
+    x = g.normal(0, 1, (batch, K)).astype(np.float32)
+    if what == "codebook_inf":
+        if kind == "oil8":
+            cb[7] = np.inf
+            w[w == 7] = 8
+            w[5, 100] = 7
+        else:
+            cb.reshape(M, K // blk, 16)[5, 3, 9] = 0x7C00
+    else:
+        x[3, 77] = np.inf if what == "x_inf" else np.nan
+    got = rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev).cpu().numpy()
+    W = w64(kind, w, cb, M, K, blk, dev).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        prod = x[:, None, :].astype(np.float64) * W[None] if kind != "tern" else np.where(
+            W[None] == 0, 0.0, x[:, None, :].astype(np.float64) * W[None])
+        want = prod.sum(-1)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf])
+    fin = np.isfinite(want)
+    assert np.abs(got[fin] - want[fin]).max() <= 1e-5 * np.abs(prod).sum(-1)[fin].max()
