@@ -192,8 +192,9 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
     const mth::Oil8Seg seg{indices, codebook, y, M};
     const bool gemm = aligned && batch >= kGemmRows && mth::oil8_gemm_x32_supported(&seg, 1, batch, K);
     const bool bt = aligned && mth::oil8_bt_supported(M, K, batch);
-    const bool walk = batch == 1 && aligned && K % 16 == 0 && K <= 4096 && M * K < (1ll << 32);
-    if (!walk && mth::oil8_rows_better(indices, M, K, batch, aligned, gemm, bt)) {
+    const bool one = batch == 1 && aligned &&  // one token: kernels of their own up to 16384 columns
+                     ((K % 16 == 0 && K <= 4096 && M * K < (1ll << 32)) || mth::oil8_long_supported(indices, x, M, K));
+    if (!one && mth::oil8_rows_better(indices, M, K, batch, aligned, gemm, bt)) {
         if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch)))
             return check_launch(mth::launch_oil8_rows(indices, codebook, x, y, M, K, batch, ws, S(stream)),
                                 "mth_oil8_gemv");
@@ -238,7 +239,8 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
     const bool gemm = aligned && ((uintptr_t)y & 15u) == 0 && batch >= kGemmRows &&
                       mth::oil4_gemm_x32_supported(batch, M, K, cb_block);
     const bool bt = aligned && mth::oil4_bt_supported(M, K, cb_block, batch);
-    const bool one = batch == 1 && aligned && K <= 4096;  // one token: its own kernels up to 4096 columns
+    const bool one = batch == 1 && aligned &&  // one token: kernels of their own
+                     (K <= 4096 || mth::oil4_one_supported(packed, codebooks, x, cb_block, M, K));
     if (!one && mth::oil4_rows_better(packed, codebooks, cb_block, M, K, batch, aligned, gemm, bt)) {
         if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch)))
             return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, ws, S(stream)),

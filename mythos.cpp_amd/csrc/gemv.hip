@@ -156,6 +156,63 @@ void oil8_gemv_k(Oil8SegArgs sg, const float* x, int K, int batch, ResidOut ro) 
     }
 }
 
+// One token, rows of more than 4096 (oil8_gemv_long): oil8_gemv_k with NSEG 16-byte pieces per lane and row, piece
+// 256 s + tid, every load of the workgroup's R rows in flight at once (at NSEG = 3 44 KB of indices and as much of x
+// per workgroup; 4 workgroups per CU).  Pieces past the row (clamped loads) are left out of the sums.  4096 x 11008:
+// one wave per output with byte loads 81.6 us, K slices on MFMA with a reduction 22 us, this kernel 11.4 us (4.0 TB/s).
+template <int R, int NSEG>
+__global__ __launch_bounds__(kWG, NSEG <= 3 ? 4 : 3) void oil8_gemv_long(const uint8_t* idx, const float* __restrict__ cb,
+                                                                         const float* x, float* __restrict__ y, int M,
+                                                                         int K) {
+    __shared__ float tab[256];
+    __shared__ float part[kWaves][R];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m0 = blockIdx.x * R;
+    float4 xq[NSEG][4];
+    const float cbv = cb[tid];
+#pragma unroll
+    for (int s = 0; s < NSEG; ++s)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xq[s][q] = ldf4(x + min((s * kWG + tid) * 16, K - 16) + 4 * q);
+    __builtin_amdgcn_sched_barrier(0);
+    uint4 w[NSEG][R];
+#pragma unroll
+    for (int s = 0; s < NSEG; ++s)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            w[s][r] = ld_stream(idx + ((uint32_t)min(m0 + r, M - 1) * (uint32_t)K + (uint32_t)min((s * kWG + tid) * 16, K - 16)));
+    __builtin_amdgcn_sched_barrier(0);
+    tab[tid] = cbv;
+    __syncthreads();
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < NSEG; ++s) {
+        const bool in = (s * kWG + tid) * 16 < K;
+        float xr[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            xr[4 * q] = xq[s][q].x, xr[4 * q + 1] = xq[s][q].y, xr[4 * q + 2] = xq[s][q].z, xr[4 * q + 3] = xq[s][q].w;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float a = 0.0f;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const uint32_t wd = u4get(w[s][r], d);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) a = fmaf(tab[(wd >> (8 * b)) & 0xffu], xr[4 * d + b], a);
+            }
+            acc[r] += in ? a : 0.0f;
+        }
+    }
+    const float s = transposed_sum<R>(acc, lane);
+    constexpr int L = MTH_WAVE / R;
+    if ((lane % L) == 0) part[wave][lane / L] = s;
+    __syncthreads();
+    if (tid < R && m0 + tid < M) y[m0 + tid] = ((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid];
+}
+
 // Generic: one wave per output element.  Row r uses weights idx + r*K and
 // activation row (r % xmod) + t; out[t*ldy + r].
 __global__ __launch_bounds__(kWG) void oil8_generic(
@@ -392,7 +449,11 @@ struct SwigluTile {
     int F;
 };
 
-template <int NW, int NPH, bool SHARED, bool PAIR = false>
+// TAIL: NW NPH 256 > K (any K % 128 == 0): loads past the row are clamped into it, x is 0 there and so are the weights
+// (their codebook's byte planes: an infinite entry must not meet a zero).  Rows of more than 4096 run on up to 16
+// waves of 2 or 4 phases: 5000 x 8192 (one wave per output before) 80 -> 11.7 us, 5000 x 9088 89 -> 17.4 us; 16384 x
+// 3968 (vector-ALU kernel before) 19.8 -> 12.3 us.
+template <int NW, int NPH, bool SHARED, bool PAIR = false, bool TAIL = false>
 __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2(const uint8_t* nib, const uint16_t* cbs,
                                                         const float* __restrict__ x, float* __restrict__ y,
                                                         int M, int K, SwigluTile sw = SwigluTile{}) {
@@ -422,12 +483,12 @@ __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2
     }
     float4 xq[2 * XS];
 #pragma unroll
-    for (int i = 0; i < 2 * XS; ++i) xq[i] = ldf4(x + k0 + lane * 8 * XS + 4 * i);
+    for (int i = 0; i < 2 * XS; ++i) xq[i] = ldf4(x + (TAIL ? min(k0 + lane * 8 * XS + 4 * i, K - 4) : k0 + lane * 8 * XS + 4 * i));
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
 
-    Oil4TileLoads<NPH, SHARED> w;
+    Oil4TileLoads<NPH, SHARED, TAIL> w;
     const int rowA = PAIR ? blockIdx.x * 8 : row0, rowB = PAIR ? sw.F + blockIdx.x * 8 : row0 + 8;
     // Phase 0's weights (and its phase pair's codebooks) now, the other phases' after the x conversion: a CU
     // returns loads in issue order, so the phase-0 data of every workgroup on the CU comes back before any
@@ -461,6 +522,7 @@ __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2
 #pragma unroll
     for (int i = 0; i < 2 * XS; ++i) {
         xv[4 * i] = xq[i].x, xv[4 * i + 1] = xq[i].y, xv[4 * i + 2] = xq[i].z, xv[4 * i + 3] = xq[i].w;
+        if (TAIL && k0 + lane * 8 * XS + 4 * i >= K) xv[4 * i] = xv[4 * i + 1] = xv[4 * i + 2] = xv[4 * i + 3] = 0.0f;
     }
     uint32_t mb = 0, mn = 0xffffffffu;  // max |x| bits; min nonzero |x| bits - 1 (0 -> all ones)
 #pragma unroll
@@ -515,7 +577,11 @@ __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2
     half8 bnext = bfrag(0);
 #pragma unroll
     for (int p = 0; p < NPH; ++p) {
-        const CbPlanes pl = SHARED ? shared_planes : w.planes(p, wl + L::bwave, lane);
+        CbPlanes pl = SHARED ? shared_planes : w.planes(p, wl + L::bwave, lane);
+        if (TAIL && k0 + 256 * p + 64 * q >= K) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pl.l[i] = pl.h[i] = 0;
+        }
         uint4 xa, yb;
         w.exchange(p, lane, xa, yb);
 #pragma unroll
@@ -544,6 +610,7 @@ __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2
 #pragma unroll
             for (int h = 0; h < XS; ++h) {
                 const int c0 = k0 + 8 * (XS * lane + h);
+                if (TAIL && c0 >= K) continue;
                 const uint32_t d = *(const uint32_t*)(nib + (int64_t)row * (K >> 1) + (c0 >> 1));
                 const uint16_t* cb = SHARED ? cbs : cbs + ((int64_t)row * nbr + (c0 >> 7)) * 16;
                 const half8 wv = lookup8(d, cb_planes(ld16(cb), ld16(cb + 8)));
@@ -762,6 +829,33 @@ bool run_oil4_v2(const uint8_t* nib, const uint16_t* cbs, const float* x, float*
         default: return false;
     }
 }
+// oil4_gemv_v2 with TAIL for any K % 128 == 0 up to 16384: waves of 2 phases up to 8192, of 4 above
+template <bool SHARED>
+bool run_oil4_tail(const uint8_t* nib, const uint16_t* cbs, const float* x, float* y, int64_t M, int64_t K,
+                   hipStream_t s) {
+    const int grid = ceil_div(M, 16);
+    const int m = (int)M, k = (int)K;
+    const bool p4 = K > 8192;
+    switch ((K + (p4 ? 1023 : 511)) / (p4 ? 1024 : 512)) {
+#define MTH_T_CASE(NW, NPH)                                                                                \
+    case NW:                                                                                               \
+        oil4_gemv_v2<NW, NPH, SHARED, false, true><<<grid, NW * 64, 0, s>>>(nib, cbs, x, y, m, k);          \
+        return true;
+#define MTH_T_CASE2(NW)                                                                                    \
+    case NW:                                                                                               \
+        if (p4)                                                                                            \
+            oil4_gemv_v2<NW, 4, SHARED, false, true><<<grid, NW * 64, 0, s>>>(nib, cbs, x, y, m, k);        \
+        else                                                                                               \
+            oil4_gemv_v2<NW, 2, SHARED, false, true><<<grid, NW * 64, 0, s>>>(nib, cbs, x, y, m, k);        \
+        return true;
+        MTH_T_CASE(1, 2) MTH_T_CASE(2, 2) MTH_T_CASE(3, 2) MTH_T_CASE(4, 2) MTH_T_CASE(5, 2) MTH_T_CASE(6, 2)
+        MTH_T_CASE(7, 2) MTH_T_CASE(8, 2) MTH_T_CASE2(9) MTH_T_CASE2(10) MTH_T_CASE2(11) MTH_T_CASE2(12)
+        MTH_T_CASE2(13) MTH_T_CASE2(14) MTH_T_CASE2(15) MTH_T_CASE2(16)
+#undef MTH_T_CASE
+#undef MTH_T_CASE2
+        default: return false;
+    }
+}
 template <int NW, int NC>
 void run_oil4_mfma(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y, int64_t M,
                    int64_t K, hipStream_t s) {
@@ -805,12 +899,23 @@ hipError_t launch_oil4_swiglu(const uint8_t* nib, const uint16_t* cbs, const flo
     return hipGetLastError();
 }
 
+// one token, rows of 4096 .. 16384 (oil8_gemv_long); 32-bit byte offsets into the indices
+bool oil8_long_supported(const uint8_t* idx, const float* x, int64_t M, int64_t K) {
+    return K % 16 == 0 && K > 4096 && K <= 16384 && M * K < (1ll << 32) && aligned16(idx) && aligned16(x);
+}
+
 hipError_t launch_oil8_gemv(const uint8_t* idx, const float* cb, const float* x, float* y,
                             int64_t M, int64_t K, int64_t batch, hipStream_t s) {
     const bool fast = (K % 16 == 0) && K <= 4096 && M * K < (1ll << 32) && aligned16(idx) && aligned16(x);
     if (fast) {
         const Oil8Seg seg{idx, cb, y, M};
         return launch_oil8_gemv_segs(&seg, 1, x, K, batch, s);
+    } else if (batch == 1 && oil8_long_supported(idx, x, M, K)) {
+        constexpr int R = 4;
+        const int grid = ceil_div(M, R);
+        if (K <= 8192) oil8_gemv_long<R, 2><<<grid, kWG, 0, s>>>(idx, cb, x, y, (int)M, (int)K);
+        else if (K <= 12288) oil8_gemv_long<R, 3><<<grid, kWG, 0, s>>>(idx, cb, x, y, (int)M, (int)K);
+        else oil8_gemv_long<R, 4><<<grid, kWG, 0, s>>>(idx, cb, x, y, (int)M, (int)K);
     } else {
         oil8_generic<<<ceil_div(M, kWaves), kWG, 0, s>>>(idx, cb, x, y, M, K, 1, batch, M);
     }
@@ -855,6 +960,13 @@ hipError_t launch_oil8_gemm_mn(const uint8_t* idx, const float* cb, const float*
     return hipGetLastError();
 }
 
+// one token on oil4_gemv_v2 (whole codebook blocks of 128 or one per tensor; 32-bit byte offsets)
+bool oil4_one_supported(const uint8_t* nib, const uint16_t* cbs, const float* x, int64_t cb_block, int64_t M,
+                        int64_t K) {
+    return (cb_block == 0 || cb_block == 128) && K % 128 == 0 && K >= 512 && K <= 16384 && M < (1ll << 31) &&
+           M * (K / 2) < (1ll << 32) && aligned16(nib) && aligned16(cbs) && aligned16(x);
+}
+
 hipError_t launch_oil4_gemv(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block,
                             const float* x, float* y, int64_t M, int64_t K, int64_t batch,
                             hipStream_t s) {
@@ -869,6 +981,10 @@ hipError_t launch_oil4_gemv(const uint8_t* nib, const uint16_t* cbs, int64_t cb_
             done = cb_block == 0 ? run_oil4_v2<2, true>(nib, cbs, x, y, M, K, s)
                                  : run_oil4_v2<2, false>(nib, cbs, x, y, M, K, s);
         if (done) return hipGetLastError();
+    }
+    if (batch == 1 && oil4_one_supported(nib, cbs, x, cb_block, M, K)) {
+        if (cb_block == 0 ? run_oil4_tail<true>(nib, cbs, x, y, M, K, s) : run_oil4_tail<false>(nib, cbs, x, y, M, K, s))
+            return hipGetLastError();
     }
     const bool mfma = batch == 1 && aligned && M < (1ll << 31) && (cb_block == 0 || cb_block % 128 == 0) &&
                       (K == 512 || K == 1024 || K == 2048 || K == 4096);

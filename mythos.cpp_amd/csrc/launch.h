@@ -20,6 +20,11 @@ int api_ok();
 // y[t*M + m] = sum_k cb[idx[m*K + k]] * x[t*K + k]          (t < batch)
 hipError_t launch_oil8_gemv(const uint8_t* idx, const float* cb, const float* x, float* y,
                             int64_t M, int64_t K, int64_t batch, hipStream_t s);
+// One token, rows of 4096 .. 16384 on a kernel of their own (launch_oil8_gemv takes it).
+bool oil8_long_supported(const uint8_t* idx, const float* x, int64_t M, int64_t K);
+// One token on the OIL4 kernel of whole rows (K % 128 == 0, 512 .. 16384; launch_oil4_gemv takes it).
+bool oil4_one_supported(const uint8_t* nib, const uint16_t* cbs, const float* x, int64_t cb_block, int64_t M,
+                        int64_t K);
 // Up to three OIL8 matrices with the same K and input, each with its own
 // codebook and output (the Q, K and V projections), in one launch:
 // seg[i].y[t*rows + m] = sum_k seg[i].cb[seg[i].idx[m*K + k]] * x[t*K + k].

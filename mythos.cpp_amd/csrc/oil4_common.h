@@ -185,7 +185,8 @@ __device__ __forceinline__ int oil4_stage_off(int r, int c) {
 
 // All weight loads of one wave for a 16-row tile and NPH phases of 256
 // columns starting at column k0, issued in consumption order.
-template <int NPH, bool SHARED>
+// TAIL: columns past the row (K) read its last 16 bytes (the caller gives them no weight).
+template <int NPH, bool SHARED, bool TAIL = false>
 struct Oil4TileLoads {
     static_assert(SHARED || NPH % 2 == 0, "codebooks load per phase pair");
     uint4 wx[NPH], wy[NPH], c0[NPH / 2 + 1], c1[NPH / 2 + 1];
@@ -218,12 +219,23 @@ struct Oil4TileLoads {
         const uint8_t* cb8 = (const uint8_t*)cbs;
 #pragma unroll
         for (int p = P0; p < P1; ++p) {
-            if (!SHARED && p % 2 == 0) {
-                c0[p / 2] = ld16(cb8 + oc0 + (p / 2) * 128);
-                c1[p / 2] = ld16(cb8 + oc1 + (p / 2) * 128);
+            if constexpr (TAIL) {
+                const uint32_t wb = min(col + 128 * p, hb - 16);
+                if (!SHARED && p % 2 == 0) {
+                    const uint32_t cbp = min(cpiece + (p / 2) * 128, nbr * 32 - 16);
+                    c0[p / 2] = ld16(cb8 + (oc0 - cpiece + cbp));
+                    c1[p / 2] = ld16(cb8 + (oc1 - cpiece + cbp));
+                }
+                wx[p] = ld_stream(nib + (ox - col + wb));
+                wy[p] = ld_stream(nib + (oy - col + wb));
+            } else {
+                if (!SHARED && p % 2 == 0) {
+                    c0[p / 2] = ld16(cb8 + oc0 + (p / 2) * 128);
+                    c1[p / 2] = ld16(cb8 + oc1 + (p / 2) * 128);
+                }
+                wx[p] = ld_stream(nib + ox + 128 * p);
+                wy[p] = ld_stream(nib + oy + 128 * p);
             }
-            wx[p] = ld_stream(nib + ox + 128 * p);
-            wy[p] = ld_stream(nib + oy + 128 * p);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
