@@ -302,6 +302,9 @@ hipError_t launch_rope_attention_slices(const Slices& q, const Slices& k, const 
 hipError_t launch_attention_rows(const float* q, const void* kc, const void* vc, bool kv_bf16, float* out,
                                  int64_t rows, int np, int p0, int heads, int kv_heads, int head_dim, int max_seq,
                                  hipStream_t s);
+// The tiled form of it (attn_prefill.hip): head_dim 64 or 128, rows % np == 0, 16-byte aligned arrays.
+hipError_t launch_attn_prefill(const float* q, const void* kc, const void* vc, bool kv_bf16, float* out, int64_t rows,
+                               int np, int p0, int heads, int kv_heads, int head_dim, int max_seq, hipStream_t s);
 // RoPE of each row's q (in place) and k; k, v appended to the caches.
 hipError_t launch_rope_kv_rows(float* q, const float* k, const float* v, const float* cos_t, const float* sin_t,
                                void* kc, void* vc, bool kv_bf16, int64_t rows, int np, int p0, int heads, int kv_heads,
