@@ -830,28 +830,30 @@ __global__ __launch_bounds__(kT) void argmax_part_k(const float* __restrict__ lo
     }
 }
 
-// Stage 2 (one workgroup): row b's result from its nc partials -> ids[b];
-// with hist, the next input token hist[b][s + 1] once the prompt is consumed
-// (s + 1 >= prompt_len); with step, then advances *step (the last launch of a
-// decode step: every earlier kernel of the step has read it).
-__global__ __launch_bounds__(kT) void argmax_final_k(const float* __restrict__ pv, const int* __restrict__ pi, int nc,
-                                                     int rows, int* __restrict__ ids, int* __restrict__ hist,
-                                                     int* step, int hist_stride, int prompt_len) {
-    __shared__ float bv[kT / 64];
-    __shared__ int bi[kT / 64];
-    const int s = step ? *step : 0;
-    for (int b = 0; b < rows; ++b) {
+// Stage 2: row b's result from its nc partials -> ids[b]; with hist, the next
+// input token hist[b][s + 1] once the prompt is consumed (s + 1 >= prompt_len);
+// with step (one workgroup), then advances *step (the last launch of a decode
+// step: every earlier kernel of the step has read it).  A wave per row: the
+// rows' loads are in flight together (16 rows of 16 partials, one workgroup
+// walking them 18.2 us, here 4.0).
+constexpr int kAfT = 1024;
+__global__ __launch_bounds__(kAfT) void argmax_final_k(const float* __restrict__ pv, const int* __restrict__ pi, int nc,
+                                                       int rows, int* __restrict__ ids, int* __restrict__ hist,
+                                                       int* step, int hist_stride, int prompt_len) {
+    const int s = step ? *step : 0, lane = threadIdx.x & 63;
+    for (int b = blockIdx.x * (kAfT / 64) + (threadIdx.x >> 6); b < rows; b += gridDim.x * (kAfT / 64)) {
         float v = -INFINITY;
         int idx = 0x7fffffff;
-        for (int c = threadIdx.x; c < nc; c += kT) amax_merge(v, idx, pv[b * nc + c], pi[b * nc + c]);
-        block_amax(v, idx, bv, bi);
-        if (threadIdx.x == 0) {
+        for (int c = lane; c < nc; c += 64) amax_merge(v, idx, pv[(int64_t)b * nc + c], pi[(int64_t)b * nc + c]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) amax_merge(v, idx, __shfl_xor(v, o, MTH_WAVE), __shfl_xor(idx, o, MTH_WAVE));
+        if (lane == 0) {
             const int best = idx == 0x7fffffff ? 0 : idx;
             if (ids) ids[b] = best;
             if (hist && s + 1 >= prompt_len && s + 1 < hist_stride) hist[(int64_t)b * hist_stride + s + 1] = best;
         }
-        __syncthreads();
     }
+    __syncthreads();  // every wave has read *step
     if (step && threadIdx.x == 0) *step = s + 1;
 }
 
@@ -1164,7 +1166,8 @@ hipError_t launch_argmax(const float* logits, int64_t rows, int64_t n, int* ids,
                          int hist_stride, int prompt_len, float* pv, int* pi, hipStream_t s) {
     const int nc = argmax_chunks(n);
     argmax_part_k<<<dim3((unsigned)nc, (unsigned)rows), kT, 0, s>>>(logits, n, kArgChunk, pv, pi);
-    argmax_final_k<<<1, kT, 0, s>>>(pv, pi, nc, (int)rows, ids, hist, step, hist_stride, prompt_len);
+    const int grid = step ? 1 : (int)((rows + kAfT / 64 - 1) / (kAfT / 64));
+    argmax_final_k<<<grid, kAfT, 0, s>>>(pv, pi, nc, (int)rows, ids, hist, step, hist_stride, prompt_len);
     return hipGetLastError();
 }
 

@@ -255,3 +255,20 @@ def test_token_rows_non_finite(kind, M, K, batch, what, mth, dev):
     fin = np.isfinite(want)
     if fin.any():
         assert np.abs(got[fin] - want[fin]).max() <= 1e-5 * np.abs(prod).sum(-1)[fin].max()
+
+
+# ----------------------------------------------------------------- argmax --
+@pytest.mark.parametrize("rows,n", [(15, 2048), (16, 2049), (17, 5000), (33, 140001)])
+def test_argmax_rows(rows, n, oracle, mth, dev):
+    """A wave per row: one short of, exactly and one past a workgroup's 16 rows, and more partials than lanes."""
+    import torch
+    print(f"argmax rows={rows} n={n}", flush=True)
+    g = np.random.default_rng(rows)
+    x = g.integers(-50, 50, (rows, n)).astype(np.float32)   # many ties: the first index wins
+    x[1] = -np.inf
+    x[2] = np.nan
+    x[3, n - 1] = 99.0
+    ids = torch.full((rows,), -1, dtype=torch.int32, device=dev)
+    mth.argmax(to_dev(x, dev), ids, rows, n)
+    torch.cuda.synchronize()
+    assert ids.cpu().tolist() == [oracle.argmax(r) for r in x]
