@@ -194,9 +194,9 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
     const bool bt = aligned && mth::oil8_bt_supported(M, K, batch);
     const bool one = batch == 1 && aligned &&  // one token: kernels of their own up to 16384 columns
                      ((K % 16 == 0 && K <= 4096 && M * K < (1ll << 32)) || mth::oil8_long_supported(indices, x, M, K));
-    if (!one && mth::oil8_rows_better(indices, M, K, batch, aligned, gemm, bt)) {
+    if (!one && mth::oil8_rows_better(&seg, 1, K, batch, aligned, gemm, bt)) {
         if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch)))
-            return check_launch(mth::launch_oil8_rows(indices, codebook, x, y, M, K, batch, ws, S(stream)),
+            return check_launch(mth::launch_oil8_rows(&seg, 1, x, K, batch, ws, S(stream)),
                                 "mth_oil8_gemv");
     }
     if (gemm) {
@@ -469,7 +469,7 @@ int mth_silu_mul_quant(const float* g, const float* u, int8_t* q, float* inv_sca
     REQUIRE(g && u && q && inv_scale, "mth_silu_mul_quant: null pointer");
     REQUIRE(rows > 0 && rows <= 65535 && gstride >= n && ustride >= n, "mth_silu_mul_quant: bad sizes");
     REQUIRE(mth::silu_mul_quant_supported(n), "mth_silu_mul_quant: n=%lld outside 1..12288", (long long)n);
-    return check_launch(mth::launch_silu_mul_quant(g, u, q, inv_scale, nullptr, rows, n, gstride, ustride, S(stream)),
+    return check_launch(mth::launch_silu_mul_quant(g, u, q, n, inv_scale, nullptr, rows, n, gstride, ustride, S(stream)),
                         "mth_silu_mul_quant");
 }
 

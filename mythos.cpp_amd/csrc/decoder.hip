@@ -66,7 +66,12 @@ struct mth_decoder {
     float *pf_x = nullptr, *pf_h = nullptr, *pf_t = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr;
     float *pf_att = nullptr, *pf_gu = nullptr, *pf_inv = nullptr;
     int8_t* pf_aq = nullptr;
-    void* pf_ws = nullptr;  // the prefill GEMMs' scratch (A fragments, row shifts, permuted int8 activations)
+    void* pf_ws = nullptr;  // the prefill GEMMs' scratch (A fragments, row shifts, K slices' partial sums)
+    size_t pf_ws_bytes = 0;
+    // bytes per row of aq and pf_aq: ffn padded to whole 256-column chunks where the int8 MFMA kernels take the down
+    // projection (down_padded)
+    int64_t ldq = 0;
+    bool down_padded = false;
 
     void drop_graph() {
         if (exec) (void)hipGraphExecDestroy(exec);
@@ -86,9 +91,14 @@ size_t round_up(size_t n) { return (n + 255) & ~(size_t)255; }
 // y[rows][M] = W x for an OIL4 weight, picking the batched kernel when it applies.
 hipError_t oil4(const mth_decoder* d, const uint8_t* w, const uint16_t* cb, const float* x, float* y, int64_t M,
                 int64_t K, hipStream_t s, int64_t rows = 0) {
+    const bool prompt = rows > 16;
     if (!rows) rows = d->batch;
     const bool aligned = (((uintptr_t)w | (uintptr_t)cb | (uintptr_t)x) & 15u) == 0;
-    if (aligned && mth::oil4_bt_supported(M, K, d->c.cb_block, rows))
+    const bool bt = aligned && mth::oil4_bt_supported(M, K, d->c.cb_block, rows);
+    if (prompt && mth::oil4_rows_better(w, cb, d->c.cb_block, M, K, rows, aligned, false, bt) &&
+        mth::rows_mfma_workspace_bytes(M, K, rows) <= d->pf_ws_bytes)
+        return mth::launch_oil4_rows(w, cb, d->c.cb_block, x, y, M, K, rows, d->pf_ws, s);
+    if (bt)
         return mth::launch_oil4_gemv_bt(w, cb, d->c.cb_block, x, y, M, K, rows, d->bt_partial, s);
     return mth::launch_oil4_gemv(w, cb, d->c.cb_block, x, y, M, K, rows, s);
 }
@@ -103,6 +113,46 @@ hipError_t oil8(const mth_decoder* d, const uint8_t* w, const float* cb, const f
     return mth::launch_oil8_gemv(w, cb, x, y, M, K, rows, s);
 }
 
+// Prompt rows times nseg OIL8 matrices on the matrix cores, whichever of the
+// row kernel and the prompt GEMM (kPfGemmRows rows and more) is the faster at
+// these sizes; false: neither takes them (16 rows and less, other shapes).
+// Prompts of two layers, hidden 2048 (with the batched GEMVs in groups of 16
+// rows up to 63 rows, the GEMM from there -> here): 24 rows 373 -> 316 us, 60
+// rows 575 -> 331, 100 rows 489 -> 361, 400 rows 823 -> 650 (the attention and
+// the K-split down projection in it).
+bool oil8_prompt(const mth_decoder* d, const mth::Oil8Seg* seg, int nseg, const float* x, int64_t rows, int64_t K,
+                 hipStream_t s, hipError_t* e) {
+    if (rows <= 16 || !d->pf_ws || ((uintptr_t)x & 15u) != 0) return false;
+    const bool gemm = rows >= kPfGemmRows && mth::oil8_gemm_x32_supported(seg, nseg, rows, K);
+    int64_t M = 0;
+    bool bt = true;
+    for (int i = 0; i < nseg; ++i) {
+        M += seg[i].rows;
+        bt = bt && ((uintptr_t)seg[i].idx & 15u) == 0 && mth::oil8_bt_supported(seg[i].rows, K, rows);
+    }
+    if (mth::oil8_rows_better(seg, nseg, K, rows, true, gemm, bt) &&
+        mth::rows_mfma_workspace_bytes(M, K, rows, nseg) <= d->pf_ws_bytes) {
+        *e = mth::launch_oil8_rows(seg, nseg, x, K, rows, d->pf_ws, s);
+        return true;
+    }
+    if (gemm) *e = mth::launch_oil8_gemm_x32(x, seg, nseg, rows, K, d->pf_ws, s);
+    return gemm;
+}
+
+// pf_ws: what the prompt kernels need for chunks of up to rows rows.
+size_t prefill_ws_bytes(const mth_decoder_config& c, int64_t rows) {
+    const int64_t H = c.hidden, F = c.ffn, QD = c.heads * c.head_dim, KD = c.kv_heads * c.head_dim;
+    size_t need = 0;
+    if (rows >= kPfGemmRows)
+        need = std::max({mth::oil4_gemm_x32_workspace_bytes(rows, H), mth::oil8_gemm_x32_workspace_bytes(rows, H),
+                         mth::oil8_gemm_x32_workspace_bytes(rows, QD)});
+    for (int64_t n = 17; n <= rows; n++)
+        need = std::max({need, mth::rows_mfma_workspace_bytes(QD + 2 * KD, H, n, 3),
+                         mth::rows_mfma_workspace_bytes(H, QD, n), mth::rows_mfma_workspace_bytes(2 * F, H, n),
+                         mth::rows_mfma_workspace_bytes(F, H, n), mth::i2s_padded_partial_bytes(H, F, n)});
+    return need;
+}
+
 // Q, K and V projections of the normed input h (rows) into q, k, v: one
 // launch over the three matrices (each with its own codebook) where the
 // kernels take them.
@@ -111,9 +161,8 @@ hipError_t qkv(const mth_decoder* d, const mth_decoder_layer& L, const float* h,
     const mth_decoder_config& c = d->c;
     const int64_t H = c.hidden, QD = c.heads * c.head_dim, KD = c.kv_heads * c.head_dim;
     const mth::Oil8Seg seg[3] = {{L.wq, L.cbq, q, QD}, {L.wk, L.cbk, k, KD}, {L.wv, L.cbv, v, KD}};
-    // prompt chunks of >= kPfGemmRows rows: the FP32-row OIL8 GEMM on MFMA
-    if (rows >= kPfGemmRows && d->pf_ws && ((uintptr_t)h & 15u) == 0 && mth::oil8_gemm_x32_supported(seg, 3, rows, H))
-        return mth::launch_oil8_gemm_x32(h, seg, 3, rows, H, d->pf_ws, s);
+    hipError_t e = hipSuccess;
+    if (oil8_prompt(d, seg, 3, h, rows, H, s, &e)) return e;
     if (((uintptr_t)h & 15u) == 0) {
         if (rows >= 2) {
             if (mth::oil8_bt_segs_fusable(seg, 3, H, rows))
@@ -122,7 +171,7 @@ hipError_t qkv(const mth_decoder* d, const mth_decoder_layer& L, const float* h,
             return mth::launch_oil8_gemv_segs(seg, 3, h, H, rows, s);
         }
     }
-    hipError_t e = oil8(d, L.wq, L.cbq, h, q, QD, H, s, rows);
+    e = oil8(d, L.wq, L.cbq, h, q, QD, H, s, rows);
     if (e == hipSuccess) e = oil8(d, L.wk, L.cbk, h, k, KD, H, s, rows);
     if (e == hipSuccess) e = oil8(d, L.wv, L.cbv, h, v, KD, H, s, rows);
     return e;
@@ -136,8 +185,8 @@ bool gate_up_fused(const mth_decoder* d, const mth_decoder_layer& L) {
 
 // The prompt as one forward pass (src/generator.cpp:36): every prompt
 // position of every sequence is a row of the same layer stack (the batched
-// GEMVs in groups of 16 rows, one RoPE + KV append and one causal attention
-// launch per layer over all rows), in chunks of pf_rows rows (whole
+// GEMVs up to 16 rows, the row kernels and GEMMs above, one RoPE + KV append
+// and one causal attention launch per layer over all rows), in chunks of pf_rows rows (whole
 // positions, all sequences); the attention of a chunk reads the earlier
 // chunks' positions from the cache.  Then the final norm, lm_head and argmax
 // of each sequence's last position: the decoder is left as after prompt_len
@@ -172,35 +221,36 @@ hipError_t enqueue_prefill(const mth_decoder* d, hipStream_t s) {
                                            (int)c.kv_heads, (int)c.head_dim, (int)c.max_seq, s));
             {
                 const mth::Oil8Seg so{L.wo, L.cbo, d->pf_t, H};
-                if (R >= kPfGemmRows && ((uintptr_t)d->pf_att & 15u) == 0 && mth::oil8_gemm_x32_supported(&so, 1, R, QD))
-                    TRY(mth::launch_oil8_gemm_x32(d->pf_att, &so, 1, R, QD, d->pf_ws, s));
-                else
-                    TRY(oil8(d, L.wo, L.cbo, d->pf_att, d->pf_t, H, QD, s, R));
+                hipError_t oe = hipSuccess;
+                if (!oil8_prompt(d, &so, 1, d->pf_att, R, QD, s, &oe))
+                    oe = oil8(d, L.wo, L.cbo, d->pf_att, d->pf_t, H, QD, s, R);
+                TRY(oe);
             }
             TRY(mth::launch_rms_norm(d->pf_x, d->pf_t, L.ffn_norm, d->pf_h, R, H, c.eps, s));
             if (gate_up_fused(d, L)) {
                 // chunks of >= kPfGemmRows rows: the FP32-row OIL4 GEMM on
                 // MFMA (each weight read once per 128 rows, not per 16)
-                if (R >= kPfGemmRows && mth::oil4_gemm_x32_supported(R, 2 * F, H, c.cb_block) &&
-                    ((((uintptr_t)L.wgate | (uintptr_t)L.cbgate) & 15u) == 0))
+                // unless the row kernel is faster (in oil4, as for fewer rows)
+                const bool aligned = (((uintptr_t)L.wgate | (uintptr_t)L.cbgate) & 15u) == 0;
+                const bool gemm = R >= kPfGemmRows && aligned && mth::oil4_gemm_x32_supported(R, 2 * F, H, c.cb_block);
+                if (gemm && !mth::oil4_rows_better(L.wgate, L.cbgate, c.cb_block, 2 * F, H, R, true, true, false))
                     TRY(mth::launch_oil4_gemm_x32(d->pf_h, L.wgate, L.cbgate, c.cb_block, d->pf_gu, R, 2 * F, H,
                                                   d->pf_ws, s));
                 else
                     TRY(oil4(d, L.wgate, L.cbgate, d->pf_h, d->pf_gu, 2 * F, H, s, R));
-                TRY(mth::launch_silu_mul_quant(d->pf_gu, d->pf_gu + F, d->pf_aq, d->pf_inv, nullptr, R, F, 2 * F,
-                                               2 * F, s));
+                TRY(mth::launch_silu_mul_quant(d->pf_gu, d->pf_gu + F, d->pf_aq, d->ldq, d->pf_inv, nullptr, R, F,
+                                               2 * F, 2 * F, s));
             } else {
                 TRY(oil4(d, L.wgate, L.cbgate, d->pf_h, d->pf_gu, F, H, s, R));
                 TRY(oil4(d, L.wup, L.cbup, d->pf_h, d->pf_gu + R * F, F, H, s, R));
-                TRY(mth::launch_silu_mul_quant(d->pf_gu, d->pf_gu + R * F, d->pf_aq, d->pf_inv, nullptr, R, F, F, F,
-                                               s));
+                TRY(mth::launch_silu_mul_quant(d->pf_gu, d->pf_gu + R * F, d->pf_aq, d->ldq, d->pf_inv, nullptr, R, F,
+                                               F, F, s));
             }
-            if (R >= kPfGemmRows && mth::i2s_gemm_mfma_ok(H, R, F) &&
-                ((((uintptr_t)L.wdown | (uintptr_t)d->pf_aq) & 15u) == 0))  // int8 MFMA GEMM, bit-exact
-                TRY(mth::launch_i2s_gemm_rows(L.wdown, L.down_scale, d->pf_aq, d->pf_inv, d->pf_t, H, R, F, s));
-            else if ((((uintptr_t)L.wdown | (uintptr_t)d->pf_aq) & 15u) == 0 && mth::i2s_bt_supported(H, F, R))
-                TRY(mth::launch_i2s_gemv_bt(L.wdown, L.down_scale, d->pf_aq, d->pf_inv, d->pf_t, H, F, R,
-                                            d->bt_partial, s));
+            // int8 MFMA, bit-exact; rows of any ffn (13 x 49 tokens, ffn 9152: walking the tokens 4.7 x the time of a
+            // prompt, of 16 decode sequences, ffn 4544, 1.44 x)
+            if (R > 1 && d->down_padded)
+                TRY(mth::launch_i2s_padded(L.wdown, L.down_scale, d->pf_aq, d->ldq, d->pf_inv, d->pf_t, H, F, R,
+                                           R <= 16 ? d->bt_partial : (float*)d->pf_ws, s));
             else
                 TRY(mth::launch_i2s_gemv(L.wdown, L.down_scale, nullptr, d->pf_aq, d->pf_inv, d->pf_t, H, F, R, s));
         }
@@ -289,7 +339,7 @@ hipError_t enqueue_step_split_norm(const mth_decoder* d, hipStream_t s) {
             continue;
         }
         TRY(mth::launch_silu_mul_quant_slices(plain_slices(d->gu, F), plain_slices(d->gu + F, F), ns_ffn, d->aq,
-                                              d->a_inv, nullptr, 1, F, s));
+                                              d->ldq, d->a_inv, nullptr, 1, F, s));
         if (!last)
             TRY(mth::launch_i2s_gemv_resid(L.wdown, L.down_scale, d->aq, d->a_inv, H, F, ro, &ns_attn.nparts, s));
         else
@@ -427,7 +477,7 @@ hipError_t enqueue_step(const mth_decoder* d, hipStream_t s) {
             // to read the gate/up slices as fast as the reduction kernel)
             TRY(oil4(d, L.wgate, L.cbgate, d->h, d->gu, 2 * F, H, s));
             if (tp) TRY(tap_copy(tp_gu, d->gu, (size_t)(B * 2 * F) * 4));
-            TRY(mth::launch_silu_mul_quant_slices(sg, su, ns_ffn, d->aq, d->a_inv, tp_act, B, F, s));
+            TRY(mth::launch_silu_mul_quant_slices(sg, su, ns_ffn, d->aq, d->ldq, d->a_inv, tp_act, B, F, s));
         } else {
             TRY(oil4(d, L.wgate, L.cbgate, d->h, d->gu, F, H, s));
             TRY(oil4(d, L.wup, L.cbup, d->h, d->gu + B * F, F, H, s));
@@ -439,22 +489,24 @@ hipError_t enqueue_step(const mth_decoder* d, hipStream_t s) {
             }
             if (splitb)
                 TRY(mth::launch_silu_mul_quant_slices(plain_slices(d->gu, F), plain_slices(d->gu + B * F, F), ns_ffn,
-                                                      d->aq, d->a_inv, tp_act, B, F, s));
+                                                      d->aq, d->ldq, d->a_inv, tp_act, B, F, s));
             else
-                TRY(mth::launch_silu_mul_quant(d->gu, d->gu + B * F, d->aq, d->a_inv, tp_act, B, F, F, F, s));
+                TRY(mth::launch_silu_mul_quant(d->gu, d->gu + B * F, d->aq, d->ldq, d->a_inv, tp_act, B, F, F, F, s));
         }
         resid = plain_slices(d->t, H);
-        if ((((uintptr_t)L.wdown | (uintptr_t)d->aq) & 15u) == 0 && mth::i2s_bt_supported(H, F, B)) {
+        if (B >= 2 && d->down_padded) {
             if (fold)
-                TRY(mth::launch_i2s_gemv_bt_slices(L.wdown, L.down_scale, d->aq, d->a_inv, d->t, H, F, B,
-                                                   d->bt_partial, &resid, s));
+                TRY(mth::launch_i2s_padded_slices(L.wdown, L.down_scale, d->aq, d->ldq, d->a_inv, d->t, H, F, B,
+                                                  d->bt_partial, &resid, s));
             else
-                TRY(mth::launch_i2s_gemv_bt(L.wdown, L.down_scale, d->aq, d->a_inv, d->t, H, F, B, d->bt_partial, s));
+                TRY(mth::launch_i2s_padded(L.wdown, L.down_scale, d->aq, d->ldq, d->a_inv, d->t, H, F, B,
+                                           d->bt_partial, s));
         } else {
             TRY(mth::launch_i2s_gemv(L.wdown, L.down_scale, nullptr, d->aq, d->a_inv, d->t, H, F, B, s));
         }
         if (tp) {
-            TRY(tap_copy(tp_aq, d->aq, (size_t)(B * F)));
+            TRY(hipMemcpy2DAsync(tp_aq, (size_t)F, d->aq, (size_t)d->ldq, (size_t)F, (size_t)B,
+                                 hipMemcpyDeviceToDevice, s));
             TRY(tap_copy(tp_inv, d->a_inv, (size_t)B * 4));
             TRY(tap_copy(tp_down, d->t, (size_t)(B * H) * 4));
         }
@@ -515,6 +567,9 @@ int mth_decoder_create(const mth_decoder_config* cfg, mth_decoder** out) {
     // prefill chunk: up to 1024 rows of (sequence, position)
     const int64_t PR = std::min<int64_t>(B * c.max_seq, 1024);
     d->pf_rows = PR;
+    d->down_padded = mth::i2s_padded_supported(H, F, std::max(PR, B));
+    d->ldq = d->down_padded ? mth::i2s_padded_cols(F) : F;
+    d->pf_ws_bytes = prefill_ws_bytes(c, PR);
     // workspace of the batched GEMVs: the largest of every projection's need
     const size_t partial = std::max({mth::oil4_bt_partial_bytes(2 * F, H), mth::oil8_bt_partial_bytes(QD + 2 * KD, H),
                                      mth::oil8_bt_partial_bytes(H, QD),
@@ -527,7 +582,7 @@ int mth_decoder_create(const mth_decoder_config* cfg, mth_decoder** out) {
         {(void**)&d->t, (size_t)(B * H) * 4},       {(void**)&d->q, (size_t)(B * QD) * 4},
         {(void**)&d->k, (size_t)(B * KD) * 4},      {(void**)&d->v, (size_t)(B * KD) * 4},
         {(void**)&d->att, (size_t)(B * QD) * 4},    {(void**)&d->gu, (size_t)(B * 2 * F) * 4},
-        {(void**)&d->aq, (size_t)(B * F)},          {(void**)&d->a_inv, (size_t)B * 4},
+        {(void**)&d->aq, (size_t)(B * d->ldq)},          {(void**)&d->a_inv, (size_t)B * 4},
         {(void**)&d->logits, (size_t)(B * c.vocab) * 4},
         {(void**)&d->arg_v, (size_t)(B * mth::argmax_chunks(c.vocab)) * 4},
         {(void**)&d->arg_i, (size_t)(B * mth::argmax_chunks(c.vocab)) * 4},
@@ -542,13 +597,10 @@ int mth_decoder_create(const mth_decoder_config* cfg, mth_decoder** out) {
         {(void**)&d->pf_t, (size_t)(PR * H) * 4},   {(void**)&d->pf_q, (size_t)(PR * QD) * 4},
         {(void**)&d->pf_k, (size_t)(PR * KD) * 4},  {(void**)&d->pf_v, (size_t)(PR * KD) * 4},
         {(void**)&d->pf_att, (size_t)(PR * QD) * 4}, {(void**)&d->pf_gu, (size_t)(PR * 2 * F) * 4},
-        {(void**)&d->pf_aq, (size_t)(PR * F)},      {(void**)&d->pf_inv, (size_t)PR * 4},
+        {(void**)&d->pf_aq, (size_t)(PR * d->ldq)},      {(void**)&d->pf_inv, (size_t)PR * 4},
         {(void**)&d->ssp, (size_t)(H / 4 + 2) * 8},  {(void**)&d->ssp2, (size_t)(H / 4 + 2) * 8},
         {(void**)&d->amx, (size_t)(B * kAmxParts) * 4},
-        {(void**)&d->pf_ws, PR >= kPfGemmRows ? std::max({mth::oil4_gemm_x32_workspace_bytes(PR, H),
-                                                          mth::oil8_gemm_x32_workspace_bytes(PR, H),
-                                                          mth::oil8_gemm_x32_workspace_bytes(PR, QD)})
-                                              : (size_t)0},
+        {(void**)&d->pf_ws, d->pf_ws_bytes},
     };
     size_t total = 0;
     for (const Slot& sl : slots) total += round_up(sl.bytes);

@@ -704,14 +704,15 @@ __global__ __launch_bounds__(NT) void attention_k(Slices q, Slices kin, Slices v
 // (src/int8_quant.cpp:8-31): max|a| (floor 1e-10), scale = 127/max,
 // q = (int8)round_half_away(a * scale), inv = max/127.  n <= kSQT * kSQ.
 constexpr int kSQT = 1024, kSQ = 12;
-// act (optional): the FP32 activations, [rows][n].
+// act (optional): the FP32 activations, [rows][n].  q: rows of ldq >= n bytes,
+// zeros from column n on (the padding the int8 MFMA kernels read).
 // g, u: the gate and up outputs as Slices (common.h), so the split-K
 // partial sums of the GEMV are added here.
 // ns (NormScale, common.h): g/u are projections of x * gamma and get the
 // RMSNorm's 1 / rms here.
 __global__ __launch_bounds__(kSQT) void silu_mul_quant_k(Slices g, Slices u, NormScale ns, int8_t* __restrict__ q,
                                                          float* __restrict__ inv_scale, float* __restrict__ act,
-                                                         int n) {
+                                                         int n, int ldq) {
     __shared__ float red[kSQT / 64];
     __shared__ double nred[kSQT / 64];
     const int r = blockIdx.x, tid = threadIdx.x;
@@ -757,12 +758,13 @@ __global__ __launch_bounds__(kSQT) void silu_mul_quant_k(Slices g, Slices u, Nor
     for (int w = 1; w < kSQT / 64; ++w) m = fmaxf(m, red[w]);
     if (m < 1e-10f) m = 1e-10f;
     const float sc = __fdiv_rn(127.0f, m);
-    int8_t* qr = q + (int64_t)r * n;
+    int8_t* qr = q + (int64_t)r * ldq;
 #pragma unroll
     for (int j = 0; j < kSQ; ++j) {
         const int i = tid + j * kSQT;
         if (i < n) qr[i] = (int8_t)quant_i8(gv[j], sc);
     }
+    for (int i = n + tid; i < ldq; i += kSQT) qr[i] = 0;
     if (act) {
         float* ar = act + (int64_t)r * n;
 #pragma unroll
@@ -1148,16 +1150,16 @@ hipError_t launch_rope_attention_slices(const Slices& q, const Slices& k, const 
 
 bool silu_mul_quant_supported(int64_t n) { return n > 0 && n <= (int64_t)kSQT * kSQ; }
 
-hipError_t launch_silu_mul_quant_slices(const Slices& g, const Slices& u, const NormScale& ns, int8_t* q,
+hipError_t launch_silu_mul_quant_slices(const Slices& g, const Slices& u, const NormScale& ns, int8_t* q, int64_t ldq,
                                         float* inv_scale, float* act, int64_t rows, int64_t n, hipStream_t s) {
-    silu_mul_quant_k<<<(unsigned)rows, kSQT, 0, s>>>(g, u, ns, q, inv_scale, act, (int)n);
+    silu_mul_quant_k<<<(unsigned)rows, kSQT, 0, s>>>(g, u, ns, q, inv_scale, act, (int)n, (int)ldq);
     return hipGetLastError();
 }
 
-hipError_t launch_silu_mul_quant(const float* g, const float* u, int8_t* q, float* inv_scale, float* act,
+hipError_t launch_silu_mul_quant(const float* g, const float* u, int8_t* q, int64_t ldq, float* inv_scale, float* act,
                                  int64_t rows, int64_t n, int64_t gstride, int64_t ustride, hipStream_t s) {
-    return launch_silu_mul_quant_slices(plain_slices(g, gstride), plain_slices(u, ustride), NormScale{}, q, inv_scale,
-                                        act, rows, n, s);
+    return launch_silu_mul_quant_slices(plain_slices(g, gstride), plain_slices(u, ustride), NormScale{}, q, ldq,
+                                        inv_scale, act, rows, n, s);
 }
 
 int argmax_chunks(int64_t n) { return (int)((n + kArgChunk - 1) / kArgChunk); }

@@ -126,6 +126,16 @@ struct RowsArgs {
     float* partial;        // [slice] of the same
     int M, K, batch, steps, cb_block;
 };
+// OIL8: up to three matrices over the same token rows (a decoder's Q, K and V), their row tiles one after another in
+// the grid; t1: the first row tile past matrix i.  Matrix i's partial sums start at partial + p0[i].
+struct RowsSegs {
+    const uint8_t* w[3];
+    const void* cb[3];
+    float* out[3];
+    int M[3], t1[3];
+    int64_t p0[3];
+    int n;
+};
 
 // a weight tile's registers of one step: 16 rows x 128 columns
 template <int FMT>
@@ -188,14 +198,26 @@ __device__ float rows_fma(const RowsArgs& p, int row, int tok, int k0, int k1) {
 }
 
 template <int FMT, int G>
-__global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p) {
+__global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) {
     constexpr int NB = 2 * G;  // 16-byte pieces of a step's B per thread (8 KB per token group)
     __shared__ __align__(16) uint8_t bs[G * 8192];
     __shared__ uint32_t tab[FMT == kOil8 ? 256 : 1];
     __shared__ float wred[kRmT / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int j = lane & 15, q = lane >> 4;
-    const int row0 = blockIdx.x * kRmRows + wave * 32, tok0 = blockIdx.y * 16 * G;
+    int bx = blockIdx.x;
+    if constexpr (FMT == kOil8) {
+        if (sg.n > 1) {
+            const int i = (bx >= sg.t1[0] ? 1 : 0) + (bx >= sg.t1[1] ? 1 : 0);
+            bx -= i == 0 ? 0 : i == 1 ? sg.t1[0] : sg.t1[1];
+            p.w = i == 0 ? sg.w[0] : i == 1 ? sg.w[1] : sg.w[2];
+            p.cb = i == 0 ? sg.cb[0] : i == 1 ? sg.cb[1] : sg.cb[2];
+            p.out = i == 0 ? sg.out[0] : i == 1 ? sg.out[1] : sg.out[2];
+            p.M = i == 0 ? sg.M[0] : i == 1 ? sg.M[1] : sg.M[2];
+            p.partial += i == 0 ? sg.p0[0] : i == 1 ? sg.p0[1] : sg.p0[2];
+        }
+    }
+    const int row0 = bx * kRmRows + wave * 32, tok0 = blockIdx.y * 16 * G;
     const int S = gridDim.z;
     const int s0 = (int)((int64_t)blockIdx.z * p.steps / S), s1 = (int)((int64_t)(blockIdx.z + 1) * p.steps / S);
     const int M = p.M, K = p.K;
@@ -261,7 +283,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p) {
     float* out = S == 1 ? p.out : p.partial + blockIdx.z * zs;
     auto at = [&](int row, int tok) { return FMT == kTern ? (int64_t)row * p.batch + tok : (int64_t)tok * M + row; };
     if (special) {
-        const int k0 = kRmStep * s0, k1 = min(K, kRmStep * s1), r0 = blockIdx.x * kRmRows;
+        const int k0 = kRmStep * s0, k1 = min(K, kRmStep * s1), r0 = bx * kRmRows;
         for (int o = tid; o < kRmRows * 16 * G; o += kRmT) {
             const int row = r0 + o % kRmRows, tok = tok0 + o / kRmRows;
             if (row < M && tok < p.batch) out[at(row, tok)] = rows_fma<FMT>(p, row, tok, k0, k1);
@@ -283,7 +305,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p) {
 #pragma unroll
         for (int g = 0; g < G; ++g) ah[t][g] = ax[t][g] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const bool edge = FMT == kTern && blockIdx.x == gridDim.x - 1;  // a tile with the matrix's last row
+    const bool edge = FMT == kTern && bx == (int)gridDim.x - 1;  // a tile with the matrix's last row
     const uint8_t* brow = bs + q * 1024 + j * 16;  // lane (token j, chunk q) of piece m: + 256 m
     auto step_body = [&](int step, RowsTile<FMT> (&w)[2]) {
 #pragma unroll
@@ -388,11 +410,17 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p) {
 }
 
 // out[i] = sum over slices z = 0, 1, ... of partial[z][i] (a fixed order); all loads before the first add.  Four
-// values per thread where both arrays are 16-byte aligned (n % 4 == 0).
+// values per thread where both arrays are 16-byte aligned (n % 4 == 0).  gridDim.y > 1: sg's matrix blockIdx.y.
 template <bool VEC>
 __global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ partial, float* __restrict__ out,
-                                                      int64_t n, int S) {
+                                                      int64_t n, int S, RowsSegs sg, int batch) {
     const int64_t i = ((int64_t)blockIdx.x * kRmT + threadIdx.x) * (VEC ? 4 : 1);
+    if (gridDim.y > 1) {
+        const int y = blockIdx.y;
+        n = (int64_t)batch * (y == 0 ? sg.M[0] : y == 1 ? sg.M[1] : sg.M[2]);
+        out = y == 0 ? sg.out[0] : y == 1 ? sg.out[1] : sg.out[2];
+        partial += y == 0 ? sg.p0[0] : y == 1 ? sg.p0[1] : sg.p0[2];
+    }
     if (i >= n) return;
     if constexpr (VEC) {
         float4 v[kRmSlices];
@@ -419,13 +447,14 @@ struct RowsPlan {
     int G, tiles, S, steps;
     int64_t rtiles;
 };
-inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch) {
+// (M rows in nseg matrices: at most nseg - 1 row tiles more than M fills)
+inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch, int nseg = 1) {
     RowsPlan p{};
     p.steps = (int)((K + kRmStep - 1) / kRmStep);
     const int64_t nt = (batch + 63) / 64;
     p.G = (int)((batch + 16 * nt - 1) / (16 * nt));  // token tiles of 16, 32, 48 or 64, as even as they go
     p.tiles = (int)((batch + 16 * p.G - 1) / (16 * p.G));
-    p.rtiles = (M + kRmRows - 1) / kRmRows;
+    p.rtiles = (M + kRmRows - 1) / kRmRows + nseg - 1;
     const int64_t wgs = p.rtiles * p.tiles;
     // K slices: about one workgroup per CU (a workgroup's fixed cost, ~5 us of load latency, table and output, is then
     // paid once per CU: 4096 x 4096 at 40 tokens 24.2 / 19.5 / 23.0 us for 4 / 8 / 16 slices); two per CU for long
@@ -440,8 +469,8 @@ inline size_t al256r(size_t n) { return (n + 255) & ~(size_t)255; }
 inline size_t rows_a16_bytes(const RowsPlan& p) { return (size_t)p.tiles * p.G * 2 * p.steps * 4096; }
 
 template <int FMT>
-hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s) {
-    const int64_t n = (int64_t)a.M * a.batch;
+hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s, const RowsSegs& sg = RowsSegs{}) {
+    int64_t n = (int64_t)a.M * a.batch;
     uint16_t* a16 = (uint16_t*)ws;
     int* rsh = (int*)((char*)ws + rows_a16_bytes(p));
     float* partial = (float*)((char*)rsh + al256r((size_t)a.batch * 4));
@@ -454,18 +483,30 @@ hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s) {
         rows_split_k<FMT == kTern, true><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps);
     else
         rows_split_k<FMT == kTern, false><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps);
-    const dim3 grid((unsigned)p.rtiles, (unsigned)p.tiles, (unsigned)p.S);
+    const dim3 grid((unsigned)(sg.n > 1 ? sg.t1[sg.n - 1] : p.rtiles), (unsigned)p.tiles, (unsigned)p.S);
     switch (p.G) {
-        case 1: rows_mfma_k<FMT, 1><<<grid, kRmT, 0, s>>>(a); break;
-        case 2: rows_mfma_k<FMT, 2><<<grid, kRmT, 0, s>>>(a); break;
-        case 3: rows_mfma_k<FMT, 3><<<grid, kRmT, 0, s>>>(a); break;
-        default: rows_mfma_k<FMT, 4><<<grid, kRmT, 0, s>>>(a); break;
+        case 1: rows_mfma_k<FMT, 1><<<grid, kRmT, 0, s>>>(a, sg); break;
+        case 2: rows_mfma_k<FMT, 2><<<grid, kRmT, 0, s>>>(a, sg); break;
+        case 3: rows_mfma_k<FMT, 3><<<grid, kRmT, 0, s>>>(a, sg); break;
+        default: rows_mfma_k<FMT, 4><<<grid, kRmT, 0, s>>>(a, sg); break;
     }
     if (p.S > 1) {
-        if (n % 4 == 0 && ((uintptr_t)a.out & 15u) == 0)
-            rows_reduce_k<true><<<(unsigned)((n / 4 + kRmT - 1) / kRmT), kRmT, 0, s>>>(partial, a.out, n, p.S);
+        bool vec4 = n % 4 == 0 && ((uintptr_t)a.out & 15u) == 0;
+        if (sg.n > 1) {
+            n = 0;
+            vec4 = true;
+            for (int i = 0; i < sg.n; ++i) {
+                n = std::max(n, (int64_t)sg.M[i] * a.batch);
+                vec4 = vec4 && (int64_t)sg.M[i] * a.batch % 4 == 0 && ((uintptr_t)sg.out[i] & 15u) == 0;
+            }
+        }
+        const unsigned ny = sg.n > 1 ? sg.n : 1;
+        if (vec4)
+            rows_reduce_k<true><<<dim3((unsigned)((n / 4 + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S,
+                                                                                                 sg, a.batch);
         else
-            rows_reduce_k<false><<<(unsigned)((n + kRmT - 1) / kRmT), kRmT, 0, s>>>(partial, a.out, n, p.S);
+            rows_reduce_k<false><<<dim3((unsigned)((n + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S, sg,
+                                                                                              a.batch);
     }
     return hipGetLastError();
 }
@@ -477,8 +518,8 @@ inline bool rows_sizes(int64_t M, int64_t K, int64_t batch) {
 
 }  // namespace
 
-size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch) {
-    const RowsPlan p = rows_plan(M, K, batch);
+size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch, int nseg) {
+    const RowsPlan p = rows_plan(M, K, batch, nseg);
     return rows_a16_bytes(p) + al256r((size_t)batch * 4) + (p.S > 1 ? (size_t)(p.S * M * batch * 4) : 0);
 }
 
@@ -503,8 +544,14 @@ double walk_us(int64_t M, int64_t K, int64_t batch, bool oil8, bool fast) {
 
 // OIL8: K % 16 == 0, 16-byte aligned indices.  gemm: the prompt GEMM takes the call (128 tokens and more); bt: the
 // batched GEMV does (16 tokens per launch pair).
-bool oil8_rows_better(const uint8_t* idx, int64_t M, int64_t K, int64_t batch, bool aligned, bool gemm, bool bt) {
-    if (!rows_sizes(M, K, batch) || K % 16 != 0 || ((uintptr_t)idx & 15u) != 0) return false;
+bool oil8_rows_better(const Oil8Seg* seg, int nseg, int64_t K, int64_t batch, bool aligned, bool gemm, bool bt) {
+    if (nseg < 1 || nseg > 3) return false;
+    int64_t M = 0;
+    for (int i = 0; i < nseg; ++i) {
+        if (seg[i].rows < 1 || ((uintptr_t)seg[i].idx & 15u) != 0) return false;
+        M += seg[i].rows;
+    }
+    if (!rows_sizes(M, K, batch) || K % 16 != 0) return false;
     const double us = rows_us(M, K, batch, 1.7);
     if (gemm) {
         // a round of 256 tiles of 128 x 64 (54 us at K = 4096), or of 256 x 64 where those fill the chip (98 us)
@@ -543,10 +590,27 @@ bool tern_rows_better(int64_t M, int64_t K, int64_t batch) {
            K * std::max(1.0, (double)M * batch / 8000.0) > 4000.0;
 }
 
-hipError_t launch_oil8_rows(const uint8_t* idx, const float* cb, const float* x, float* y, int64_t M, int64_t K,
-                            int64_t batch, void* ws, hipStream_t s) {
-    RowsArgs a{idx, cb, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, 0};
-    return rows_run<kOil8>(a, rows_plan(M, K, batch), ws, s);
+hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, void* ws,
+                            hipStream_t s) {
+    RowsSegs sg{};
+    int64_t M = 0, tiles = 0;
+    for (int i = 0; i < nseg; ++i) M += seg[i].rows;
+    const RowsPlan p = rows_plan(M, K, batch, nseg);
+    sg.n = nseg;
+    M = 0;
+    for (int i = 0; i < 3; ++i) {
+        const Oil8Seg& g = seg[i < nseg ? i : nseg - 1];
+        sg.w[i] = g.idx, sg.cb[i] = g.cb, sg.out[i] = g.y;
+        sg.M[i] = (int)g.rows;
+        sg.p0[i] = p.S * M * batch;
+        if (i < nseg) {
+            M += g.rows;
+            tiles += (g.rows + kRmRows - 1) / kRmRows;
+        }
+        sg.t1[i] = (int)tiles;
+    }
+    RowsArgs a{seg[0].idx, seg[0].cb, nullptr, nullptr, x, seg[0].y, nullptr, (int)seg[0].rows, (int)K, (int)batch, 0, 0};
+    return rows_run<kOil8>(a, p, ws, s, sg);
 }
 hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
                             int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s) {

@@ -111,8 +111,6 @@ bool i2s_bt_supported(int64_t M, int64_t K, int64_t batch);
 size_t i2s_bt_partial_bytes(int64_t M, int64_t K);
 hipError_t launch_i2s_gemv_bt(const uint8_t* packed, float w_scale, const int8_t* act, const float* act_scale, float* y,
                               int64_t M, int64_t K, int64_t batch, float* partial, hipStream_t s);
-// Batches of at most 16 without the slice reduction (Slices with the I2_S
-// epilogue, common.h).
 // Batches of 2..16 with FP32 activations quantised inside the launch (the
 // decode step): act[t * lda + k] and amax[t][nmx] as
 // launch_oil4_gemv_bt_swiglu writes them; inv[t] = max|act| / 127 is
@@ -125,9 +123,6 @@ hipError_t launch_i2s_gemv_bt_f32act(const uint8_t* packed, float w_scale, const
 hipError_t launch_i2s_gemv_bt_f32act_y(const uint8_t* packed, float w_scale, const float* act, int64_t lda,
                                        const float* amax, int nmx, float* inv, float* y, int64_t M, int64_t K,
                                        int64_t batch, float* partial, hipStream_t s);
-hipError_t launch_i2s_gemv_bt_slices(const uint8_t* packed, float w_scale, const int8_t* act, const float* act_scale,
-                                    float* y, int64_t M, int64_t K, int64_t batch, float* partial, Slices* out,
-                                    hipStream_t s);
 // Token rows of any K % 4 == 0, FP32 rows (x: quantised per token) or int8 rows (act, act_scale): the
 // rows as padded int8 in ws (i2s_rows_workspace_bytes), then the batched kernel (up to 16 tokens) or the int8
 // MFMA GEMM; the same bits as launch_i2s_gemv.
@@ -136,6 +131,18 @@ size_t i2s_rows_workspace_bytes(int64_t M, int64_t K, int64_t batch);
 hipError_t launch_i2s_rows(const uint8_t* packed, float w_scale, const float* x, const int8_t* act,
                            const float* act_scale, float* y, int64_t M, int64_t K, int64_t batch, void* ws,
                            hipStream_t s);
+// The same product from int8 rows that lie lda bytes apart (a multiple of 16, at least i2s_padded_cols(K)) and end in
+// zeros from column K on, at a 16-byte aligned address: no copy.  partial: i2s_padded_partial_bytes.  _slices
+// (at most 16 rows): without the slice reduction (Slices with the I2_S epilogue, common.h).
+int64_t i2s_padded_cols(int64_t K);
+bool i2s_padded_supported(int64_t M, int64_t K, int64_t batch);
+size_t i2s_padded_partial_bytes(int64_t M, int64_t K, int64_t batch);
+hipError_t launch_i2s_padded(const uint8_t* packed, float w_scale, const int8_t* act, int64_t lda,
+                             const float* act_scale, float* y, int64_t M, int64_t K, int64_t batch, float* partial,
+                             hipStream_t s);
+hipError_t launch_i2s_padded_slices(const uint8_t* packed, float w_scale, const int8_t* act, int64_t lda,
+                                    const float* act_scale, float* y, int64_t M, int64_t K, int64_t batch,
+                                    float* partial, Slices* out, hipStream_t s);
 // Batch 1, int8 activations, with the residual epilogue (ResidOut,
 // common.h) in place of y; *nparts: partials per token.
 bool i2s_resid_supported(const uint8_t* packed, const int8_t* act, int64_t M, int64_t K);
@@ -160,12 +167,6 @@ hipError_t launch_i2s_gemm(const uint8_t* w, const float* a, float* o,
 bool i2s_gemm_mfma_ok(int64_t M, int64_t N, int64_t K);
 hipError_t launch_i2s_gemm_vnni(const uint8_t* w, const int8_t* a, float* o,
                                 int64_t M, int64_t N, int64_t K, hipStream_t s);
-// The prompt prefill's down projection on int8 MFMA: y [N][M] = the I2_S
-// GEMV of every token row n of the int8 activations a [N][K] with act scale
-// inv[n] (bit-identical to launch_i2s_gemv per row); i2s_gemm_mfma_ok(M, N, K)
-// and 16-byte aligned w, a (else hipErrorInvalidValue).
-hipError_t launch_i2s_gemm_rows(const uint8_t* w, float w_scale, const int8_t* a, const float* inv, float* y, int64_t M,
-                                int64_t N, int64_t K, hipStream_t s);
 hipError_t launch_tl1_gemm(const uint8_t* w, const float* a, float* o,
                            int64_t M, int64_t N, int64_t K, hipStream_t s);
 hipError_t launch_tl2_gemm(const uint8_t* w, const float* a, float* o,
@@ -225,15 +226,16 @@ hipError_t launch_oil8_gemm_x32(const float* a, const Oil8Seg* seg, int nseg, in
 // y [batch][M] (ternary: out [M][batch]) for any M and batch; OIL8 rows of a multiple of 16, OIL4 rows and codebook
 // blocks of a multiple of 32 (16-byte aligned weights), ternary rows of a multiple of 4 (any alignment).
 // ws: rows_mfma_workspace_bytes.
-size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch);
+size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch, int nseg = 1);  // M: all matrices' rows
 // Whether this route is the faster one (and takes the call): against the prompt GEMM (gemm), the batched GEMV (bt) or
 // the kernels that walk the tokens (x aligned to 16 bytes: aligned).
-bool oil8_rows_better(const uint8_t* idx, int64_t M, int64_t K, int64_t batch, bool aligned, bool gemm, bool bt);
+// nseg matrices of one K in one launch (OIL8): each with its own codebook and output [batch][rows].
+bool oil8_rows_better(const Oil8Seg* seg, int nseg, int64_t K, int64_t batch, bool aligned, bool gemm, bool bt);
 bool oil4_rows_better(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, int64_t M, int64_t K, int64_t batch,
                       bool aligned, bool gemm, bool bt);
 bool tern_rows_better(int64_t M, int64_t K, int64_t batch);
-hipError_t launch_oil8_rows(const uint8_t* idx, const float* cb, const float* x, float* y, int64_t M, int64_t K,
-                            int64_t batch, void* ws, hipStream_t s);
+hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, void* ws,
+                            hipStream_t s);
 hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
                             int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s);
 hipError_t launch_tern_rows(const uint8_t* w, const float* x, float* out, int64_t M, int64_t K, int64_t batch,
@@ -312,13 +314,13 @@ hipError_t launch_rope_kv_rows(float* q, const float* k, const float* v, const f
 // x[r] = emb[hist[r / np][p0 + r % np]]
 hipError_t launch_embed_rows(const float* emb, const int* hist, int hist_stride, float* x, int64_t rows, int np, int p0,
                              int dim, int vocab, hipStream_t s);
-// silu(g) * u then quantize_per_token: q [rows][n] int8, inv_scale [rows];
+// silu(g) * u then quantize_per_token: q [rows][ldq] int8 (ldq >= n, zeros from column n on), inv_scale [rows];
 // act (nullable) receives the FP32 activations [rows][n].
 bool silu_mul_quant_supported(int64_t n);
 // g/u as Slices (common.h)
-hipError_t launch_silu_mul_quant_slices(const Slices& g, const Slices& u, const NormScale& ns, int8_t* q,
+hipError_t launch_silu_mul_quant_slices(const Slices& g, const Slices& u, const NormScale& ns, int8_t* q, int64_t ldq,
                                         float* inv_scale, float* act, int64_t rows, int64_t n, hipStream_t s);
-hipError_t launch_silu_mul_quant(const float* g, const float* u, int8_t* q, float* inv_scale, float* act,
+hipError_t launch_silu_mul_quant(const float* g, const float* u, int8_t* q, int64_t ldq, float* inv_scale, float* act,
                                  int64_t rows, int64_t n, int64_t gstride, int64_t ustride, hipStream_t s);
 // Greedy argmax in two launches; pv/pi: rows * argmax_chunks(n) partials.
 // With hist: writes the next input token; with step: advances it last.

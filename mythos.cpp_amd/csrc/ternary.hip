@@ -1650,15 +1650,23 @@ inline bool rows_pay(bool f32, bool whole, int64_t M, int64_t K, int64_t batch) 
 }
 }  // namespace
 
+int64_t i2s_padded_cols(int64_t K) { return rows_kp(K); }
+
+bool i2s_padded_supported(int64_t M, int64_t K, int64_t batch) {
+    return batch >= 1 && K % 4 == 0 && K >= 64 && K < (1 << 24) / 128 && M < (1ll << 31) && M * (K / 4) >= 16 &&
+           M * (K / 4) < (1ll << 32) - 256 && batch * rows_kp(K) < (1ll << 32) &&
+           ((M + TGM - 1) / TGM) * ((batch + TGN - 1) / TGN) < (1ll << 31) && batch <= 65535;
+}
+
+size_t i2s_padded_partial_bytes(int64_t M, int64_t K, int64_t batch) { return rows_partial(M, K, batch); }
+
 bool i2s_rows_supported(const uint8_t* packed, const void* x, bool f32, int64_t M, int64_t K, int64_t batch) {
     // int8 rows the batched kernel takes as they are (a decode group of whole aligned chunks) stay on it; exact
     // integer sums in FP32 (K < 2^17) and 32-bit lane offsets as i2s_gemm_mfma_ok
     if (!f32 && batch <= kIbTok && i2s_bt_supported(M, K, batch) && aligned16(packed) && aligned16(x)) return false;
     const bool whole = K % 64 == 0 && K <= 64 * 256 && aligned16(packed) && aligned16(x);
     if (batch == 1 && whole) return false;
-    return batch >= 1 && rows_pay(f32, whole, M, K, batch) && K % 4 == 0 && K >= 64 && K < (1 << 24) / 128 && M < (1ll << 31) &&
-           M * (K / 4) >= 16 && M * (K / 4) < (1ll << 32) - 256 && batch * rows_kp(K) < (1ll << 32) &&
-           ((M + TGM - 1) / TGM) * ((batch + TGN - 1) / TGN) < (1ll << 31) && batch <= 65535;
+    return rows_pay(f32, whole, M, K, batch) && i2s_padded_supported(M, K, batch);
 }
 
 size_t i2s_rows_workspace_bytes(int64_t M, int64_t K, int64_t batch) {
@@ -1686,6 +1694,13 @@ hipError_t launch_i2s_rows(const uint8_t* packed, float w_scale, const float* x,
         a = act;
         lda = K;
     }
+    return launch_i2s_padded(packed, w_scale, a, lda, act_scale, y, M, K, batch, partial, s);
+}
+
+hipError_t launch_i2s_padded(const uint8_t* packed, float w_scale, const int8_t* a, int64_t lda, const float* act_scale,
+                             float* y, int64_t M, int64_t K, int64_t batch, float* partial, hipStream_t s) {
+    if (!i2s_padded_supported(M, K, batch) || lda % 16 != 0 || lda < rows_kp(K) || !aligned16(a))
+        return hipErrorInvalidValue;
     const bool tail = K % 256 != 0 || !aligned16(packed);
     const int m = (int)M, k = (int)K, n = (int)batch;
     if (batch <= kIbTok) {
@@ -1713,11 +1728,18 @@ hipError_t launch_i2s_rows(const uint8_t* packed, float w_scale, const float* x,
     return hipGetLastError();
 }
 
-hipError_t launch_i2s_gemv_bt_slices(const uint8_t* packed, float w_scale, const int8_t* act, const float* act_scale,
-                                    float* y, int64_t M, int64_t K, int64_t batch, float* partial, Slices* out,
-                                    hipStream_t s) {
+hipError_t launch_i2s_padded_slices(const uint8_t* packed, float w_scale, const int8_t* a, int64_t lda,
+                                    const float* act_scale, float* y, int64_t M, int64_t K, int64_t batch,
+                                    float* partial, Slices* out, hipStream_t s) {
+    if (!i2s_padded_supported(M, K, batch) || batch > kIbTok || lda % 16 != 0 || lda < rows_kp(K) || !aligned16(a))
+        return hipErrorInvalidValue;
     const int S = ib_slices(M, K);
-    i2s_gemv_bt<kIbChunks, kIbWaves><<<dim3(ceil_div(M, kIbRows), (unsigned)S), kIbWaves * 64, 0, s>>>(packed, w_scale, act, K, act_scale, y, partial,
+    const dim3 grid(ceil_div(M, kIbRows), (unsigned)S);
+    if (K % 256 != 0 || !aligned16(packed))
+        i2s_gemv_bt<kIbChunks, kIbWaves, false, true><<<grid, kIbWaves * 64, 0, s>>>(
+            packed, w_scale, a, lda, act_scale, y, partial, (int)M, (int)K, (int)batch);
+    else
+        i2s_gemv_bt<kIbChunks, kIbWaves><<<grid, kIbWaves * 64, 0, s>>>(packed, w_scale, a, lda, act_scale, y, partial,
                                                                         (int)M, (int)K, (int)batch);
     *out = S == 1 ? plain_slices(y, M) : Slices{partial, M, kIbTok * M, S, w_scale, act_scale};
     return hipGetLastError();
@@ -1768,14 +1790,6 @@ hipError_t launch_i2s_gemm_vnni(const uint8_t* w, const int8_t* a, float* o, int
         return hipGetLastError();
     }
     i2s_gemm_vnni_k<<<ceil_div(M * N, kWaves), kWG, 0, s>>>(w, a, o, M, N, K);
-    return hipGetLastError();
-}
-
-hipError_t launch_i2s_gemm_rows(const uint8_t* w, float w_scale, const int8_t* a, const float* inv, float* y, int64_t M,
-                                int64_t N, int64_t K, hipStream_t s) {
-    if (!i2s_gemm_mfma_ok(M, N, K) || (((uintptr_t)w | (uintptr_t)a) & 15u) != 0) return hipErrorInvalidValue;
-    const unsigned grid = (unsigned)(((M + TGM - 1) / TGM) * ((N + TGN - 1) / TGN));
-    i2s_gemm_mfma<true><<<grid, TGT, 0, s>>>(w, a, y, (int)M, (int)N, (int)K, (int)K, w_scale, inv);
     return hipGetLastError();
 }
 

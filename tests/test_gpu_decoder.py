@@ -602,3 +602,35 @@ def test_config5_prefill(B, oracle):
     cfg = synth.decoder_config(layers=2, max_seq=72)
     model = scaled_down(synth.decoder_model(cfg, config=93))
     prefill_vs_oracle(cfg, model, B, 64, "f32", oracle, seed=94 + B)
+
+
+# ffn 1100: its last 256-column chunk holds 76 columns and a code row 275 bytes; 1088: 64 columns
+@pytest.mark.parametrize("ffn,batch,P,kv", [(1100, 3, 5, "f32"), (1088, 1, 40, "f32"), (1100, 16, 3, "bf16"),
+                                            (1088, 3, 30, "f32"), (1024, 1, 17, "f32"), (1024, 2, 33, "f32")])
+def test_prompt_rows_and_partial_chunks(ffn, batch, P, kv, oracle):
+    """Prompts of 15 .. 90 rows (the batched GEMVs' groups up to 16 rows, the row
+    kernels from 17 rows on, Q / K / V as one launch of three matrices), and
+    down projections whose rows end within a 256-column chunk (activations
+    padded with zeros by the quantisation), then decode steps; the bars and the
+    scaled-down FFN of test_prefill_chunks_and_gqa."""
+    cfg = synth.decoder_config(**dict(MID, ffn=ffn, max_seq=P + 6, heads=8, kv_heads=4, head_dim=64))
+    model = scaled_down(synth.decoder_model(cfg, config=71, random_gamma=True), 16)
+    prefill_vs_oracle(cfg, model, batch, P, kv, oracle, seed=72, ltol=TOL if kv == "f32" else 1e-3)
+
+
+@pytest.mark.parametrize("ffn,batch", [(1100, 2), (1088, 16)])
+def test_partial_chunks_per_layer(ffn, batch, oracle):
+    """The same down projections in a decode step, int8 activations and products bit for bit."""
+    cfg = synth.decoder_config(**dict(MID, ffn=ffn))
+    model = synth.decoder_model(cfg, config=73, random_gamma=True)
+    print(f"decoder ffn={ffn} batch={batch}", flush=True)
+    prompts = synth.decoder_prompts(cfg, batch, 3, config=74)
+    dec = make(cfg, model, batch)
+    dec.start(prompts)
+    dec.enable_taps()
+    orc = oracle.decoder(oracle_cfg(cfg), model)
+    caches = [orc.new_cache() for _ in range(batch)]
+    for pos in range(3):
+        dec.step(1)
+        check_layers(dec, orc, oracle, cfg, model, caches, prompts, pos)
+    dec.close()
