@@ -248,12 +248,18 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
     }
     if (gemm) {
         // >= 128 tokens: the MFMA GEMM (each weight read once per 128 tokens)
+        // (partial tiles: where the workspace cannot grow, a kernel below that needs less or none)
         void* ws = nullptr;
         const size_t need = mth::oil4_gemm_x32_workspace_bytes(batch, K);
-        const hipError_t e = workspace(S(stream), need, &ws);
-        if (e != hipSuccess) return workspace_fail("mth_oil4_gemv", e, need);
-        return check_launch(mth::launch_oil4_gemm_x32(x, packed, codebooks, cb_block, y, batch, M, K, ws, S(stream)),
-                            "mth_oil4_gemv");
+        if (mth::oil4_whole_tiles(M, K)) {
+            const hipError_t e = workspace(S(stream), need, &ws);
+            if (e != hipSuccess) return workspace_fail("mth_oil4_gemv", e, need);
+        } else {
+            ws = workspace_or_null(S(stream), need);
+        }
+        if (ws)
+            return check_launch(mth::launch_oil4_gemm_x32(x, packed, codebooks, cb_block, y, batch, M, K, ws, S(stream)),
+                                "mth_oil4_gemv");
     }
     if (bt) {
         void* partial = nullptr;
@@ -312,16 +318,27 @@ int mth_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* packed, const u
                     "mth_oil4_gemm_prefill: M=%lld N=%lld K=%lld cb_block=%lld not supported "
                     "(needs K %% 32 == 0, cb_block %% 32 == 0, 16-byte aligned inputs)",
                     (long long)M, (long long)N, (long long)K, (long long)cb_block);
-    // workspace: the per-row shifts of A, then (FP16-A kernels) A in FP16
+    if (mth::oil4_rows_bf16_better(N, K, M, mth::oil4_prefill_us(M, N, K, cb_block))) {
+        if (void* ws = workspace_or_null(S(stream), mth::rows_bf16_workspace_bytes(N, K, M)))
+            return check_launch(mth::launch_oil4_rows_bf16(packed, codebooks, cb_block, a_bf16, c_bf16, N, K, M, ws,
+                                                           S(stream)),
+                                "mth_oil4_gemm_prefill");
+    }
+    // workspace: the per-row shifts of A, then (FP16-A kernels) A in FP16; partial tiles: where it cannot grow to that,
+    // the kernels that need the shifts alone
+    const size_t shifts = mth::oil4_prefill_shift_bytes(M);
     const size_t a16 = mth::oil4_prefill_workspace_bytes(M, N, K, cb_block);
-    const size_t need = mth::oil4_prefill_shift_bytes(M) + a16;
-    void* ws = nullptr;
-    const hipError_t e = workspace(S(stream), need, &ws);
-    if (e != hipSuccess) return workspace_fail("mth_oil4_gemm_prefill", e, need);
-    if (a16)
+    const bool whole = mth::oil4_whole_tiles(N, K);
+    void* ws = a16 && !whole ? workspace_or_null(S(stream), shifts + a16) : nullptr;
+    if (a16 && (ws || whole)) {
+        const hipError_t e = ws ? hipSuccess : workspace(S(stream), shifts + a16, &ws);
+        if (e != hipSuccess) return workspace_fail("mth_oil4_gemm_prefill", e, shifts + a16);
         return check_launch(mth::launch_oil4_gemm_prefill_a16(a_bf16, packed, codebooks, cb_block, c_bf16, M, N, K, ws,
                                                              S(stream)),
                             "mth_oil4_gemm_prefill");
+    }
+    const hipError_t e = workspace(S(stream), shifts, &ws);
+    if (e != hipSuccess) return workspace_fail("mth_oil4_gemm_prefill", e, shifts);
     return check_launch(mth::launch_oil4_gemm_prefill(a_bf16, packed, codebooks, cb_block, c_bf16, M, N, K, (int*)ws,
                                                       S(stream)),
                         "mth_oil4_gemm_prefill");

@@ -14,6 +14,8 @@
 //   * v_mfma_f32_16x16x32_f16 with FP32 accumulation; bf16 (RNE) output.
 // Tile: 128 (m) x 128 (n) x 32 (k) per 256-thread workgroup, 2x2 waves of
 // 64x64, register double-buffered global loads.
+#include <algorithm>
+
 #include "common.h"
 #include "launch.h"
 #include "oil4_common.h"
@@ -33,13 +35,6 @@ __device__ __forceinline__ uint32_t bf16x2_to_f16x2(uint32_t v, int s) {
     const float lo = ldexpf(__uint_as_float(v << 16), s), hi = ldexpf(__uint_as_float(v & 0xffff0000u), s);
     const _Float16 hl = (_Float16)lo, hh = (_Float16)hi;
     return (uint32_t)__builtin_bit_cast(uint16_t, hl) | ((uint32_t)__builtin_bit_cast(uint16_t, hh) << 16);
-}
-
-__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u && (u & 0x007fffffu)) return (uint16_t)((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
 }
 
 // Per-row power-of-two shifts of A (one workgroup per row): rsh[m] = s with
@@ -194,17 +189,6 @@ __device__ __forceinline__ int pf_off(int r, int c) { return r * 128 + 16 * (c ^
 
 // 8 bf16 -> 8 FP16 of a * 2^s (through FP32: v_cvt_pk_f16_f32 rounds to
 // nearest even; exact inside FP16's range)
-__device__ __forceinline__ half8 bf16x8_to_f16(uint4 v, int s) {
-    half8 r;
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        r[2 * i] = (_Float16)ldexpf(__uint_as_float(w[i] << 16), s);
-        r[2 * i + 1] = (_Float16)ldexpf(__uint_as_float(w[i] & 0xffff0000u), s);
-    }
-    return r;
-}
-
 template <int BN>
 struct PfLds {
     static constexpr int a = PBM * 128;  // one A tile (double-buffered)
@@ -394,7 +378,9 @@ __global__ __launch_bounds__(256) void oil4_prefill_a16(const uint16_t* __restri
 // thread of the pair, the halves exchanged with a DPP lane swap.  Workgroups
 // on one XCD share an M tile (WG i runs on XCD i % 8), so an XCD's L2 holds
 // one M tile's rows of A.  C is staged through LDS as bf16 and written in
-// 16-byte pieces.
+// 16-byte pieces.  Partial tiles (EDGE) against the kernels they ran on before
+// (one call): 512 x 14336 x 1664 78 -> 40 us, 512 x 20000 x 4096 217 -> 116,
+// 835 x 8064 x 1664 81 -> 43; FP32 rows, 500 x 14352 x 1920 4523 -> 82.
 template <int BN, int BS, bool X32 = false>
 struct Pf2Lds {
     static constexpr int w = BN * 128;                   // one K step's dequantised W tile
@@ -410,17 +396,20 @@ struct Pf2Lds {
 // CW: consumer waves (4: 64 rows each, one per SIMD; 8: 32 rows each, two per SIMD beside the producer wave);
 // the workgroup has ws_threads(CW) threads.
 constexpr int ws_threads(int cw) { return 64 * (cw + 4); }
-template <int BN, int PA, int BS, bool X32 = false, int CW = 4>
+// EDGE 0: K % 256 == 0 and N % BN == 0; 1: N % 16 == 0, columns past N of the last tile repeat weight row N - 1 and are
+// not stored; 2: that and K % 256 == 128, two steps after the last unrolled four.
+template <int BN, int PA, int BS, bool X32 = false, int CW = 4, int EDGE = 0>
 __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t* __restrict__ A16, const uint8_t* nib,
                                                        const uint16_t* cbs, int cb_block, void* __restrict__ Cv,
                                                        int M, int N, int K, const int* __restrict__ rsh, int Mr = 0) {
     using L = Pf2Lds<BN, BS, X32>;
+    constexpr bool TAIL = EDGE == 2;
     constexpr int NT = BN / 16, PW = 4;
     static_assert(PA == 2 || PA == 4, "A ring index");
     static_assert(BS == 1 || BS == 2 || BS == 4, "barrier interval");
     __shared__ __align__(16) uint8_t lds[L::bytes];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int tm = (M + PBM - 1) / PBM, tn = N / BN;
+    const int tm = (M + PBM - 1) / PBM, tn = EDGE ? (N + BN - 1) / BN : N / BN;
     int mt, nt;
     {
         const int id = blockIdx.x, total = tm * tn;
@@ -434,8 +423,9 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
         }
     }
     const int m0 = mt * PBM, n0 = nt * BN;
-    const int steps = K / PBK;
+    const int steps = K / PBK, steps4 = TAIL ? steps - 2 : steps;
 
+    static_assert(!TAIL || BS <= 2, "the tail's barriers");
     static_assert(CW == 4 || CW == 8, "consumer waves");
     constexpr int NG = 16 / CW;  // 16-row groups per consumer wave
     constexpr int NTH = ws_threads(CW);
@@ -444,7 +434,7 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
         const int t = tid - 64 * CW;
         const bool wt = t < 2 * BN;
         const int wn = t >> 1, wh = t & 1;
-        const int wrow = n0 + (wt ? wn : 0);
+        const int wrow = EDGE ? min(n0 + (wt ? wn : 0), N - 1) : n0 + (wt ? wn : 0);
         const uint8_t* wnib = nib + (int64_t)wrow * (K >> 1) + 16 * wh;
         const uint16_t* wcb = cbs + (int64_t)wrow * (K / cb_block) * 16 + 8 * wh;
         const int pairs = steps >> 1;
@@ -486,7 +476,7 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
             produce(3, I3{});
         }
         __syncthreads();
-        for (int s0 = 0; s0 < steps; s0 += 4) {
+        for (int s0 = 0; s0 < steps4; s0 += 4) {
             // steps s0 + BS .. s0 + 3 + BS while the consumers run s0 .. s0 + 3 (tiles of steps >= steps are unused)
             produce(s0 + BS, std::integral_constant<int, BS % 4>{});
             if constexpr (BS == 1) __syncthreads();
@@ -495,6 +485,13 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
             produce(s0 + 2 + BS, std::integral_constant<int, (2 + BS) % 4>{});
             if constexpr (BS == 1) __syncthreads();
             produce(s0 + 3 + BS, std::integral_constant<int, (3 + BS) % 4>{});
+            __syncthreads();
+        }
+        if constexpr (TAIL) {  // the last two steps
+            if constexpr (BS == 1) {
+                produce(steps4 + 1, I1{});
+                __syncthreads();
+            }
             __syncthreads();
         }
         __syncthreads();  // consumers stage C
@@ -524,6 +521,7 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int step = s0 + u;
+                if (TAIL && u == 2 && step >= steps) break;
                 const uint8_t* cur = lds + (step % (2 * BS)) * L::w;
                 load_a(min(step + PA - 1, steps - 1), (u + PA - 1) % PA);  // into the set of A(step - 1)
 #pragma unroll
@@ -586,7 +584,7 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
             const int c = tid + it * NTH;
             if (c >= 128 * CPR) break;
             const int r = c / CPR, q = c % CPR, row = 128 * mt + r;
-            if (row < Mr) {
+            if (row < Mr && (!EDGE || n0 + 4 * q < N)) {
                 const int sh = shv[it];
                 const float4 hi = *(const float4*)(st + r * BN + 4 * q), lo = *(const float4*)(st + (r + 128) * BN + 4 * q);
                 // oil4_hi_lo: an infinite hi sum (an infinite codebook entry) is the result, as the reference's
@@ -602,7 +600,7 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
         constexpr int CPR = BN * 2 / 16;
         for (int c = tid; c < 256 * CPR; c += NTH) {
             const int r = c / CPR, q = c % CPR;
-            if (m0 + r < M) *(uint4*)(C + (int64_t)(m0 + r) * N + n0 + 8 * q) = *(const uint4*)(st + r * BN + 8 * q);
+            if (m0 + r < M && (!EDGE || n0 + 8 * q < N)) *(uint4*)(C + (int64_t)(m0 + r) * N + n0 + 8 * q) = *(const uint4*)(st + r * BN + 8 * q);
         }
     }
 }
@@ -665,20 +663,23 @@ __global__ __launch_bounds__(256) void oil4_prefill_a16x(const float* __restrict
     }
 }
 
-// BN of oil4_prefill_ws for N (N % BN == 0), best fill of 256 CUs, or 0
-inline int pick_bn_v2(int64_t M, int64_t N) {
+// BN of oil4_prefill_ws: the best fill of 256 CUs among the widths that divide N, or, where none does (N % 16 == 0),
+// among all with the last tile's idle columns counted as idle CUs; 0 for other N.  K % 256 != 0: not 112, whose
+// registers spill around the shorter last round (300 x 14336 x 1664: 69 us, on 128 columns 36)
+inline int pick_bn_v2(int64_t M, int64_t N, int64_t K) {
     const int cand[4] = {128, 112, 96, 64};
     int best = 0;
     double beff = -1.0;
-    for (int bn : cand) {
-        if (N % bn) continue;
-        const int64_t tiles = (N / bn) * ((M + PBM - 1) / PBM);
-        const double eff = (double)tiles / (double)(((tiles + 255) / 256) * 256);
-        if (eff > beff + 1e-9) {
-            beff = eff;
-            best = bn;
+    for (int pass = 0; pass < 2 && best == 0; ++pass)
+        for (int bn : cand) {
+            if ((pass == 0 ? N % bn != 0 : N % 16 != 0) || (bn == 112 && K % (4 * PBK) != 0)) continue;
+            const int64_t tn = (N + bn - 1) / bn, tiles = tn * ((M + PBM - 1) / PBM);
+            const double eff = (double)tiles / (double)(((tiles + 255) / 256) * 256) * (double)N / (double)(tn * bn);
+            if (eff > beff + 1e-9) {
+                beff = eff;
+                best = bn;
+            }
         }
-    }
     return best;
 }
 
@@ -701,18 +702,54 @@ inline int pick_bn(int64_t M, int64_t N) {
 
 }  // namespace
 
-// oil4_prefill_ws serves K % 256 == 0, codebook blocks of a multiple of 128 and an N that one of the tile widths
-// divides; the workspace is A in FP16 fragment order (ceil(M / 16) * 16 rows)
+// oil4_prefill_ws serves K % 128 == 0, codebook blocks of a multiple of 128 and N % 16 == 0; the workspace is A in FP16 fragment order (ceil(M / 16) * 16 rows)
 size_t oil4_prefill_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t cb_block) {
-    const bool v2 = K % (4 * PBK) == 0 && cb_block % (2 * PBK) == 0 && pick_bn_v2(M, N) != 0 && M < (1ll << 31) &&
-                    ((M + PBM - 1) / PBM) * (N / 64) < (1ll << 31) && M * K < (1ll << 40);
+    const bool v2 = K % (2 * PBK) == 0 && cb_block % (2 * PBK) == 0 && pick_bn_v2(M, N, K) != 0 && M < (1ll << 31) &&
+                    ((M + PBM - 1) / PBM) * (N / 64 + 1) < (1ll << 31) && M * K < (1ll << 40);
     return v2 ? (size_t)(((M + 15) / 16) * 16 * K * 2) : 0;
+}
+
+// Measured at 100 .. 2000 tokens: oil4_prefill_ws 10.6 .. 16.5 us per 1024 columns and round of 256 tiles of 64 .. 128
+// columns, oil4_prefill_mfma 27 us, oil4_gemm_prefill_k 36 us per 440 of its 128 x 128 tiles.
+double oil4_prefill_us(int64_t M, int64_t N, int64_t K, int64_t cb_block) {
+    const int64_t tm = (M + PBM - 1) / PBM;
+    auto rounds = [](int64_t tiles) { return (double)((tiles + 255) / 256); };
+    if (oil4_prefill_workspace_bytes(M, N, K, cb_block) != 0) {
+        const int bn = pick_bn_v2(M, N, K);
+        return 6.5 + rounds(tm * ((N + bn - 1) / bn)) * (K / 1024.0) * (5.2 + 0.088 * bn);
+    }
+    if (K % (4 * PBK) == 0 && cb_block % PBK == 0) {
+        const int bn = pick_bn(M, N);
+        return rounds(tm * ((N + bn - 1) / bn)) * (K / 1024.0) * 27.0;
+    }
+    return std::max(1.0, (double)((M + BM - 1) / BM * ((N + BN - 1) / BN)) / 440.0) * (K / 1024.0) * 36.0;
+}
+
+bool oil4_whole_tiles(int64_t N, int64_t K) {
+    return K % (4 * PBK) == 0 && (N % 128 == 0 || N % 112 == 0 || N % 96 == 0 || N % 64 == 0);
 }
 
 size_t oil4_prefill_shift_bytes(int64_t M) { return (size_t)((M * 4 + 255) / 256 * 256); }
 
 static void launch_rowshift(const uint16_t* a_bf16, int* rsh, int64_t M, int64_t K, hipStream_t s) {
     oil4_prefill_rowshift<<<(unsigned)M, 256, 0, s>>>(a_bf16, rsh, (int)M, (int)K);
+}
+
+template <int EDGE>
+static void run_prefill_ws(int bn, unsigned grid, const uint16_t* a16, const uint8_t* nib, const uint16_t* cbs,
+                           int64_t cb_block, uint16_t* c, int64_t M, int64_t N, int64_t K, const int* rsh,
+                           hipStream_t s) {
+    const int cbk = (int)cb_block, m = (int)M, n = (int)N, k = (int)K;
+    constexpr int T4 = ws_threads(4);
+    switch (bn) {
+        case 128: oil4_prefill_ws<128, 2, 1, false, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh); break;
+        case 112:
+            if constexpr (EDGE < 2)
+                oil4_prefill_ws<112, 4, 2, false, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh);
+            break;
+        case 96: oil4_prefill_ws<96, 4, 2, false, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh); break;
+        default: oil4_prefill_ws<64, 4, 2, false, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh); break;
+    }
 }
 
 hipError_t launch_oil4_gemm_prefill_a16(const uint16_t* a_bf16, const uint8_t* nib, const uint16_t* cbs,
@@ -722,16 +759,11 @@ hipError_t launch_oil4_gemm_prefill_a16(const uint16_t* a_bf16, const uint8_t* n
     uint16_t* a16 = (uint16_t*)((char*)ws + oil4_prefill_shift_bytes(M));
     const int64_t groups = (M + 15) / 16;
     oil4_prefill_a16<<<(unsigned)(((groups + 7) / 8) * 128), 256, 0, s>>>(a_bf16, a16, (int)M, (int)K, rsh);
-    const int bn = pick_bn_v2(M, N);
-    const unsigned grid = (unsigned)(((M + PBM - 1) / PBM) * (N / bn));
-    const int cbk = (int)cb_block, m = (int)M, n = (int)N, k = (int)K;
-    constexpr int T4 = ws_threads(4);
-    switch (bn) {
-        case 128: oil4_prefill_ws<128, 2, 1><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c_bf16, m, n, k, rsh); break;
-        case 112: oil4_prefill_ws<112, 4, 2><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c_bf16, m, n, k, rsh); break;
-        case 96: oil4_prefill_ws<96, 4, 2><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c_bf16, m, n, k, rsh); break;
-        default: oil4_prefill_ws<64, 4, 2><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c_bf16, m, n, k, rsh); break;
-    }
+    const int bn = pick_bn_v2(M, N, K);
+    const unsigned grid = (unsigned)(((M + PBM - 1) / PBM) * ((N + bn - 1) / bn));
+    if (K % (4 * PBK) == 0 && N % bn == 0) run_prefill_ws<0>(bn, grid, a16, nib, cbs, cb_block, c_bf16, M, N, K, rsh, s);
+    else if (K % (4 * PBK) == 0) run_prefill_ws<1>(bn, grid, a16, nib, cbs, cb_block, c_bf16, M, N, K, rsh, s);
+    else run_prefill_ws<2>(bn, grid, a16, nib, cbs, cb_block, c_bf16, M, N, K, rsh, s);
     return hipGetLastError();
 }
 
@@ -755,6 +787,41 @@ size_t oil4_gemm_x32_workspace_bytes(int64_t Mr, int64_t K) {
     return oil4_prefill_shift_bytes(Mr) + (size_t)(mv * K * 2);
 }
 
+// 128-column tiles whenever they fill a round of 256 CUs: they halve the
+// A fragment loads per product and the W tile is dequantised for twice the
+// columns per barrier (measured at 1024 rows x 22016 x 4096: 528 -> 461 us
+// against the best-fill 64-column tiles), on 8 consumer waves of 32 rows
+// (two per SIMD: one issues MFMAs while the other waits; 468 -> 434 us;
+// at config 4's 512 x 14336 x 4096 they measured slower, 70 -> 73-78 us)
+static int x32_bn(int64_t tiles, int64_t N, int64_t K) {
+    return (N % 128 == 0 && tiles * (N / 128) >= 256) ? 128 : pick_bn_v2(256 * tiles, N, K);
+}
+
+// 11.7 us (64 columns) .. 15.5 us (128) per 1024 columns and round of 256 tiles
+double oil4_gemm_x32_us(int64_t Mr, int64_t N, int64_t K) {
+    const int64_t tiles = (Mr + 127) / 128;
+    const int bn = x32_bn(tiles, N, K);
+    if (bn == 0) return 1e9;
+    return 5.0 + (double)((tiles * ((N + bn - 1) / bn) + 255) / 256) * (K / 1024.0) * (7.9 + 0.0594 * bn);
+}
+
+template <int EDGE>
+static void run_prefill_x32(int bn, unsigned grid, const uint16_t* a16, const uint8_t* nib, const uint16_t* cbs,
+                            int64_t cb_block, float* c, int64_t mv, int64_t N, int64_t K, const int* rsh, int64_t Mr,
+                            hipStream_t s) {
+    const int cbk = (int)cb_block, m = (int)mv, n = (int)N, k = (int)K, mr = (int)Mr;
+    constexpr int T4 = ws_threads(4), T8 = ws_threads(8);
+    switch (bn) {
+        case 128: oil4_prefill_ws<128, 4, 1, true, 8, EDGE><<<grid, T8, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
+        case 112:
+            if constexpr (EDGE < 2)
+                oil4_prefill_ws<112, 4, 2, true, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr);
+            break;
+        case 96: oil4_prefill_ws<96, 4, 2, true, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
+        default: oil4_prefill_ws<64, 4, 2, true, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
+    }
+}
+
 hipError_t launch_oil4_gemm_x32(const float* a, const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, float* c,
                                 int64_t Mr, int64_t N, int64_t K, void* ws, hipStream_t s) {
     if (!oil4_gemm_x32_supported(Mr, N, K, cb_block)) return hipErrorInvalidValue;
@@ -763,27 +830,13 @@ hipError_t launch_oil4_gemm_x32(const float* a, const uint8_t* nib, const uint16
     const int* rsh = (const int*)ws;
     const uint16_t* a16 = (const uint16_t*)((const char*)ws + oil4_prefill_shift_bytes(Mr));
     const int64_t tiles = (Mr + 127) / 128, mv = 256 * tiles;
-    // 128-column tiles whenever they fill a round of 256 CUs: they halve the
-    // A fragment loads per product and the W tile is dequantised for twice the
-    // columns per barrier (measured at 1024 rows x 22016 x 4096: 528 -> 461 us
-    // against the best-fill 64-column tiles), on 8 consumer waves of 32 rows
-    // (two per SIMD: one issues MFMAs while the other waits; 468 -> 434 us;
-    // at config 4's 512 x 14336 x 4096 they measured slower, 70 -> 73-78 us)
-    const int bn = (N % 128 == 0 && tiles * (N / 128) >= 256) ? 128 : pick_bn_v2(mv, N);
-    const unsigned grid = (unsigned)(tiles * (N / bn));
-    const int cbk = (int)cb_block, m = (int)mv, n = (int)N, k = (int)K, mr = (int)Mr;
-    constexpr int T4 = ws_threads(4);
-    switch (bn) {
-        case 128:
-            oil4_prefill_ws<128, 4, 1, true, 8><<<grid, ws_threads(8), 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr);
-            break;
-        case 112: oil4_prefill_ws<112, 4, 2, true><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
-        case 96: oil4_prefill_ws<96, 4, 2, true><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
-        default: oil4_prefill_ws<64, 4, 2, true><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
-    }
+    const int bn = x32_bn(tiles, N, K);
+    const unsigned grid = (unsigned)(tiles * ((N + bn - 1) / bn));
+    if (K % (4 * PBK) == 0 && N % bn == 0) run_prefill_x32<0>(bn, grid, a16, nib, cbs, cb_block, c, mv, N, K, rsh, Mr, s);
+    else if (K % (4 * PBK) == 0) run_prefill_x32<1>(bn, grid, a16, nib, cbs, cb_block, c, mv, N, K, rsh, Mr, s);
+    else run_prefill_x32<2>(bn, grid, a16, nib, cbs, cb_block, c, mv, N, K, rsh, Mr, s);
     return hipGetLastError();
 }
-
 bool oil4_gemm_prefill_supported(int64_t M, int64_t N, int64_t K, int64_t cb_block) {
     return K % BK == 0 && cb_block % BK == 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31) &&
            (M + BM - 1) / BM < 65536;

@@ -26,7 +26,8 @@
 // full chip, LDS for OIL8 (a step's 256 gathers of ~6 cycles and its B reads, 1.35 us per step for two workgroups a
 // CU at 48 tokens) and half of the MFMA rate for the others (0.83 us).  Measured against the routes before it (one
 // call, eager): OIL8 4000 x 4096, 40 tokens 32.9 -> 19.3 us; 2000 x 8976, 256 tokens 9.9 ms -> 52 us; OIL4 5000 x
-// 9088 (codebooks per 64), 64 tokens 5.4 ms -> 36 us; ternary 4096 x 4096, 300 tokens 5.8 ms -> 36 us.
+// 9088 (codebooks per 64), 64 tokens 5.4 ms -> 36 us; ternary 4096 x 4096, 300 tokens 5.8 ms -> 36 us.  bf16 rows (one
+// part and product): 100 tokens x 1200 x 4096 103 -> 18 us, 160 x 5120 x 4096 50 -> 33 us.
 #include <algorithm>
 
 #include "common.h"
@@ -40,7 +41,10 @@ constexpr int kRmStep = 128;              // columns per step
 constexpr int kRmRows = 128, kRmT = 256;  // weight rows and threads per workgroup
 constexpr int kRmSlices = 16;             // most K slices (rows_reduce_k)
 
-enum RowsFmt { kOil8, kOil4, kTern };
+// kOil4B: OIL4 weights, bf16 token rows (one FP16 part), bf16 outputs
+enum RowsFmt { kOil8, kOil4, kTern, kOil4B };
+template <int FMT>
+constexpr int kParts = FMT == kOil4B ? 1 : 2;  // FP16 parts of a token row
 
 // ---- token rows -> FP16 hi / lo B fragments ------------------------------------
 // Row t: shift s with max|x| 2^s in [2^14, 2^15) into rsh[t] (kRowNonFinite for a row holding Inf / NaN), then
@@ -115,14 +119,49 @@ __global__ __launch_bounds__(kRmT) void rows_split_k(const float* __restrict__ x
     }
 }
 
+// bf16 rows, K % 32 == 0, 16-byte aligned: one part per group (2^s x, rounded to FP16 only 2^-24 below the row's
+// maximum and less); rows with an Inf or a NaN: s = 0, the value in the part.
+__global__ __launch_bounds__(kRmT) void rows_half_k(const uint16_t* __restrict__ x, uint16_t* __restrict__ a16,
+                                                    int* __restrict__ rsh, int K, int chunks) {
+    __shared__ uint32_t red[kRmT / 64];
+    const int tid = threadIdx.x, row = blockIdx.x;
+    const uint16_t* xr = x + (int64_t)row * K;
+    const int n8 = 4 * chunks;  // 8-column pieces, zeros past K
+    auto load = [&](int c) { return 8 * c < K ? ld16(xr + 8 * c) : make_uint4(0, 0, 0, 0); };
+    uint4 v[2 * kRsN];
+#pragma unroll
+    for (int j = 0; j < 2 * kRsN; ++j) v[j] = load(tid + j * kRmT);
+    uint32_t mb = 0;
+    auto most = [&](uint4 w) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mb = max(mb, max(u4get(w, e) & 0x7fffu, (u4get(w, e) >> 16) & 0x7fffu));
+    };
+#pragma unroll
+    for (int j = 0; j < 2 * kRsN; ++j) most(v[j]);
+    for (int c = tid + 2 * kRsN * kRmT; c < n8; c += kRmT) most(load(c));
+    mb = group_reduce<64>(mb, UMaxOp{});
+    if ((tid & 63) == 0) red[tid >> 6] = mb;
+    __syncthreads();
+    const int sh = fp16_scale_shift(__uint_as_float(max(max(red[0], red[1]), max(red[2], red[3])) << 16));
+    if (tid == 0) rsh[row] = sh;
+    uint16_t* dst = a16 + (int64_t)(row >> 4) * chunks * 512 + 8 * (row & 15);
+    auto store = [&](int c, uint4 w) {
+        *(half8*)(dst + (int64_t)(c >> 2) * 512 + 128 * (c & 3)) = bf16x8_to_f16(w, sh);
+    };
+#pragma unroll
+    for (int j = 0; j < 2 * kRsN; ++j)
+        if (tid + j * kRmT < n8) store(tid + j * kRmT, v[j]);
+    for (int c = tid + 2 * kRsN * kRmT; c < n8; c += kRmT) store(c, load(c));
+}
+
 // ---- the product ----------------------------------------------------------------
 struct RowsArgs {
     const uint8_t* w;      // OIL8 indices [M][K], OIL4 nibbles [M][K / 2], ternary codes [M][K / 4]
     const void* cb;        // OIL8: 256 floats; OIL4: FP16 codebooks
     const uint16_t* a16;   // rows_split_k's fragments
     const int* rsh;
-    const float* x;        // [batch][K]
-    float* out;            // [batch][M] (ternary: [M][batch])
+    const float* x;        // [batch][K] (FP32 rows)
+    float* out;            // [batch][M] (ternary: [M][batch]; kOil4B: bf16)
     float* partial;        // [slice] of the same
     int M, K, batch, steps, cb_block;
 };
@@ -148,6 +187,8 @@ template <>
 struct RowsTile<kOil4> {
     uint4 n, c0, c1;  // the lane's row: nibbles of columns 32 q .., its block's 16 entries
 };
+template <>
+struct RowsTile<kOil4B> : RowsTile<kOil4> {};
 template <>
 struct RowsTile<kTern> {
     uint2 c;  // the lane's row: codes of columns 32 q ..
@@ -179,7 +220,7 @@ __device__ float rows_fma(const RowsArgs& p, int row, int tok, int k0, int k1) {
         const uint8_t* w = p.w + (int64_t)row * p.K;
         const float* cb = (const float*)p.cb;
         for (int k = k0; k < k1; ++k) s = fmaf(cb[w[k]], x[k], s);
-    } else if constexpr (FMT == kOil4) {
+    } else if constexpr (FMT == kOil4 || FMT == kOil4B) {
         const uint8_t* w = p.w + (int64_t)row * (p.K >> 1);
         const uint16_t* cb = (const uint16_t*)p.cb;
         for (int k = k0; k < k1; ++k) {
@@ -199,8 +240,10 @@ __device__ float rows_fma(const RowsArgs& p, int row, int tok, int k0, int k1) {
 
 template <int FMT, int G>
 __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) {
-    constexpr int NB = 2 * G;  // 16-byte pieces of a step's B per thread (8 KB per token group)
-    __shared__ __align__(16) uint8_t bs[G * 8192];
+    constexpr int P = kParts<FMT>;
+    constexpr bool O4 = FMT == kOil4 || FMT == kOil4B;
+    constexpr int NB = P * G;  // 16-byte pieces of a step's B per thread (4 KB per token group and part)
+    __shared__ __align__(16) uint8_t bs[P * G * 4096];
     __shared__ uint32_t tab[FMT == kOil8 ? 256 : 1];
     __shared__ float wred[kRmT / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -234,7 +277,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
                 const int col = min(kRmStep * st + 16 * (2 * q + (j >> 3)), K - 16);
                 dst[t].x = ld_stream(p.w + (int64_t)min(row0 + 16 * t + (j & 7), M - 1) * K + col);
                 dst[t].y = ld_stream(p.w + (int64_t)min(row0 + 16 * t + 8 + (j & 7), M - 1) * K + col);
-            } else if constexpr (FMT == kOil4) {
+            } else if constexpr (O4) {
                 const int64_t row = min(row0 + 16 * t + j, M - 1);
                 const int col = min(kRmStep * st + 32 * q, K - 32);
                 dst[t].n = ld_stream(p.w + row * (K >> 1) + (col >> 1));
@@ -251,7 +294,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
     uint4 bv[NB];
     // B: thread's pieces tid + 256 i of [group][part][4 KB of the step's 4 chunks]
     const int64_t part_bytes = (int64_t)p.steps * 4096;
-    const uint8_t* a16 = (const uint8_t*)p.a16 + (int64_t)(tok0 >> 4) * 2 * part_bytes + 16 * tid;
+    const uint8_t* a16 = (const uint8_t*)p.a16 + (int64_t)(tok0 >> 4) * P * part_bytes + 16 * tid;
     auto load_b = [&](int step) {
         const uint8_t* base = a16 + (int64_t)min(step, s1 - 1) * 4096;
 #pragma unroll
@@ -277,12 +320,12 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
         if (lane == 0) wred[wave] = m;
     }
 #pragma unroll
-    for (int g = 0; g < G; ++g) fin = fin && rs[g] != kRowNonFinite;
+    for (int g = 0; g < G; ++g) fin = fin && (FMT == kOil4B || rs[g] != kRowNonFinite);
     const bool special = __syncthreads_or(!fin) != 0;
     const int64_t zs = (int64_t)p.batch * M;
     float* out = S == 1 ? p.out : p.partial + blockIdx.z * zs;
     auto at = [&](int row, int tok) { return FMT == kTern ? (int64_t)row * p.batch + tok : (int64_t)tok * M + row; };
-    if (special) {
+    if (FMT != kOil4B && special) {
         const int k0 = kRmStep * s0, k1 = min(K, kRmStep * s1), r0 = bx * kRmRows;
         for (int o = tid; o < kRmRows * 16 * G; o += kRmT) {
             const int row = r0 + o % kRmRows, tok = tok0 + o / kRmRows;
@@ -296,7 +339,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
         tab[tid] = rows_hl(ldexpf(cbv, sw));
     }
     CbPlanes shared_planes;
-    if constexpr (FMT == kOil4)
+    if constexpr (O4)
         if (!p.cb_block) shared_planes = cb_planes(wt[0][0].c0, wt[0][0].c1);
 
     floatx4 ah[2][G], ax[2][G];  // hi x hi; the other products
@@ -324,7 +367,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
                                    dpp_mix<0xc>(cur[t].x.z, cur[t].y.z), dpp_mix<0xc>(cur[t].x.w, cur[t].y.w));
                 wb[t] = make_uint4(dpp_mix<0x3>(cur[t].y.x, cur[t].x.x), dpp_mix<0x3>(cur[t].y.y, cur[t].x.y),
                                    dpp_mix<0x3>(cur[t].y.z, cur[t].x.z), dpp_mix<0x3>(cur[t].y.w, cur[t].x.w));
-            } else if constexpr (FMT == kOil4) {
+            } else if constexpr (O4) {
                 pl[t] = p.cb_block ? cb_planes(cur[t].c0, cur[t].c1) : shared_planes;
                 if (kRmStep * step + 32 * q >= K) {  // columns past the row: weight 0 (an Inf entry would meet 0)
 #pragma unroll
@@ -340,8 +383,8 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
             half8 bh[G], bl[G];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                bh[g] = *(const half8*)(brow + g * 8192 + 256 * m);
-                bl[g] = *(const half8*)(brow + g * 8192 + 4096 + 256 * m);
+                bh[g] = *(const half8*)(brow + g * P * 4096 + 256 * m);
+                if constexpr (P == 2) bl[g] = *(const half8*)(brow + g * 8192 + 4096 + 256 * m);
             }
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
@@ -363,7 +406,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
                     }
                     Ah = __builtin_bit_cast(half8, hv);
                     Al = __builtin_bit_cast(half8, lv);
-                } else if constexpr (FMT == kOil4) {
+                } else if constexpr (O4) {
                     Ah = lookup8_natural(u4get(cur[t].n, m), pl[t]);
                 } else {
                     Ah = rows_tern8(m < 2 ? cur[t].c.x : cur[t].c.y, 2 * (m & 1));
@@ -371,7 +414,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
                     ah[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh[g], ah[t][g], 0, 0, 0);
-                    ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bl[g], ax[t][g], 0, 0, 0);
+                    if constexpr (P == 2) ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bl[g], ax[t][g], 0, 0, 0);
                     if constexpr (FMT == kOil8)
                         ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, bh[g], ax[t][g], 0, 0, 0);
                 }
@@ -396,7 +439,24 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
             float v[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                v[i] = ldexpf(FMT == kOil8 ? ah[t][g][i] + ax[t][g][i] : oil4_hi_lo(ah[t][g][i], ax[t][g][i]), -sh);
+                v[i] = ldexpf(P == 1 ? ah[t][g][i]
+                              : FMT == kOil8 ? ah[t][g][i] + ax[t][g][i] : oil4_hi_lo(ah[t][g][i], ax[t][g][i]), -sh);
+            if constexpr (FMT == kOil4B) {
+                if (S == 1) {
+                    uint16_t* d16 = (uint16_t*)p.out + (int64_t)tok * M + row;
+                    uint16_t h[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) h[i] = f32_to_bf16_rne(v[i]);
+                    if (row + 3 < M && ((uintptr_t)d16 & 7u) == 0) {
+                        *(uint2*)d16 = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (row + i < M) d16[i] = h[i];
+                    }
+                    continue;
+                }
+            }
             float* dst = out + at(row, tok);
             if (FMT != kTern && row + 3 < M && ((uintptr_t)dst & 15u) == 0) {
                 *(float4*)dst = make_float4(v[0], v[1], v[2], v[3]);
@@ -410,8 +470,8 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
 }
 
 // out[i] = sum over slices z = 0, 1, ... of partial[z][i] (a fixed order); all loads before the first add.  Four
-// values per thread where both arrays are 16-byte aligned (n % 4 == 0).  gridDim.y > 1: sg's matrix blockIdx.y.
-template <bool VEC>
+// values per thread where both arrays are 16-byte aligned (n % 4 == 0).  HALF: out is bf16.  gridDim.y > 1: sg's matrix blockIdx.y.
+template <bool VEC, bool HALF = false>
 __global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ partial, float* __restrict__ out,
                                                       int64_t n, int S, RowsSegs sg, int batch) {
     const int64_t i = ((int64_t)blockIdx.x * kRmT + threadIdx.x) * (VEC ? 4 : 1);
@@ -430,7 +490,11 @@ __global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ 
 #pragma unroll
         for (int z = 1; z < kRmSlices; ++z)
             if (z < S) s = make_float4(s.x + v[z].x, s.y + v[z].y, s.z + v[z].z, s.w + v[z].w);
-        *(float4*)(out + i) = s;
+        if constexpr (HALF)
+            *(uint2*)((uint16_t*)out + i) = make_uint2(f32_to_bf16_rne(s.x) | ((uint32_t)f32_to_bf16_rne(s.y) << 16),
+                                                       f32_to_bf16_rne(s.z) | ((uint32_t)f32_to_bf16_rne(s.w) << 16));
+        else
+            *(float4*)(out + i) = s;
     } else {
         float v[kRmSlices];
 #pragma unroll
@@ -439,7 +503,8 @@ __global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ 
 #pragma unroll
         for (int z = 1; z < kRmSlices; ++z)
             if (z < S) s += v[z];
-        out[i] = s;
+        if constexpr (HALF) ((uint16_t*)out)[i] = f32_to_bf16_rne(s);
+        else out[i] = s;
     }
 }
 
@@ -466,20 +531,24 @@ inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch, int nseg = 1) {
     return p;
 }
 inline size_t al256r(size_t n) { return (n + 255) & ~(size_t)255; }
-inline size_t rows_a16_bytes(const RowsPlan& p) { return (size_t)p.tiles * p.G * 2 * p.steps * 4096; }
+inline size_t rows_a16_bytes(const RowsPlan& p, int parts = 2) {
+    return (size_t)p.tiles * p.G * parts * p.steps * 4096;
+}
 
 template <int FMT>
 hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s, const RowsSegs& sg = RowsSegs{}) {
     int64_t n = (int64_t)a.M * a.batch;
     uint16_t* a16 = (uint16_t*)ws;
-    int* rsh = (int*)((char*)ws + rows_a16_bytes(p));
+    int* rsh = (int*)((char*)ws + rows_a16_bytes(p, kParts<FMT>));
     float* partial = (float*)((char*)rsh + al256r((size_t)a.batch * 4));
     a.a16 = a16;
     a.rsh = rsh;
     a.partial = partial;
     a.steps = p.steps;
     const bool vec = ((uintptr_t)a.x & 15u) == 0 && a.K % 4 == 0;
-    if (vec)
+    if constexpr (FMT == kOil4B)
+        rows_half_k<<<(unsigned)a.batch, kRmT, 0, s>>>((const uint16_t*)a.x, a16, rsh, a.K, 4 * p.steps);
+    else if (vec)
         rows_split_k<FMT == kTern, true><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps);
     else
         rows_split_k<FMT == kTern, false><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps);
@@ -501,11 +570,12 @@ hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s, cons
             }
         }
         const unsigned ny = sg.n > 1 ? sg.n : 1;
+        constexpr bool HALF = FMT == kOil4B;
         if (vec4)
-            rows_reduce_k<true><<<dim3((unsigned)((n / 4 + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S,
+            rows_reduce_k<true, HALF><<<dim3((unsigned)((n / 4 + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S,
                                                                                                  sg, a.batch);
         else
-            rows_reduce_k<false><<<dim3((unsigned)((n + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S, sg,
+            rows_reduce_k<false, HALF><<<dim3((unsigned)((n + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S, sg,
                                                                                               a.batch);
     }
     return hipGetLastError();
@@ -521,6 +591,11 @@ inline bool rows_sizes(int64_t M, int64_t K, int64_t batch) {
 size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch, int nseg) {
     const RowsPlan p = rows_plan(M, K, batch, nseg);
     return rows_a16_bytes(p) + al256r((size_t)batch * 4) + (p.S > 1 ? (size_t)(p.S * M * batch * 4) : 0);
+}
+
+size_t rows_bf16_workspace_bytes(int64_t M, int64_t K, int64_t batch) {
+    const RowsPlan p = rows_plan(M, K, batch);
+    return rows_a16_bytes(p, 1) + al256r((size_t)batch * 4) + (p.S > 1 ? (size_t)(p.S * M * batch * 4) : 0);
 }
 
 // ---- which route: estimated microseconds (eager calls, MI355X) ------------------
@@ -564,21 +639,14 @@ bool oil8_rows_better(const Oil8Seg* seg, int nseg, int64_t K, int64_t batch, bo
     return us < walk_us(M, K, batch, true, aligned && K <= 4096);
 }
 
-// OIL4: K % 32 == 0, codebook blocks of a multiple of 32 columns, 16-byte aligned weights.  Wider GEMM tiles (128
-// columns, 15.5 us per 1024 columns and round) as launch_oil4_gemm_x32 picks them.
+// OIL4: K % 32 == 0, codebook blocks of a multiple of 32 columns, 16-byte aligned weights.
 bool oil4_rows_better(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, int64_t M, int64_t K, int64_t batch,
                       bool aligned, bool gemm, bool bt) {
     if (!rows_sizes(M, K, batch) || K % 32 != 0 || cb_block % 32 != 0 || cb_block >= (1 << 30) ||
         (((uintptr_t)nib | (uintptr_t)cbs) & 15u) != 0)
         return false;
     const double us = rows_us(M, K, batch, 1.85);
-    if (gemm) {
-        const int64_t tiles = (batch + 127) / 128;
-        const bool w128 = M % 128 == 0;
-        const int64_t t = tiles * (M / (w128 ? 128 : 64));
-        const double g = 5.0 + (w128 && t >= 128 ? 15.5 : 11.7) * (K / 1024.0) * ((t + 255) / 256);
-        return us < g;
-    }
+    if (gemm) return us < oil4_gemm_x32_us(batch, M, K);
     if (bt) return batch > 16;  // 17 tokens: 18 .. 49 us against 15 .. 48 us
     return us < walk_us(M, K, batch, false, aligned && K <= 4096);
 }
@@ -588,6 +656,19 @@ bool oil4_rows_better(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block,
 bool tern_rows_better(int64_t M, int64_t K, int64_t batch) {
     return rows_sizes(M, K, batch) && K % 4 == 0 && M * (K / 4) >= 8 &&
            K * std::max(1.0, (double)M * batch / 8000.0) > 4000.0;
+}
+
+// bf16 prompt rows (M: weight rows), K % 32 == 0 and codebook blocks of a multiple of 32 columns: against the tiled
+// kernels' estimate (oil4_prefill_us).  Here 13.5 us for any little work, 3 us for the slice reduction, 1.05 us per step
+// of a 128 x 64 tile on the busiest CU (measured at 100 .. 2000 tokens x 1200 .. 28672 x 1664 .. 8192: within 15 %, hence the
+// margin).  Few tokens or rows: the tiled kernels' 256-token tiles leave CUs idle and split no K (158 x 5120 x 3840:
+// 47 us there, 33 here; 300 x 14336 x 3840: 68 and 105).
+bool oil4_rows_bf16_better(int64_t M, int64_t K, int64_t batch, double tiled_us) {
+    if (!rows_sizes(M, K, batch) || K % 32 != 0) return false;
+    const RowsPlan p = rows_plan(M, K, batch);
+    const double most = (double)((p.rtiles * p.tiles * p.S + 255) / 256);  // workgroups on the busiest CU
+    const double us = 13.5 + (p.S > 1 ? 3.0 : 0.0) + 1.05 * most * p.steps / p.S;
+    return 1.12 * us < tiled_us;
 }
 
 hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, void* ws,
@@ -616,6 +697,12 @@ hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_
                             int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s) {
     RowsArgs a{nib, cbs, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, (int)cb_block};
     return rows_run<kOil4>(a, rows_plan(M, K, batch), ws, s);
+}
+hipError_t launch_oil4_rows_bf16(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const uint16_t* x,
+                                 uint16_t* y, int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s) {
+    RowsArgs a{nib, cbs, nullptr, nullptr, (const float*)x, (float*)y, nullptr, (int)M, (int)K, (int)batch, 0,
+               (int)cb_block};
+    return rows_run<kOil4B>(a, rows_plan(M, K, batch), ws, s);
 }
 hipError_t launch_tern_rows(const uint8_t* w, const float* x, float* out, int64_t M, int64_t K, int64_t batch,
                             void* ws, hipStream_t s) {

@@ -186,6 +186,10 @@ size_t oil4_prefill_shift_bytes(int64_t M);
 hipError_t launch_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* nib, const uint16_t* cbs,
                                     int64_t cb_block, uint16_t* c_bf16,
                                     int64_t M, int64_t N, int64_t K, int* rsh, hipStream_t s);
+bool oil4_whole_tiles(int64_t N, int64_t K);  // no partial tile of columns or round of K steps
+double oil4_gemm_x32_us(int64_t Mr, int64_t N, int64_t K);  // launch_oil4_gemm_x32's
+// the tiled prompt kernels' estimated time (microseconds), for oil4_rows_bf16_better
+double oil4_prefill_us(int64_t M, int64_t N, int64_t K, int64_t cb_block);
 bool oil4_gemm_prefill_supported(int64_t M, int64_t N, int64_t K, int64_t cb_block);
 // The FP16-A kernels (oil4_prefill_a16 + oil4_prefill_ws) for K % 256 == 0, cb_block % 64 == 0
 // and N a multiple of 64, 96, 112 or 128: needs a workspace of
@@ -233,6 +237,11 @@ size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch, int nseg =
 bool oil8_rows_better(const Oil8Seg* seg, int nseg, int64_t K, int64_t batch, bool aligned, bool gemm, bool bt);
 bool oil4_rows_better(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, int64_t M, int64_t K, int64_t batch,
                       bool aligned, bool gemm, bool bt);
+// bf16 rows in, bf16 out; ws: rows_bf16_workspace_bytes.  tiled_us: oil4_prefill_us of the shape
+bool oil4_rows_bf16_better(int64_t M, int64_t K, int64_t batch, double tiled_us);
+size_t rows_bf16_workspace_bytes(int64_t M, int64_t K, int64_t batch);
+hipError_t launch_oil4_rows_bf16(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const uint16_t* x,
+                                 uint16_t* y, int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s);
 bool tern_rows_better(int64_t M, int64_t K, int64_t batch);
 hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, void* ws,
                             hipStream_t s);

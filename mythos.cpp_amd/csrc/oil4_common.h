@@ -274,4 +274,23 @@ struct Oil4TileLoads {
     }
 };
 
+__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
+    uint32_t u = __float_as_uint(f);
+    if ((u & 0x7f800000u) == 0x7f800000u && (u & 0x007fffffu)) return (uint16_t)((u >> 16) | 0x40u);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return (uint16_t)(u >> 16);
+}
+
+// eight bf16 -> FP16 of a * 2^s
+__device__ __forceinline__ half8 bf16x8_to_f16(uint4 v, int s) {
+    half8 r;
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        r[2 * i] = (_Float16)ldexpf(__uint_as_float(w[i] << 16), s);
+        r[2 * i + 1] = (_Float16)ldexpf(__uint_as_float(w[i] & 0xffff0000u), s);
+    }
+    return r;
+}
+
 }  // namespace mth

@@ -272,3 +272,108 @@ def test_argmax_rows(rows, n, oracle, mth, dev):
     mth.argmax(to_dev(x, dev), ids, rows, n)
     torch.cuda.synchronize()
     assert ids.cpu().tolist() == [oracle.argmax(r) for r in x]
+
+
+# ---------------------------------------------------------- bf16 prompts --
+# one token and one row; one past and one short of a 128 x 64 tile; odd row counts (2-byte aligned output rows); a last
+# step of 32 and of 96 columns, codebooks per 32; K split over workgroups and not
+@pytest.mark.parametrize("M,N,K,block", [(1, 1, 32, 32), (15, 127, 96, 32), (17, 129, 256, 64), (64, 128, 1120, 32),
+                                         (65, 130, 4192, 32), (130, 60, 640, 128), (200, 9000, 160, 32)])
+def test_prefill_rows(M, N, K, block, mth, dev):
+    """mth_oil4_gemm_prefill on the row kernel, rows of very different magnitudes: the bars of test_gpu_prefill."""
+    import torch
+    from test_gpu_prefill import check
+    print(f"prefill rows M={M} N={N} K={K} block={block}", flush=True)
+    a, packed, cbs = synth.prefill(M, N, K, block)
+    A = torch.from_numpy(synth.bf16_to_f32(a).reshape(M, K)) * torch.exp2(torch.arange(M) % 41 - 20.0)[:, None]
+    c = torch.zeros(M * N, dtype=torch.bfloat16, device=dev)
+    mth.oil4_gemm_prefill(A.bfloat16().to(dev), to_dev(packed, dev), to_dev(cbs, dev), block, c, M, N, K)
+    torch.cuda.synchronize()
+    W = synth.dequant_oil4(packed, cbs, N, K, block).astype(np.float64)
+    A = A.bfloat16().double().numpy()
+    check(c.view(torch.int16).cpu().numpy().view(np.uint16).reshape(M, N), A @ W.T, np.abs(A) @ np.abs(W).T, "rows")
+
+
+# 16 tokens; row counts that pick every tile width with a last tile of 16 columns and more: 64 (1616), 96 (24016),
+# 112 (28016, 128 where K % 256 != 0), 128 (32016); K of two steps, of whole rounds of four and two past them
+@pytest.mark.parametrize("x32", [False, True])
+@pytest.mark.parametrize("M,N,K", [(16, 1616, 128), (300, 1616, 640), (16, 24016, 256), (16, 24016, 384),
+                                   (16, 28016, 512), (16, 28016, 384), (16, 32016, 256), (16, 32016, 384),
+                                   (1100, 4096, 384)])
+def test_prefill_tile_edges(M, N, K, x32, mth, dev):
+    """The tiled prompt kernels (bf16 rows; FP32 rows of hi and lo parts) where the last tile or the last round of steps
+    is partial.  FP32 rows: the parts keep 2^-22 of a product and the sums round less than K / 16 times."""
+    import ctypes as C
+    import torch
+    from test_gpu_prefill import check
+    print(f"prefill tile edges M={M} N={N} K={K} x32={x32}", flush=True)
+    a, packed, cbs = synth.prefill(M, N, K, 128)
+    A = torch.from_numpy(synth.bf16_to_f32(a).reshape(M, K).copy())
+    if x32:
+        A = A * (1.0 + torch.rand(M, K, generator=torch.Generator().manual_seed(K)))
+    L, P = mth.lib, C.c_void_p
+    size = {}
+    for name, sym, n in (("ws", "_ZN3mth28oil4_prefill_workspace_bytesEllll", 4), ("shift", "_ZN3mth24oil4_prefill_shift_bytesEl", 1),
+                         ("x32", "_ZN3mth29oil4_gemm_x32_workspace_bytesEll", 2)):
+        f = getattr(L, sym)
+        f.argtypes, f.restype = [C.c_int64] * n, C.c_size_t
+        size[name] = f
+    f = (L._ZN3mth20launch_oil4_gemm_x32EPKfPKhPKtlPflllPvP12ihipStream_t if x32 else
+         L._ZN3mth28launch_oil4_gemm_prefill_a16EPKtPKhS1_lPtlllPvP12ihipStream_t)
+    f.argtypes, f.restype = [P, P, P, C.c_int64, P, C.c_int64, C.c_int64, C.c_int64, P, P], C.c_int
+    need = size["x32"](M, K) if x32 else size["shift"](M) + size["ws"](M, N, K, 128)
+    assert need > 0
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    x = A.to(dev) if x32 else A.bfloat16().to(dev)
+    w, cb = to_dev(packed, dev), to_dev(cbs, dev)
+    c = torch.full((M * N + 64,), float("nan"), dtype=torch.float32 if x32 else torch.bfloat16, device=dev)
+    assert f(x.data_ptr(), w.data_ptr(), cb.data_ptr(), 128, c.data_ptr(), M, N, K, ws.data_ptr(),
+             torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(c[M * N:]).all())
+    W = torch.from_numpy(synth.dequant_oil4(packed, cbs, N, K, 128)).to(dev).double()
+    xd = x.double()
+    ref, absw = (xd @ W.T.contiguous()).cpu().numpy(), (xd.abs() @ W.abs().T.contiguous()).cpu().numpy()
+    got = c[:M * N].cpu().reshape(M, N)
+    if x32:
+        assert bool((np.abs(got.double().numpy() - ref) <= (K / 16 + 8) * 2.0 ** -24 * absw).all())
+    else:
+        check(got.view(torch.int16).numpy().view(np.uint16), ref, absw, "tile edges")
+
+
+@pytest.mark.parametrize("entry", ["prefill", "gemv"])
+def test_partial_tiles_under_capture(entry, mth, dev):
+    """A capture on a stream whose workspace holds the row shifts alone: partial tiles take the kernels that need no
+    more, and every replay gives the same values."""
+    import torch
+    from test_gpu_prefill import check
+    M, N, K = 300, 7056, 384
+    print(f"partial tiles under capture {entry}", flush=True)
+    a, packed, cbs = synth.prefill(M, N, K, 128)
+    w, cb = to_dev(packed, dev), to_dev(cbs, dev)
+    A = torch.from_numpy(synth.bf16_to_f32(a).reshape(M, K).copy()).to(dev)
+    x = A.bfloat16() if entry == "prefill" else A
+    c = torch.zeros(M * N, dtype=x.dtype, device=dev)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    mth.workspace_reserve((4 * M + 255) // 256 * 256, stream=s)
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr, stream=s):
+        if entry == "prefill":
+            mth.oil4_gemm_prefill(x, w, cb, 128, c, M, N, K)
+        else:
+            mth.oil4_gemv(w, cb, 128, x, c, N, K, M)
+    W = torch.from_numpy(synth.dequant_oil4(packed, cbs, N, K, 128)).to(dev).double()
+    ref = (A.double() @ W.T.contiguous()).cpu().numpy()
+    absw = (A.double().abs() @ W.abs().T.contiguous()).cpu().numpy()
+    for rep in range(3):
+        c.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            gr.replay()
+        torch.cuda.synchronize()
+        got = c.cpu().reshape(M, N)
+        if entry == "prefill":
+            check(got.view(torch.int16).numpy().view(np.uint16), ref, absw, f"replay {rep}")
+        else:
+            assert bool((np.abs(got.double().numpy() - ref) <= (K / 16 + 8) * 2.0 ** -24 * absw).all()), rep
