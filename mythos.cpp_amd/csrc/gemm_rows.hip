@@ -607,6 +607,13 @@ double rows_us(int64_t M, int64_t K, int64_t batch, double step_us) {
     const double steps = (double)p.rtiles * p.tiles * p.steps / 256.0;
     return 14.8 + std::max(steps * step_us * (p.G + 1) / 5.0 - 4.0, 0.0);
 }
+// the same for whole rounds of a full chip, against a tiled GEMM: the busiest CU's steps, and the slices' partial sums
+// written and read (within 15 % at 128 .. 512 tokens x 4096 .. 32000 x 2048 .. 4096)
+double rows_busy_us(int64_t M, int64_t K, int64_t batch, double step_us) {
+    const RowsPlan p = rows_plan(M, K, batch);
+    const double most = (double)((p.rtiles * p.tiles * p.S + 255) / 256);
+    return 10.8 + most * p.steps / p.S * step_us * (p.G + 1) / 5.0 + (p.S > 1 ? 2e-6 * p.S * M * batch : 0.0);
+}
 // the kernels that walk tokens one after another (a launch of their own: 8.7 us eagerly).  Measured at M = 512 ..
 // 16384, 1 .. 16 tokens: OIL8 rows of up to 4096 0.98 .. 11.9 us per token, OIL4 rows of up to 2048 / 4096 1.85 / 3.9
 // us per token up to 4400 rows, longer rows (one wave per output) 2.8 / 3.2 us per 1024 columns up to 1600 / 2900 rows
@@ -627,14 +634,15 @@ bool oil8_rows_better(const Oil8Seg* seg, int nseg, int64_t K, int64_t batch, bo
         M += seg[i].rows;
     }
     if (!rows_sizes(M, K, batch) || K % 16 != 0) return false;
-    const double us = rows_us(M, K, batch, 1.7);
     if (gemm) {
-        // a round of 256 tiles of 128 x 64 (54 us at K = 4096), or of 256 x 64 where those fill the chip (98 us)
+        // a round of 256 tiles of 128 x 64 (54 us at K = 4096), or of 256 x 64 where those fill the chip (98 us; 384
+        // tiles, 476 tokens x 12288, 150 us, and 204 us here)
         const int64_t t = M / 64, wide = (batch + 255) / 256 * t, narrow = (batch + 127) / 128 * t;
-        const double g = wide >= 256 ? 5.0 + 23.3 * (K / 1024.0) * ((wide + 255) / 256)
+        const double g = wide >= 256 ? 5.0 + 23.3 * (K / 1024.0) * (wide / 256.0)
                                      : 5.0 + (12.2 + narrow / 110.0) * (K / 1024.0);
-        return us < g;
+        return 1.05 * rows_busy_us(M, K, batch, 1.7) < g;
     }
+    const double us = rows_us(M, K, batch, 1.7);
     if (bt) return batch > 16;  // 17 tokens: 19 .. 49 us against 15 .. 31 us
     return us < walk_us(M, K, batch, true, aligned && K <= 4096);
 }
@@ -645,8 +653,8 @@ bool oil4_rows_better(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block,
     if (!rows_sizes(M, K, batch) || K % 32 != 0 || cb_block % 32 != 0 || cb_block >= (1 << 30) ||
         (((uintptr_t)nib | (uintptr_t)cbs) & 15u) != 0)
         return false;
+    if (gemm) return 1.05 * rows_busy_us(M, K, batch, 1.6) < oil4_gemm_x32_us(batch, M, K);
     const double us = rows_us(M, K, batch, 1.85);
-    if (gemm) return us < oil4_gemm_x32_us(batch, M, K);
     if (bt) return batch > 16;  // 17 tokens: 18 .. 49 us against 15 .. 48 us
     return us < walk_us(M, K, batch, false, aligned && K <= 4096);
 }
