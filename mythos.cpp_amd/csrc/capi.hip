@@ -96,12 +96,29 @@ hipError_t workspace(hipStream_t s, size_t need, void** out) {
 }
 
 // The stream's workspace for a faster route that the call can do without: null where it cannot grow now (the
-// stream is capturing, or the allocation failed), and the call then takes the route that needs less.
-void* workspace_or_null(hipStream_t s, size_t need) {
+// stream is capturing, or the allocation failed), and the call then takes the route that needs less.  graphs: whether
+// a captured call may use what the stream holds; not for calls that need no workspace on the other route, whose graphs
+// may be replayed beside other work of the stream they were captured on.
+void* workspace_or_null(hipStream_t s, size_t need, bool graphs) {
     void* p = nullptr;
+    if (!graphs) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
     if (workspace(s, need, &p) == hipSuccess) return p;
     (void)hipGetLastError();
     return nullptr;
+}
+
+// Held while a call enqueues the launches that hand data on through the workspace: threads that share a stream do not
+// come between them.  One of 64 locks by stream.
+std::mutex& ws_launches(hipStream_t s) {
+    static std::mutex mu[64];
+    const uintptr_t v = (uintptr_t)s;
+    return mu[((v >> 6) ^ (v >> 12) ^ (v >> 18)) & 63u];
 }
 
 int workspace_fail(const char* what, hipError_t e, size_t need) {
@@ -188,6 +205,7 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
     REQUIRE(indices && codebook && x && y, "mth_oil8_gemv: null pointer");
     REQUIRE(M > 0 && K > 0 && batch > 0 && M < kMaxDim && K < kMaxDim && batch <= 65536,
             "mth_oil8_gemv: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const bool aligned = (((uintptr_t)indices | (uintptr_t)x) & 15u) == 0;
     const mth::Oil8Seg seg{indices, codebook, y, M};
     const bool gemm = aligned && batch >= kGemmRows && mth::oil8_gemm_x32_supported(&seg, 1, batch, K);
@@ -195,7 +213,7 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
     const bool one = batch == 1 && aligned &&  // one token: kernels of their own up to 16384 columns
                      ((K % 16 == 0 && K <= 4096 && M * K < (1ll << 32)) || mth::oil8_long_supported(indices, x, M, K));
     if (!one && mth::oil8_rows_better(&seg, 1, K, batch, aligned, gemm, bt)) {
-        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch)))
+        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), batch > 1))
             return check_launch(mth::launch_oil8_rows(&seg, 1, x, K, batch, ws, S(stream)),
                                 "mth_oil8_gemv");
     }
@@ -235,15 +253,17 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
     REQUIRE(cb_block >= 0, "mth_oil4_gemv: cb_block=%lld < 0", (long long)cb_block);
     REQUIRE(cb_block == 0 || K % cb_block == 0, "mth_oil4_gemv: K=%lld not a multiple of cb_block=%lld",
             (long long)K, (long long)cb_block);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const bool aligned = (((uintptr_t)packed | (uintptr_t)codebooks | (uintptr_t)x) & 15u) == 0;
     const bool gemm = aligned && ((uintptr_t)y & 15u) == 0 && batch >= kGemmRows &&
                       mth::oil4_gemm_x32_supported(batch, M, K, cb_block);
     const bool bt = aligned && mth::oil4_bt_supported(M, K, cb_block, batch);
     const bool one = batch == 1 && aligned &&  // one token: kernels of their own
                      (K <= 4096 || mth::oil4_one_supported(packed, codebooks, x, cb_block, M, K));
+    const bool redo = !bt && !(gemm && mth::oil4_whole_tiles(M, K));
     if (!one && mth::oil4_rows_better(packed, codebooks, cb_block, M, K, batch, aligned, gemm, bt)) {
-        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch)))
-            return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, ws, S(stream)),
+        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), batch > 1))
+            return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, redo, ws, S(stream)),
                                 "mth_oil4_gemv");
     }
     if (gemm) {
@@ -255,7 +275,7 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
             const hipError_t e = workspace(S(stream), need, &ws);
             if (e != hipSuccess) return workspace_fail("mth_oil4_gemv", e, need);
         } else {
-            ws = workspace_or_null(S(stream), need);
+            ws = workspace_or_null(S(stream), need, true);
         }
         if (ws)
             return check_launch(mth::launch_oil4_gemm_x32(x, packed, codebooks, cb_block, y, batch, M, K, ws, S(stream)),
@@ -312,6 +332,7 @@ int mth_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* packed, const u
     REQUIRE(K % 2 == 0, "mth_oil4_gemm_prefill: K=%lld must be even", (long long)K);
     REQUIRE(cb_block > 0 && K % cb_block == 0, "mth_oil4_gemm_prefill: K=%lld not a multiple of cb_block=%lld",
             (long long)K, (long long)cb_block);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const bool aligned = (((uintptr_t)a_bf16 | (uintptr_t)packed | (uintptr_t)codebooks | (uintptr_t)c_bf16) & 15u) == 0;
     if (!aligned || !mth::oil4_gemm_prefill_supported(M, N, K, cb_block))
         return fail(MTH_EUNSUPPORTED,
@@ -319,7 +340,7 @@ int mth_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* packed, const u
                     "(needs K %% 32 == 0, cb_block %% 32 == 0, 16-byte aligned inputs)",
                     (long long)M, (long long)N, (long long)K, (long long)cb_block);
     if (mth::oil4_rows_bf16_better(N, K, M, mth::oil4_prefill_us(M, N, K, cb_block))) {
-        if (void* ws = workspace_or_null(S(stream), mth::rows_bf16_workspace_bytes(N, K, M)))
+        if (void* ws = workspace_or_null(S(stream), mth::rows_bf16_workspace_bytes(N, K, M), true))
             return check_launch(mth::launch_oil4_rows_bf16(packed, codebooks, cb_block, a_bf16, c_bf16, N, K, M, ws,
                                                            S(stream)),
                                 "mth_oil4_gemm_prefill");
@@ -329,7 +350,7 @@ int mth_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* packed, const u
     const size_t shifts = mth::oil4_prefill_shift_bytes(M);
     const size_t a16 = mth::oil4_prefill_workspace_bytes(M, N, K, cb_block);
     const bool whole = mth::oil4_whole_tiles(N, K);
-    void* ws = a16 && !whole ? workspace_or_null(S(stream), shifts + a16) : nullptr;
+    void* ws = a16 && !whole ? workspace_or_null(S(stream), shifts + a16, true) : nullptr;
     if (a16 && (ws || whole)) {
         const hipError_t e = ws ? hipSuccess : workspace(S(stream), shifts + a16, &ws);
         if (e != hipSuccess) return workspace_fail("mth_oil4_gemm_prefill", e, shifts + a16);
@@ -373,8 +394,9 @@ int mth_i2s_gemv(const uint8_t* packed, float w_scale, const int8_t* act, const 
     REQUIRE(M > 0 && K > 0 && batch > 0 && M < kMaxDim && K < (1ll << 24) && batch <= 65536,
             "mth_i2s_gemv: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
     REQUIRE(K % 4 == 0, "mth_i2s_gemv: K=%lld must be a multiple of 4", (long long)K);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     if (mth::i2s_rows_supported(packed, act, false, M, K, batch)) {
-        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch)))
+        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch), batch > 1))
             return check_launch(mth::launch_i2s_rows(packed, w_scale, nullptr, act, act_scale, y, M, K, batch, ws,
                                                      S(stream)),
                                 "mth_i2s_gemv");
@@ -399,8 +421,9 @@ int mth_i2s_gemv_f32(const uint8_t* packed, float w_scale, const float* x, float
     REQUIRE(M > 0 && K > 0 && batch > 0 && M < kMaxDim && K < (1ll << 24) && batch <= 65536,
             "mth_i2s_gemv_f32: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
     REQUIRE(K % 4 == 0, "mth_i2s_gemv_f32: K=%lld must be a multiple of 4", (long long)K);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     if (mth::i2s_rows_supported(packed, x, true, M, K, batch)) {
-        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch)))
+        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch), false))
             return check_launch(mth::launch_i2s_rows(packed, w_scale, x, nullptr, nullptr, y, M, K, batch, ws,
                                                      S(stream)),
                                 "mth_i2s_gemv_f32");
@@ -413,8 +436,9 @@ int mth_i2s_gemm(const uint8_t* w, const float* act, float* out, int64_t M, int6
                  mth_stream_t stream) {
     REQUIRE(w && act && out, "mth_i2s_gemm: null pointer");
     REQUIRE(M > 0 && N > 0 && K > 0 && M * N < kMaxDim && K < kMaxDim, "mth_i2s_gemm: bad sizes");
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     if (mth::tern_rows_better(M, K, N)) {
-        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, N)))
+        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, N), false))
             return check_launch(mth::launch_tern_rows(w, act, out, M, K, N, ws, S(stream)), "mth_i2s_gemm");
     }
     return check_launch(mth::launch_i2s_gemm(w, act, out, M, N, K, S(stream)), "mth_i2s_gemm");
@@ -439,6 +463,7 @@ int mth_tl2_gemm(const uint8_t* w, const float* act, float* out, int64_t M, int6
     REQUIRE(w && act && out, "mth_tl2_gemm: null pointer");
     REQUIRE(M > 0 && N > 0 && K > 0 && M * N < kMaxDim && K < (1ll << 24), "mth_tl2_gemm: bad sizes");
     REQUIRE(K % 3 == 0, "mth_tl2_gemm: K=%lld must be a multiple of 3", (long long)K);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const size_t need = mth::tl2_workspace_bytes(w, M, N, K);
     if (need) {
         void* ws = nullptr;
@@ -528,6 +553,7 @@ int mth_oil4_gemv_swiglu_batch(const uint8_t* packed, const uint16_t* codebooks,
             "mth_oil4_gemv_swiglu_batch: F=%lld K=%lld cb_block=%lld not supported (F %% 4 == 0, K %% 512 == 0, "
             "512 <= K <= 8192, cb_block 0 or 128)",
             (long long)F, (long long)K, (long long)cb_block);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     void* partial = nullptr;
     const size_t need = mth::oil4_bt_partial_bytes(2 * F, K);
     const hipError_t e = workspace(S(stream), need, &partial);
@@ -548,6 +574,7 @@ int mth_i2s_gemv_act_batch(const uint8_t* packed, float w_scale, const float* ac
     REQUIRE((((uintptr_t)packed | (uintptr_t)act) & 15u) == 0,
             "mth_i2s_gemv_act_batch: packed and act must be 16-byte aligned");
     REQUIRE(mth::i2s_bt_supported(M, K, batch), "mth_i2s_gemv_act_batch: K=%lld not a multiple of 256", (long long)K);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     void* partial = nullptr;
     const size_t need = mth::i2s_bt_partial_bytes(M, K);
     const hipError_t e = workspace(S(stream), need, &partial);
@@ -667,10 +694,11 @@ int mth_attention_decode(const float* q, const float* kcache, const float* vcach
             (long long)head_dim, (long long)max_seq);
     REQUIRE(ctx >= 1 && ctx <= max_seq, "mth_attention_decode: ctx=%lld outside 1..%lld", (long long)ctx,
             (long long)max_seq);
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     if (mth::attention_split_supported(q, kcache, vcache, batch, (int)heads, (int)kv_heads, (int)head_dim, (int)ctx,
                                        (int)max_seq)) {
         if (void* ws = workspace_or_null(S(stream), mth::attention_split_workspace_bytes(batch, (int)heads, (int)kv_heads,
-                                                                                         (int)head_dim, (int)ctx)))
+                                                                                         (int)head_dim, (int)ctx), false))
             return check_launch(mth::launch_attention_split(q, kcache, vcache, out, (int)ctx, batch, (int)heads,
                                                             (int)kv_heads, (int)head_dim, (int)max_seq, ws, S(stream)),
                                 "mth_attention_decode");
@@ -683,6 +711,7 @@ int mth_attention_decode(const float* q, const float* kcache, const float* vcach
 int mth_argmax(const float* logits, int32_t* ids, int64_t rows, int64_t n, mth_stream_t stream) {
     REQUIRE(logits && ids, "mth_argmax: null pointer");
     REQUIRE(rows > 0 && rows <= 65535 && n > 0 && n < (1ll << 31), "mth_argmax: bad sizes");
+    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     void* ws = nullptr;
     const size_t nc = (size_t)mth::argmax_chunks(n) * (size_t)rows;
     const hipError_t e = workspace(S(stream), nc * 8, &ws);

@@ -97,7 +97,7 @@ hipError_t oil4(const mth_decoder* d, const uint8_t* w, const uint16_t* cb, cons
     const bool bt = aligned && mth::oil4_bt_supported(M, K, d->c.cb_block, rows);
     if (prompt && mth::oil4_rows_better(w, cb, d->c.cb_block, M, K, rows, aligned, false, bt) &&
         mth::rows_mfma_workspace_bytes(M, K, rows) <= d->pf_ws_bytes)
-        return mth::launch_oil4_rows(w, cb, d->c.cb_block, x, y, M, K, rows, d->pf_ws, s);
+        return mth::launch_oil4_rows(w, cb, d->c.cb_block, x, y, M, K, rows, !bt, d->pf_ws, s);
     if (bt)
         return mth::launch_oil4_gemv_bt(w, cb, d->c.cb_block, x, y, M, K, rows, d->bt_partial, s);
     return mth::launch_oil4_gemv(w, cb, d->c.cb_block, x, y, M, K, rows, s);

@@ -12,7 +12,10 @@
 // lo x lo lies below FP32's rounding).  Products are exact in FP32, sums FP32
 // on v_mfma_f32_16x16x32_f16, the hi x hi products and the rest in accumulators
 // of their own.  A token tile that holds Inf or NaN, or a non-finite OIL8
-// codebook, takes FP32 FMAs over the reference's products instead.
+// codebook, takes FP32 FMAs over the reference's products instead, as does an
+// OIL4 output that comes out NaN (redo: shapes that no other FP16 hi / lo
+// kernel takes, which give NaN where infinite entries meet such values).  bf16 rows are one FP16 part, as
+// in the tiled prompt kernels.
 //
 // Tiling.  A workgroup of 4 waves takes 128 weight rows (32 per wave: two A
 // tiles share every B read, which otherwise bounds the kernel: a tile-step
@@ -164,6 +167,7 @@ struct RowsArgs {
     float* out;            // [batch][M] (ternary: [M][batch]; kOil4B: bf16)
     float* partial;        // [slice] of the same
     int M, K, batch, steps, cb_block;
+    bool redo;             // kOil4: FP32 products for an output that comes out NaN
 };
 // OIL8: up to three matrices over the same token rows (a decoder's Q, K and V), their row tiles one after another in
 // the grid; t1: the first row tile past matrix i.  Matrix i's partial sums start at partial + p0[i].
@@ -441,6 +445,13 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
             for (int i = 0; i < 4; ++i)
                 v[i] = ldexpf(P == 1 ? ah[t][g][i]
                               : FMT == kOil8 ? ah[t][g][i] + ax[t][g][i] : oil4_hi_lo(ah[t][g][i], ax[t][g][i]), -sh);
+            if constexpr (FMT == kOil4) {
+                // NaN: also an infinite entry times a value whose parts are 0, where the reference's product is infinite
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (p.redo && v[i] != v[i] && row + i < M)
+                        v[i] = rows_fma<FMT>(p, row + i, tok, kRmStep * s0, min(K, kRmStep * s1));
+            }
             if constexpr (FMT == kOil4B) {
                 if (S == 1) {
                     uint16_t* d16 = (uint16_t*)p.out + (int64_t)tok * M + row;
@@ -702,8 +713,8 @@ hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_
     return rows_run<kOil8>(a, p, ws, s, sg);
 }
 hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
-                            int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s) {
-    RowsArgs a{nib, cbs, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, (int)cb_block};
+                            int64_t M, int64_t K, int64_t batch, bool redo, void* ws, hipStream_t s) {
+    RowsArgs a{nib, cbs, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, (int)cb_block, redo};
     return rows_run<kOil4>(a, rows_plan(M, K, batch), ws, s);
 }
 hipError_t launch_oil4_rows_bf16(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const uint16_t* x,

@@ -377,3 +377,27 @@ def test_partial_tiles_under_capture(entry, mth, dev):
             check(got.view(torch.int16).numpy().view(np.uint16), ref, absw, f"replay {rep}")
         else:
             assert bool((np.abs(got.double().numpy() - ref) <= (K / 16 + 8) * 2.0 ** -24 * absw).all()), rep
+
+
+def test_token_rows_oil4_infinite_entry(mth, dev):
+    """An infinite codebook entry times values 2^-60 below their row's largest (0 in both FP16 parts): +-Inf, as one
+    FP32 product gives, and NaN where entries of both signs meet."""
+    import torch
+    M, K, batch = 130, 1120, 20
+    print("token rows OIL4 infinite entry", flush=True)
+    g = np.random.default_rng(8)
+    nib = g.integers(2, 16, (M, K), dtype=np.uint8)          # entries 0 (+Inf) and 1 (-Inf) only where placed
+    nib[3, 100] = nib[129, 1119] = nib[5, 40] = 0
+    nib[7, 64] = nib[5, 1000] = 1
+    cb = g.normal(0, 0.02, 16).astype(np.float16)
+    cb[0], cb[1] = np.inf, -np.inf
+    x = (1.0 + g.random((batch, K))).astype(np.float32)
+    x[:, [100, 1119, 40, 64, 1000]] = 2.0 ** -60
+    y = empty(batch * M, torch.float32, dev)
+    mth.oil4_gemv(to_dev(nib[:, 0::2] | (nib[:, 1::2] << 4), dev), to_dev(cb.view(np.uint16), dev), 0, to_dev(x, dev), y,
+                  M, K, batch)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().reshape(batch, M)
+    assert (got[:, [3, 129]] == np.inf).all() and (got[:, 7] == -np.inf).all() and np.isnan(got[:, 5]).all()
+    rest = [m for m in range(M) if m not in (3, 5, 7, 129)]
+    assert np.isfinite(got[:, rest]).all()
