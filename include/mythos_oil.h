@@ -14,20 +14,28 @@
  * 4 * K bytes per token rounded up to 128 (OIL4) or 256 (OIL8) tokens,
  * plus 4 bytes per token),
  * mth_argmax, mth_oil4_gemm_prefill (per-row shifts of A,
- * 4 bytes per row, and an FP16 copy of A in MFMA fragment order,
- * ceil(M/16)*16*K*2 bytes, for K % 256 == 0, codebook blocks of a multiple
- * of 128 and N a multiple of 64, 96 or 112), mth_tl2_gemm (each activation
+ * 4 bytes per row rounded up to 256 in all, and an FP16 copy of A in MFMA
+ * fragment order, ceil(M/16)*16*K*2 bytes, for K % 256 == 0, codebook blocks
+ * of a multiple of 128 and N a multiple of 64, 96 or 112), mth_tl2_gemm (each activation
  * row quantised once: N * ceil(K/4) * 4 bytes plus 4 bytes per row, when
  * ceil(K/4) % 16 == 0) keep intermediate data in a device workspace
  * the library owns, one per (device, stream).  The first call that needs more
  * than the stream's workspace holds allocates a larger one (hipMalloc, at
  * least double the old size) and retires the old block WITHOUT freeing it, so
  * work queued earlier and HIP graphs captured earlier from that stream keep
- * valid addresses until the process ends.  No other entry point allocates.
+ * valid addresses until the process ends.
  * Inside a stream capture a call never allocates: if the workspace is too
  * small it fails with MTH_EUNSUPPORTED, so reserve the size beforehand with
  * mth_workspace_reserve (or make one uncaptured call of the largest shape).
- * Calls on one stream share its workspace; a captured graph uses the
+ * Some sizes have a faster route that keeps more there: the calls above at
+ * odd sizes and token counts, mth_attention_decode over long contexts,
+ * mth_i2s_gemm, mth_i2s_gemv_f32 and single-token calls of odd sizes.  Such a
+ * call never fails for want of it: where the workspace cannot grow it runs as
+ * the sizes above say.  mth_attention_decode, mth_i2s_gemm, mth_i2s_gemv_f32
+ * and single-token calls use no workspace at all inside a capture.  No other
+ * entry point allocates.
+ * Calls on one stream share its workspace (threads may share the stream: a
+ * call's launches are enqueued together); a captured graph uses the
  * workspace of the stream it was captured on and must not be replayed
  * concurrently with other work that uses that stream's workspace.
  *
@@ -83,11 +91,11 @@ int mth_oil8_gemm(const uint8_t* indices, const float* codebook, const float* ac
 /* Decode GEMV over one OIL8 weight matrix shared by `batch` tokens (the
  * reference's oil8_gemm with N = 1, once per token, src/kernel_oil8.cpp:30-60):
  *   y[t*M + m] = sum_k codebook[indices[m*K + k]] * x[t*K + k],  t < batch.
- * Fast path: K % 16 == 0, K <= 4096, indices and x 16-byte aligned.  Batches
- * of >= 128 tokens with M % 64 == 0, K % 256 == 0 and 16-byte aligned y run
+ * Fast path: K % 16 == 0 and 16-byte aligned indices; batch 1: up to 16384
+ * columns, and a 16-byte aligned x.  Batches of >= 128 tokens with M % 64 == 0, K % 256 == 0 and 16-byte aligned y may run
  * as the prompt prefill's MFMA GEMM (FP16 hi / lo parts of x and codebook,
- * FP32 sums: the FP32 bar; rows or codebooks holding Inf / NaN take FP32
- * products). */
+ * FP32 sums: the FP32 bar, as for every batch; rows or codebooks holding Inf
+ * / NaN take FP32 products). */
 int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x, float* y,
                   int64_t M, int64_t K, int64_t batch, mth_stream_t stream);
 
@@ -108,11 +116,12 @@ int mth_oil4_gemm(const uint8_t* packed, const uint16_t* codebook, const float* 
  *   y[t*M + m] = sum_k f32(codebooks[(m*(K/cb_block) + k/cb_block)*16 + nib(m,k)]) * x[t*K + k]
  * packed: M rows of K/2 bytes, nibble order as above.  cb_block = 0 selects
  * a single shared 16-entry codebook.  Requires K even and, for cb_block > 0,
- * K % cb_block == 0.  Fast path: K % 32 == 0, K <= 4096, cb_block % 32 == 0,
- * 16-byte aligned packed / codebooks / x.  Batches of >= 128 tokens with
- * cb_block a multiple of 128, K % 256 == 0, M a multiple of 64, 96, 112 or
- * 128 and 16-byte aligned y run as the prompt prefill's MFMA GEMM (FP16 hi /
- * lo parts of x, FP32 sums). */
+ * K % cb_block == 0.  Fast path: K % 32 == 0, cb_block % 32 == 0, 16-byte
+ * aligned packed / codebooks; batch 1: K <= 4096, or codebooks per 128 columns
+ * (cb_block 128 or 0) and K up to 16384, and a 16-byte aligned x.  Batches of
+ * >= 128 tokens with cb_block a multiple of 128, K % 128 == 0, M % 16 == 0 and
+ * 16-byte aligned y may run as the prompt prefill's MFMA GEMM (FP16 hi / lo
+ * parts of x, FP32 sums). */
 int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_block,
                   const float* x, float* y, int64_t M, int64_t K, int64_t batch,
                   mth_stream_t stream);
@@ -120,7 +129,9 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
 /* mth_oil4_gemv for callers that cannot allocate device memory (code under
  * HIP graph capture, serving loops, harnesses that forbid hipMalloc).  No
  * counterpart in the reference (its CPU kernels need no scratch).  Same
- * arguments, results and kernels as mth_oil4_gemv; the batched path's K-slice
+ * arguments as mth_oil4_gemv and the same results up to FP32 rounding (bit
+ * for bit up to 16 tokens where K % 512 == 0); batches above 16 tokens run
+ * in groups of 16, odd sizes token by token.  The batched path's K-slice
  * partial sums (16 tokens x M rows x K/1024 slices of FP32 for K >= 2048)
  * live in a fixed 8 MiB device array per GPU instead of the workspace, and
  * the call never allocates.  Shapes whose partial sums exceed 8 MiB (e.g.
@@ -143,7 +154,9 @@ int mth_oil4_gemv_noalloc(const uint8_t* packed, const uint16_t* codebooks, int6
  * exactly before its bf16 rounding, so activations of any magnitude keep
  * their bits.  K % 32 == 0, cb_block % 32 == 0, 16-byte aligned inputs
  * (MTH_EUNSUPPORTED otherwise).  Uses the stream's workspace (4 bytes per row
- * of A, plus an FP16 copy of A for the tile shapes above). */
+ * of A, plus an FP16 copy of A for the tile shapes above, and where it can
+ * grow also for N % 16 == 0 with K % 128 == 0 and for few rows or columns,
+ * there with the K slices' partial sums). */
 int mth_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* packed, const uint16_t* codebooks,
                           int64_t cb_block, uint16_t* c_bf16, int64_t M, int64_t N, int64_t K,
                           mth_stream_t stream);
@@ -172,7 +185,8 @@ int mth_i2s_gemv(const uint8_t* packed, float w_scale, const int8_t* act, const 
                  float* y, int64_t M, int64_t K, int64_t batch, mth_stream_t stream);
 
 /* Fused decode op: quantize_per_token(x_t) then mth_i2s_gemv with
- * act_scale = inv_scale, in one launch.  Requires K % 4 == 0.  Bit-exact. */
+ * act_scale = inv_scale (one launch for little work; else the tokens are
+ * quantised once, then int8 MFMA).  Requires K % 4 == 0.  Bit-exact. */
 int mth_i2s_gemv_f32(const uint8_t* packed, float w_scale, const float* x, float* y,
                      int64_t M, int64_t K, int64_t batch, mth_stream_t stream);
 
