@@ -35,7 +35,10 @@
  * and single-token calls use no workspace at all inside a capture.  No other
  * entry point allocates.
  * Calls on one stream share its workspace (threads may share the stream: a
- * call's launches are enqueued together); a captured graph uses the
+ * call's launches are enqueued together).  hipStreamPerThread is one handle
+ * for a stream of its own in every thread: the routes that a call can do
+ * without are not taken there, and calls that need the workspace must come
+ * from one thread.  A captured graph uses the
  * workspace of the stream it was captured on and must not be replayed
  * concurrently with other work that uses that stream's workspace.
  *

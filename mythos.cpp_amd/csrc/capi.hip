@@ -98,9 +98,11 @@ hipError_t workspace(hipStream_t s, size_t need, void** out) {
 // The stream's workspace for a faster route that the call can do without: null where it cannot grow now (the
 // stream is capturing, or the allocation failed), and the call then takes the route that needs less.  graphs: whether
 // a captured call may use what the stream holds; not for calls that need no workspace on the other route, whose graphs
-// may be replayed beside other work of the stream they were captured on.
+// may be replayed beside other work of the stream they were captured on.  hipStreamPerThread: null, since that one
+// handle is another stream in every thread, and a block kept by handle would be shared by streams that run together.
 void* workspace_or_null(hipStream_t s, size_t need, bool graphs) {
     void* p = nullptr;
+    if (s == hipStreamPerThread) return nullptr;
     if (!graphs) {
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {

@@ -140,6 +140,43 @@ def test_attention_split_specials(mth, dev):
         assert ((got - want).norm() / want.norm()).item() <= 4e-6
 
 
+def test_attention_on_per_thread_streams(mth, dev):
+    """hipStreamPerThread is one handle for a stream per thread: long-context
+    attention of four threads at once on it, each on its own queries."""
+    import threading
+    import types
+    import torch
+    B, H, KVH, D, ctx, n, reps = 2, 32, 8, 128, 1500, 4, 20
+    print("attention on per-thread streams", flush=True)
+    g = torch.Generator(device=dev).manual_seed(9)
+    q = torch.randn(n, B, H, D, generator=g, device=dev)
+    kc, vc = (torch.randn(B, KVH, ctx, D, generator=g, device=dev) for _ in range(2))
+    out = torch.full((n, reps, B, H, D), float("nan"), device=dev)
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(i):
+        try:
+            for r in range(reps):
+                mth.attention_decode(q[i], kc, vc, out[i, r], B, H, KVH, D, ctx, ctx,
+                                     stream=types.SimpleNamespace(cuda_stream=2))
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(n)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    k, v = (x.double()[:, torch.arange(H, device=dev) % KVH] for x in (kc, vc))
+    for i in range(n):
+        p = torch.softmax((k * q[i].double()[:, :, None, :]).sum(-1) / D ** 0.5, -1)
+        want = (p[..., None] * v).sum(-2)
+        assert bool(((out[i].double() - want).norm(dim=(-1, -2)) <= 4e-6 * want.norm(dim=(-1, -2))).all()), i
+
+
 # ----------------------------------------------------- token rows on MFMA --
 def w64(kind, w, cb, M, K, blk, dev):
     """[M][K] float64 weights."""

@@ -1,0 +1,64 @@
+"""Which kernels a call launches and what it keeps in the workspace, with the
+HIP runtime replaced by a recorder (recorded.py): no GPU.
+"""
+import itertools
+
+import recorded
+
+W, CB, X, Y, Z = (0x100000000000 * (i + 1) for i in range(5))   # 16-byte aligned device addresses, never touched
+ROWS = ("rows_split", "rows_half", "rows_mfma", "rows_reduce")
+PER_THREAD = 2                                                   # hipStreamPerThread
+stream = itertools.count(0x10000, 0x100)                         # a fresh stream: no workspace yet
+
+
+def oil8(M, K, b, s, x=X):
+    return {"fn": "mth_oil8_gemv", "args": [W, CB, x, Y, M, K, b, s]}
+
+
+def oil4(M, K, b, s, blk=128):
+    return {"fn": "mth_oil4_gemv", "args": [W, CB, blk, X, Y, M, K, b, s]}
+
+
+def i2s(M, K, b, s):
+    return {"fn": "mth_i2s_gemv", "args": [W, 1.0, X, CB, Y, M, K, b, s]}
+
+
+def i2s_f32(M, K, b, s):
+    return {"fn": "mth_i2s_gemv_f32", "args": [W, 1.0, X, Y, M, K, b, s]}
+
+
+def i2s_gemm(M, N, K, s):
+    return {"fn": "mth_i2s_gemm", "args": [W, X, Y, M, N, K, s]}
+
+
+def attention(b, h, kvh, D, ctx, s):
+    return {"fn": "mth_attention_decode", "args": [X, W, CB, Y, b, h, kvh, D, ctx, ctx, s]}
+
+
+def kernels(r):
+    assert r["rc"] == 0, r["error"]
+    return [n for n, _ in r["kernels"]]
+
+
+def on(r, *names):
+    """Whether one of the call's kernels has one of these names in its own."""
+    return any(n in k for k in kernels(r) for n in names)
+
+
+# one call of each entry point whose other route keeps nothing in the workspace, and its workspace kernels
+def without_workspace(s):
+    return [(attention(2, 32, 8, 128, 6000, s), "attn_split_k"), (i2s_gemm(4096, 300, 4096, s), "rows_mfma_k"),
+            (i2s_f32(4096, 11008, 16, s), "i2s_quant_rows_k"), (oil8(64, 17024, 1, s), "rows_mfma_k"),
+            (oil4(7529, 10240, 1, s, 64), "rows_mfma_k")]
+
+
+def test_per_thread_stream_shares_no_workspace():
+    """hipStreamPerThread is one handle for a stream of its own in every
+    thread: calls that can do without the workspace, which is kept by handle,
+    do so there."""
+    calls = without_workspace(PER_THREAD)
+    for (c, name), r in zip(calls, recorded.run([c for c, _ in calls])):
+        assert not on(r, name) and r["mallocs"] == 0, (c, kernels(r))
+    calls = without_workspace(next(stream))                      # an ordinary stream: the route with workspace
+    for (c, name), r in zip(calls, recorded.run([c for c, _ in calls])):
+        assert on(r, name), (c, kernels(r))
