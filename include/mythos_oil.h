@@ -122,9 +122,9 @@ int mth_oil4_gemm(const uint8_t* packed, const uint16_t* codebook, const float* 
  * K % cb_block == 0.  Fast path: K % 32 == 0, cb_block % 32 == 0, 16-byte
  * aligned packed / codebooks; batch 1: K <= 4096, or codebooks per 128 columns
  * (cb_block 128 or 0) and K up to 16384, and a 16-byte aligned x.  Batches of
- * >= 128 tokens with cb_block a multiple of 128, K % 128 == 0, M % 16 == 0 and
- * 16-byte aligned y may run as the prompt prefill's MFMA GEMM (FP16 hi / lo
- * parts of x, FP32 sums). */
+ * >= 128 tokens with cb_block a multiple of 128, K % 256 == 0, M a multiple of
+ * 64, 96 or 112 and 16-byte aligned y may run as the prompt prefill's MFMA GEMM
+ * (FP16 hi / lo parts of x, FP32 sums). */
 int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_block,
                   const float* x, float* y, int64_t M, int64_t K, int64_t batch,
                   mth_stream_t stream);

@@ -262,26 +262,20 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
     const bool bt = aligned && mth::oil4_bt_supported(M, K, cb_block, batch);
     const bool one = batch == 1 && aligned &&  // one token: kernels of their own
                      (K <= 4096 || mth::oil4_one_supported(packed, codebooks, x, cb_block, M, K));
-    const bool redo = !bt && !(gemm && mth::oil4_whole_tiles(M, K));
     if (!one && mth::oil4_rows_better(packed, codebooks, cb_block, M, K, batch, aligned, gemm, bt)) {
         if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), batch > 1))
-            return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, redo, ws, S(stream)),
+            return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, !bt && !gemm, ws,
+                                                      S(stream)),
                                 "mth_oil4_gemv");
     }
     if (gemm) {
         // >= 128 tokens: the MFMA GEMM (each weight read once per 128 tokens)
-        // (partial tiles: where the workspace cannot grow, a kernel below that needs less or none)
         void* ws = nullptr;
         const size_t need = mth::oil4_gemm_x32_workspace_bytes(batch, K);
-        if (mth::oil4_whole_tiles(M, K)) {
-            const hipError_t e = workspace(S(stream), need, &ws);
-            if (e != hipSuccess) return workspace_fail("mth_oil4_gemv", e, need);
-        } else {
-            ws = workspace_or_null(S(stream), need, true);
-        }
-        if (ws)
-            return check_launch(mth::launch_oil4_gemm_x32(x, packed, codebooks, cb_block, y, batch, M, K, ws, S(stream)),
-                                "mth_oil4_gemv");
+        const hipError_t e = workspace(S(stream), need, &ws);
+        if (e != hipSuccess) return workspace_fail("mth_oil4_gemv", e, need);
+        return check_launch(mth::launch_oil4_gemm_x32(x, packed, codebooks, cb_block, y, batch, M, K, ws, S(stream)),
+                            "mth_oil4_gemv");
     }
     if (bt) {
         void* partial = nullptr;

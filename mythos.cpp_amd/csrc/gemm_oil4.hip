@@ -380,7 +380,7 @@ __global__ __launch_bounds__(256) void oil4_prefill_a16(const uint16_t* __restri
 // one M tile's rows of A.  C is staged through LDS as bf16 and written in
 // 16-byte pieces.  Partial tiles (EDGE) against the kernels they ran on before
 // (one call): 512 x 14336 x 1664 78 -> 40 us, 512 x 20000 x 4096 217 -> 116,
-// 835 x 8064 x 1664 81 -> 43; FP32 rows, 500 x 14352 x 1920 4523 -> 82.
+// 835 x 8064 x 1664 81 -> 43.
 template <int BN, int BS, bool X32 = false>
 struct Pf2Lds {
     static constexpr int w = BN * 128;                   // one K step's dequantised W tile
@@ -426,6 +426,7 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
     const int steps = K / PBK, steps4 = TAIL ? steps - 2 : steps;
 
     static_assert(!TAIL || BS <= 2, "the tail's barriers");
+    static_assert(!X32 || EDGE == 0, "FP32 rows: whole tiles");
     static_assert(CW == 4 || CW == 8, "consumer waves");
     constexpr int NG = 16 / CW;  // 16-row groups per consumer wave
     constexpr int NTH = ws_threads(CW);
@@ -584,7 +585,7 @@ __global__ __launch_bounds__(ws_threads(CW)) void oil4_prefill_ws(const uint16_t
             const int c = tid + it * NTH;
             if (c >= 128 * CPR) break;
             const int r = c / CPR, q = c % CPR, row = 128 * mt + r;
-            if (row < Mr && (!EDGE || n0 + 4 * q < N)) {
+            if (row < Mr) {
                 const int sh = shv[it];
                 const float4 hi = *(const float4*)(st + r * BN + 4 * q), lo = *(const float4*)(st + (r + 128) * BN + 4 * q);
                 // oil4_hi_lo: an infinite hi sum (an infinite codebook entry) is the result, as the reference's
@@ -779,7 +780,8 @@ hipError_t launch_prefill_a16x(const float* a, int64_t Mr, int64_t K, void* ws, 
 
 bool oil4_gemm_x32_supported(int64_t Mr, int64_t N, int64_t K, int64_t cb_block) {
     const int64_t mv = 256 * ((Mr + 127) / 128);
-    return Mr >= 1 && cb_block > 0 && oil4_prefill_workspace_bytes(mv, N, K, cb_block) != 0 && K <= (1 << 20);
+    return Mr >= 1 && cb_block > 0 && oil4_whole_tiles(N, K) && oil4_prefill_workspace_bytes(mv, N, K, cb_block) != 0 &&
+           K <= (1 << 20);
 }
 
 size_t oil4_gemm_x32_workspace_bytes(int64_t Mr, int64_t K) {
@@ -802,24 +804,7 @@ double oil4_gemm_x32_us(int64_t Mr, int64_t N, int64_t K) {
     const int64_t tiles = (Mr + 127) / 128;
     const int bn = x32_bn(tiles, N, K);
     if (bn == 0) return 1e9;
-    return 5.0 + (double)((tiles * ((N + bn - 1) / bn) + 255) / 256) * (K / 1024.0) * (7.9 + 0.0594 * bn);
-}
-
-template <int EDGE>
-static void run_prefill_x32(int bn, unsigned grid, const uint16_t* a16, const uint8_t* nib, const uint16_t* cbs,
-                            int64_t cb_block, float* c, int64_t mv, int64_t N, int64_t K, const int* rsh, int64_t Mr,
-                            hipStream_t s) {
-    const int cbk = (int)cb_block, m = (int)mv, n = (int)N, k = (int)K, mr = (int)Mr;
-    constexpr int T4 = ws_threads(4), T8 = ws_threads(8);
-    switch (bn) {
-        case 128: oil4_prefill_ws<128, 4, 1, true, 8, EDGE><<<grid, T8, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
-        case 112:
-            if constexpr (EDGE < 2)
-                oil4_prefill_ws<112, 4, 2, true, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr);
-            break;
-        case 96: oil4_prefill_ws<96, 4, 2, true, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
-        default: oil4_prefill_ws<64, 4, 2, true, 4, EDGE><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
-    }
+    return 5.0 + (double)((tiles * (N / bn) + 255) / 256) * (K / 1024.0) * (7.9 + 0.0594 * bn);
 }
 
 hipError_t launch_oil4_gemm_x32(const float* a, const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, float* c,
@@ -831,12 +816,18 @@ hipError_t launch_oil4_gemm_x32(const float* a, const uint8_t* nib, const uint16
     const uint16_t* a16 = (const uint16_t*)((const char*)ws + oil4_prefill_shift_bytes(Mr));
     const int64_t tiles = (Mr + 127) / 128, mv = 256 * tiles;
     const int bn = x32_bn(tiles, N, K);
-    const unsigned grid = (unsigned)(tiles * ((N + bn - 1) / bn));
-    if (K % (4 * PBK) == 0 && N % bn == 0) run_prefill_x32<0>(bn, grid, a16, nib, cbs, cb_block, c, mv, N, K, rsh, Mr, s);
-    else if (K % (4 * PBK) == 0) run_prefill_x32<1>(bn, grid, a16, nib, cbs, cb_block, c, mv, N, K, rsh, Mr, s);
-    else run_prefill_x32<2>(bn, grid, a16, nib, cbs, cb_block, c, mv, N, K, rsh, Mr, s);
+    const unsigned grid = (unsigned)(tiles * (N / bn));
+    const int cbk = (int)cb_block, m = (int)mv, n = (int)N, k = (int)K, mr = (int)Mr;
+    constexpr int T4 = ws_threads(4), T8 = ws_threads(8);
+    switch (bn) {
+        case 128: oil4_prefill_ws<128, 4, 1, true, 8><<<grid, T8, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
+        case 112: oil4_prefill_ws<112, 4, 2, true><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
+        case 96: oil4_prefill_ws<96, 4, 2, true><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
+        default: oil4_prefill_ws<64, 4, 2, true><<<grid, T4, 0, s>>>(a16, nib, cbs, cbk, c, m, n, k, rsh, mr); break;
+    }
     return hipGetLastError();
 }
+
 bool oil4_gemm_prefill_supported(int64_t M, int64_t N, int64_t K, int64_t cb_block) {
     return K % BK == 0 && cb_block % BK == 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31) &&
            (M + BM - 1) / BM < 65536;

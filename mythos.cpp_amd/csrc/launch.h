@@ -203,7 +203,8 @@ hipError_t launch_oil4_gemm_prefill_a16(const uint16_t* a_bf16, const uint8_t* n
 // The prompt prefill's OIL4 projection with FP32 rows (FP32 accurate, the
 // decode GEMVs' arithmetic on MFMA): c [Mr][N] = a [Mr][K] W^T, each row of a
 // split into FP16 hi + lo after a power-of-two scale (two products per
-// weight, sums FP32).  ws: oil4_gemm_x32_workspace_bytes(Mr, K).
+// weight, sums FP32).  Whole tiles (oil4_whole_tiles), codebook blocks of a
+// multiple of 128.  ws: oil4_gemm_x32_workspace_bytes(Mr, K).
 bool oil4_gemm_x32_supported(int64_t Mr, int64_t N, int64_t K, int64_t cb_block);
 size_t oil4_gemm_x32_workspace_bytes(int64_t Mr, int64_t K);
 hipError_t launch_oil4_gemm_x32(const float* a, const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, float* c,

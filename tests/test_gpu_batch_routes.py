@@ -338,8 +338,8 @@ def test_prefill_rows(M, N, K, block, mth, dev):
                                    (16, 28016, 512), (16, 28016, 384), (16, 32016, 256), (16, 32016, 384),
                                    (1100, 4096, 384)])
 def test_prefill_tile_edges(M, N, K, x32, mth, dev):
-    """The tiled prompt kernels (bf16 rows; FP32 rows of hi and lo parts) where the last tile or the last round of steps
-    is partial.  FP32 rows: the parts keep 2^-22 of a product and the sums round less than K / 16 times."""
+    """bf16 rows on the tiled prompt kernels where the last tile or the last round of steps is partial; FP32 rows of the
+    same shapes: the parts keep 2^-22 of a product and the sums round less than K / 16 times."""
     import ctypes as C
     import torch
     from test_gpu_prefill import check
@@ -348,24 +348,25 @@ def test_prefill_tile_edges(M, N, K, x32, mth, dev):
     A = torch.from_numpy(synth.bf16_to_f32(a).reshape(M, K).copy())
     if x32:
         A = A * (1.0 + torch.rand(M, K, generator=torch.Generator().manual_seed(K)))
-    L, P = mth.lib, C.c_void_p
-    size = {}
-    for name, sym, n in (("ws", "_ZN3mth28oil4_prefill_workspace_bytesEllll", 4), ("shift", "_ZN3mth24oil4_prefill_shift_bytesEl", 1),
-                         ("x32", "_ZN3mth29oil4_gemm_x32_workspace_bytesEll", 2)):
-        f = getattr(L, sym)
-        f.argtypes, f.restype = [C.c_int64] * n, C.c_size_t
-        size[name] = f
-    f = (L._ZN3mth20launch_oil4_gemm_x32EPKfPKhPKtlPflllPvP12ihipStream_t if x32 else
-         L._ZN3mth28launch_oil4_gemm_prefill_a16EPKtPKhS1_lPtlllPvP12ihipStream_t)
-    f.argtypes, f.restype = [P, P, P, C.c_int64, P, C.c_int64, C.c_int64, C.c_int64, P, P], C.c_int
-    need = size["x32"](M, K) if x32 else size["shift"](M) + size["ws"](M, N, K, 128)
-    assert need > 0
-    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
     x = A.to(dev) if x32 else A.bfloat16().to(dev)
     w, cb = to_dev(packed, dev), to_dev(cbs, dev)
     c = torch.full((M * N + 64,), float("nan"), dtype=torch.float32 if x32 else torch.bfloat16, device=dev)
-    assert f(x.data_ptr(), w.data_ptr(), cb.data_ptr(), 128, c.data_ptr(), M, N, K, ws.data_ptr(),
-             torch.cuda.current_stream().cuda_stream) == 0
+    if x32:
+        mth.oil4_gemv(w, cb, 128, x, c[:M * N], N, K, M)
+    else:
+        L, P = mth.lib, C.c_void_p
+        size = {}
+        for name, sym, n in (("ws", "_ZN3mth28oil4_prefill_workspace_bytesEllll", 4),
+                             ("shift", "_ZN3mth24oil4_prefill_shift_bytesEl", 1)):
+            f = getattr(L, sym)
+            f.argtypes, f.restype = [C.c_int64] * n, C.c_size_t
+            size[name] = f
+        f = L._ZN3mth28launch_oil4_gemm_prefill_a16EPKtPKhS1_lPtlllPvP12ihipStream_t
+        f.argtypes, f.restype = [P, P, P, C.c_int64, P, C.c_int64, C.c_int64, C.c_int64, P, P], C.c_int
+        assert size["ws"](M, N, K, 128) > 0
+        ws = torch.zeros(size["shift"](M) + size["ws"](M, N, K, 128), dtype=torch.uint8, device=dev)
+        assert f(x.data_ptr(), w.data_ptr(), cb.data_ptr(), 128, c.data_ptr(), M, N, K, ws.data_ptr(),
+                 torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
     assert bool(torch.isnan(c[M * N:]).all())
     W = torch.from_numpy(synth.dequant_oil4(packed, cbs, N, K, 128)).to(dev).double()
@@ -416,12 +417,14 @@ def test_partial_tiles_under_capture(entry, mth, dev):
             assert bool((np.abs(got.double().numpy() - ref) <= (K / 16 + 8) * 2.0 ** -24 * absw).all()), rep
 
 
-def test_token_rows_oil4_infinite_entry(mth, dev):
+# a few rows of no whole tile; token counts of a prompt with rows and columns that are no whole tiles of its kernels
+@pytest.mark.parametrize("M,K,batch,blk", [(130, 1120, 20, 0), (1616, 1280, 200, 128), (1616, 1280, 500, 128),
+                                           (208, 1152, 300, 128), (1616, 1408, 500, 128)])
+def test_token_rows_oil4_infinite_entry(M, K, batch, blk, mth, dev):
     """An infinite codebook entry times values 2^-60 below their row's largest (0 in both FP16 parts): +-Inf, as one
     FP32 product gives, and NaN where entries of both signs meet."""
     import torch
-    M, K, batch = 130, 1120, 20
-    print("token rows OIL4 infinite entry", flush=True)
+    print(f"token rows OIL4 infinite entry M={M} K={K} batch={batch}", flush=True)
     g = np.random.default_rng(8)
     nib = g.integers(2, 16, (M, K), dtype=np.uint8)          # entries 0 (+Inf) and 1 (-Inf) only where placed
     nib[3, 100] = nib[129, 1119] = nib[5, 40] = 0
@@ -431,8 +434,8 @@ def test_token_rows_oil4_infinite_entry(mth, dev):
     x = (1.0 + g.random((batch, K))).astype(np.float32)
     x[:, [100, 1119, 40, 64, 1000]] = 2.0 ** -60
     y = empty(batch * M, torch.float32, dev)
-    mth.oil4_gemv(to_dev(nib[:, 0::2] | (nib[:, 1::2] << 4), dev), to_dev(cb.view(np.uint16), dev), 0, to_dev(x, dev), y,
-                  M, K, batch)
+    cbs = np.tile(cb.view(np.uint16), M * (K // blk) if blk else 1)
+    mth.oil4_gemv(to_dev(nib[:, 0::2] | (nib[:, 1::2] << 4), dev), to_dev(cbs, dev), blk, to_dev(x, dev), y, M, K, batch)
     torch.cuda.synchronize()
     got = y.cpu().numpy().reshape(batch, M)
     assert (got[:, [3, 129]] == np.inf).all() and (got[:, 7] == -np.inf).all() and np.isnan(got[:, 5]).all()

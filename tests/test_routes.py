@@ -62,3 +62,15 @@ def test_per_thread_stream_shares_no_workspace():
     calls = without_workspace(next(stream))                      # an ordinary stream: the route with workspace
     for (c, name), r in zip(calls, recorded.run([c for c, _ in calls])):
         assert on(r, name), (c, kernels(r))
+
+
+def test_partial_tiles_of_fp32_rows():
+    """FP32 token rows whose columns or K steps are no whole tiles of the
+    prompt GEMM keep off it (an infinite codebook entry would meet a part that
+    is 0 there); whole tiles run on it."""
+    calls = [oil4(M, K, b, next(stream)) for M in (1616, 8016, 14352, 24016) for K in (384, 640, 768, 1280, 1920)
+             for b in (128, 200, 500)]
+    for c, r in zip(calls, recorded.run(calls)):
+        assert not on(r, "oil4_prefill_ws"), (c, kernels(r))
+    r = recorded.run([oil4(22016, 4096, 512, next(stream))])[0]
+    assert on(r, "oil4_prefill_ws"), kernels(r)
