@@ -11,7 +11,13 @@
 // and token), OIL8 codebook entries are split the same way (three products;
 // lo x lo lies below FP32's rounding).  Products are exact in FP32, sums FP32
 // on v_mfma_f32_16x16x32_f16, the hi x hi products and the rest in accumulators
-// of their own.  A token tile that holds Inf or NaN, or a non-finite OIL8
+// of their own.  OIL8 and OIL4 add the hi x hi products of a step of 128 columns
+// up from zero and then to the slice's sum: one accumulator per slice rounds at
+// its full size some K / 10 times, and at 4080 .. 13696 columns in one slice was
+// 4.1e-7 .. 7.4e-7 of the norm off (64-bit sums), where the FP32 FMAs of the
+// kernels that walk the tokens are 1.1e-7 .. 2.7e-7 and this 1.4e-7 .. 2.1e-7
+// (OIL8 2 % slower, OIL4 the same time; the ternary sums were below the FP32
+// kernel's without it).  A token tile that holds Inf or NaN, or a non-finite OIL8
 // codebook, takes FP32 FMAs over the reference's products instead, as does an
 // OIL4 output that comes out NaN (redo: shapes that no other FP16 hi / lo
 // kernel takes, which give NaN where infinite entries meet such values).  bf16 rows are one FP16 part, as
@@ -246,6 +252,7 @@ template <int FMT, int G>
 __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) {
     constexpr int P = kParts<FMT>;
     constexpr bool O4 = FMT == kOil4 || FMT == kOil4B;
+    constexpr bool STEP = FMT == kOil8 || FMT == kOil4;  // hi x hi sums of a step, added up outside
     constexpr int NB = P * G;  // 16-byte pieces of a step's B per thread (4 KB per token group and part)
     __shared__ __align__(16) uint8_t bs[P * G * 4096];
     __shared__ uint32_t tab[FMT == kOil8 ? 256 : 1];
@@ -382,46 +389,81 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
                 cur[t].c = codes8_at(cur[t].c, pos, tend);
             }
         }
+        // piece m (columns 8 m .. of every 32) of tile t as A operands: hi, and OIL8's lo
+        auto weights = [&](int t, int m, half8& Ah, half8& Al) {
+            if constexpr (FMT == kOil8) {
+                const uint32_t w0 = m == 0 ? wa[t].x : m == 1 ? wa[t].z : m == 2 ? wb[t].x : wb[t].z;
+                const uint32_t w1 = m == 0 ? wa[t].y : m == 1 ? wa[t].w : m == 2 ? wb[t].y : wb[t].w;
+                uint32_t gv[8];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            half8 bh[G], bl[G];
+                for (int e = 0; e < 4; ++e) {
+                    gv[e] = tab[(w0 >> (8 * e)) & 0xffu];
+                    gv[4 + e] = tab[(w1 >> (8 * e)) & 0xffu];
+                }
+                u32x4 hv, lv;
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    hv[d] = __builtin_amdgcn_perm(gv[2 * d + 1], gv[2 * d], 0x05040100u);
+                    lv[d] = __builtin_amdgcn_perm(gv[2 * d + 1], gv[2 * d], 0x07060302u);
+                }
+                Ah = __builtin_bit_cast(half8, hv);
+                Al = __builtin_bit_cast(half8, lv);
+            } else if constexpr (O4) {
+                Ah = lookup8_natural(u4get(cur[t].n, m), pl[t]);
+            } else {
+                Ah = rows_tern8(m < 2 ? cur[t].c.x : cur[t].c.y, 2 * (m & 1));
+            }
+        };
+        // the token operands of piece m and group g
+        auto tokens = [&](int m, int g, half8& bh, half8& bl) {
+            bh = *(const half8*)(brow + g * P * 4096 + 256 * m);
+            if constexpr (P == 2) bl = *(const half8*)(brow + g * 8192 + 4096 + 256 * m);
+        };
+        // tile t's products with group g; h: the hi x hi sums (a step's alone, or from the slice's start)
+        auto product = [&](int m, int t, int g, half8 Ah, half8 Al, half8 bh, half8 bl, floatx4& h) {
+            h = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh, STEP && m == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : h, 0, 0, 0);
+            if constexpr (P == 2) ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bl, ax[t][g], 0, 0, 0);
+            if constexpr (FMT == kOil8) ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, bh, ax[t][g], 0, 0, 0);
+        };
+        if constexpr (FMT == kOil4) {  // the step's A operands first: a group's step sums are then 8 registers
+            half8 Ah[4][2], Al;
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) weights(t, m, Ah[m][t], Al);
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                bh[g] = *(const half8*)(brow + g * P * 4096 + 256 * m);
-                if constexpr (P == 2) bl[g] = *(const half8*)(brow + g * 8192 + 4096 + 256 * m);
+                floatx4 st[2];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    half8 bh, bl;
+                    tokens(m, g, bh, bl);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) product(m, t, g, Ah[m][t], Al, bh, bl, st[t]);
+                }
+                ah[0][g] += st[0];
+                ah[1][g] += st[1];
             }
+        } else {
+            floatx4 st[2][G];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                half8 Ah, Al;
-                if constexpr (FMT == kOil8) {
-                    const uint32_t w0 = m == 0 ? wa[t].x : m == 1 ? wa[t].z : m == 2 ? wb[t].x : wb[t].z;
-                    const uint32_t w1 = m == 0 ? wa[t].y : m == 1 ? wa[t].w : m == 2 ? wb[t].y : wb[t].w;
-                    uint32_t gv[8];
+            for (int m = 0; m < 4; ++m) {
+                half8 bh[G], bl[G];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        gv[e] = tab[(w0 >> (8 * e)) & 0xffu];
-                        gv[4 + e] = tab[(w1 >> (8 * e)) & 0xffu];
-                    }
-                    u32x4 hv, lv;
+                for (int g = 0; g < G; ++g) tokens(m, g, bh[g], bl[g]);
 #pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        hv[d] = __builtin_amdgcn_perm(gv[2 * d + 1], gv[2 * d], 0x05040100u);
-                        lv[d] = __builtin_amdgcn_perm(gv[2 * d + 1], gv[2 * d], 0x07060302u);
-                    }
-                    Ah = __builtin_bit_cast(half8, hv);
-                    Al = __builtin_bit_cast(half8, lv);
-                } else if constexpr (O4) {
-                    Ah = lookup8_natural(u4get(cur[t].n, m), pl[t]);
-                } else {
-                    Ah = rows_tern8(m < 2 ? cur[t].c.x : cur[t].c.y, 2 * (m & 1));
+                for (int t = 0; t < 2; ++t) {
+                    half8 Ah, Al;
+                    weights(t, m, Ah, Al);
+#pragma unroll
+                    for (int g = 0; g < G; ++g) product(m, t, g, Ah, Al, bh[g], bl[g], STEP ? st[t][g] : ah[t][g]);
                 }
+            }
+            if constexpr (STEP) {
 #pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    ah[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh[g], ah[t][g], 0, 0, 0);
-                    if constexpr (P == 2) ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bl[g], ax[t][g], 0, 0, 0);
-                    if constexpr (FMT == kOil8)
-                        ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, bh[g], ax[t][g], 0, 0, 0);
-                }
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int g = 0; g < G; ++g) ah[t][g] += st[t][g];
             }
         }
         __syncthreads();

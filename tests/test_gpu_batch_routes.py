@@ -257,6 +257,33 @@ def test_token_rows(kind, M, K, batch, blk, shift, mth, dev):
     assert bool(((got - want).norm(dim=1) <= 1e-6 * nrm + 1e-30).all())
 
 
+# whole rows in one slice, the longest chains of sums: 4080 .. 8192 columns, each token tile width
+@pytest.mark.parametrize("kind,M,K,batch,blk", [("oil8", 12000, 4080, 200, 0), ("oil8", 33000, 6000, 16, 0),
+                                                ("oil4", 12000, 4224, 200, 64), ("oil4", 12016, 2688, 140, 128),
+                                                ("oil4", 33000, 8192, 17, 64), ("oil4", 16500, 4224, 96, 64),
+                                                ("tern", 8000, 4096, 300, 0)])
+def test_token_rows_error(kind, M, K, batch, blk, mth, dev):
+    """The sums' error against float64, of normal values: FP32 FMAs in 64 lanes (the kernels that take these sizes one
+    token after another) are 1.1e-7 .. 2.2e-7 of the norm off, one chain of all products 2.7e-7 .. 6e-7.  2^-22: a part
+    pair's own rounding."""
+    import torch
+    print(f"token rows error {kind} M={M} K={K} batch={batch}", flush=True)
+    g = np.random.default_rng(M + K)
+    w, cb = rows_inputs(kind, M, K, blk, g)
+    x = g.normal(0, 1, (batch, K)).astype(np.float32)
+    got = rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev).double()
+    err = ref = 0.0
+    X = torch.from_numpy(x).to(dev).double()
+    step = 3000
+    for i in range(0, M, step):
+        n = min(M, i + step) - i
+        c = cb if kind != "oil4" else cb[16 * (K // blk) * i:16 * (K // blk) * (i + n)]
+        want = X @ w64(kind, w[i:i + n], c, n, K, blk, dev).T.contiguous()
+        err += float((got[:, i:i + n] - want).square().sum())
+        ref += float(want.square().sum())
+    assert (err / ref) ** 0.5 <= 2.0 ** -22, (err / ref) ** 0.5
+
+
 @pytest.mark.parametrize("kind", ["oil8", "oil4", "tern"])
 @pytest.mark.parametrize("M,K,batch", [(300, 4096, 40), (40, 4736, 1)])
 @pytest.mark.parametrize("what", ["x_inf", "x_nan", "codebook_inf"])
