@@ -132,7 +132,7 @@ bool oil8_prompt(const mth_decoder* d, const mth::Oil8Seg* seg, int nseg, const 
     }
     if (mth::oil8_rows_better(seg, nseg, K, rows, true, gemm, bt) &&
         mth::rows_mfma_workspace_bytes(M, K, rows, nseg) <= d->pf_ws_bytes) {
-        *e = mth::launch_oil8_rows(seg, nseg, x, K, rows, d->pf_ws, s);
+        *e = mth::launch_oil8_rows(seg, nseg, x, K, rows, !bt && !gemm, d->pf_ws, s);
         return true;
     }
     if (gemm) *e = mth::launch_oil8_gemm_x32(x, seg, nseg, rows, K, d->pf_ws, s);

@@ -9,7 +9,9 @@
 // scaled by a power of two and split into FP16 hi + lo (rows_split_k, once per
 // call); OIL4 and ternary weights are exact in FP16 (two products per weight
 // and token), OIL8 codebook entries are split the same way (three products;
-// lo x lo lies below FP32's rounding).  Products are exact in FP32, sums FP32
+// lo x lo lies below FP32's rounding).  lo parts are held times 2^11, so that a
+// value keeps its 22 bits down to 2^-28 of its row's (its codebook's) maximum.
+// Products are exact in FP32, sums FP32
 // on v_mfma_f32_16x16x32_f16, the hi x hi products and the rest in accumulators
 // of their own.  OIL8 and OIL4 add the hi x hi products of a step of 128 columns
 // up from zero and then to the slice's sum: one accumulator per slice rounds at
@@ -17,10 +19,12 @@
 // 4.1e-7 .. 7.4e-7 of the norm off (64-bit sums), where the FP32 FMAs of the
 // kernels that walk the tokens are 1.1e-7 .. 2.7e-7 and this 1.4e-7 .. 2.1e-7
 // (OIL8 2 % slower, OIL4 the same time; the ternary sums were below the FP32
-// kernel's without it).  A token tile that holds Inf or NaN, or a non-finite OIL8
-// codebook, takes FP32 FMAs over the reference's products instead, as does an
-// OIL4 output that comes out NaN (redo: shapes that no other FP16 hi / lo
-// kernel takes, which give NaN where infinite entries meet such values).  bf16 rows are one FP16 part, as
+// kernel's without it).  A token row that
+// holds Inf or NaN, or that spans more than 28 binades at a shape whose other
+// route is FP32 products (fp32: its largest values may meet weights of 0), takes
+// FP32 FMAs over the reference's products instead, as do all rows of a
+// non-finite OIL8 codebook and (fp32) an OIL4 output that comes out NaN, where
+// an infinite entry may have met a value that both parts miss.  bf16 rows are one FP16 part, as
 // in the tiled prompt kernels.
 //
 // Tiling.  A workgroup of 4 waves takes 128 weight rows (32 per wave: two A
@@ -56,17 +60,18 @@ template <int FMT>
 constexpr int kParts = FMT == kOil4B ? 1 : 2;  // FP16 parts of a token row
 
 // ---- token rows -> FP16 hi / lo B fragments ------------------------------------
-// Row t: shift s with max|x| 2^s in [2^14, 2^15) into rsh[t] (kRowNonFinite for a row holding Inf / NaN), then
-// 2^s x = hi + lo, group t / 16, part (hi, lo), 32-column chunk c: 1 KB of [8-column piece m][token t % 16][8].
+// Row t: shift s with max|x| 2^s in [2^14, 2^15) into rsh[t] (kRowFp32 for a row holding Inf / NaN and, with guard, for
+// one whose nonzero values span more than 28 binades), then 2^s x = hi + 2^-11 lo, group t / 16, part (hi, lo), 32-column chunk c: 1 KB of [8-column piece m][token t % 16][8].
 // TERN: the pieces hold the columns in the order of the ternary codes' planes (element e of piece m: column
 // 16 (m / 2) + 2 (m % 2) + e / 4 + 4 (e % 4) of the chunk).  Columns past K are zeros; rows past the batch are not
 // written (their products only reach their own, discarded, outputs).  One workgroup per row, the row read once
 // (16384 columns in registers; the rest of a longer row twice).
 constexpr int kRsN = 4;
+constexpr int kRowFp32 = kRowNonFinite;
 template <bool TERN, bool VEC>
 __global__ __launch_bounds__(kRmT) void rows_split_k(const float* __restrict__ x, uint16_t* __restrict__ a16,
-                                                     int* __restrict__ rsh, int K, int chunks) {
-    __shared__ uint32_t red[kRmT / 64];
+                                                     int* __restrict__ rsh, int K, int chunks, bool guard) {
+    __shared__ uint32_t red[kRmT / 64], redn[kRmT / 64];
     const int tid = threadIdx.x, row = blockIdx.x;
     const float* xr = x + (int64_t)row * K;
     const int n16 = 2 * chunks;  // 16-column groups
@@ -86,22 +91,29 @@ __global__ __launch_bounds__(kRmT) void rows_split_k(const float* __restrict__ x
     float v[kRsN][16], u[16];
 #pragma unroll
     for (int j = 0; j < kRsN; ++j) load(tid + j * kRmT, v[j]);
-    uint32_t mb = 0;
+    uint32_t mb = 0, mn = 0;  // max |x| bits; 2^32 - the least nonzero |x| bits (0: all zeros)
+    auto range = [&](const float (&f)[16]) {
 #pragma unroll
-    for (int j = 0; j < kRsN; ++j)
+        for (int i = 0; i < 16; ++i) {
+            const uint32_t ab = __float_as_uint(f[i]) & 0x7fffffffu;
+            mb = max(mb, ab);
+            mn = max(mn, 0u - ab);
+        }
+    };
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mb = max(mb, __float_as_uint(v[j][i]) & 0x7fffffffu);
+    for (int j = 0; j < kRsN; ++j) range(v[j]);
     for (int g = tid + kRsN * kRmT; g < n16; g += kRmT) {
         load(g, u);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mb = max(mb, __float_as_uint(u[i]) & 0x7fffffffu);
+        range(u);
     }
     mb = group_reduce<64>(mb, UMaxOp{});
-    if ((tid & 63) == 0) red[tid >> 6] = mb;
+    mn = group_reduce<64>(mn, UMaxOp{});
+    if ((tid & 63) == 0) red[tid >> 6] = mb, redn[tid >> 6] = mn;
     __syncthreads();
     mb = max(max(red[0], red[1]), max(red[2], red[3]));
+    mn = 0u - max(max(redn[0], redn[1]), max(redn[2], redn[3]));
     const int sh = fp16_scale_shift(__uint_as_float(mb));
-    if (tid == 0) rsh[row] = mb >= 0x7f800000u ? kRowNonFinite : sh;
+    if (tid == 0) rsh[row] = mb >= 0x7f800000u || (guard && (int)(mb >> 23) - (int)(mn >> 23) > 28) ? kRowFp32 : sh;
     uint16_t* hi = a16 + (int64_t)(row >> 4) * 2 * chunks * 512 + 8 * (row & 15);
     uint16_t* lo = hi + (int64_t)chunks * 512;
     auto store = [&](int g, const float (&f)[16]) {
@@ -112,7 +124,7 @@ __global__ __launch_bounds__(kRmT) void rows_split_k(const float* __restrict__ x
             for (int e = 0; e < 8; ++e) {
                 const float xs = ldexpf(f[TERN ? 2 * p + (e >> 2) + 4 * (e & 3) : 8 * p + e], sh);
                 h[e] = (_Float16)xs;
-                l[e] = (_Float16)(xs - (float)h[e]);
+                l[e] = (_Float16)((xs - (float)h[e]) * 2048.0f);
             }
             const int64_t off = (int64_t)(g >> 1) * 512 + 128 * (2 * (g & 1) + p);
             *(half8*)(hi + off) = h;
@@ -173,7 +185,7 @@ struct RowsArgs {
     float* out;            // [batch][M] (ternary: [M][batch]; kOil4B: bf16)
     float* partial;        // [slice] of the same
     int M, K, batch, steps, cb_block;
-    bool redo;             // kOil4: FP32 products for an output that comes out NaN
+    bool fp32;             // FP32 products for rows of a wide range, and for an OIL4 output that comes out NaN
 };
 // OIL8: up to three matrices over the same token rows (a decoder's Q, K and V), their row tiles one after another in
 // the grid; t1: the first row tile past matrix i.  Matrix i's partial sums start at partial + p0[i].
@@ -206,7 +218,7 @@ struct RowsTile<kTern> {
 
 __device__ __forceinline__ uint32_t rows_hl(float c) {
     const _Float16 h = (_Float16)c;
-    const _Float16 l = (_Float16)(c - (float)h);
+    const _Float16 l = (_Float16)((c - (float)h) * 2048.0f);
     return (uint32_t)__builtin_bit_cast(uint16_t, h) | ((uint32_t)__builtin_bit_cast(uint16_t, l) << 16);
 }
 
@@ -330,19 +342,21 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
         const float m = wave_max(fabsf(cbv));
         if (lane == 0) wred[wave] = m;
     }
-#pragma unroll
-    for (int g = 0; g < G; ++g) fin = fin && (FMT == kOil4B || rs[g] != kRowNonFinite);
-    const bool special = __syncthreads_or(!fin) != 0;
     const int64_t zs = (int64_t)p.batch * M;
     float* out = S == 1 ? p.out : p.partial + blockIdx.z * zs;
     auto at = [&](int row, int tok) { return FMT == kTern ? (int64_t)row * p.batch + tok : (int64_t)tok * M + row; };
-    if (FMT != kOil4B && special) {
-        const int k0 = kRmStep * s0, k1 = min(K, kRmStep * s1), r0 = bx * kRmRows;
-        for (int o = tid; o < kRmRows * 16 * G; o += kRmT) {
-            const int row = r0 + o % kRmRows, tok = tok0 + o / kRmRows;
-            if (row < M && tok < p.batch) out[at(row, tok)] = rows_fma<FMT>(p, row, tok, k0, k1);
+    // the tile's outputs of one token with FP32 products: two threads per weight row, half of the slice each
+    auto fp32_token = [&](int tok) {
+        const int row = bx * kRmRows + (tid >> 1), k0 = kRmStep * s0, k1 = min(K, kRmStep * s1), mid = (k0 + k1) / 2;
+        float v = row < M ? rows_fma<FMT>(p, row, tok, tid & 1 ? mid : k0, tid & 1 ? k1 : mid) : 0.0f;
+        v += lane_xor1(v);
+        if (row < M && (tid & 1) == 0) out[at(row, tok)] = v;
+    };
+    if constexpr (FMT == kOil8) {
+        if (__syncthreads_or(!fin)) {
+            for (int tok = tok0; tok < min(tok0 + 16 * G, p.batch); ++tok) fp32_token(tok);
+            return;
         }
-        return;
     }
     int sw = 0;
     if constexpr (FMT == kOil8) {
@@ -477,21 +491,22 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
 #pragma unroll
     for (int g = 0; g < G; ++g) {
         const int tok = tok0 + 16 * g + j;
-        if (tok >= p.batch) continue;
+        if (tok >= p.batch || (FMT != kOil4B && rs[g] == kRowFp32)) continue;
         const int sh = rs[g] + sw;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const int row = row0 + 16 * t + 4 * q;
             float v[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                v[i] = ldexpf(P == 1 ? ah[t][g][i]
-                              : FMT == kOil8 ? ah[t][g][i] + ax[t][g][i] : oil4_hi_lo(ah[t][g][i], ax[t][g][i]), -sh);
+            for (int i = 0; i < 4; ++i) {
+                const float hi = ah[t][g][i], lo = ax[t][g][i] * 0x1p-11f;
+                v[i] = ldexpf(P == 1 ? hi : FMT == kOil8 ? hi + lo : oil4_hi_lo(hi, lo), -sh);
+            }
             if constexpr (FMT == kOil4) {
                 // NaN: also an infinite entry times a value whose parts are 0, where the reference's product is infinite
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (p.redo && v[i] != v[i] && row + i < M)
+                    if (p.fp32 && v[i] != v[i] && row + i < M)
                         v[i] = rows_fma<FMT>(p, row + i, tok, kRmStep * s0, min(K, kRmStep * s1));
             }
             if constexpr (FMT == kOil4B) {
@@ -519,6 +534,13 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
                     if (row + i < M) out[at(row + i, tok)] = v[i];
             }
         }
+    }
+    if constexpr (FMT != kOil4B) {  // (every wave holds the tile's shifts)
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            for (uint64_t m = __builtin_amdgcn_ballot_w64(q == 0 && tok0 + 16 * g + j < p.batch && rs[g] == kRowFp32); m;
+                 m &= m - 1)
+                fp32_token(tok0 + 16 * g + __builtin_ctzll(m));
     }
 }
 
@@ -602,9 +624,9 @@ hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s, cons
     if constexpr (FMT == kOil4B)
         rows_half_k<<<(unsigned)a.batch, kRmT, 0, s>>>((const uint16_t*)a.x, a16, rsh, a.K, 4 * p.steps);
     else if (vec)
-        rows_split_k<FMT == kTern, true><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps);
+        rows_split_k<FMT == kTern, true><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps, a.fp32);
     else
-        rows_split_k<FMT == kTern, false><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps);
+        rows_split_k<FMT == kTern, false><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps, a.fp32);
     const dim3 grid((unsigned)(sg.n > 1 ? sg.t1[sg.n - 1] : p.rtiles), (unsigned)p.tiles, (unsigned)p.S);
     switch (p.G) {
         case 1: rows_mfma_k<FMT, 1><<<grid, kRmT, 0, s>>>(a, sg); break;
@@ -732,7 +754,7 @@ bool oil4_rows_bf16_better(int64_t M, int64_t K, int64_t batch, double tiled_us)
     return 1.12 * us < tiled_us;
 }
 
-hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, void* ws,
+hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, bool fp32, void* ws,
                             hipStream_t s) {
     RowsSegs sg{};
     int64_t M = 0, tiles = 0;
@@ -751,23 +773,24 @@ hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_
         }
         sg.t1[i] = (int)tiles;
     }
-    RowsArgs a{seg[0].idx, seg[0].cb, nullptr, nullptr, x, seg[0].y, nullptr, (int)seg[0].rows, (int)K, (int)batch, 0, 0};
+    RowsArgs a{seg[0].idx, seg[0].cb, nullptr, nullptr, x, seg[0].y, nullptr, (int)seg[0].rows, (int)K, (int)batch, 0, 0,
+               fp32};
     return rows_run<kOil8>(a, p, ws, s, sg);
 }
 hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
-                            int64_t M, int64_t K, int64_t batch, bool redo, void* ws, hipStream_t s) {
-    RowsArgs a{nib, cbs, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, (int)cb_block, redo};
+                            int64_t M, int64_t K, int64_t batch, bool fp32, void* ws, hipStream_t s) {
+    RowsArgs a{nib, cbs, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, (int)cb_block, fp32};
     return rows_run<kOil4>(a, rows_plan(M, K, batch), ws, s);
 }
 hipError_t launch_oil4_rows_bf16(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const uint16_t* x,
                                  uint16_t* y, int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s) {
     RowsArgs a{nib, cbs, nullptr, nullptr, (const float*)x, (float*)y, nullptr, (int)M, (int)K, (int)batch, 0,
-               (int)cb_block};
+               (int)cb_block, false};
     return rows_run<kOil4B>(a, rows_plan(M, K, batch), ws, s);
 }
 hipError_t launch_tern_rows(const uint8_t* w, const float* x, float* out, int64_t M, int64_t K, int64_t batch,
                             void* ws, hipStream_t s) {
-    RowsArgs a{w, nullptr, nullptr, nullptr, x, out, nullptr, (int)M, (int)K, (int)batch, 0, 0};
+    RowsArgs a{w, nullptr, nullptr, nullptr, x, out, nullptr, (int)M, (int)K, (int)batch, 0, 0, true};
     return rows_run<kTern>(a, rows_plan(M, K, batch), ws, s);
 }
 

@@ -244,11 +244,12 @@ size_t rows_bf16_workspace_bytes(int64_t M, int64_t K, int64_t batch);
 hipError_t launch_oil4_rows_bf16(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const uint16_t* x,
                                  uint16_t* y, int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s);
 bool tern_rows_better(int64_t M, int64_t K, int64_t batch);
-hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, void* ws,
+// fp32: the call's other route is FP32 products; rows that span more than 28 binades then take them here too, and so does
+// an OIL4 output that comes out NaN (an infinite codebook entry times a value that both parts miss)
+hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, bool fp32, void* ws,
                             hipStream_t s);
-// redo: FP32 products where an output comes out NaN (an infinite codebook entry times a value that both parts miss)
 hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
-                            int64_t M, int64_t K, int64_t batch, bool redo, void* ws, hipStream_t s);
+                            int64_t M, int64_t K, int64_t batch, bool fp32, void* ws, hipStream_t s);
 hipError_t launch_tern_rows(const uint8_t* w, const float* x, float* out, int64_t M, int64_t K, int64_t batch,
                             void* ws, hipStream_t s);
 

@@ -321,6 +321,47 @@ def test_token_rows_non_finite(kind, M, K, batch, what, mth, dev):
         assert np.abs(got[fin] - want[fin]).max() <= 1e-5 * np.abs(prod).sum(-1)[fin].max()
 
 
+# one, two and four token groups; K split over workgroups and not; more than one token tile; a K remainder
+@pytest.mark.parametrize("kind,M,K,batch,blk", [("oil8", 300, 1040, 12, 0), ("oil8", 200, 6448, 70, 0),
+                                                ("oil4", 130, 1120, 33, 32), ("oil4", 1616, 1920, 200, 128),
+                                                ("oil4", 500, 9088, 20, 64), ("tern", 300, 4100, 9, 0),
+                                                ("tern", 4096, 1024, 130, 0)])
+@pytest.mark.parametrize("span", [2.0 ** 20, 2.0 ** 27, 2.0 ** 40])
+def test_token_rows_wide_range(kind, M, K, batch, blk, span, mth, dev):
+    """Values far above the rest of their row that meet weights of 0 in half of the outputs: those keep the precision
+    of the rest, as FP32 products do.  Other tokens of the tile are as without them, bit for bit."""
+    import torch
+    print(f"token rows wide range {kind} M={M} K={K} batch={batch} span={span}", flush=True)
+    g = np.random.default_rng(M + K)
+    w, cb = rows_inputs(kind, M, K, blk, g)
+    per = {"oil8": 1, "oil4": 2, "tern": 4}[kind]
+    cols, zero = np.array([0, K // 2, K - 1]), M // 2
+    if kind == "oil8":
+        cb[7] = 0.0
+        w[:zero, cols] = 7
+    elif kind == "oil4":
+        cb.reshape(-1, 16)[:, 5] = 0
+        for c in cols:
+            w[:zero, c // 2] = (w[:zero, c // 2] & (0xF0 if c % 2 == 0 else 0x0F)) | (5 << (4 * (c % 2)))
+    else:
+        for c in cols:
+            w[:zero, c // 4] = (w[:zero, c // 4] & ~np.uint8(3 << (2 * (c % 4)))) | (1 << (2 * (c % 4)))
+    x = (1 + g.random((batch, K))).astype(np.float32) * g.choice([-1, 1], (batch, K)).astype(np.float32)
+    plain = rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev)
+    wide = [0, batch // 2, batch - 1]
+    for t in wide:
+        x[t, cols] *= span
+    got = rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev)
+    rest = [t for t in range(batch) if t not in wide]
+    assert torch.equal(got[rest], plain[rest])
+    W, X = w64(kind, w, cb, M, K, blk, dev), torch.from_numpy(x).to(dev).double()
+    want, absw = X @ W.T.contiguous(), X.abs() @ W.abs().T.contiguous()
+    got = got.double()
+    assert bool(((got - want).abs() <= 1e-5 * absw + 1e-30).all())
+    err = (got - want)[wide][:, :zero].norm(dim=1) / want[wide][:, :zero].norm(dim=1)
+    assert bool((err <= 1e-6).all()), err
+
+
 # ----------------------------------------------------------------- argmax --
 @pytest.mark.parametrize("rows,n", [(15, 2048), (16, 2049), (17, 5000), (33, 140001)])
 def test_argmax_rows(rows, n, oracle, mth, dev):
