@@ -452,7 +452,11 @@ struct SwigluTile {
 // TAIL: NW NPH 256 > K (any K % 128 == 0): loads past the row are clamped into it, x is 0 there and so are the weights
 // (their codebook's byte planes: an infinite entry must not meet a zero).  Rows of more than 4096 run on up to 16
 // waves of 2 or 4 phases: 5000 x 8192 (one wave per output before) 80 -> 11.7 us, 5000 x 9088 89 -> 17.4 us; 16384 x
-// 3968 (vector-ALU kernel before) 19.8 -> 12.3 us.
+// 3968 (vector-ALU kernel before) 19.8 -> 12.3 us.  As FP32 products served these rows before, every kTailSum MFMAs add
+// up from zero (one accumulator over a wave's 16 or 32 rounds at its full size: 640 .. 1664 columns 1.46e-7 .. 1.55e-7
+// off 64-bit sums, the FP32 kernels 1.19e-7 .. 1.21e-7, this 1.03e-7 .. 1.06e-7 for 1 % of the time; 2 at a time 1.0e-7
+// for 2.5 %), and lo parts are held times 2^11, which keeps 22 bits of a value down to 2^-28 of the wave's maximum.
+constexpr int kTailSum = 4;
 template <int NW, int NPH, bool SHARED, bool PAIR = false, bool TAIL = false>
 __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2(const uint8_t* nib, const uint16_t* cbs,
                                                         const float* __restrict__ x, float* __restrict__ y,
@@ -553,7 +557,8 @@ __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2
         for (int t = 0; t < 8; t += 2) {
             const f2v xs = {ldexpf(xv[8 * h + oil4_elem_col(t)], sh), ldexpf(xv[8 * h + oil4_elem_col(t + 1)], sh)};
             const h2v hh = __builtin_convertvector(xs, h2v);
-            const h2v ll = __builtin_convertvector(f2v{xs[0] - (float)hh[0], xs[1] - (float)hh[1]}, h2v);
+            const f2v rs = {xs[0] - (float)hh[0], xs[1] - (float)hh[1]};
+            const h2v ll = __builtin_convertvector(TAIL ? f2v{rs[0] * 2048.0f, rs[1] * 2048.0f} : rs, h2v);
             vh[t] = hh[0], vh[t + 1] = hh[1];
             vl[t] = ll[0], vl[t + 1] = ll[1];
         }
@@ -573,7 +578,7 @@ __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2
     const int xb = ((j & 1) ? L::lo_off : 0) + q * 16;
     auto bfrag = [&](int pm) { return *(const half8*)(wl + xb + pm * 64); };
 
-    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, sum = acc;  // sum (TAIL): acc of every kTailSum products, added up
     half8 bnext = bfrag(0);
 #pragma unroll
     for (int p = 0; p < NPH; ++p) {
@@ -590,13 +595,18 @@ __global__ __launch_bounds__(NW * 64, PAIR && NW >= 4 ? 5 : 1) void oil4_gemv_v2
             const half8 b = bnext;
             if (pm + 1 < NPH * 8) bnext = bfrag(pm + 1);  // one MFMA ahead
             const half8 a = lookup8(m < 4 ? u4get(xa, m) : u4get(yb, m - 4), pl);
+            if (TAIL && m % kTailSum == 0) {
+                sum += acc;
+                acc = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc, 0, 0, 0);
         }
     }
+    if (TAIL) acc += sum;
     // D[4q+i][n]: rows' hi (n = 0) + lo (n = 1) parts (oil4_hi_lo)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float s = oil4_hi_lo(acc[i], lane_xor1(acc[i]));
+        const float s = oil4_hi_lo(acc[i], lane_xor1(acc[i]) * (TAIL ? 0x1p-11f : 1.0f));
         if (j == 0) part[wave * 16 + 4 * q + i] = ldexpf(s, -sh);
     }
     if (lossy) {

@@ -325,7 +325,8 @@ def test_token_rows_non_finite(kind, M, K, batch, what, mth, dev):
 @pytest.mark.parametrize("kind,M,K,batch,blk", [("oil8", 300, 1040, 12, 0), ("oil8", 200, 6448, 70, 0),
                                                 ("oil4", 130, 1120, 33, 32), ("oil4", 1616, 1920, 200, 128),
                                                 ("oil4", 500, 9088, 20, 64), ("tern", 300, 4100, 9, 0),
-                                                ("tern", 4096, 1024, 130, 0)])
+                                                ("tern", 4096, 1024, 130, 0), ("oil4", 500, 1664, 1, 128),
+                                                ("oil4", 500, 9088, 1, 0)])
 @pytest.mark.parametrize("span", [2.0 ** 20, 2.0 ** 27, 2.0 ** 40])
 def test_token_rows_wide_range(kind, M, K, batch, blk, span, mth, dev):
     """Values far above the rest of their row that meet weights of 0 in half of the outputs: those keep the precision
@@ -348,7 +349,7 @@ def test_token_rows_wide_range(kind, M, K, batch, blk, span, mth, dev):
             w[:zero, c // 4] = (w[:zero, c // 4] & ~np.uint8(3 << (2 * (c % 4)))) | (1 << (2 * (c % 4)))
     x = (1 + g.random((batch, K))).astype(np.float32) * g.choice([-1, 1], (batch, K)).astype(np.float32)
     plain = rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev)
-    wide = [0, batch // 2, batch - 1]
+    wide = sorted({0, batch // 2, batch - 1})
     for t in wide:
         x[t, cols] *= span
     got = rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev)
@@ -360,6 +361,21 @@ def test_token_rows_wide_range(kind, M, K, batch, blk, span, mth, dev):
     assert bool(((got - want).abs() <= 1e-5 * absw + 1e-30).all())
     err = (got - want)[wide][:, :zero].norm(dim=1) / want[wide][:, :zero].norm(dim=1)
     assert bool((err <= 1e-6).all()), err
+
+
+@pytest.mark.parametrize("K,blk", [(640, 128), (1152, 128), (1664, 0), (3968, 128), (9088, 128)])
+def test_one_token_error(K, blk, mth, dev):
+    """One token's sums against float64: FP32 products in 64 lanes are 1.2e-7 (640 .. 1664 columns) .. 2.3e-7 (9088) of
+    the norm off; parts of 22 bits (4e-8) in short sums stay below that."""
+    import torch
+    M = 8000
+    print(f"one token error K={K} blk={blk}", flush=True)
+    g = np.random.default_rng(K)
+    w, cb = rows_inputs("oil4", M, K, blk, g)
+    x = g.normal(0, 1, (1, K)).astype(np.float32)
+    got = rows_call("oil4", mth, w, cb, x, M, K, 1, blk, dev).double()
+    want = torch.from_numpy(x).to(dev).double() @ w64("oil4", w, cb, M, K, blk, dev).T.contiguous()
+    assert float((got - want).norm() / want.norm()) <= 1.3e-7
 
 
 # ----------------------------------------------------------------- argmax --
