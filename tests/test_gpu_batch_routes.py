@@ -378,6 +378,22 @@ def test_one_token_error(K, blk, mth, dev):
     assert float((got - want).norm() / want.norm()) <= 1.3e-7
 
 
+@pytest.mark.parametrize("M,K,batch", [(4096, 4096, 512), (12288, 4096, 1024), (8192, 1024, 300)])
+def test_prompt_gemm_oil8_error(M, K, batch, mth, dev):
+    """The OIL8 prompt GEMM's sums against float64, tiles of 128 and of 256 rows.  An MFMA rounds its accumulator once
+    per 8 columns, by 2.5e-8 of its size in the mean square, at sizes that grow to the full (half of it in the mean
+    square); the parts' own rounding is 8e-8.  A tenth more for the sample."""
+    import torch
+    print(f"prompt GEMM error M={M} K={K} batch={batch}", flush=True)
+    g = np.random.default_rng(K)
+    w, cb = rows_inputs("oil8", M, K, 0, g)
+    x = g.normal(0, 1, (batch, K)).astype(np.float32)
+    got = rows_call("oil8", mth, w, cb, x, M, K, batch, 0, dev).double()
+    want = torch.from_numpy(x).to(dev).double() @ w64("oil8", w, cb, M, K, 0, dev).T.contiguous()
+    err = float((got - want).norm() / want.norm())
+    assert err <= 1.1 * (K / 16 * 2.5e-8 ** 2 + 8e-8 ** 2) ** 0.5, err
+
+
 # ----------------------------------------------------------------- argmax --
 @pytest.mark.parametrize("rows,n", [(15, 2048), (16, 2049), (17, 5000), (33, 140001)])
 def test_argmax_rows(rows, n, oracle, mth, dev):
