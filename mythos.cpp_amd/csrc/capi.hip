@@ -216,7 +216,7 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
                      ((K % 16 == 0 && K <= 4096 && M * K < (1ll << 32)) || mth::oil8_long_supported(indices, x, M, K));
     if (!one && mth::oil8_rows_better(&seg, 1, K, batch, aligned, gemm, bt)) {
         if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), batch > 1))
-            return check_launch(mth::launch_oil8_rows(&seg, 1, x, K, batch, !bt && !gemm, ws, S(stream)),
+            return check_launch(mth::launch_oil8_rows(&seg, 1, x, K, batch, !bt && !gemm, ws, S(stream), true),
                                 "mth_oil8_gemv");
     }
     if (gemm) {
@@ -265,7 +265,7 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
     if (!one && mth::oil4_rows_better(packed, codebooks, cb_block, M, K, batch, aligned, gemm, bt)) {
         if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), batch > 1))
             return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, !bt && !gemm, ws,
-                                                      S(stream)),
+                                                      S(stream), true),
                                 "mth_oil4_gemv");
     }
     if (gemm) {

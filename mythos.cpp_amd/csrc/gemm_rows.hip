@@ -587,8 +587,8 @@ struct RowsPlan {
     int G, tiles, S, steps;
     int64_t rtiles;
 };
-// (M rows in nseg matrices: at most nseg - 1 row tiles more than M fills)
-inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch, int nseg = 1) {
+// (M rows in nseg matrices: at most nseg - 1 row tiles more than M fills; alone: a call's only product)
+inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch, int nseg = 1, bool alone = false) {
     RowsPlan p{};
     p.steps = (int)((K + kRmStep - 1) / kRmStep);
     const int64_t nt = (batch + 63) / 64;
@@ -603,6 +603,10 @@ inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch, int nseg = 1) {
     const int64_t per = wgs > 256 ? 1 : wgs > 128 ? (p.steps >= 16 ? 512 / wgs : 1)
                       : wgs >= 64 && p.steps >= 48 ? 512 / wgs : 256 / wgs;
     p.S = (int)std::max<int64_t>(1, std::min<int64_t>({per, p.steps / 2, kRmSlices}));
+    // alone, up to 512 columns and 48 tokens per tile: one slice, since the reduction's launch (3 us of host time) costs
+    // more than two steps more in a chain (M = 256 .. 16384, 17 .. 32 tokens 15.1 .. 15.8 us with two slices, 12.3 .. 13.1
+    // with one, 64 tokens 15.1 and 15.9); within a prompt's queue the split is the faster (60 tokens of hidden 512: 5 %).
+    if (alone && p.steps <= 4 && p.G <= 3) p.S = 1;
     return p;
 }
 inline size_t al256r(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -718,7 +722,9 @@ bool oil8_rows_better(const Oil8Seg* seg, int nseg, int64_t K, int64_t batch, bo
         return 1.05 * rows_busy_us(M, K, batch, 1.7) < g;
     }
     const double us = rows_us(M, K, batch, 1.7);
-    if (bt) return batch > 16;  // 17 tokens: 19 .. 49 us against 15 .. 31 us
+    // 16 tokens per launch, or launch pair where K is split (K > 512), against two launches or three: 17 tokens of K =
+    // 1024 .. 4096 20 .. 86 us against 15 .. 48, of K = 512 14.7 .. 16.0 against 12.3 .. 12.9
+    if (bt) return batch > 16;
     return us < walk_us(M, K, batch, true, aligned && K <= 4096);
 }
 
@@ -730,7 +736,9 @@ bool oil4_rows_better(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block,
         return false;
     if (gemm) return 1.05 * rows_busy_us(M, K, batch, 1.6) < oil4_gemm_x32_us(batch, M, K);
     const double us = rows_us(M, K, batch, 1.85);
-    if (bt) return batch > 16;  // 17 tokens: 18 .. 49 us against 15 .. 48 us
+    // as for OIL8: 17 tokens of K = 1024 .. 4096 18 .. 94 us against 15 .. 52.  K = 512 in two launches: 11.5 .. 12.3 us up
+    // to 16384 rows against 12.4 .. 12.7, 15.4 us at 32000 against 12.9 (about 2 x (4.4 us + 1e-4 us per row))
+    if (bt) return batch > 16 && !(K == 512 && batch <= 32 && M < 18000);
     return us < walk_us(M, K, batch, false, aligned && K <= 4096);
 }
 
@@ -755,11 +763,11 @@ bool oil4_rows_bf16_better(int64_t M, int64_t K, int64_t batch, double tiled_us)
 }
 
 hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, bool fp32, void* ws,
-                            hipStream_t s) {
+                            hipStream_t s, bool alone) {
     RowsSegs sg{};
     int64_t M = 0, tiles = 0;
     for (int i = 0; i < nseg; ++i) M += seg[i].rows;
-    const RowsPlan p = rows_plan(M, K, batch, nseg);
+    const RowsPlan p = rows_plan(M, K, batch, nseg, alone);
     sg.n = nseg;
     M = 0;
     for (int i = 0; i < 3; ++i) {
@@ -778,9 +786,9 @@ hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_
     return rows_run<kOil8>(a, p, ws, s, sg);
 }
 hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
-                            int64_t M, int64_t K, int64_t batch, bool fp32, void* ws, hipStream_t s) {
+                            int64_t M, int64_t K, int64_t batch, bool fp32, void* ws, hipStream_t s, bool alone) {
     RowsArgs a{nib, cbs, nullptr, nullptr, x, y, nullptr, (int)M, (int)K, (int)batch, 0, (int)cb_block, fp32};
-    return rows_run<kOil4>(a, rows_plan(M, K, batch), ws, s);
+    return rows_run<kOil4>(a, rows_plan(M, K, batch, 1, alone), ws, s);
 }
 hipError_t launch_oil4_rows_bf16(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const uint16_t* x,
                                  uint16_t* y, int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s) {

@@ -245,11 +245,13 @@ hipError_t launch_oil4_rows_bf16(const uint8_t* nib, const uint16_t* cbs, int64_
                                  uint16_t* y, int64_t M, int64_t K, int64_t batch, void* ws, hipStream_t s);
 bool tern_rows_better(int64_t M, int64_t K, int64_t batch);
 // fp32: the call's other route is FP32 products; rows that span more than 28 binades then take them here too, and so does
-// an OIL4 output that comes out NaN (an infinite codebook entry times a value that both parts miss)
+// an OIL4 output that comes out NaN (an infinite codebook entry times a value that both parts miss).  alone: the launches
+// are a call's only ones (one less where that is the faster)
 hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_t K, int64_t batch, bool fp32, void* ws,
-                            hipStream_t s);
+                            hipStream_t s, bool alone = false);
 hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
-                            int64_t M, int64_t K, int64_t batch, bool fp32, void* ws, hipStream_t s);
+                            int64_t M, int64_t K, int64_t batch, bool fp32, void* ws, hipStream_t s,
+                            bool alone = false);
 hipError_t launch_tern_rows(const uint8_t* w, const float* x, float* out, int64_t M, int64_t K, int64_t batch,
                             void* ws, hipStream_t s);
 

@@ -74,3 +74,16 @@ def test_partial_tiles_of_fp32_rows():
         assert not on(r, "oil4_prefill_ws"), (c, kernels(r))
     r = recorded.run([oil4(22016, 4096, 512, next(stream))])[0]
     assert on(r, "oil4_prefill_ws"), kernels(r)
+
+
+def test_token_rows_take_no_more_launches():
+    """17 .. 127 tokens at shapes the batched GEMVs take (16 tokens per launch,
+    with a reduction where K is split): the route taken has no more launches."""
+    calls, most = [], []
+    for K in (512, 1024, 2048, 4096):
+        for M in (256, 2048, 8192, 16384, 32000):
+            for b in (17, 32, 33, 48, 64, 127):
+                calls += [oil8(M, K, b, next(stream)), oil4(M, K, b, next(stream)), oil4(M, K, b, next(stream), 0)]
+                most += 3 * [(b + 15) // 16 * (1 if K == 512 else 2)]
+    for c, n, r in zip(calls, most, recorded.run(calls)):
+        assert len(kernels(r)) <= n, (c, kernels(r))
