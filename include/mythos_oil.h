@@ -31,9 +31,10 @@
  * odd sizes and token counts, mth_attention_decode over long contexts,
  * mth_i2s_gemm, mth_i2s_gemv_f32 and single-token calls of odd sizes.  Such a
  * call never fails for want of it: where the workspace cannot grow it runs as
- * the sizes above say.  mth_attention_decode, mth_i2s_gemm, mth_i2s_gemv_f32
- * and single-token calls use no workspace at all inside a capture.  No other
- * entry point allocates.
+ * the sizes above say.  Inside a capture a call whose route by these sizes
+ * keeps nothing there (mth_attention_decode, mth_i2s_gemm, mth_i2s_gemv_f32,
+ * single tokens, odd sizes) uses no workspace at all.  No other entry point
+ * allocates.
  * Calls on one stream share its workspace (threads may share the stream: a
  * call's launches are enqueued together).  hipStreamPerThread is one handle
  * for a stream of its own in every thread: the routes that a call can do

@@ -97,9 +97,10 @@ hipError_t workspace(hipStream_t s, size_t need, void** out) {
 
 // The stream's workspace for a faster route that the call can do without: null where it cannot grow now (the
 // stream is capturing, or the allocation failed), and the call then takes the route that needs less.  graphs: whether
-// a captured call may use what the stream holds; not for calls that need no workspace on the other route, whose graphs
-// may be replayed beside other work of the stream they were captured on.  hipStreamPerThread: null, since that one
-// handle is another stream in every thread, and a block kept by handle would be shared by streams that run together.
+// the other route keeps something there too; only then does a captured call use what the stream holds, since the graph
+// of a call without workspace may be replayed beside other work of the stream it was captured on.  hipStreamPerThread:
+// null, since that one handle is another stream in every thread, and a block kept by handle would be shared by streams
+// that run together.
 void* workspace_or_null(hipStream_t s, size_t need, bool graphs) {
     void* p = nullptr;
     if (s == hipStreamPerThread) return nullptr;
@@ -215,7 +216,8 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
     const bool one = batch == 1 && aligned &&  // one token: kernels of their own up to 16384 columns
                      ((K % 16 == 0 && K <= 4096 && M * K < (1ll << 32)) || mth::oil8_long_supported(indices, x, M, K));
     if (!one && mth::oil8_rows_better(&seg, 1, K, batch, aligned, gemm, bt)) {
-        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), batch > 1))
+        const bool graphs = gemm || (bt && mth::oil8_bt_partial_bytes(M, K) != 0);
+        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), graphs))
             return check_launch(mth::launch_oil8_rows(&seg, 1, x, K, batch, !bt && !gemm, ws, S(stream), true),
                                 "mth_oil8_gemv");
     }
@@ -263,7 +265,8 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
     const bool one = batch == 1 && aligned &&  // one token: kernels of their own
                      (K <= 4096 || mth::oil4_one_supported(packed, codebooks, x, cb_block, M, K));
     if (!one && mth::oil4_rows_better(packed, codebooks, cb_block, M, K, batch, aligned, gemm, bt)) {
-        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), batch > 1))
+        const bool graphs = gemm || (bt && mth::oil4_bt_partial_bytes(M, K) != 0);
+        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), graphs))
             return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, !bt && !gemm, ws,
                                                       S(stream), true),
                                 "mth_oil4_gemv");
@@ -391,14 +394,15 @@ int mth_i2s_gemv(const uint8_t* packed, float w_scale, const int8_t* act, const 
             "mth_i2s_gemv: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
     REQUIRE(K % 4 == 0, "mth_i2s_gemv: K=%lld must be a multiple of 4", (long long)K);
     const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
+    const bool bt = (((uintptr_t)packed | (uintptr_t)act) & 15u) == 0 && mth::i2s_bt_supported(M, K, batch);
     if (mth::i2s_rows_supported(packed, act, false, M, K, batch)) {
-        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch), batch > 1))
+        const bool graphs = bt && mth::i2s_bt_partial_bytes(M, K) != 0;
+        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch), graphs))
             return check_launch(mth::launch_i2s_rows(packed, w_scale, nullptr, act, act_scale, y, M, K, batch, ws,
                                                      S(stream)),
                                 "mth_i2s_gemv");
     }
-    const bool aligned = (((uintptr_t)packed | (uintptr_t)act) & 15u) == 0;
-    if (aligned && mth::i2s_bt_supported(M, K, batch)) {
+    if (bt) {
         void* partial = nullptr;
         const size_t need = mth::i2s_bt_partial_bytes(M, K);
         const hipError_t e = workspace(S(stream), need, &partial);

@@ -87,3 +87,22 @@ def test_token_rows_take_no_more_launches():
                 most += 3 * [(b + 15) // 16 * (1 if K == 512 else 2)]
     for c, n, r in zip(calls, most, recorded.run(calls)):
         assert len(kernels(r)) <= n, (c, kernels(r))
+
+
+def test_graphs_hold_no_workspace_of_calls_without():
+    """Captured on a stream that holds a large workspace: calls whose other
+    route keeps nothing there record no address of it, calls that need it do."""
+    st = next(stream)
+    calls = [{"fn": "mth_workspace_reserve", "args": [1 << 30, st]}]
+    calls += [c for c, _ in without_workspace(st)]
+    calls += [oil8(300, 1040, 40, st), oil8(512, 512, 40, st), oil8(300, 4112, 2, st), oil4(500, 1024, 40, st, 64),
+              oil4(500, 640, 40, st), oil4(512, 512, 40, st), oil4(1616, 384, 200, st), i2s(130, 1028, 20, st),
+              i2s(64, 260, 300, st), i2s(512, 256, 40, st)]
+    needs = len(calls)
+    calls += [oil8(4096, 4096, 40, st), oil4(4096, 4096, 40, st), i2s(4096, 4096, 40, st)]
+    for c in calls[1:]:
+        c["capture"] = st
+    out = recorded.run(calls)
+    for i, (c, r) in enumerate(zip(calls, out)):
+        used = on(r, *ROWS, "i2s_pad_rows_k", "i2s_quant_rows_k", "i2s_gemm_mfma", "attn_combine", "reduce")
+        assert used == (i >= needs) and (i == 0 or r["mallocs"] == 0), (c, kernels(r))
