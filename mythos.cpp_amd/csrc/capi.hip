@@ -64,35 +64,52 @@ constexpr int64_t kGemmRows = 128;
 struct Workspace {
     void* base = nullptr;
     size_t bytes = 0;
+    std::mutex mu;  // held by a call from here until its launches are enqueued
 };
-std::mutex g_ws_mu;
-std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
+std::mutex g_ws_mu;  // the map and the list; never held while another lock is taken or the runtime is called
+std::map<std::pair<int, hipStream_t>, Workspace> g_ws;  // (its nodes stay where they are)
 std::vector<void*> g_ws_retired;  // superseded blocks: valid until the process ends
 
-// hipSuccess, or hipErrorStreamCaptureUnsupported when growing under capture
-hipError_t workspace(hipStream_t s, size_t need, void** out) {
-    *out = nullptr;
-    if (need == 0) return hipSuccess;
+// A call's hold on its stream's workspace: the block, and the stream's lock while the call enqueues the launches that
+// hand data on through it, so that threads that share a stream do not come between them.  Calls that keep nothing
+// there take no lock.
+struct WsHold {
+    std::unique_lock<std::mutex> order;
+    void* p = nullptr;
+    hipError_t e = hipSuccess;
+};
+
+// e: hipErrorStreamCaptureUnsupported when growing under capture
+WsHold workspace(hipStream_t s, size_t need) {
+    WsHold h;
+    if (need == 0) return h;
     int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> g(g_ws_mu);
-    Workspace& w = g_ws[{dev, s}];
-    if (w.bytes < need) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        e = hipStreamIsCapturing(s, &st);
-        if (e != hipSuccess) return e;
-        if (st != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
-        const size_t bytes = std::max(need, 2 * w.bytes);
-        void* p = nullptr;
-        e = hipMalloc(&p, bytes);
-        if (e != hipSuccess) return e;
-        if (w.base) g_ws_retired.push_back(w.base);
-        w.base = p;
-        w.bytes = bytes;
+    if ((h.e = hipGetDevice(&dev)) != hipSuccess) return h;
+    Workspace* w = nullptr;
+    {
+        const std::lock_guard<std::mutex> g(g_ws_mu);
+        w = &g_ws[{dev, s}];
     }
-    *out = w.base;
-    return hipSuccess;
+    h.order = std::unique_lock<std::mutex>(w->mu);
+    if (w->bytes < need) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if ((h.e = hipStreamIsCapturing(s, &st)) != hipSuccess) return h;
+        if (st != hipStreamCaptureStatusNone) {
+            h.e = hipErrorStreamCaptureUnsupported;
+            return h;
+        }
+        const size_t bytes = std::max(need, 2 * w->bytes);
+        void* p = nullptr;
+        if ((h.e = hipMalloc(&p, bytes)) != hipSuccess) return h;
+        if (w->base) {
+            const std::lock_guard<std::mutex> g(g_ws_mu);
+            g_ws_retired.push_back(w->base);
+        }
+        w->base = p;
+        w->bytes = bytes;
+    }
+    h.p = w->base;
+    return h;
 }
 
 // The stream's workspace for a faster route that the call can do without: null where it cannot grow now (the
@@ -101,27 +118,19 @@ hipError_t workspace(hipStream_t s, size_t need, void** out) {
 // of a call without workspace may be replayed beside other work of the stream it was captured on.  hipStreamPerThread:
 // null, since that one handle is another stream in every thread, and a block kept by handle would be shared by streams
 // that run together.
-void* workspace_or_null(hipStream_t s, size_t need, bool graphs) {
-    void* p = nullptr;
-    if (s == hipStreamPerThread) return nullptr;
+WsHold workspace_or_null(hipStream_t s, size_t need, bool graphs) {
+    if (s == hipStreamPerThread) return WsHold{};
     if (!graphs) {
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
             (void)hipGetLastError();
-            return nullptr;
+            return WsHold{};
         }
     }
-    if (workspace(s, need, &p) == hipSuccess) return p;
+    WsHold h = workspace(s, need);
+    if (h.e == hipSuccess) return h;
     (void)hipGetLastError();
-    return nullptr;
-}
-
-// Held while a call enqueues the launches that hand data on through the workspace: threads that share a stream do not
-// come between them.  One of 64 locks by stream.
-std::mutex& ws_launches(hipStream_t s) {
-    static std::mutex mu[64];
-    const uintptr_t v = (uintptr_t)s;
-    return mu[((v >> 6) ^ (v >> 12) ^ (v >> 18)) & 63u];
+    return WsHold{};
 }
 
 int workspace_fail(const char* what, hipError_t e, size_t need) {
@@ -189,9 +198,8 @@ int mth_version(void) { return (2 << 16) | 0; }
 
 int mth_workspace_reserve(int64_t bytes, mth_stream_t stream) {
     REQUIRE(bytes >= 0 && bytes < kMaxDim, "mth_workspace_reserve: bad size %lld", (long long)bytes);
-    void* p = nullptr;
-    const hipError_t e = workspace(S(stream), (size_t)bytes, &p);
-    if (e != hipSuccess) return workspace_fail("mth_workspace_reserve", e, (size_t)bytes);
+    const WsHold h = workspace(S(stream), (size_t)bytes);
+    if (h.e != hipSuccess) return workspace_fail("mth_workspace_reserve", h.e, (size_t)bytes);
     return ok();
 }
 
@@ -208,7 +216,6 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
     REQUIRE(indices && codebook && x && y, "mth_oil8_gemv: null pointer");
     REQUIRE(M > 0 && K > 0 && batch > 0 && M < kMaxDim && K < kMaxDim && batch <= 65536,
             "mth_oil8_gemv: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const bool aligned = (((uintptr_t)indices | (uintptr_t)x) & 15u) == 0;
     const mth::Oil8Seg seg{indices, codebook, y, M};
     const bool gemm = aligned && batch >= kGemmRows && mth::oil8_gemm_x32_supported(&seg, 1, batch, K);
@@ -217,24 +224,22 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
                      ((K % 16 == 0 && K <= 4096 && M * K < (1ll << 32)) || mth::oil8_long_supported(indices, x, M, K));
     if (!one && mth::oil8_rows_better(&seg, 1, K, batch, aligned, gemm, bt)) {
         const bool graphs = gemm || (bt && mth::oil8_bt_partial_bytes(M, K) != 0);
-        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), graphs))
-            return check_launch(mth::launch_oil8_rows(&seg, 1, x, K, batch, !bt && !gemm, ws, S(stream), true),
+        if (const WsHold ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), graphs); ws.p)
+            return check_launch(mth::launch_oil8_rows(&seg, 1, x, K, batch, !bt && !gemm, ws.p, S(stream), true),
                                 "mth_oil8_gemv");
     }
     if (gemm) {
         // >= 128 tokens: the MFMA GEMM (each weight read once per 128 tokens)
-        void* ws = nullptr;
         const size_t need = mth::oil8_gemm_x32_workspace_bytes(batch, K);
-        const hipError_t e = workspace(S(stream), need, &ws);
-        if (e != hipSuccess) return workspace_fail("mth_oil8_gemv", e, need);
-        return check_launch(mth::launch_oil8_gemm_x32(x, &seg, 1, batch, K, ws, S(stream)), "mth_oil8_gemv");
+        const WsHold ws = workspace(S(stream), need);
+        if (ws.e != hipSuccess) return workspace_fail("mth_oil8_gemv", ws.e, need);
+        return check_launch(mth::launch_oil8_gemm_x32(x, &seg, 1, batch, K, ws.p, S(stream)), "mth_oil8_gemv");
     }
     if (bt) {
-        void* partial = nullptr;
         const size_t need = mth::oil8_bt_partial_bytes(M, K);
-        const hipError_t e = workspace(S(stream), need, &partial);
-        if (e != hipSuccess) return workspace_fail("mth_oil8_gemv", e, need);
-        return check_launch(mth::launch_oil8_gemv_bt(indices, codebook, x, y, M, K, batch, (float*)partial, S(stream)),
+        const WsHold ws = workspace(S(stream), need);
+        if (ws.e != hipSuccess) return workspace_fail("mth_oil8_gemv", ws.e, need);
+        return check_launch(mth::launch_oil8_gemv_bt(indices, codebook, x, y, M, K, batch, (float*)ws.p, S(stream)),
                             "mth_oil8_gemv");
     }
     return check_launch(mth::launch_oil8_gemv(indices, codebook, x, y, M, K, batch, S(stream)), "mth_oil8_gemv");
@@ -257,7 +262,6 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
     REQUIRE(cb_block >= 0, "mth_oil4_gemv: cb_block=%lld < 0", (long long)cb_block);
     REQUIRE(cb_block == 0 || K % cb_block == 0, "mth_oil4_gemv: K=%lld not a multiple of cb_block=%lld",
             (long long)K, (long long)cb_block);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const bool aligned = (((uintptr_t)packed | (uintptr_t)codebooks | (uintptr_t)x) & 15u) == 0;
     const bool gemm = aligned && ((uintptr_t)y & 15u) == 0 && batch >= kGemmRows &&
                       mth::oil4_gemm_x32_supported(batch, M, K, cb_block);
@@ -266,26 +270,24 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
                      (K <= 4096 || mth::oil4_one_supported(packed, codebooks, x, cb_block, M, K));
     if (!one && mth::oil4_rows_better(packed, codebooks, cb_block, M, K, batch, aligned, gemm, bt)) {
         const bool graphs = gemm || (bt && mth::oil4_bt_partial_bytes(M, K) != 0);
-        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), graphs))
-            return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, !bt && !gemm, ws,
+        if (const WsHold ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, batch), graphs); ws.p)
+            return check_launch(mth::launch_oil4_rows(packed, codebooks, cb_block, x, y, M, K, batch, !bt && !gemm, ws.p,
                                                       S(stream), true),
                                 "mth_oil4_gemv");
     }
     if (gemm) {
         // >= 128 tokens: the MFMA GEMM (each weight read once per 128 tokens)
-        void* ws = nullptr;
         const size_t need = mth::oil4_gemm_x32_workspace_bytes(batch, K);
-        const hipError_t e = workspace(S(stream), need, &ws);
-        if (e != hipSuccess) return workspace_fail("mth_oil4_gemv", e, need);
-        return check_launch(mth::launch_oil4_gemm_x32(x, packed, codebooks, cb_block, y, batch, M, K, ws, S(stream)),
+        const WsHold ws = workspace(S(stream), need);
+        if (ws.e != hipSuccess) return workspace_fail("mth_oil4_gemv", ws.e, need);
+        return check_launch(mth::launch_oil4_gemm_x32(x, packed, codebooks, cb_block, y, batch, M, K, ws.p, S(stream)),
                             "mth_oil4_gemv");
     }
     if (bt) {
-        void* partial = nullptr;
         const size_t need = mth::oil4_bt_partial_bytes(M, K);
-        const hipError_t e = workspace(S(stream), need, &partial);
-        if (e != hipSuccess) return workspace_fail("mth_oil4_gemv", e, need);
-        return check_launch(mth::launch_oil4_gemv_bt(packed, codebooks, cb_block, x, y, M, K, batch, (float*)partial,
+        const WsHold ws = workspace(S(stream), need);
+        if (ws.e != hipSuccess) return workspace_fail("mth_oil4_gemv", ws.e, need);
+        return check_launch(mth::launch_oil4_gemv_bt(packed, codebooks, cb_block, x, y, M, K, batch, (float*)ws.p,
                                                      S(stream)),
                             "mth_oil4_gemv");
     }
@@ -331,7 +333,6 @@ int mth_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* packed, const u
     REQUIRE(K % 2 == 0, "mth_oil4_gemm_prefill: K=%lld must be even", (long long)K);
     REQUIRE(cb_block > 0 && K % cb_block == 0, "mth_oil4_gemm_prefill: K=%lld not a multiple of cb_block=%lld",
             (long long)K, (long long)cb_block);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const bool aligned = (((uintptr_t)a_bf16 | (uintptr_t)packed | (uintptr_t)codebooks | (uintptr_t)c_bf16) & 15u) == 0;
     if (!aligned || !mth::oil4_gemm_prefill_supported(M, N, K, cb_block))
         return fail(MTH_EUNSUPPORTED,
@@ -339,8 +340,8 @@ int mth_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* packed, const u
                     "(needs K %% 32 == 0, cb_block %% 32 == 0, 16-byte aligned inputs)",
                     (long long)M, (long long)N, (long long)K, (long long)cb_block);
     if (mth::oil4_rows_bf16_better(N, K, M, mth::oil4_prefill_us(M, N, K, cb_block))) {
-        if (void* ws = workspace_or_null(S(stream), mth::rows_bf16_workspace_bytes(N, K, M), true))
-            return check_launch(mth::launch_oil4_rows_bf16(packed, codebooks, cb_block, a_bf16, c_bf16, N, K, M, ws,
+        if (const WsHold ws = workspace_or_null(S(stream), mth::rows_bf16_workspace_bytes(N, K, M), true); ws.p)
+            return check_launch(mth::launch_oil4_rows_bf16(packed, codebooks, cb_block, a_bf16, c_bf16, N, K, M, ws.p,
                                                            S(stream)),
                                 "mth_oil4_gemm_prefill");
     }
@@ -349,17 +350,17 @@ int mth_oil4_gemm_prefill(const uint16_t* a_bf16, const uint8_t* packed, const u
     const size_t shifts = mth::oil4_prefill_shift_bytes(M);
     const size_t a16 = mth::oil4_prefill_workspace_bytes(M, N, K, cb_block);
     const bool whole = mth::oil4_whole_tiles(N, K);
-    void* ws = a16 && !whole ? workspace_or_null(S(stream), shifts + a16, true) : nullptr;
-    if (a16 && (ws || whole)) {
-        const hipError_t e = ws ? hipSuccess : workspace(S(stream), shifts + a16, &ws);
-        if (e != hipSuccess) return workspace_fail("mth_oil4_gemm_prefill", e, shifts + a16);
-        return check_launch(mth::launch_oil4_gemm_prefill_a16(a_bf16, packed, codebooks, cb_block, c_bf16, M, N, K, ws,
-                                                             S(stream)),
-                            "mth_oil4_gemm_prefill");
+    if (a16) {
+        const WsHold ws = whole ? workspace(S(stream), shifts + a16) : workspace_or_null(S(stream), shifts + a16, true);
+        if (ws.e != hipSuccess) return workspace_fail("mth_oil4_gemm_prefill", ws.e, shifts + a16);
+        if (ws.p)
+            return check_launch(mth::launch_oil4_gemm_prefill_a16(a_bf16, packed, codebooks, cb_block, c_bf16, M, N, K,
+                                                                 ws.p, S(stream)),
+                                "mth_oil4_gemm_prefill");
     }
-    const hipError_t e = workspace(S(stream), shifts, &ws);
-    if (e != hipSuccess) return workspace_fail("mth_oil4_gemm_prefill", e, shifts);
-    return check_launch(mth::launch_oil4_gemm_prefill(a_bf16, packed, codebooks, cb_block, c_bf16, M, N, K, (int*)ws,
+    const WsHold ws = workspace(S(stream), shifts);
+    if (ws.e != hipSuccess) return workspace_fail("mth_oil4_gemm_prefill", ws.e, shifts);
+    return check_launch(mth::launch_oil4_gemm_prefill(a_bf16, packed, codebooks, cb_block, c_bf16, M, N, K, (int*)ws.p,
                                                       S(stream)),
                         "mth_oil4_gemm_prefill");
 }
@@ -393,21 +394,19 @@ int mth_i2s_gemv(const uint8_t* packed, float w_scale, const int8_t* act, const 
     REQUIRE(M > 0 && K > 0 && batch > 0 && M < kMaxDim && K < (1ll << 24) && batch <= 65536,
             "mth_i2s_gemv: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
     REQUIRE(K % 4 == 0, "mth_i2s_gemv: K=%lld must be a multiple of 4", (long long)K);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const bool bt = (((uintptr_t)packed | (uintptr_t)act) & 15u) == 0 && mth::i2s_bt_supported(M, K, batch);
     if (mth::i2s_rows_supported(packed, act, false, M, K, batch)) {
         const bool graphs = bt && mth::i2s_bt_partial_bytes(M, K) != 0;
-        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch), graphs))
-            return check_launch(mth::launch_i2s_rows(packed, w_scale, nullptr, act, act_scale, y, M, K, batch, ws,
+        if (const WsHold ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch), graphs); ws.p)
+            return check_launch(mth::launch_i2s_rows(packed, w_scale, nullptr, act, act_scale, y, M, K, batch, ws.p,
                                                      S(stream)),
                                 "mth_i2s_gemv");
     }
     if (bt) {
-        void* partial = nullptr;
         const size_t need = mth::i2s_bt_partial_bytes(M, K);
-        const hipError_t e = workspace(S(stream), need, &partial);
-        if (e != hipSuccess) return workspace_fail("mth_i2s_gemv", e, need);
-        return check_launch(mth::launch_i2s_gemv_bt(packed, w_scale, act, act_scale, y, M, K, batch, (float*)partial,
+        const WsHold ws = workspace(S(stream), need);
+        if (ws.e != hipSuccess) return workspace_fail("mth_i2s_gemv", ws.e, need);
+        return check_launch(mth::launch_i2s_gemv_bt(packed, w_scale, act, act_scale, y, M, K, batch, (float*)ws.p,
                                                     S(stream)),
                             "mth_i2s_gemv");
     }
@@ -421,10 +420,9 @@ int mth_i2s_gemv_f32(const uint8_t* packed, float w_scale, const float* x, float
     REQUIRE(M > 0 && K > 0 && batch > 0 && M < kMaxDim && K < (1ll << 24) && batch <= 65536,
             "mth_i2s_gemv_f32: bad sizes M=%lld K=%lld batch=%lld", (long long)M, (long long)K, (long long)batch);
     REQUIRE(K % 4 == 0, "mth_i2s_gemv_f32: K=%lld must be a multiple of 4", (long long)K);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     if (mth::i2s_rows_supported(packed, x, true, M, K, batch)) {
-        if (void* ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch), false))
-            return check_launch(mth::launch_i2s_rows(packed, w_scale, x, nullptr, nullptr, y, M, K, batch, ws,
+        if (const WsHold ws = workspace_or_null(S(stream), mth::i2s_rows_workspace_bytes(M, K, batch), false); ws.p)
+            return check_launch(mth::launch_i2s_rows(packed, w_scale, x, nullptr, nullptr, y, M, K, batch, ws.p,
                                                      S(stream)),
                                 "mth_i2s_gemv_f32");
     }
@@ -436,10 +434,9 @@ int mth_i2s_gemm(const uint8_t* w, const float* act, float* out, int64_t M, int6
                  mth_stream_t stream) {
     REQUIRE(w && act && out, "mth_i2s_gemm: null pointer");
     REQUIRE(M > 0 && N > 0 && K > 0 && M * N < kMaxDim && K < kMaxDim, "mth_i2s_gemm: bad sizes");
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     if (mth::tern_rows_better(M, K, N)) {
-        if (void* ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, N), false))
-            return check_launch(mth::launch_tern_rows(w, act, out, M, K, N, ws, S(stream)), "mth_i2s_gemm");
+        if (const WsHold ws = workspace_or_null(S(stream), mth::rows_mfma_workspace_bytes(M, K, N), false); ws.p)
+            return check_launch(mth::launch_tern_rows(w, act, out, M, K, N, ws.p, S(stream)), "mth_i2s_gemm");
     }
     return check_launch(mth::launch_i2s_gemm(w, act, out, M, N, K, S(stream)), "mth_i2s_gemm");
 }
@@ -463,13 +460,11 @@ int mth_tl2_gemm(const uint8_t* w, const float* act, float* out, int64_t M, int6
     REQUIRE(w && act && out, "mth_tl2_gemm: null pointer");
     REQUIRE(M > 0 && N > 0 && K > 0 && M * N < kMaxDim && K < (1ll << 24), "mth_tl2_gemm: bad sizes");
     REQUIRE(K % 3 == 0, "mth_tl2_gemm: K=%lld must be a multiple of 3", (long long)K);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     const size_t need = mth::tl2_workspace_bytes(w, M, N, K);
     if (need) {
-        void* ws = nullptr;
-        const hipError_t e = workspace(S(stream), need, &ws);
-        if (e != hipSuccess) return workspace_fail("mth_tl2_gemm", e, need);
-        return check_launch(mth::launch_tl2_gemm_ws(w, act, out, M, N, K, ws, S(stream)), "mth_tl2_gemm");
+        const WsHold ws = workspace(S(stream), need);
+        if (ws.e != hipSuccess) return workspace_fail("mth_tl2_gemm", ws.e, need);
+        return check_launch(mth::launch_tl2_gemm_ws(w, act, out, M, N, K, ws.p, S(stream)), "mth_tl2_gemm");
     }
     return check_launch(mth::launch_tl2_gemm(w, act, out, M, N, K, S(stream)), "mth_tl2_gemm");
 }
@@ -553,13 +548,11 @@ int mth_oil4_gemv_swiglu_batch(const uint8_t* packed, const uint16_t* codebooks,
             "mth_oil4_gemv_swiglu_batch: F=%lld K=%lld cb_block=%lld not supported (F %% 4 == 0, K %% 512 == 0, "
             "512 <= K <= 8192, cb_block 0 or 128)",
             (long long)F, (long long)K, (long long)cb_block);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
-    void* partial = nullptr;
     const size_t need = mth::oil4_bt_partial_bytes(2 * F, K);
-    const hipError_t e = workspace(S(stream), need, &partial);
-    if (e != hipSuccess) return workspace_fail("mth_oil4_gemv_swiglu_batch", e, need);
+    const WsHold ws = workspace(S(stream), need);
+    if (ws.e != hipSuccess) return workspace_fail("mth_oil4_gemv_swiglu_batch", ws.e, need);
     return check_launch(mth::launch_oil4_gemv_bt_swiglu(packed, codebooks, cb_block, x, mth::NormScale{}, gu, amax, F,
-                                                        K, batch, (float*)partial, S(stream)),
+                                                        K, batch, (float*)ws.p, S(stream)),
                         "mth_oil4_gemv_swiglu_batch");
 }
 
@@ -574,13 +567,11 @@ int mth_i2s_gemv_act_batch(const uint8_t* packed, float w_scale, const float* ac
     REQUIRE((((uintptr_t)packed | (uintptr_t)act) & 15u) == 0,
             "mth_i2s_gemv_act_batch: packed and act must be 16-byte aligned");
     REQUIRE(mth::i2s_bt_supported(M, K, batch), "mth_i2s_gemv_act_batch: K=%lld not a multiple of 256", (long long)K);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
-    void* partial = nullptr;
     const size_t need = mth::i2s_bt_partial_bytes(M, K);
-    const hipError_t e = workspace(S(stream), need, &partial);
-    if (e != hipSuccess) return workspace_fail("mth_i2s_gemv_act_batch", e, need);
+    const WsHold ws = workspace(S(stream), need);
+    if (ws.e != hipSuccess) return workspace_fail("mth_i2s_gemv_act_batch", ws.e, need);
     return check_launch(mth::launch_i2s_gemv_bt_f32act_y(packed, w_scale, act, lda, amax, mth::oil4_bt_swiglu_parts(K),
-                                                         inv_scale, y, M, K, batch, (float*)partial, S(stream)),
+                                                         inv_scale, y, M, K, batch, (float*)ws.p, S(stream)),
                         "mth_i2s_gemv_act_batch");
 }
 
@@ -694,13 +685,12 @@ int mth_attention_decode(const float* q, const float* kcache, const float* vcach
             (long long)head_dim, (long long)max_seq);
     REQUIRE(ctx >= 1 && ctx <= max_seq, "mth_attention_decode: ctx=%lld outside 1..%lld", (long long)ctx,
             (long long)max_seq);
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
     if (mth::attention_split_supported(q, kcache, vcache, batch, (int)heads, (int)kv_heads, (int)head_dim, (int)ctx,
                                        (int)max_seq)) {
-        if (void* ws = workspace_or_null(S(stream), mth::attention_split_workspace_bytes(batch, (int)heads, (int)kv_heads,
-                                                                                         (int)head_dim, (int)ctx), false))
+        const size_t need = mth::attention_split_workspace_bytes(batch, (int)heads, (int)kv_heads, (int)head_dim, (int)ctx);
+        if (const WsHold ws = workspace_or_null(S(stream), need, false); ws.p)
             return check_launch(mth::launch_attention_split(q, kcache, vcache, out, (int)ctx, batch, (int)heads,
-                                                            (int)kv_heads, (int)head_dim, (int)max_seq, ws, S(stream)),
+                                                            (int)kv_heads, (int)head_dim, (int)max_seq, ws.p, S(stream)),
                                 "mth_attention_decode");
     }
     return check_launch(mth::launch_attention(q, kcache, vcache, out, nullptr, (int)ctx - 1, batch, (int)heads,
@@ -711,13 +701,11 @@ int mth_attention_decode(const float* q, const float* kcache, const float* vcach
 int mth_argmax(const float* logits, int32_t* ids, int64_t rows, int64_t n, mth_stream_t stream) {
     REQUIRE(logits && ids, "mth_argmax: null pointer");
     REQUIRE(rows > 0 && rows <= 65535 && n > 0 && n < (1ll << 31), "mth_argmax: bad sizes");
-    const std::lock_guard<std::mutex> order(ws_launches(S(stream)));
-    void* ws = nullptr;
     const size_t nc = (size_t)mth::argmax_chunks(n) * (size_t)rows;
-    const hipError_t e = workspace(S(stream), nc * 8, &ws);
-    if (e != hipSuccess) return workspace_fail("mth_argmax", e, nc * 8);
-    return check_launch(mth::launch_argmax(logits, rows, n, ids, nullptr, nullptr, 0, 0, (float*)ws,
-                                           (int*)((char*)ws + nc * 4), S(stream)),
+    const WsHold ws = workspace(S(stream), nc * 8);
+    if (ws.e != hipSuccess) return workspace_fail("mth_argmax", ws.e, nc * 8);
+    return check_launch(mth::launch_argmax(logits, rows, n, ids, nullptr, nullptr, 0, 0, (float*)ws.p,
+                                           (int*)((char*)ws.p + nc * 4), S(stream)),
                         "mth_argmax");
 }
 

@@ -2,6 +2,8 @@
 HIP runtime replaced by a recorder (recorded.py): no GPU.
 """
 import itertools
+import os
+import textwrap
 
 import recorded
 
@@ -106,3 +108,81 @@ def test_graphs_hold_no_workspace_of_calls_without():
     for i, (c, r) in enumerate(zip(calls, out)):
         used = on(r, *ROWS, "i2s_pad_rows_k", "i2s_quant_rows_k", "i2s_gemm_mfma", "attn_combine", "reduce")
         assert used == (i >= needs) and (i == 0 or r["mallocs"] == 0), (c, kernels(r))
+
+
+def threads(body):
+    """A child with the recorder and the library loaded; body's `call(id, fn,
+    args)` makes a call in a thread of its own."""
+    head = """
+        import sys, threading, time
+        sys.path.insert(0, %r)
+        import recorded, test_routes as t
+        rec, lib = recorded.library()
+        def call(i, c):
+            def work():
+                rec.rec_thread_id(i)
+                assert getattr(lib, c["fn"])(*c["args"]) == 0
+            th = threading.Thread(target=work, daemon=True)
+            th.start()
+            return th
+        def until_waiting():
+            end = time.time() + 20
+            while not rec.rec_waiting():
+                assert time.time() < end
+                time.sleep(0.01)
+        A, B = 0x10000000, 0x10000000 + (1 << 40)
+    """ % os.path.dirname(os.path.abspath(__file__))
+    recorded.child(["-c", textwrap.dedent(head) + textwrap.dedent(body)])
+
+
+def test_a_full_queue_holds_up_no_other_stream():
+    """While one thread waits for room in its stream's queue, calls on other
+    streams go on, whether they use the workspace or not, and so do calls on
+    that stream's handle that take no workspace."""
+    threads("""
+        rec.rec_hold(A)
+        first = call(1, t.oil8(4096, 4096, 1, A))       # one launch, no workspace
+        until_waiting()
+        rest = [call(2, c) for c in (t.oil8(4096, 4096, 1, B), t.oil4(11008, 4096, 1, B), t.i2s_gemm(4096, 300, 4096, B),
+                                     t.attention(2, 32, 8, 128, 6000, B), t.oil8(4096, 4096, 40, B))]
+        for th in rest:
+            th.join(20)
+            assert not th.is_alive()
+        assert first.is_alive()
+        rec.rec_release()
+        first.join(20)
+        rec.rec_hold(A)
+        first = call(1, t.i2s_gemm(4096, 300, 4096, A))  # three launches through the workspace
+        until_waiting()
+        rest = [call(2, c) for c in (t.i2s_gemm(4096, 300, 4096, B), t.oil8(4096, 4096, 40, B))]
+        for th in rest:
+            th.join(20)
+            assert not th.is_alive()
+        rec.rec_release()
+        first.join(20)
+        assert not first.is_alive()
+    """)
+
+
+def test_threads_that_share_a_stream_enqueue_in_turn():
+    """Calls that hand data on through a stream's workspace: no other call's
+    launches come between theirs."""
+    threads("""
+        calls = [t.i2s_gemm(4096, 300, 4096, A), t.attention(2, 32, 8, 128, 6000, A), t.oil8(4096, 4096, 40, A),
+                 t.oil4(1616, 1920, 200, A), t.i2s_f32(4096, 11008, 16, A), t.oil4(4096, 4096, 8, A)]
+        for rep in range(20):
+            rec.rec_reset()
+            rec.rec_hold(A)
+            all_ = [call(1, calls[rep % len(calls)])]
+            until_waiting()
+            all_ += [call(2 + i, c) for i, c in enumerate(calls)]
+            time.sleep(0.05)
+            assert rec.rec_launches() == 1
+            rec.rec_release()
+            for th in all_:
+                th.join(20)
+                assert not th.is_alive()
+            ids = [rec.rec_thread(i) for i in range(rec.rec_launches())]
+            runs = [i for k, i in enumerate(ids) if k == 0 or ids[k - 1] != i]
+            assert len(runs) == len(set(runs)) == 1 + len(calls), ids
+    """)
