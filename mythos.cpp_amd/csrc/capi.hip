@@ -100,7 +100,12 @@ WsHold workspace(hipStream_t s, size_t need) {
         }
         const size_t bytes = std::max(need, 2 * w->bytes);
         void* p = nullptr;
-        if ((h.e = hipMalloc(&p, bytes)) != hipSuccess) return h;
+        // (relaxed: an allocation would invalidate the capture of another thread, in the default mode)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        h.e = hipMalloc(&p, bytes);
+        if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (h.e != hipSuccess) return h;
         if (w->base) {
             const std::lock_guard<std::mutex> g(g_ws_mu);
             g_ws_retired.push_back(w->base);

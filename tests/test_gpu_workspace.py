@@ -84,3 +84,51 @@ def test_growth_under_capture_is_refused_then_reserve(oracle, mth, dev):
             g2.replay()
         torch.cuda.synchronize()
         check(y, h, M, K, B, oracle, f"reserved graph replay {rep}")
+
+
+@pytest.mark.parametrize("mode", ["global", "thread_local", "relaxed"])
+def test_growth_beside_another_threads_capture(mode, mth, dev):
+    """A thread captures; another one's first calls on streams of its own need
+    a workspace.  Both go well: the capture stays valid, its replays give the
+    eager result, and the other thread's results are right."""
+    import threading
+    import torch
+    print(f"workspace growth beside a capture, {mode}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(4)
+    K, M, B, H, D, ctx = 2048, 512, 1, 8, 128, 2000
+    w = torch.randint(0, 256, (M, K), generator=g, device=dev, dtype=torch.uint8)
+    cb, x = torch.randn(256, generator=g, device=dev), torch.randn(K, generator=g, device=dev)
+    y, eager = torch.empty(M, device=dev), torch.empty(M, device=dev)
+    q = torch.randn(B, H, D, generator=g, device=dev)
+    kc, vc = (torch.randn(B, H, ctx, D, generator=g, device=dev) for _ in range(2))
+    out, want = torch.empty(B, H, D, device=dev), torch.empty(B, H, D, device=dev)
+    mth.oil8_gemv(w, cb, x, eager, M, K, 1)
+    mth.attention_decode(q, kc, vc, want, B, H, H, D, ctx, ctx)
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    errors = []
+
+    def other():
+        try:
+            mth.attention_decode(q, kc, vc, out, B, H, H, D, ctx, ctx, stream=s2)
+            mth.workspace_reserve(1 << 26, stream=s2)
+        except Exception as e:
+            errors.append(e)
+
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr, stream=s1, capture_error_mode=mode):
+        mth.oil8_gemv(w, cb, x, y, M, K, 1)
+        t = threading.Thread(target=other)
+        t.start()
+        t.join()
+        mth.oil8_gemv(w, cb, x, y, M, K, 1)
+    assert not errors, errors
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s1):
+            gr.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager)

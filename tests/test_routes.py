@@ -137,8 +137,7 @@ def threads(body):
 
 def test_a_full_queue_holds_up_no_other_stream():
     """While one thread waits for room in its stream's queue, calls on other
-    streams go on, whether they use the workspace or not, and so do calls on
-    that stream's handle that take no workspace."""
+    streams go on, whether they use the workspace or not."""
     threads("""
         rec.rec_hold(A)
         first = call(1, t.oil8(4096, 4096, 1, A))       # one launch, no workspace
@@ -185,4 +184,18 @@ def test_threads_that_share_a_stream_enqueue_in_turn():
             ids = [rec.rec_thread(i) for i in range(rec.rec_launches())]
             runs = [i for k, i in enumerate(ids) if k == 0 or ids[k - 1] != i]
             assert len(runs) == len(set(runs)) == 1 + len(calls), ids
+    """)
+
+
+def test_workspace_grows_in_relaxed_capture_mode():
+    """An allocation in the default mode invalidates a capture that another
+    thread has open; the mode is the thread's own again afterwards."""
+    threads("""
+        import ctypes as C
+        for c in (t.attention(2, 32, 8, 128, 6000, A), {"fn": "mth_workspace_reserve", "args": [1 << 28, B]}):
+            rec.rec_reset()
+            assert getattr(lib, c["fn"])(*c["args"]) == 0
+            assert rec.rec_mallocs() == 1 and rec.rec_malloc_mode() == 2   # hipStreamCaptureModeRelaxed
+            mode = C.c_int(0)
+            assert rec.hipThreadExchangeStreamCaptureMode(C.byref(mode)) == 0 and mode.value == 0
     """)
