@@ -19,7 +19,13 @@
 // 4.1e-7 .. 7.4e-7 of the norm off (64-bit sums), where the FP32 FMAs of the
 // kernels that walk the tokens are 1.1e-7 .. 2.7e-7 and this 1.4e-7 .. 2.1e-7
 // (OIL8 2 % slower, OIL4 the same time; the ternary sums were below the FP32
-// kernel's without it).  A token row that
+// kernel's without it).  The OIL8 kernel that walks the tokens in rows of up to
+// 4096 columns sums 16 products per lane and is 0.96e-7 .. 1.09e-7 off.  Where it
+// is the other route (fp32) FINE adds lo x lo, starts every product of 32
+// columns from zero and keeps the roundings of the additions: 0.89e-7 .. 0.97e-7
+// (without FINE 1.18e-7 .. 1.5e-7) on token tiles of at most 48, for 3 .. 30 % of
+// the time (40 tokens x 12000 x 4080 38 -> 46 us, walking them 349 us).
+// A token row that
 // holds Inf or NaN, or that spans more than 28 binades at a shape whose other
 // route is FP32 products (fp32: its largest values may meet weights of 0), takes
 // FP32 FMAs over the reference's products instead, as do all rows of a
@@ -53,6 +59,7 @@ namespace {
 constexpr int kRmStep = 128;              // columns per step
 constexpr int kRmRows = 128, kRmT = 256;  // weight rows and threads per workgroup
 constexpr int kRmSlices = 16;             // most K slices (rows_reduce_k)
+constexpr int kRmFineCols = 4096;         // OIL8 rows of up to so many columns: FINE where the other route is FP32
 
 // kOil4B: OIL4 weights, bf16 token rows (one FP16 part), bf16 outputs
 enum RowsFmt { kOil8, kOil4, kTern, kOil4B };
@@ -260,7 +267,7 @@ __device__ float rows_fma(const RowsArgs& p, int row, int tok, int k0, int k1) {
     return s;
 }
 
-template <int FMT, int G>
+template <int FMT, int G, bool FINE = false>
 __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) {
     constexpr int P = kParts<FMT>;
     constexpr bool O4 = FMT == kOil4 || FMT == kOil4B;
@@ -435,9 +442,18 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
         };
         // tile t's products with group g; h: the hi x hi sums (a step's alone, or from the slice's start)
         auto product = [&](int m, int t, int g, half8 Ah, half8 Al, half8 bh, half8 bl, floatx4& h) {
-            h = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh, STEP && m == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : h, 0, 0, 0);
+            if constexpr (FINE) {
+                const floatx4 r = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh, floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                h = m == 0 ? r : h + r;
+            } else {
+                h = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh, STEP && m == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : h, 0, 0, 0);
+            }
             if constexpr (P == 2) ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bl, ax[t][g], 0, 0, 0);
             if constexpr (FMT == kOil8) ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, bh, ax[t][g], 0, 0, 0);
+            if constexpr (FINE) {  // (2^22 lo x lo: one of them at 2^-11 of its scale, exact where it counts)
+                const half8 a = Al * (_Float16)0x1p-11f;
+                ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl, ax[t][g], 0, 0, 0);
+            }
         };
         if constexpr (FMT == kOil4) {  // the step's A operands first: a group's step sums are then 8 registers
             half8 Ah[4][2], Al;
@@ -477,7 +493,15 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
-                    for (int g = 0; g < G; ++g) ah[t][g] += st[t][g];
+                    for (int g = 0; g < G; ++g) {
+                        if constexpr (FINE) {  // the addition's rounding joins the small products
+                            const floatx4 s = ah[t][g] + st[t][g];
+                            ax[t][g] += (st[t][g] - (s - ah[t][g])) * 2048.0f;
+                            ah[t][g] = s;
+                        } else {
+                            ah[t][g] += st[t][g];
+                        }
+                    }
             }
         }
         __syncthreads();
@@ -544,9 +568,16 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
     }
 }
 
+// what t = a + b left out of a + b (exact; 0 where t is not finite, so that t stays the result)
+__device__ __forceinline__ float rows_rest(float a, float b, float t) {
+    const float z = t - a, r = (a - (t - z)) + (b - z);
+    return __builtin_isfinite(t) ? r : 0.0f;
+}
+
+// FINE: with the roundings of the additions added up beside.
 // out[i] = sum over slices z = 0, 1, ... of partial[z][i] (a fixed order); all loads before the first add.  Four
 // values per thread where both arrays are 16-byte aligned (n % 4 == 0).  HALF: out is bf16.  gridDim.y > 1: sg's matrix blockIdx.y.
-template <bool VEC, bool HALF = false>
+template <bool VEC, bool HALF = false, bool FINE = false>
 __global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ partial, float* __restrict__ out,
                                                       int64_t n, int S, RowsSegs sg, int batch) {
     const int64_t i = ((int64_t)blockIdx.x * kRmT + threadIdx.x) * (VEC ? 4 : 1);
@@ -561,10 +592,17 @@ __global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ 
         float4 v[kRmSlices];
 #pragma unroll
         for (int z = 0; z < kRmSlices; ++z) v[z] = z < S ? ldf4(partial + z * n + i) : make_float4(0, 0, 0, 0);
-        float4 s = v[0];
+        float4 s = v[0], e = make_float4(0, 0, 0, 0);
 #pragma unroll
         for (int z = 1; z < kRmSlices; ++z)
-            if (z < S) s = make_float4(s.x + v[z].x, s.y + v[z].y, s.z + v[z].z, s.w + v[z].w);
+            if (z < S) {
+                const float4 t = make_float4(s.x + v[z].x, s.y + v[z].y, s.z + v[z].z, s.w + v[z].w);
+                if constexpr (FINE)
+                    e = make_float4(e.x + rows_rest(s.x, v[z].x, t.x), e.y + rows_rest(s.y, v[z].y, t.y),
+                                    e.z + rows_rest(s.z, v[z].z, t.z), e.w + rows_rest(s.w, v[z].w, t.w));
+                s = t;
+            }
+        if constexpr (FINE) s = make_float4(s.x + e.x, s.y + e.y, s.z + e.z, s.w + e.w);
         if constexpr (HALF)
             *(uint2*)((uint16_t*)out + i) = make_uint2(f32_to_bf16_rne(s.x) | ((uint32_t)f32_to_bf16_rne(s.y) << 16),
                                                        f32_to_bf16_rne(s.z) | ((uint32_t)f32_to_bf16_rne(s.w) << 16));
@@ -574,10 +612,15 @@ __global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ 
         float v[kRmSlices];
 #pragma unroll
         for (int z = 0; z < kRmSlices; ++z) v[z] = z < S ? partial[z * n + i] : 0.0f;
-        float s = v[0];
+        float s = v[0], e = 0.0f;
 #pragma unroll
         for (int z = 1; z < kRmSlices; ++z)
-            if (z < S) s += v[z];
+            if (z < S) {
+                const float t = s + v[z];
+                if constexpr (FINE) e += rows_rest(s, v[z], t);
+                s = t;
+            }
+        if constexpr (FINE) s += e;
         if constexpr (HALF) ((uint16_t*)out)[i] = f32_to_bf16_rne(s);
         else out[i] = s;
     }
@@ -587,11 +630,12 @@ struct RowsPlan {
     int G, tiles, S, steps;
     int64_t rtiles;
 };
-// (M rows in nseg matrices: at most nseg - 1 row tiles more than M fills; alone: a call's only product)
-inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch, int nseg = 1, bool alone = false) {
+// (M rows in nseg matrices: at most nseg - 1 row tiles more than M fills; alone: a call's only product; fine: token
+// tiles of at most 48, whose sums the FINE kernels hold in registers)
+inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch, int nseg = 1, bool alone = false, bool fine = false) {
     RowsPlan p{};
     p.steps = (int)((K + kRmStep - 1) / kRmStep);
-    const int64_t nt = (batch + 63) / 64;
+    const int64_t most = fine ? 48 : 64, nt = (batch + most - 1) / most;
     p.G = (int)((batch + 16 * nt - 1) / (16 * nt));  // token tiles of 16, 32, 48 or 64, as even as they go
     p.tiles = (int)((batch + 16 * p.G - 1) / (16 * p.G));
     p.rtiles = (M + kRmRows - 1) / kRmRows + nseg - 1;
@@ -614,7 +658,7 @@ inline size_t rows_a16_bytes(const RowsPlan& p, int parts = 2) {
     return (size_t)p.tiles * p.G * parts * p.steps * 4096;
 }
 
-template <int FMT>
+template <int FMT, bool FINE = false>
 hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s, const RowsSegs& sg = RowsSegs{}) {
     int64_t n = (int64_t)a.M * a.batch;
     uint16_t* a16 = (uint16_t*)ws;
@@ -633,10 +677,12 @@ hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s, cons
         rows_split_k<FMT == kTern, false><<<(unsigned)a.batch, kRmT, 0, s>>>(a.x, a16, rsh, a.K, 4 * p.steps, a.fp32);
     const dim3 grid((unsigned)(sg.n > 1 ? sg.t1[sg.n - 1] : p.rtiles), (unsigned)p.tiles, (unsigned)p.S);
     switch (p.G) {
-        case 1: rows_mfma_k<FMT, 1><<<grid, kRmT, 0, s>>>(a, sg); break;
-        case 2: rows_mfma_k<FMT, 2><<<grid, kRmT, 0, s>>>(a, sg); break;
-        case 3: rows_mfma_k<FMT, 3><<<grid, kRmT, 0, s>>>(a, sg); break;
-        default: rows_mfma_k<FMT, 4><<<grid, kRmT, 0, s>>>(a, sg); break;
+        case 1: rows_mfma_k<FMT, 1, FINE><<<grid, kRmT, 0, s>>>(a, sg); break;
+        case 2: rows_mfma_k<FMT, 2, FINE><<<grid, kRmT, 0, s>>>(a, sg); break;
+        case 3: rows_mfma_k<FMT, 3, FINE><<<grid, kRmT, 0, s>>>(a, sg); break;
+        default:
+            if constexpr (FINE) return hipErrorInvalidValue;  // (rows_plan: fine)
+            else rows_mfma_k<FMT, 4><<<grid, kRmT, 0, s>>>(a, sg);
     }
     if (p.S > 1) {
         bool vec4 = n % 4 == 0 && ((uintptr_t)a.out & 15u) == 0;
@@ -651,10 +697,10 @@ hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s, cons
         const unsigned ny = sg.n > 1 ? sg.n : 1;
         constexpr bool HALF = FMT == kOil4B;
         if (vec4)
-            rows_reduce_k<true, HALF><<<dim3((unsigned)((n / 4 + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S,
+            rows_reduce_k<true, HALF, FINE><<<dim3((unsigned)((n / 4 + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S,
                                                                                                  sg, a.batch);
         else
-            rows_reduce_k<false, HALF><<<dim3((unsigned)((n + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S, sg,
+            rows_reduce_k<false, HALF, FINE><<<dim3((unsigned)((n + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S, sg,
                                                                                               a.batch);
     }
     return hipGetLastError();
@@ -668,8 +714,12 @@ inline bool rows_sizes(int64_t M, int64_t K, int64_t batch) {
 }  // namespace
 
 size_t rows_mfma_workspace_bytes(int64_t M, int64_t K, int64_t batch, int nseg) {
-    const RowsPlan p = rows_plan(M, K, batch, nseg);
-    return rows_a16_bytes(p) + al256r((size_t)batch * 4) + (p.S > 1 ? (size_t)(p.S * M * batch * 4) : 0);
+    size_t need = 0;
+    for (const bool fine : {false, true}) {
+        const RowsPlan p = rows_plan(M, K, batch, nseg, false, fine);
+        need = std::max(need, rows_a16_bytes(p) + al256r((size_t)batch * 4) + (p.S > 1 ? (size_t)(p.S * M * batch * 4) : 0));
+    }
+    return need;
 }
 
 size_t rows_bf16_workspace_bytes(int64_t M, int64_t K, int64_t batch) {
@@ -721,7 +771,7 @@ bool oil8_rows_better(const Oil8Seg* seg, int nseg, int64_t K, int64_t batch, bo
                                      : 5.0 + (12.2 + narrow / 110.0) * (K / 1024.0);
         return 1.05 * rows_busy_us(M, K, batch, 1.7) < g;
     }
-    const double us = rows_us(M, K, batch, 1.7);
+    const double us = rows_us(M, K, batch, bt || K > kRmFineCols ? 1.7 : 2.1);
     // 16 tokens per launch, or launch pair where K is split (K > 512), against two launches or three: 17 tokens of K =
     // 1024 .. 4096 20 .. 86 us against 15 .. 48, of K = 512 14.7 .. 16.0 against 12.3 .. 12.9
     if (bt) return batch > 16;
@@ -767,7 +817,8 @@ hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_
     RowsSegs sg{};
     int64_t M = 0, tiles = 0;
     for (int i = 0; i < nseg; ++i) M += seg[i].rows;
-    const RowsPlan p = rows_plan(M, K, batch, nseg, alone);
+    const bool fine = fp32 && K <= kRmFineCols;
+    const RowsPlan p = rows_plan(M, K, batch, nseg, alone, fine);
     sg.n = nseg;
     M = 0;
     for (int i = 0; i < 3; ++i) {
@@ -783,7 +834,7 @@ hipError_t launch_oil8_rows(const Oil8Seg* seg, int nseg, const float* x, int64_
     }
     RowsArgs a{seg[0].idx, seg[0].cb, nullptr, nullptr, x, seg[0].y, nullptr, (int)seg[0].rows, (int)K, (int)batch, 0, 0,
                fp32};
-    return rows_run<kOil8>(a, p, ws, s, sg);
+    return fine ? rows_run<kOil8, true>(a, p, ws, s, sg) : rows_run<kOil8>(a, p, ws, s, sg);
 }
 hipError_t launch_oil4_rows(const uint8_t* nib, const uint16_t* cbs, int64_t cb_block, const float* x, float* y,
                             int64_t M, int64_t K, int64_t batch, bool fp32, void* ws, hipStream_t s, bool alone) {

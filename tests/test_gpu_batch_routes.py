@@ -363,6 +363,23 @@ def test_token_rows_wide_range(kind, M, K, batch, blk, span, mth, dev):
     assert bool((err <= 1e-6).all()), err
 
 
+# one slice and several (two to eight), token tiles of 16 to 48, an odd row count
+@pytest.mark.parametrize("M,K,batch", [(4000, 528, 18), (3001, 944, 49), (12000, 2064, 200), (4000, 4080, 64),
+                                       (8000, 4080, 10)])
+def test_token_rows_oil8_short_error(M, K, batch, mth, dev):
+    """OIL8 rows of up to 4096 columns off the batched GEMV's shapes: no further from float64 than the kernel that takes
+    one token after another in FP32 (0.96e-7 .. 1.1e-7 of the norm)."""
+    import torch
+    print(f"token rows OIL8 error M={M} K={K} batch={batch}", flush=True)
+    g = np.random.default_rng(M + K)
+    w, cb = rows_inputs("oil8", M, K, 0, g)
+    x = g.normal(0, 1, (batch, K)).astype(np.float32)
+    got = rows_call("oil8", mth, w, cb, x, M, K, batch, 0, dev).double()
+    want = torch.from_numpy(x).to(dev).double() @ w64("oil8", w, cb, M, K, 0, dev).T.contiguous()
+    err = float((got - want).norm() / want.norm())
+    assert err <= 1.03e-7, err
+
+
 @pytest.mark.parametrize("K,blk", [(640, 128), (1152, 128), (1664, 0), (3968, 128), (9088, 128)])
 def test_one_token_error(K, blk, mth, dev):
     """One token's sums against float64: FP32 products in 64 lanes are 1.2e-7 (640 .. 1664 columns) .. 2.3e-7 (9088) of

@@ -86,14 +86,15 @@ def test_growth_under_capture_is_refused_then_reserve(oracle, mth, dev):
         check(y, h, M, K, B, oracle, f"reserved graph replay {rep}")
 
 
+@pytest.mark.parametrize("own", [True, False])             # a stream of its own, or the default stream
 @pytest.mark.parametrize("mode", ["global", "thread_local", "relaxed"])
-def test_growth_beside_another_threads_capture(mode, mth, dev):
+def test_growth_beside_another_threads_capture(mode, own, mth, dev):
     """A thread captures; another one's first calls on streams of its own need
     a workspace.  Both go well: the capture stays valid, its replays give the
     eager result, and the other thread's results are right."""
     import threading
     import torch
-    print(f"workspace growth beside a capture, {mode}", flush=True)
+    print(f"workspace growth beside a capture, {mode}, {own}", flush=True)
     g = torch.Generator(device=dev).manual_seed(4)
     K, M, B, H, D, ctx = 2048, 512, 1, 8, 128, 2000
     w = torch.randint(0, 256, (M, K), generator=g, device=dev, dtype=torch.uint8)
@@ -104,14 +105,15 @@ def test_growth_beside_another_threads_capture(mode, mth, dev):
     out, want = torch.empty(B, H, D, device=dev), torch.empty(B, H, D, device=dev)
     mth.oil8_gemv(w, cb, x, eager, M, K, 1)
     mth.attention_decode(q, kc, vc, want, B, H, H, D, ctx, ctx)
-    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream() if own else torch.cuda.default_stream()
     torch.cuda.synchronize()
     errors = []
 
     def other():
         try:
             mth.attention_decode(q, kc, vc, out, B, H, H, D, ctx, ctx, stream=s2)
-            mth.workspace_reserve(1 << 26, stream=s2)
+            if own:
+                mth.workspace_reserve(1 << 26, stream=s2)
         except Exception as e:
             errors.append(e)
 
