@@ -1637,16 +1637,24 @@ inline size_t rows_partial(int64_t M, int64_t K, int64_t batch) {
     const int S = rows_slices(M, K, batch);
     return S > 1 ? (size_t)(S * batch * M * 4) : 0;
 }
-// Whether the two or three launches of launch_i2s_rows (12 us eagerly without a K split, 15 us with one) beat the
-// one launch of the kernels that walk the tokens one after another (8 us eagerly for any little work).  Those take
-// per token (measured at M = 512 .. 8192, K = 512 .. 8256, 1 .. 16 tokens): the codes of any alignment about
-// K (3300 + M) / 2e6 us; whole 64-column pieces of int8 tokens (K + 1500)(1800 + M) / 1.2e7 us; quantising FP32
-// tokens 0.25 us + K / 3000 us and M K / 1e7 us.  At 12 tokens and more the walk was never faster.
+// Whether the two or three launches of launch_i2s_rows (12.1 us eagerly without a K split, 15.3 us with one) beat the
+// one launch of the kernels that walk the tokens one after another (8 .. 9 us eagerly for any little work).  Those take
+// about 2 us and per token (measured at M = 512 .. 8192, K = 64 .. 9152, 2 .. 16 tokens; int8 tokens: 1250 shapes):
+//   int8, codes of any alignment: (0.2 + 1.5e-3 K) us, by (M + 1500) / 4300 above 2800 rows;
+//   int8, whole 64-column pieces: 0.67 us up to 1024 columns (1.0 for up to 131072 codes), 1.1 up to 2048
+//     and, where few rows leave CUs idle, 4096, 0.23 + 0.41 per 1024 beyond; more rows than 4096 a second round of
+//     workgroups;
+//   quantising FP32 tokens: 0.25 us + K / 3000 us, and M K / 1e7 us.  At 12 FP32 tokens and more it was never faster.
 inline bool rows_pay(bool f32, bool whole, int64_t M, int64_t K, int64_t batch) {
-    if (batch >= 12) return true;
-    if (!whole) return batch * K * (3300 + M) >= 30000000;
+    if (batch >= (f32 ? 12 : kIbTok + 1)) return true;
+    if (f32 && !whole) return batch * K * (3300 + M) >= 30000000;
     if (f32) return batch * (K + 3000) >= 44000 || batch * M * K >= 120000000;
-    return batch * (K + 1500) * (1800 + M) >= 175000000;
+    double us;
+    if (!whole) us = (0.2 + 1.5e-3 * K) * std::max(1.0, (M + 1500) / 4300.0);
+    else if (K <= 2048) us = (K <= 1024 ? (M * K <= 131072 ? 1.0 : 0.67) : 1.1) * (M > 4096 ? 1.4 : 1.0);
+    else if (M <= 1024) us = K <= 4096 ? 1.1 : 1.78;
+    else us = (0.23 + 0.41 * (K / 1024.0)) * std::max(1.0, (M + 600) / 4700.0);
+    return 2.1 + batch * us >= (ib_slices(M, K) > 1 ? 15.3 : 12.1);
 }
 }  // namespace
 

@@ -91,6 +91,18 @@ def test_token_rows_take_no_more_launches():
         assert len(kernels(r)) <= n, (c, kernels(r))
 
 
+def test_few_int8_ternary_tokens_take_the_faster_route():
+    """A few int8 tokens at shapes where the walk over the tokens and the token
+    rows (two launches, three with a K split) were timed: the faster of the two."""
+    walk = [(1024, 832, 13), (4096, 320, 12), (512, 260, 12), (1024, 260, 14), (4096, 1984, 9), (8192, 1984, 6),
+            (4096, 2052, 2), (1024, 9152, 6), (4096, 3136, 7), (8192, 832, 8)]      # 9.4 .. 12.6 us; rows 12 .. 16.9
+    rows = [(512, 192, 14), (4096, 832, 16), (4096, 4096, 8), (8192, 9152, 3), (1024, 9152, 10), (4096, 388, 12),
+            (8192, 5188, 2), (1024, 260, 17), (64, 64, 17)]                         # 12 .. 15.7 us; the walk 12.5 .. 36
+    calls = [i2s(M, K, b, next(stream)) for M, K, b in walk + rows]
+    for i, (c, r) in enumerate(zip(calls, recorded.run(calls))):
+        assert (len(kernels(r)) > 1) == (i >= len(walk)), (c, kernels(r))
+
+
 def test_graphs_hold_no_workspace_of_calls_without():
     """Captured on a stream that holds a large workspace: calls whose other
     route keeps nothing there record no address of it, calls that need it do."""
