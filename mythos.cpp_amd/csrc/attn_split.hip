@@ -266,11 +266,11 @@ bool attention_split_supported(const float* q, const float* kc, const float* vc,
     // without shared K / V rows the split only adds its partial sums there (70.8 -> 75.7 us at 16 x 32 x 800 x 128; at
     // 128 workgroups 145 -> 138 us at 6000 positions), with them it pays from ctx * D = 80000 (17.5 -> 19.5 us at
     // 51200, 38.7 -> 31.9 at 102400).  Rows of 64 on the one-launch kernel's 16 waves (few workgroups, a cache of more
-    // than 1024 positions) take 10.1 us at 64000, 15 us at 128000.
+    // than 1024 positions): 10.9 .. 11.4 us there and 11.4 .. 12.1 split at 80640, 12.0 .. 12.9 and 11.0 .. 12.2 at 89600.
     const int64_t work = (int64_t)ctx * head_dim, wgs = batch * heads;
     const int hg = as_hg(heads, kv_heads);
     const bool waves16 = head_dim == 64 && max_seq > 1024 && wgs <= 128;
-    if (work < (wgs > 256 || waves16 ? 80000 : 42000) || (hg == 1 && wgs > 160)) return false;
+    if (work < (waves16 ? 88000 : wgs > 256 ? 80000 : 42000) || (hg == 1 && wgs > 160)) return false;
     return as_plan(batch, heads, kv_heads, head_dim, ctx).S > 1;
 }
 

@@ -103,6 +103,14 @@ def test_few_int8_ternary_tokens_take_the_faster_route():
         assert (len(kernels(r)) > 1) == (i >= len(walk)), (c, kernels(r))
 
 
+def test_attention_of_64_columns_splits_where_it_pays():
+    """Few heads of 64 columns over a cache of more than 1024 positions: one
+    launch to 1374 positions (at 1260: 10.9 .. 11.4 us against 11.4 .. 12.1),
+    two from 1375 (at 1400: 12.0 .. 12.9 against 11.0 .. 12.2)."""
+    calls = [attention(1, 32, 8, 64, ctx, next(stream)) for ctx in (1260, 1306, 1374, 1375, 1400, 6000)]
+    assert [len(kernels(r)) for r in recorded.run(calls)] == [1, 1, 1, 2, 2, 2]
+
+
 def test_graphs_hold_no_workspace_of_calls_without():
     """Captured on a stream that holds a large workspace: calls whose other
     route keeps nothing there record no address of it, calls that need it do."""
