@@ -133,9 +133,13 @@ int mth_oil4_gemv(const uint8_t* packed, const uint16_t* codebooks, int64_t cb_b
 /* mth_oil4_gemv for callers that cannot allocate device memory (code under
  * HIP graph capture, serving loops, harnesses that forbid hipMalloc).  No
  * counterpart in the reference (its CPU kernels need no scratch).  Same
- * arguments as mth_oil4_gemv and the same results up to FP32 rounding (bit
- * for bit up to 16 tokens where K % 512 == 0); batches above 16 tokens run
- * in groups of 16, odd sizes token by token.  The batched path's K-slice
+ * arguments as mth_oil4_gemv, and its results up to FP32 rounding.  Bit for
+ * bit (the same kernels) with 16-byte aligned inputs and M * K < 2^33 for one
+ * token of K <= 4096, and with codebooks per 128 columns or one per tensor for
+ * one token of K % 128 == 0, K <= 16384 and for 2 .. 16 tokens of K % 512 == 0,
+ * K <= 8192.  There more tokens run in groups of 16; other sizes run token by
+ * token, without the routes that mth_oil4_gemv may take in its workspace (they
+ * differ by FP32 rounding, and are faster).  The batched path's K-slice
  * partial sums (16 tokens x M rows x K/1024 slices of FP32 for K >= 2048)
  * live in a fixed 8 MiB device array per GPU instead of the workspace, and
  * the call never allocates.  Shapes whose partial sums exceed 8 MiB (e.g.

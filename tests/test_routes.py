@@ -111,6 +111,18 @@ def test_attention_of_64_columns_splits_where_it_pays():
     assert [len(kernels(r)) for r in recorded.run(calls)] == [1, 1, 1, 2, 2, 2]
 
 
+def test_noalloc_runs_the_same_kernels():
+    """mth_oil4_gemv_noalloc's results are mth_oil4_gemv's bit for bit at these
+    sizes because both launch the same kernels."""
+    sizes = [(b, K) for b, Ks in ((1, (32, 544, 4096, 4224, 11008, 16384)), (2, (512, 7680, 8192)), (16, (512, 4096)))
+             for K in Ks]
+    calls = [oil4(M, K, b, next(stream), blk) for b, K in sizes for M in (1, 700, 5000) for blk in (0, 128)
+             if blk == 0 or K % blk == 0]
+    calls += [oil4(700, K, 1, next(stream), 32) for K in (32, 1056, 4096)]
+    for c, a, b in zip(calls, recorded.run(calls), recorded.run([dict(c, fn="mth_oil4_gemv_noalloc") for c in calls])):
+        assert a["kernels"] == b["kernels"] and b["mallocs"] == 0 and kernels(b), c
+
+
 def test_graphs_hold_no_workspace_of_calls_without():
     """Captured on a stream that holds a large workspace: calls whose other
     route keeps nothing there record no address of it, calls that need it do."""
