@@ -177,6 +177,46 @@ def test_attention_on_per_thread_streams(mth, dev):
         assert bool(((out[i].double() - want).norm(dim=(-1, -2)) <= 4e-6 * want.norm(dim=(-1, -2))).all()), i
 
 
+@pytest.mark.parametrize("what", ["attention", "i2s_gemm"])
+def test_captured_calls_without_workspace(what, mth, dev):
+    """Captured on a stream that already holds a workspace, these run on the kernels that use none: every replay, with
+    eager calls of the workspace route on the same stream between them, gives the same bits."""
+    import torch
+    print(f"captured {what}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(4)
+    s = torch.cuda.Stream()
+    if what == "attention":
+        B, H, KVH, D, ctx = 2, 32, 8, 128, 1500
+        q = torch.randn(B, H, D, generator=g, device=dev)
+        kc, vc = (torch.randn(B, KVH, ctx, D, generator=g, device=dev) for _ in range(2))
+        eager, out = torch.empty(B, H, D, device=dev), torch.empty(B, H, D, device=dev)
+        call = lambda o: mth.attention_decode(q, kc, vc, o, B, H, KVH, D, ctx, ctx)
+    else:
+        M, N, K = 300, 40, 4096
+        w = torch.randint(0, 256, (M, K // 4), generator=g, device=dev, dtype=torch.uint8)
+        x = torch.randn(N, K, generator=g, device=dev)
+        eager, out = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
+        call = lambda o: mth.i2s_gemm(w, x, o, M, N, K)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        call(eager)
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr, stream=s):
+        call(out)
+    first = None
+    for rep in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            call(eager)
+            gr.replay()
+            call(eager)
+        torch.cuda.synchronize()
+        assert float((out - eager).norm() / eager.norm()) <= 2e-6, rep
+        first = out.clone() if first is None else first
+        assert torch.equal(out, first), rep
+
+
 # ----------------------------------------------------- token rows on MFMA --
 def w64(kind, w, cb, M, K, blk, dev):
     """[M][K] float64 weights."""
@@ -411,6 +451,157 @@ def test_prompt_gemm_oil8_error(M, K, batch, mth, dev):
     assert err <= 1.1 * (K / 16 * 2.5e-8 ** 2 + 8e-8 ** 2) ** 0.5, err
 
 
+# ------------------------------------------------ the row kernels by themselves --
+# Sizes at their edges that the entry points' estimates give to other kernels: the launches called directly, in a
+# workspace of exactly the size they ask for, with guards behind it and behind the output.
+SYMS = {
+    "ws": ("_ZN3mth25rows_mfma_workspace_bytesEllli", "llli"),
+    "ws_bf16": ("_ZN3mth25rows_bf16_workspace_bytesElll", "lll"),
+    "ws_i2s": ("_ZN3mth24i2s_rows_workspace_bytesElll", "lll"),
+    "oil8": ("_ZN3mth16launch_oil8_rowsEPKNS_7Oil8SegEiPKfllbPvP12ihipStream_tb", "pipllbppb"),
+    "oil4": ("_ZN3mth16launch_oil4_rowsEPKhPKtlPKfPflllbPvP12ihipStream_tb", "pplpplllbppb"),
+    "oil4_bf16": ("_ZN3mth21launch_oil4_rows_bf16EPKhPKtlS3_PtlllPvP12ihipStream_t", "pplpplllpp"),
+    "tern": ("_ZN3mth16launch_tern_rowsEPKhPKfPflllPvP12ihipStream_t", "ppplllpp"),
+    "i2s": ("_ZN3mth15launch_i2s_rowsEPKhfPKfPKaS3_PflllPvP12ihipStream_t", "pfpppplllpp"),
+}
+
+
+def direct(mth, name, *args):
+    import ctypes as C
+    sym, sig = SYMS[name]
+    f = getattr(mth.lib, sym)
+    f.argtypes = [{"p": C.c_void_p, "l": C.c_int64, "i": C.c_int, "b": C.c_bool, "f": C.c_float}[c] for c in sig]
+    f.restype = C.c_size_t if name.startswith("ws") else C.c_int
+    return f(*args)
+
+
+class Guarded:
+    """Workspace and outputs with untouched bytes behind them (`ok`), on the current stream."""
+    def __init__(self, dev, ws_bytes):
+        import torch
+        self.bufs = [(torch.full((ws_bytes + 1024,), 0xA5, dtype=torch.uint8, device=dev), ws_bytes)]
+        self.ws, self.stream = self.bufs[0][0].data_ptr(), torch.cuda.current_stream().cuda_stream
+
+    def out(self, n, dtype, dev):
+        import torch
+        size = n * torch.empty(0, dtype=dtype).element_size()
+        t = torch.full((size + 1024,), 0xA5, dtype=torch.uint8, device=dev)
+        self.bufs.append((t, size))
+        return t[:size].view(dtype)
+
+    def ok(self):
+        import torch
+        torch.cuda.synchronize()
+        return all(bool((t[n:] == 0xA5).all()) for t, n in self.bufs)
+
+
+def rows_close(got, want, absw):
+    assert bool(((got.double() - want).abs() <= 1e-5 * absw + 1e-30).all())
+    assert bool(((got.double() - want).norm(dim=1) <= 1e-6 * want.norm(dim=1) + 1e-30).all())
+
+
+@pytest.mark.parametrize("kind,M,K,batch,blk,shift", [
+    ("oil8", 1, 32, 1, 0, 0), ("oil8", 129, 2064, 17, 0, 0), ("oil8", 127, 144, 33, 0, 4),
+    ("oil8", 257, 4096, 48, 0, 0), ("oil8", 256, 4080, 49, 0, 0), ("oil8", 130, 4112, 64, 0, 0),
+    ("oil8", 33000, 272, 5, 0, 0),
+    ("oil4", 1, 32, 1, 32, 0), ("oil4", 129, 544, 17, 32, 4), ("oil4", 130, 2080, 65, 0, 0),
+    ("tern", 1, 32, 1, 0, 0), ("tern", 129, 1028, 40, 0, 0), ("tern", 33, 100, 17, 0, 4), ("tern", 200, 2052, 64, 0, 4),
+])
+def test_row_kernels_by_themselves(kind, M, K, batch, blk, shift, mth, dev):
+    """As test_token_rows, on the row kernel whatever the estimates say; with and without the FP32 guard (for OIL8 rows
+    of up to 4096 columns: its FINE kernels) and with a K split and without where the call chooses."""
+    import torch
+    g = np.random.default_rng(M + K + batch)
+    w, cb = rows_inputs(kind, M, K, blk, g)
+    x = (g.normal(0, 1, (batch, K)) * np.exp2(g.integers(-40, 40, batch))[:, None]).astype(np.float32)
+    if batch > 2:
+        x[batch // 2] = 0.0
+    W, X = w64(kind, w, cb, M, K, blk, dev), torch.from_numpy(x).to(dev).double()
+    want, absw = X @ W.T.contiguous(), X.abs() @ W.abs().T.contiguous()
+    wd, xd = offset(to_dev(w, dev), shift if kind == "tern" else 0), offset(to_dev(x, dev), shift)
+    cd = to_dev(cb, dev) if cb is not None else None
+    for fp32 in ((False, True) if kind != "tern" else (True,)):
+        for alone in ((False, True) if kind != "tern" else (False,)):
+            print(f"row kernel {kind} M={M} K={K} batch={batch} blk={blk} fp32={fp32} alone={alone}", flush=True)
+            b = Guarded(dev, direct(mth, "ws", M, K, batch, 1))
+            y = b.out(batch * M, torch.float32, dev)
+            if kind == "oil8":
+                seg = np.array([wd.data_ptr(), cd.data_ptr(), y.data_ptr(), M], dtype=np.int64)
+                rc = direct(mth, kind, seg.ctypes.data, 1, xd.data_ptr(), K, batch, fp32, b.ws, b.stream, alone)
+            elif kind == "oil4":
+                rc = direct(mth, kind, wd.data_ptr(), cd.data_ptr(), blk, xd.data_ptr(), y.data_ptr(), M, K, batch, fp32,
+                            b.ws, b.stream, alone)
+            else:
+                rc = direct(mth, kind, wd.data_ptr(), xd.data_ptr(), y.data_ptr(), M, K, batch, b.ws, b.stream)
+            assert rc == 0 and b.ok()
+            rows_close(y.reshape(batch, M) if kind != "tern" else y.reshape(M, batch).T, want, absw)
+
+
+# a K split and none, the FINE kernels and the others; an odd matrix (scalar stores and reduction) between even ones
+@pytest.mark.parametrize("K,batch,fp32", [(1040, 20, True), (1040, 20, False), (4112, 33, True), (288, 50, True)])
+def test_row_kernel_three_matrices(K, batch, fp32, mth, dev):
+    import torch
+    Ms = (5, 129, 256)
+    print(f"row kernel, three matrices, K={K} batch={batch} fp32={fp32}", flush=True)
+    g = np.random.default_rng(K)
+    x = g.normal(0, 1, (batch, K)).astype(np.float32)
+    x[0, :3] *= 2.0 ** 40
+    xd = to_dev(x, dev)
+    mats = [rows_inputs("oil8", M, K, 0, g) for M in Ms]
+    on = [(to_dev(w, dev), to_dev(cb, dev)) for w, cb in mats]
+    b = Guarded(dev, direct(mth, "ws", sum(Ms), K, batch, 3))
+    ys = [b.out(batch * M, torch.float32, dev) for M in Ms]
+    seg = np.array([[w.data_ptr(), cb.data_ptr(), y.data_ptr(), M] for (w, cb), y, M in zip(on, ys, Ms)], dtype=np.int64)
+    assert direct(mth, "oil8", seg.ctypes.data, 3, xd.data_ptr(), K, batch, fp32, b.ws, b.stream, False) == 0 and b.ok()
+    X = torch.from_numpy(x).to(dev).double()
+    for (w, cb), y, M in zip(mats, ys, Ms):
+        W = w64("oil8", w, cb, M, K, 0, dev)
+        rows_close(y.reshape(batch, M), X @ W.T.contiguous(), X.abs() @ W.abs().T.contiguous())
+
+
+# stores of whole pairs, of single values (odd rows) and of both (rows not a multiple of 4) in one slice, many
+# workgroups; K split with an odd and an even count of outputs
+@pytest.mark.parametrize("M,N,K,block", [(1, 1, 32, 32), (15, 127, 96, 32), (17, 129, 256, 128), (33, 130, 384, 128),
+                                         (200, 4225, 992, 32), (3, 127, 512, 64), (200, 9000, 160, 32), (5, 132, 1056, 32)])
+def test_row_kernel_bf16_by_itself(M, N, K, block, mth, dev):
+    """As test_prefill_rows, on the row kernel whatever the estimates say."""
+    import torch
+    from test_gpu_prefill import check
+    print(f"row kernel bf16 M={M} N={N} K={K} block={block}", flush=True)
+    a, packed, cbs = synth.prefill(M, N, K, block)
+    A = torch.from_numpy(synth.bf16_to_f32(a).reshape(M, K)) * torch.exp2(torch.arange(M) % 41 - 20.0)[:, None]
+    x, w, cb = A.bfloat16().to(dev), to_dev(packed, dev), to_dev(cbs, dev)
+    b = Guarded(dev, direct(mth, "ws_bf16", N, K, M))
+    c = b.out(M * N, torch.bfloat16, dev)
+    assert direct(mth, "oil4_bf16", w.data_ptr(), cb.data_ptr(), block, x.data_ptr(), c.data_ptr(), N, K, M, b.ws,
+                  b.stream) == 0 and b.ok()
+    W = synth.dequant_oil4(packed, cbs, N, K, block).astype(np.float64)
+    A = A.bfloat16().double().numpy()
+    check(c.view(torch.int16).cpu().numpy().view(np.uint16).reshape(M, N), A @ W.T, np.abs(A) @ np.abs(W).T, "rows")
+
+
+@pytest.mark.parametrize("M,K,batch,shift", [(1, 64, 2, 0), (64, 260, 5, 0), (128, 512, 3, 4), (129, 1028, 16, 4),
+                                             (33, 68, 17, 4)])
+def test_ternary_rows_by_themselves(M, K, batch, shift, oracle, mth, dev):
+    """As test_ternary_rows_bit_exact, on the padded rows whatever the estimates say."""
+    import torch
+    print(f"ternary rows by themselves M={M} K={K} batch={batch} shift={shift}", flush=True)
+    g = np.random.default_rng(M + K + batch)
+    packed = g.integers(0, 256, (M, K // 4), dtype=np.uint8)
+    x = (g.normal(0, 1, (batch, K)) * np.exp2(g.integers(-40, 40, batch))[:, None]).astype(np.float32)
+    q, inv = g.integers(-128, 128, (batch, K), dtype=np.int8), g.uniform(0.001, 2.0, batch).astype(np.float32)
+    p, xd, qd = (offset(to_dev(t, dev), shift) for t in (packed, x, q))
+    sc = to_dev(inv, dev)
+    for f32 in (True, False):
+        b = Guarded(dev, direct(mth, "ws_i2s", M, K, batch))
+        y = b.out(batch * M, torch.float32, dev)
+        assert direct(mth, "i2s", p.data_ptr(), WS, xd.data_ptr() if f32 else None, None if f32 else qd.data_ptr(),
+                      None if f32 else sc.data_ptr(), y.data_ptr(), M, K, batch, b.ws, b.stream) == 0 and b.ok()
+        want = (oracle.i2s_gemv_f32(packed.ravel(), WS, x, M, K, batch, threads=8) if f32 else
+                np.stack([oracle.i2s_gemv_rows(packed.ravel(), WS, q[t], inv[t], M, K, threads=8) for t in range(batch)]))
+        assert np.array_equal(y.cpu().numpy().reshape(batch, M), want), f32
+
+
 # ----------------------------------------------------------------- argmax --
 @pytest.mark.parametrize("rows,n", [(15, 2048), (16, 2049), (17, 5000), (33, 140001)])
 def test_argmax_rows(rows, n, oracle, mth, dev):
@@ -434,7 +625,8 @@ def test_argmax_rows(rows, n, oracle, mth, dev):
 @pytest.mark.parametrize("M,N,K,block", [(1, 1, 32, 32), (15, 127, 96, 32), (17, 129, 256, 64), (64, 128, 1120, 32),
                                          (65, 130, 4192, 32), (130, 60, 640, 128), (200, 9000, 160, 32)])
 def test_prefill_rows(M, N, K, block, mth, dev):
-    """mth_oil4_gemm_prefill on the row kernel, rows of very different magnitudes: the bars of test_gpu_prefill."""
+    """mth_oil4_gemm_prefill at sizes of the row kernel and around them, rows of very different magnitudes: the bars of
+    test_gpu_prefill."""
     import torch
     from test_gpu_prefill import check
     print(f"prefill rows M={M} N={N} K={K} block={block}", flush=True)
