@@ -2,7 +2,7 @@
 """bench.py — MI355X throughput of the quantized GEMV/GEMM hot path.
 
 One "step" is one launch of the hot-path kernel over one batch of synthetic
-input.  The headline workload is BASELINE config 2 (OIL4 GEMV, W 11008x4096,
+input.  The headline workload is config 2 (OIL4 GEMV, W 11008x4096,
 per-128-weight FP16 codebooks, batch 1); the other configs are reported in
 "extra", config 5 (the 32-layer decoder, greedy, batch 1 and 16) as tokens
 per second.  Method, per workload:
@@ -405,7 +405,7 @@ def main():
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py: this build measures one GPU only (--gpus {args.gpus} requested); "
-              "the path shards by weight rows with no exchange, see DESIGN.md", file=sys.stderr)
+              "the path shards by weight rows with no exchange", file=sys.stderr)
         sys.exit(2)
 
     import torch

@@ -115,8 +115,8 @@ int mth_oil8_gemv(const uint8_t* indices, const float* codebook, const float* x,
 int mth_oil4_gemm(const uint8_t* packed, const uint16_t* codebook, const float* act, float* out,
                   int64_t M, int64_t N, int64_t K, mth_stream_t stream);
 
-/* Decode GEMV with per-block FP16 codebooks (the layout the BASELINE configs
- * use; the reference kernel takes one codebook per call):
+/* Decode GEMV with per-block FP16 codebooks (one per 128
+ * columns in use; the reference kernel takes one codebook per call):
  *   y[t*M + m] = sum_k f32(codebooks[(m*(K/cb_block) + k/cb_block)*16 + nib(m,k)]) * x[t*K + k]
  * packed: M rows of K/2 bytes, nibble order as above.  cb_block = 0 selects
  * a single shared 16-entry codebook.  Requires K even and, for cb_block > 0,
@@ -229,7 +229,7 @@ int mth_tl2_gemm(const uint8_t* w, const float* act, float* out, int64_t M, int6
  * (w0, w1[, w2]) in {-1,0,1}^group, row-major, = clamp_int8(sum a_i*w_i). */
 int mth_tl_precompute_lut(const int8_t* act, int8_t* lut, int64_t K, int group, mth_stream_t stream);
 
-/* ---- FP32 decode-step operators (config-5 decoder) ----------------------- */
+/* ---- FP32 decode-step operators (the decoder's) ----------------------- */
 
 /* oil::math::rms_norm (include/oil/math.h:24, src/math.cpp:182-205) over rows
  * of dim: double sum of squares, y = (float)(x / sqrt(ss/dim + eps)) * gamma.

@@ -187,8 +187,6 @@ constexpr int PBM = 256, PBK = 64;
 // byte offset of 16-byte chunk c (0..7) of row r in a 128-byte-row tile
 __device__ __forceinline__ int pf_off(int r, int c) { return r * 128 + 16 * (c ^ ((r & 7) ^ ((r >> 3) & 1))); }
 
-// 8 bf16 -> 8 FP16 of a * 2^s (through FP32: v_cvt_pk_f16_f32 rounds to
-// nearest even; exact inside FP16's range)
 template <int BN>
 struct PfLds {
     static constexpr int a = PBM * 128;  // one A tile (double-buffered)
@@ -703,7 +701,8 @@ inline int pick_bn(int64_t M, int64_t N) {
 
 }  // namespace
 
-// oil4_prefill_ws serves K % 128 == 0, codebook blocks of a multiple of 128 and N % 16 == 0; the workspace is A in FP16 fragment order (ceil(M / 16) * 16 rows)
+// oil4_prefill_ws serves K % 128 == 0, codebook blocks of a multiple of 128 and N % 16 == 0; the workspace is A in FP16
+// fragment order (ceil(M / 16) * 16 rows)
 size_t oil4_prefill_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t cb_block) {
     const bool v2 = K % (2 * PBK) == 0 && cb_block % (2 * PBK) == 0 && pick_bn_v2(M, N, K) != 0 && M < (1ll << 31) &&
                     ((M + PBM - 1) / PBM) * (N / 64 + 1) < (1ll << 31) && M * K < (1ll << 40);

@@ -42,8 +42,9 @@
 // K slices, whose sums rows_reduce_k adds in order.
 //
 // Bound: per workgroup ~5 us before the first step and after the last (load latency, table, output) and then, on a
-// full chip, LDS for OIL8 (a step's 256 gathers of ~6 cycles and its B reads, 1.35 us per step for two workgroups a
-// CU at 48 tokens) and half of the MFMA rate for the others (0.83 us).  Measured against the routes before it (one
+// full chip, LDS for OIL8 (counters at 48 tokens: a workgroup's step keeps it busy for 2180 cycles, 256 gathers of 5.5
+// and 770 for B, 0.9 of the 1.36 us that a CU takes per step) and half of the MFMA rate for the others (64 tokens: 1024
+// matrix cycles per SIMD, 0.43 of 0.83 us).  Measured against the routes before it (one
 // call, eager): OIL8 4000 x 4096, 40 tokens 32.9 -> 19.3 us; 2000 x 8976, 256 tokens 9.9 ms -> 52 us; OIL4 5000 x
 // 9088 (codebooks per 64), 64 tokens 5.4 ms -> 36 us; ternary 4096 x 4096, 300 tokens 5.8 ms -> 36 us.  bf16 rows (one
 // part and product): 100 tokens x 1200 x 4096 103 -> 18 us, 160 x 5120 x 4096 50 -> 33 us.
@@ -68,8 +69,8 @@ constexpr int kParts = FMT == kOil4B ? 1 : 2;  // FP16 parts of a token row
 
 // ---- token rows -> FP16 hi / lo B fragments ------------------------------------
 // Row t: shift s with max|x| 2^s in [2^14, 2^15) into rsh[t] (kRowFp32 for a row holding Inf / NaN and, with guard, for
-// one whose nonzero values span more than 28 binades), then 2^s x = hi + 2^-11 lo, group t / 16, part (hi, lo), 32-column chunk c: 1 KB of [8-column piece m][token t % 16][8].
-// TERN: the pieces hold the columns in the order of the ternary codes' planes (element e of piece m: column
+// one whose nonzero values span more than 28 binades), then 2^s x = hi + 2^-11 lo, group t / 16, part (hi, lo),
+// 32-column chunk c: 1 KB of [8-column piece m][token t % 16][8].  TERN: the pieces hold the columns in the order of the ternary codes' planes (element e of piece m: column
 // 16 (m / 2) + 2 (m % 2) + e / 4 + 4 (e % 4) of the chunk).  Columns past K are zeros; rows past the batch are not
 // written (their products only reach their own, discarded, outputs).  One workgroup per row, the row read once
 // (16384 columns in registers; the rest of a longer row twice).
@@ -443,10 +444,12 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
         // tile t's products with group g; h: the hi x hi sums (a step's alone, or from the slice's start)
         auto product = [&](int m, int t, int g, half8 Ah, half8 Al, half8 bh, half8 bl, floatx4& h) {
             if constexpr (FINE) {
-                const floatx4 r = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh, floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                const floatx4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+                const floatx4 r = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh, zero, 0, 0, 0);
                 h = m == 0 ? r : h + r;
             } else {
-                h = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh, STEP && m == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : h, 0, 0, 0);
+                if (STEP && m == 0) h = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                h = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bh, h, 0, 0, 0);
             }
             if constexpr (P == 2) ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, bl, ax[t][g], 0, 0, 0);
             if constexpr (FMT == kOil8) ax[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, bh, ax[t][g], 0, 0, 0);
@@ -576,7 +579,8 @@ __device__ __forceinline__ float rows_rest(float a, float b, float t) {
 
 // FINE: with the roundings of the additions added up beside.
 // out[i] = sum over slices z = 0, 1, ... of partial[z][i] (a fixed order); all loads before the first add.  Four
-// values per thread where both arrays are 16-byte aligned (n % 4 == 0).  HALF: out is bf16.  gridDim.y > 1: sg's matrix blockIdx.y.
+// values per thread where both arrays are 16-byte aligned (n % 4 == 0).  HALF: out is bf16.  gridDim.y > 1: sg's matrix
+// blockIdx.y.
 template <bool VEC, bool HALF = false, bool FINE = false>
 __global__ __launch_bounds__(kRmT) void rows_reduce_k(const float* __restrict__ partial, float* __restrict__ out,
                                                       int64_t n, int S, RowsSegs sg, int batch) {
@@ -648,8 +652,9 @@ inline RowsPlan rows_plan(int64_t M, int64_t K, int64_t batch, int nseg = 1, boo
                       : wgs >= 64 && p.steps >= 48 ? 512 / wgs : 256 / wgs;
     p.S = (int)std::max<int64_t>(1, std::min<int64_t>({per, p.steps / 2, kRmSlices}));
     // alone, up to 512 columns and 48 tokens per tile: one slice, since the reduction's launch (3 us of host time) costs
-    // more than two steps more in a chain (M = 256 .. 16384, 17 .. 32 tokens 15.1 .. 15.8 us with two slices, 12.3 .. 13.1
-    // with one, 64 tokens 15.1 and 15.9); within a prompt's queue the split is the faster (60 tokens of hidden 512: 5 %).
+    // more than two steps more in a chain (M = 256 .. 16384, 17 .. 32 tokens 15.1 .. 15.8 us with two slices, 12.3 ..
+    // 13.1 with one, 64 tokens 15.1 and 15.9); within a prompt's queue the split is the faster (60 tokens of hidden 512:
+    // 5 %).
     if (alone && p.steps <= 4 && p.G <= 3) p.S = 1;
     return p;
 }
@@ -697,11 +702,11 @@ hipError_t rows_run(RowsArgs a, const RowsPlan& p, void* ws, hipStream_t s, cons
         const unsigned ny = sg.n > 1 ? sg.n : 1;
         constexpr bool HALF = FMT == kOil4B;
         if (vec4)
-            rows_reduce_k<true, HALF, FINE><<<dim3((unsigned)((n / 4 + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S,
-                                                                                                 sg, a.batch);
+            rows_reduce_k<true, HALF, FINE><<<dim3((unsigned)((n / 4 + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(
+                partial, a.out, n, p.S, sg, a.batch);
         else
-            rows_reduce_k<false, HALF, FINE><<<dim3((unsigned)((n + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(partial, a.out, n, p.S, sg,
-                                                                                              a.batch);
+            rows_reduce_k<false, HALF, FINE><<<dim3((unsigned)((n + kRmT - 1) / kRmT), ny), kRmT, 0, s>>>(
+                partial, a.out, n, p.S, sg, a.batch);
     }
     return hipGetLastError();
 }

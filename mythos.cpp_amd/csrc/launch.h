@@ -191,10 +191,10 @@ double oil4_gemm_x32_us(int64_t Mr, int64_t N, int64_t K);  // launch_oil4_gemm_
 // the tiled prompt kernels' estimated time (microseconds), for oil4_rows_bf16_better
 double oil4_prefill_us(int64_t M, int64_t N, int64_t K, int64_t cb_block);
 bool oil4_gemm_prefill_supported(int64_t M, int64_t N, int64_t K, int64_t cb_block);
-// The FP16-A kernels (oil4_prefill_a16 + oil4_prefill_ws) for K % 256 == 0, cb_block % 64 == 0
-// and N a multiple of 64, 96, 112 or 128: needs a workspace of
-// oil4_prefill_shift_bytes(M) + oil4_prefill_workspace_bytes (the row shifts,
-// then A converted to FP16; 0 = shape not covered).
+// The FP16-A kernels (oil4_prefill_a16 + oil4_prefill_ws) for K % 128 == 0, cb_block % 128 == 0
+// and N % 16 == 0 (whole tiles: K % 256 == 0 and N a multiple of 64, 96, 112 or 128): needs a
+// workspace of oil4_prefill_shift_bytes(M) + oil4_prefill_workspace_bytes (the row shifts, then A
+// converted to FP16; 0 = shape not covered).
 size_t oil4_prefill_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t cb_block);
 hipError_t launch_oil4_gemm_prefill_a16(const uint16_t* a_bf16, const uint8_t* nib, const uint16_t* cbs,
                                        int64_t cb_block, uint16_t* c_bf16, int64_t M, int64_t N, int64_t K,

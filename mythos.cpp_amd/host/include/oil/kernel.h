@@ -54,8 +54,8 @@ void tiled_gemm(const float* A, const float* B, float* C, int M, int N, int K);
 void avx2_gemm(const float* A, const float* B, float* C, int M, int N, int K);
 void avx2_tiled_gemm(const float* A, const float* B, float* C, int M, int N, int K);
 
-// ---- extensions (no reference counterpart): the decode formats of the
-// BASELINE configs, host-pointer + synchronous like the functions above ----
+// ---- extensions (no reference counterpart): the decoder's
+// formats, host-pointer + synchronous like the functions above ----
 
 // y[t*M + m] = sum_k codebooks[(m*(K/cb_block) + k/cb_block)*16 + nib] * x[t*K + k]
 void oil4_gemv_blocked(const uint8_t* packed, const uint16_t* codebooks, int cb_block, const float* x,

@@ -1,4 +1,4 @@
-"""Seeded synthetic inputs for the BASELINE configurations (host side).
+"""Seeded synthetic inputs for the measured configurations (host side).
 
 One stream per configuration: MYTHOS.cpp's RNG (xoroshiro128+ seeded by
 splitmix64, src/random.cpp:7-51) with seed 0x5EED0000 + config, drawn in

@@ -474,7 +474,7 @@ def test_config5_b1_exact_path(config5, oracle):
 
 
 def test_config5_b16_exact_path(config5, oracle):
-    """The BASELINE config-5 stack (32 layers, hidden 4096, ffn 11008, vocab
+    """The config-5 stack (32 layers, hidden 4096, ffn 11008, vocab
     32000) at batch 16 with every ternary down weight 0: the FFN output is
     exactly 0 on both sides, so no int8 rounding boundary is involved; the
     attention half of every block (norms, OIL8 Q/K/V/O on the batched MFMA

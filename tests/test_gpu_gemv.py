@@ -1,7 +1,7 @@
 """GPU parity: decode GEMV kernels (OIL8, OIL4, I2_S) through the C ABI
 against the CPU oracle on the same seeded inputs.
 
-Bars (BASELINE north star): OIL8 FP32 within 1e-5 relative (norm-wise and
+Bars: OIL8 FP32 within 1e-5 relative (norm-wise and
 per element against sum|w*x|); OIL4 within 2e-3 (asserted here at 1e-5,
 since the kernel accumulates in FP32 with exact FP16 codebook values);
 ternary / int8 paths bit-exact.

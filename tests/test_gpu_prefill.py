@@ -2,7 +2,7 @@
 oracle (small shapes, every element) and against a float64 contraction of the
 dequantised weights (config 4 shape, sampled rows and all columns).
 
-Tolerance (BASELINE north star): 2e-3 relative for the OIL4/bf16 path.  The
+Tolerance: 2e-3 relative for the OIL4/bf16 path.  The
 production kernel (K a multiple of 256, the codebook block a multiple of 128,
 N a multiple of 128, 112, 96 or 64) uses the FP16 codebook entries exactly and
 converts A bf16 -> FP16 (exact in range), sums in FP32; the output is rounded
