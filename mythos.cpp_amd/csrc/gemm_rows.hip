@@ -25,13 +25,14 @@
 // columns from zero and keeps the roundings of the additions: 0.89e-7 .. 0.97e-7
 // (without FINE 1.18e-7 .. 1.5e-7) on token tiles of at most 48, for 3 .. 30 % of
 // the time (40 tokens x 12000 x 4080 38 -> 46 us, walking them 349 us).
-// A token row that
-// holds Inf or NaN, or that spans more than 28 binades at a shape whose other
-// route is FP32 products (fp32: its largest values may meet weights of 0), takes
-// FP32 FMAs over the reference's products instead, as do all rows of a
-// non-finite OIL8 codebook and (fp32) an OIL4 output that comes out NaN, where
-// an infinite entry may have met a value that both parts miss.  bf16 rows are one FP16 part, as
-// in the tiled prompt kernels.
+// A token row that holds Inf or NaN takes FP32 FMAs over the reference's
+// products instead, as do all rows of a non-finite OIL8 codebook.  Where the
+// other route is FP32 products (fp32), so do single outputs: of a token row (or
+// an OIL8 codebook) that spans more than 28 binades those so small that only
+// values with fewer bits can have made them (its largest met weights of 0), and
+// an OIL4 output that comes out NaN, where an infinite entry may have met a
+// value that both parts miss.  bf16 rows are one FP16 part, as in the tiled
+// prompt kernels.
 //
 // Tiling.  A workgroup of 4 waves takes 128 weight rows (32 per wave: two A
 // tiles share every B read, which otherwise bounds the kernel: a tile-step
@@ -68,14 +69,14 @@ template <int FMT>
 constexpr int kParts = FMT == kOil4B ? 1 : 2;  // FP16 parts of a token row
 
 // ---- token rows -> FP16 hi / lo B fragments ------------------------------------
-// Row t: shift s with max|x| 2^s in [2^14, 2^15) into rsh[t] (kRowFp32 for a row holding Inf / NaN and, with guard, for
-// one whose nonzero values span more than 28 binades), then 2^s x = hi + 2^-11 lo, group t / 16, part (hi, lo),
-// 32-column chunk c: 1 KB of [8-column piece m][token t % 16][8].  TERN: the pieces hold the columns in the order of the ternary codes' planes (element e of piece m: column
-// 16 (m / 2) + 2 (m % 2) + e / 4 + 4 (e % 4) of the chunk).  Columns past K are zeros; rows past the batch are not
-// written (their products only reach their own, discarded, outputs).  One workgroup per row, the row read once
-// (16384 columns in registers; the rest of a longer row twice).
+// Row t: shift s with max|x| 2^s in [2^14, 2^15) into rsh[t] (kRowFp32 for a row holding Inf / NaN; s + kRowWide, with
+// guard, for one whose nonzero values span more than 28 binades), then 2^s x = hi + 2^-11 lo, group t / 16, part (hi,
+// lo), 32-column chunk c: 1 KB of [8-column piece m][token t % 16][8].  TERN: the pieces hold the columns in the order
+// of the ternary codes' planes (element e of piece m: column 16 (m / 2) + 2 (m % 2) + e / 4 + 4 (e % 4) of the chunk).
+// Columns past K are zeros; rows past the batch are not written (their products only reach their own, discarded,
+// outputs).  One workgroup per row, the row read once (16384 columns in registers; the rest of a longer row twice).
 constexpr int kRsN = 4;
-constexpr int kRowFp32 = kRowNonFinite;
+constexpr int kRowFp32 = kRowNonFinite, kRowWide = 1 << 16;
 template <bool TERN, bool VEC>
 __global__ __launch_bounds__(kRmT) void rows_split_k(const float* __restrict__ x, uint16_t* __restrict__ a16,
                                                      int* __restrict__ rsh, int K, int chunks, bool guard) {
@@ -121,7 +122,8 @@ __global__ __launch_bounds__(kRmT) void rows_split_k(const float* __restrict__ x
     mb = max(max(red[0], red[1]), max(red[2], red[3]));
     mn = 0u - max(max(redn[0], redn[1]), max(redn[2], redn[3]));
     const int sh = fp16_scale_shift(__uint_as_float(mb));
-    if (tid == 0) rsh[row] = mb >= 0x7f800000u || (guard && (int)(mb >> 23) - (int)(mn >> 23) > 28) ? kRowFp32 : sh;
+    if (tid == 0)
+        rsh[row] = mb >= 0x7f800000u ? kRowFp32 : guard && (int)(mb >> 23) - (int)(mn >> 23) > 28 ? sh + kRowWide : sh;
     uint16_t* hi = a16 + (int64_t)(row >> 4) * 2 * chunks * 512 + 8 * (row & 15);
     uint16_t* lo = hi + (int64_t)chunks * 512;
     auto store = [&](int g, const float (&f)[16]) {
@@ -193,7 +195,7 @@ struct RowsArgs {
     float* out;            // [batch][M] (ternary: [M][batch]; kOil4B: bf16)
     float* partial;        // [slice] of the same
     int M, K, batch, steps, cb_block;
-    bool fp32;             // FP32 products for rows of a wide range, and for an OIL4 output that comes out NaN
+    bool fp32;             // FP32 products for the outputs that a wide range may have left inexact and OIL4's NaN
 };
 // OIL8: up to three matrices over the same token rows (a decoder's Q, K and V), their row tiles one after another in
 // the grid; t1: the first row tile past matrix i.  Matrix i's partial sums start at partial + p0[i].
@@ -241,26 +243,26 @@ __device__ __forceinline__ half8 rows_tern8(uint32_t d, int f) {
     return __builtin_bit_cast(half8, r);
 }
 
-// FP32 products over columns [k0, k1) of one output, the reference's arithmetic in column order.
+// FP32 products over every inc-th column of [k0, k1) of one output, the reference's arithmetic in column order.
 template <int FMT>
-__device__ float rows_fma(const RowsArgs& p, int row, int tok, int k0, int k1) {
+__device__ float rows_fma(const RowsArgs& p, int row, int tok, int k0, int k1, int inc = 1) {
     const float* x = p.x + (int64_t)tok * p.K;
     float s = 0.0f;
     if constexpr (FMT == kOil8) {
         const uint8_t* w = p.w + (int64_t)row * p.K;
         const float* cb = (const float*)p.cb;
-        for (int k = k0; k < k1; ++k) s = fmaf(cb[w[k]], x[k], s);
+        for (int k = k0; k < k1; k += inc) s = fmaf(cb[w[k]], x[k], s);
     } else if constexpr (FMT == kOil4 || FMT == kOil4B) {
         const uint8_t* w = p.w + (int64_t)row * (p.K >> 1);
         const uint16_t* cb = (const uint16_t*)p.cb;
-        for (int k = k0; k < k1; ++k) {
+        for (int k = k0; k < k1; k += inc) {
             const int e = (w[k >> 1] >> (4 * (k & 1))) & 15;
             const int64_t b = p.cb_block ? (int64_t)row * (p.K / p.cb_block) + k / p.cb_block : 0;
             s = fmaf(h2f(cb[b * 16 + e]), x[k], s);
         }
     } else {
         const uint8_t* w = p.w + (int64_t)row * (p.K >> 2);
-        for (int k = k0; k < k1; ++k) {
+        for (int k = k0; k < k1; k += inc) {
             const int c = (w[k >> 2] >> (2 * (k & 3))) & 3;
             s += c == 1 ? 0.0f : (c == 0 ? -x[k] : x[k]);
         }
@@ -277,6 +279,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
     __shared__ __align__(16) uint8_t bs[P * G * 4096];
     __shared__ uint32_t tab[FMT == kOil8 ? 256 : 1];
     __shared__ float wred[kRmT / 64];
+    __shared__ uint32_t wleast[kRmT / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int j = lane & 15, q = lane >> 4;
     int bx = blockIdx.x;
@@ -348,7 +351,8 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
     if constexpr (FMT == kOil8) {
         fin = __builtin_isfinite(cbv);
         const float m = wave_max(fabsf(cbv));
-        if (lane == 0) wred[wave] = m;
+        const uint32_t least = group_reduce<64>(0u - (__float_as_uint(cbv) & 0x7fffffffu), UMaxOp{});  // (rows_split_k)
+        if (lane == 0) wred[wave] = m, wleast[wave] = least;
     }
     const int64_t zs = (int64_t)p.batch * M;
     float* out = S == 1 ? p.out : p.partial + blockIdx.z * zs;
@@ -514,6 +518,27 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
         if (step + 1 < s1) step_body(step + 1, wt[1]);
     }
 
+    uint32_t wide = 0;  // this lane's tokens of a wide range
+    if constexpr (FMT != kOil4B) {
+        if (p.fp32) {
+            bool wide_cb = false;
+            if constexpr (FMT == kOil8) {
+                const uint32_t least = 0u - max(max(wleast[0], wleast[1]), max(wleast[2], wleast[3]));
+                wide_cb = least != 0 && 141 - sw - (int)(least >> 23) > 28;  // (141 - sw: the largest entry's exponent)
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const bool w = rs[g] > kRowWide / 2 && rs[g] != kRowFp32;  // (a shift is -128 .. 165)
+                if (w) rs[g] -= kRowWide;
+                if (w || wide_cb) wide |= 1u << g;
+            }
+        }
+    }
+    // the scaled sum of row 16 t + 4 q + i and token 16 g + j
+    auto scaled = [&](int t, int g, int i) {
+        const float hi = ah[t][g][i], lo = ax[t][g][i] * 0x1p-11f;
+        return P == 1 ? hi : FMT == kOil8 ? hi + lo : oil4_hi_lo(hi, lo);
+    };
     // ---- D: lane (j, q) holds rows 4q + i of token j
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -525,17 +550,7 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
             const int row = row0 + 16 * t + 4 * q;
             float v[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float hi = ah[t][g][i], lo = ax[t][g][i] * 0x1p-11f;
-                v[i] = ldexpf(P == 1 ? hi : FMT == kOil8 ? hi + lo : oil4_hi_lo(hi, lo), -sh);
-            }
-            if constexpr (FMT == kOil4) {
-                // NaN: also an infinite entry times a value whose parts are 0, where the reference's product is infinite
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (p.fp32 && v[i] != v[i] && row + i < M)
-                        v[i] = rows_fma<FMT>(p, row + i, tok, kRmStep * s0, min(K, kRmStep * s1));
-            }
+            for (int i = 0; i < 4; ++i) v[i] = ldexpf(scaled(t, g, i), -sh);
             if constexpr (FMT == kOil4B) {
                 if (S == 1) {
                     uint16_t* d16 = (uint16_t*)p.out + (int64_t)tok * M + row;
@@ -568,6 +583,66 @@ __global__ __launch_bounds__(kRmT, 2) void rows_mfma_k(RowsArgs p, RowsSegs sg) 
             for (uint64_t m = __builtin_amdgcn_ballot_w64(q == 0 && tok0 + 16 * g + j < p.batch && rs[g] == kRowFp32); m;
                  m &= m - 1)
                 fp32_token(tok0 + 16 * g + __builtin_ctzll(m));
+        bool nan = false;  // OIL4: also an infinite entry times a value whose parts are 0, where the product is infinite
+        if constexpr (FMT == kOil4) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                float z = 0.0f;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) z = fmaf(0.0f, ax[t][g][i], fmaf(0.0f, ah[t][g][i], z));
+                nan = nan || (p.fp32 && z != 0.0f && tok0 + 16 * g + j < p.batch);  // (past it: whatever was there)
+            }
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(wide != 0 || nan) == 0, 1)) return;
+        // A value below 2^-28 of its row's maximum (scaled: 2^-14) is held to 2^-36 only.  FP32 products are as far off
+        // as n of those are together from outputs of sqrt(n) 2^-13 of the largest weight: an output below that is done
+        // again, by the wave.  (All outputs of such a token in FP32, in every workgroup: 40 tokens x 4000 x 4080, 1, 10 and
+        // 40 of them of a wide range, 86, 660 and 2530 us; this 23 us for any of them, and walking all tokens 125.)
+        const int k0 = kRmStep * s0, k1 = min(K, kRmStep * s1);
+        const float n = sqrtf((float)(k1 - k0)) * 0x1p-13f;
+        float top = FMT == kOil8 ? 0x1p15f : 1.0f;  // OIL4: the largest entry of row lane % 32's blocks in the slice
+        if constexpr (O4) {
+            const int blk = p.cb_block ? p.cb_block : K, b1 = (k1 - 1) / blk;
+            const uint16_t* cb = (const uint16_t*)p.cb;
+            if (p.cb_block) cb += (int64_t)min(row0 + (lane & 31), M - 1) * (K / blk) * 16;
+            top = 0.0f;
+#pragma unroll 4
+            for (int b = k0 / blk + (lane >> 5); b <= b1; b += 2) {
+                const uint4 c[2] = {ld16(cb + 16 * b), ld16(cb + 16 * b + 8)};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const uint32_t d = u4get(c[e >> 2], e & 3);
+                    top = fmaxf(top, fmaxf(fabsf(h2f(d & 0xffffu)), fabsf(h2f(d >> 16))));
+                }
+            }
+            top = fmaxf(top, __shfl_xor(top, 32, 64));
+        }
+        uint32_t again = 0;  // this lane's outputs (8 g + 4 t + i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float least = n * (O4 ? __shfl(top, 16 * t + 4 * q + i, 64) : top);
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const float d = scaled(t, g, i);
+                    const bool redo = (((wide >> g) & 1u) != 0 && !(fabsf(d) >= least)) || (FMT == kOil4 && d != d);
+                    if (redo && row0 + 16 * t + 4 * q + i < M && tok0 + 16 * g + j < p.batch && rs[g] != kRowFp32)
+                        again |= 1u << (8 * g + 4 * t + i);
+                }
+            }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores above: the same addresses follow
+        for (uint64_t m = __builtin_amdgcn_ballot_w64(again != 0); m; m &= m - 1) {
+            const int l = __builtin_ctzll(m);
+            for (uint32_t e = __builtin_amdgcn_readlane(again, l); e; e &= e - 1) {
+                const int b = __builtin_ctz(e), tok = tok0 + 16 * (b >> 3) + (l & 15);
+                const int row = row0 + 16 * ((b >> 2) & 1) + 4 * (l >> 4) + (b & 3);
+                const float v = group_sum<64>(rows_fma<FMT>(p, row, tok, k0 + lane, k1, 64));
+                if (lane == 0) out[at(row, tok)] = v;
+            }
+        }
     }
 }
 

@@ -403,6 +403,41 @@ def test_token_rows_wide_range(kind, M, K, batch, blk, span, mth, dev):
     assert bool((err <= 1e-6).all()), err
 
 
+@pytest.mark.parametrize("kind,M,K,batch,blk", [("oil8", 4000, 4080, 64, 0), ("oil8", 200, 6448, 70, 0),
+                                                ("oil4", 12000, 4224, 200, 64), ("oil4", 500, 9088, 20, 64),
+                                                ("tern", 4096, 4096, 100, 0)])
+def test_token_rows_wide_range_elsewhere(kind, M, K, batch, blk, mth, dev):
+    """Every token spans 40 binades, its small values beside large ones in every output: as close to float64 as without
+    them (2^-22, test_token_rows_error), none of it summed in one chain."""
+    import torch
+    print(f"token rows wide range elsewhere {kind} M={M} K={K} batch={batch}", flush=True)
+    g = np.random.default_rng(M + K)
+    w, cb = rows_inputs(kind, M, K, blk, g)
+    x = g.normal(0, 1, (batch, K)).astype(np.float32)
+    x[:, ::7] *= np.float32(2.0 ** -40)
+    got = rows_call(kind, mth, w, cb, x, M, K, batch, blk, dev).double()
+    want = torch.from_numpy(x).to(dev).double() @ w64(kind, w, cb, M, K, blk, dev).T.contiguous()
+    err = float((got - want).norm() / want.norm())
+    assert err <= 2.0 ** -22, err
+
+
+@pytest.mark.parametrize("M,K,batch", [(300, 1040, 12), (129, 6448, 70), (4000, 272, 40)])
+def test_token_rows_wide_codebook(M, K, batch, mth, dev):
+    """OIL8 codebook entries 2^-36 of the others: rows that hold those alone keep the precision of FP32 products."""
+    import torch
+    print(f"token rows wide codebook M={M} K={K} batch={batch}", flush=True)
+    g = np.random.default_rng(K)
+    w, cb = rows_inputs("oil8", M, K, 0, g)
+    cb[:16] = (g.normal(0, 1, 16) * 2.0 ** -42).astype(np.float32)
+    w[: M // 2] %= 16
+    w[M // 2:] = np.maximum(w[M // 2:], 16)
+    x = g.normal(0, 1, (batch, K)).astype(np.float32)
+    got = rows_call("oil8", mth, w, cb, x, M, K, batch, 0, dev).double()
+    want = torch.from_numpy(x).to(dev).double() @ w64("oil8", w, cb, M, K, 0, dev).T.contiguous()
+    for rows in (slice(0, M // 2), slice(M // 2, M)):
+        assert float((got[:, rows] - want[:, rows]).norm() / want[:, rows].norm()) <= 2.0 ** -22, rows
+
+
 # one slice and several (two to eight), token tiles of 16 to 48, an odd row count
 @pytest.mark.parametrize("M,K,batch", [(4000, 528, 18), (3001, 944, 49), (12000, 2064, 200), (4000, 4080, 64),
                                        (8000, 4080, 10)])
