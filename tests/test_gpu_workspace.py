@@ -92,6 +92,7 @@ def test_growth_beside_another_threads_capture(mode, own, mth, dev):
     """A thread captures; another one's first calls on streams of its own need
     a workspace.  Both go well: the capture stays valid, its replays give the
     eager result, and the other thread's results are right."""
+    import gc
     import threading
     import torch
     print(f"workspace growth beside a capture, {mode}, {own}", flush=True)
@@ -118,6 +119,7 @@ def test_growth_beside_another_threads_capture(mode, own, mth, dev):
             errors.append(e)
 
     gr = torch.cuda.CUDAGraph()
+    assert not gc.isenabled()                              # conftest: nothing is destroyed inside the capture
     with torch.cuda.graph(gr, stream=s1, capture_error_mode=mode):
         mth.oil8_gemv(w, cb, x, y, M, K, 1)
         t = threading.Thread(target=other)
